@@ -78,11 +78,15 @@ typedef struct spr_stats {
     int64_t learned_fallbacks; /* LEARNED: frames whose exact total exceeded the allocation and were
                                   rendered with the plain method (the allocation then grows) */
     /* Which kernel routes the last frame took (each route has its own kernel or mode): */
-    int64_t n_wave_chains;     /* crossing chains solved by a whole wave each (896 or more crossings,
-                                  and each launch's costliest classes while they hold at most 512) */
+    int64_t n_wave_chains;     /* crossing chains that the lanes of a wave share.  Frames of 2^23
+                                  intersections and more: chains solved by a whole wave each (896
+                                  or more crossings, and each launch's costliest classes while they
+                                  hold at most 512); smaller frames: chains cut into segments that
+                                  are solved side by side */
     int64_t n_heavy_pieces;    /* monotone pieces merged by a 256-thread workgroup each (more than
-                                  1024 entries, or whose last segment waits on a chain of 256 or
-                                  more crossings of the next piece) */
+                                  1024 entries, or, in frames of 2^23 intersections and more, whose
+                                  last segment waits on a chain of 256 or more crossings of the
+                                  next piece) */
     int64_t n_long_bands;      /* sort bands of more than 512 words (one wave at 16 or 32 words per
                                   lane; 256-thread LDS sorts in frames that export a stage) */
     int64_t n_big_bands;       /* sort bands of more than 2048 words (global merge-path sort) */

@@ -320,8 +320,9 @@ __host__ __device__ inline float next_up(float x) {
 // bisect_axis under (1), with every decision "v < cut" (cut = c for a start below the line,
 // next_up(c) on the negated axis); c itself decides the fallback to t_min (|B(tm) - c| > 1),
 // reported in *ok.
-// FULL unrolls the 24 steps (the straight-line form of the common path).
-template <uint32_t T, bool FULL = false>
+// UNROLL steps are written out at a time: 24 for the common path of kernels that run it many times
+// over, few where instruction fetch would cost more than the loop.
+template <uint32_t T, int UNROLL = 4>
 __host__ __device__ inline float bisect_below(const CurveAxis& ax, float cut, float c, float t_min, float t1, bool* ok) {
     const float c0 = ax.c[0], c1 = ax.c[1], c2 = ax.c[2], c3 = ax.c[3];
     float t0 = t_min, tm = t_min, vtm = 0.0f;
@@ -332,13 +333,8 @@ __host__ __device__ inline float bisect_below(const CurveAxis& ax, float cut, fl
         t0 = right ? tm : t0;
         t1 = right ? t1 : tm;
     };
-    if constexpr (FULL) {
-#pragma unroll
-        for (int j = 0; j < kCubicIters; ++j) step();
-    } else {
-#pragma unroll 4
-        for (int j = 0; j < kCubicIters; ++j) step();
-    }
+#pragma unroll UNROLL
+    for (int j = 0; j < kCubicIters; ++j) step();
     *ok = !(fabsf(vtm - c) > 1.0f);
     return *ok ? tm : t_min;
 }
@@ -364,7 +360,7 @@ __device__ inline float solve_axis(uint32_t type, const CurveAxis& ax, float c, 
 // names the usual case (such a chain, start side known, t_min in range), for which
 // next_common() is the same computation in straight-line form: a wave whose lanes are all in
 // that case runs it without divergent branches.
-template <uint32_t T>
+template <uint32_t T, int UNROLL = kCubicIters>
 struct ChainSolver {
     CurveAxis a, an;
     bool fast, neg, known;
@@ -377,7 +373,7 @@ struct ChainSolver {
     __host__ __device__ bool common(float t_min) const { return T != kLine && fast && known && fast_t(t_min); }
     __host__ __device__ float next_common(float line, float t_min, float t1) {
         const float cn = neg ? -line : line;
-        return bisect_below<T, true>(an, neg ? next_up(cn) : cn, cn, t_min, t1, &known);
+        return bisect_below<T, UNROLL>(an, neg ? next_up(cn) : cn, cn, t_min, t1, &known);
     }
     __host__ __device__ float next(float line, float t_min, float t1) {
         if (T == kLine) return solve_line(a, line, t_min, t1);

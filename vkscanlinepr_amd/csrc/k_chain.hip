@@ -1,4 +1,5 @@
-// k_chain.hip -- intersection write (make_intersection_1.comp:217-447) for gfx950.
+// k_chain.hip -- intersection write (make_intersection_1.comp:217-447) for gfx950, in passes over
+// whole chains: the form of large frames (k_curves.hip is that of the others).
 //
 // Inside one monotone piece the reference interleaves x-grid and y-grid crossings, but every
 // bisection for the next crossing on one axis starts from the previous crossing of the SAME axis
@@ -87,21 +88,13 @@ __global__ __launch_bounds__(kBlock) void k_chain_prep(
     const int32_t* __restrict__ visible, const float4* __restrict__ cuts,
     const uint32_t* __restrict__ ncuts, const int32_t* __restrict__ offsets, uint32_t C, int w,
     int h, ChainDesc* __restrict__ chains, PieceDesc* __restrict__ pieces, uint8_t* __restrict__ chain_cls,
-    int32_t* __restrict__ class_count, Budget budget, bool budgeted, const int2* __restrict__ pcanvas) {
+    int32_t* __restrict__ class_count, const int32_t* __restrict__ over, const int2* __restrict__ pcanvas) {
     __shared__ int32_t hist[kClasses];
     if (threadIdx.x < kClasses) hist[threadIdx.x] = 0;
     __syncthreads();
-    // a frame over its budget (or whose int32 total wrapped) writes nothing past any buffer: every
-    // curve takes the culled route (no chain, no piece)
-    bool skip = false;
-    if (budgeted) {
-        const int32_t total = offsets[C];
-        skip = total < 0 || (int64_t)total > budget.entries;
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            *budget.live = skip ? 0 : total;
-            *budget.over = skip ? 1 : 0;
-        }
-    }
+    // a frame over its budget writes nothing past any buffer: every curve takes the culled route (no
+    // chain, no piece)
+    const bool skip = over && *over != 0;
     // grid-stride over curves; the class histogram is flushed once per workgroup
     for (uint32_t c = blockIdx.x * kBlock + threadIdx.x; c < C; c += gridDim.x * kBlock) {
         const uint32_t path = cpath[c];
@@ -1030,13 +1023,12 @@ hipError_t launch_chain_prep(const float2* tpos, const uint32_t* cpos, const uin
                              const float* cweight, const uint32_t* cpath, const int32_t* visible, const float4* cuts,
                              const uint32_t* ncuts, const int32_t* offsets, uint32_t C, int w, int h,
                              ChainDesc* chains, PieceDesc* pieces, uint8_t* chain_cls, int32_t* class_count,
-                             int n_cu, hipStream_t s, const Budget* budget, const int2* pcanvas) {
+                             int n_cu, hipStream_t s, const int32_t* over, const int2* pcanvas) {
     if (C == 0) return hipSuccess;
     unsigned g = grid_for((int64_t)C);
     if (g > (unsigned)n_cu * 8) g = (unsigned)n_cu * 8;
-    const Budget b = budget ? *budget : Budget{0, nullptr, nullptr};
     k_chain_prep<<<g, kBlock, 0, s>>>(tpos, cpos, ctype, cweight, cpath, visible, cuts, ncuts, offsets, C, w, h, chains,
-                                      pieces, chain_cls, class_count, b, budget != nullptr, pcanvas);
+                                      pieces, chain_cls, class_count, over, pcanvas);
     return hipGetLastError();
 }
 

@@ -1,5 +1,5 @@
 // k_geometry.hip -- transform + cull, monotonisation + count, and fragment-key generation
-// (gfx950).  The intersection write between count and keys lives in k_chain.hip.
+// (gfx950).  The intersection write between count and keys lives in k_curves.hip.
 #include "device_common.hpp"
 #include "kernels.hpp"
 
@@ -32,6 +32,30 @@ __global__ void k_fill_u32_dev(uint32_t* __restrict__ p, int64_t n_max, const in
     const int64_t n = min(n_max, mult * (int64_t)*n_dev + add);
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         p[i] = v;
+}
+
+// Clears what the second half of a frame counts in, finds the curve that holds each window's
+// first entry and holds the exact total against the budget: one launch for all of it.
+__global__ __launch_bounds__(kBlock) void k_frame_init(const FrameInit I) {
+    const int64_t stride = (int64_t)gridDim.x * kBlock, t0 = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    for (int k = 0; k < I.n_fills; ++k) {
+        const FrameInit::Fill& f = I.fill[k];
+        int64_t n = f.n;
+        if (f.n_dev) n = min(n, (int64_t)f.mult * *f.n_dev + f.add);
+        for (int64_t i = t0; i < n; i += stride) f.p[i] = f.value;
+    }
+    for (int64_t c = t0; c < (int64_t)I.C; c += stride) {
+        const int64_t o0 = I.offsets[c], o1 = I.offsets[c + 1];
+        if (o0 < 0) continue;
+        for (int64_t b = (o0 + I.window - 1) / I.window; b < I.n_first && b * I.window < o1; ++b)
+            I.first[b] = (int32_t)c;
+    }
+    if (I.budget.entries && t0 == 0) {
+        const int32_t total = I.offsets[I.C];
+        const bool skip = total < 0 || (int64_t)total > I.budget.entries;
+        *I.budget.live = skip ? 0 : total;
+        *I.budget.over = skip ? 1 : 0;
+    }
 }
 
 // transform_pos.comp:33-85.  The per-path outcode OR is reduced inside the wave first (points of
@@ -244,6 +268,15 @@ hipError_t launch_fill_u32_dev(uint32_t* p, int64_t n_max, const int32_t* n_dev,
 hipError_t launch_gather_summary(const SummarySrc& src, int32_t* dst, hipStream_t s) {
     if (src.n <= 0 || src.n > kSummaryMax) return hipErrorInvalidValue;
     k_gather_summary<<<1, 64, 0, s>>>(src, dst);
+    return hipGetLastError();
+}
+
+hipError_t launch_frame_init(const FrameInit& I, hipStream_t s) {
+    int64_t n = I.C;
+    for (int k = 0; k < I.n_fills; ++k) n = n > I.fill[k].n ? n : I.fill[k].n;
+    unsigned g = grid_for(n);
+    if (g > 2048u) g = 2048u;
+    k_frame_init<<<g, kBlock, 0, s>>>(I);
     return hipGetLastError();
 }
 

@@ -102,19 +102,21 @@ constexpr int kCcFill = kChainClasses, kCcOff = 2 * kChainClasses, kCcNLong = 3 
 // entries, which never wait on them, are finished by a concurrent stream meanwhile.
 constexpr int kHeavyCrossings = 256;
 // A frame whose buffers were sized before its counts were known (no host synchronisation): the
-// chain prep compares the exact total offsets[C] with the budget; a frame over budget writes no
-// chain and no piece (as if every path were culled), sets *over and leaves 0 in *live, the number
-// of entry positions the later kernels read; a frame within budget leaves the total in *live.
+// frame init compares the exact total offsets[C] with the budget; a frame over budget sets *over
+// and leaves 0 in *live, the number of entries that the later kernels write and read; a frame
+// within budget leaves the total in *live.
 struct Budget {
     int64_t entries;
     int32_t* live;
     int32_t* over;
 };
+// The chain passes (k_chain.hip): frames of kChainFrame entries and more.  over (optional): frames
+// with *over != 0 write no chain and no piece.
 hipError_t launch_chain_prep(const float2* tpos, const uint32_t* cpos, const uint32_t* ctype,
                              const float* cweight, const uint32_t* cpath, const int32_t* visible, const float4* cuts,
                              const uint32_t* ncuts, const int32_t* offsets, uint32_t C, int w, int h,
                              ChainDesc* chains, PieceDesc* pieces, uint8_t* chain_cls, int32_t* class_count,
-                             int n_cu, hipStream_t s, const Budget* budget = nullptr, const int2* pcanvas = nullptr);
+                             int n_cu, hipStream_t s, const int32_t* over = nullptr, const int2* pcanvas = nullptr);
 // n_long / n_long_light: the wave-solved chains at the head of the heavy / light launch's range.
 hipError_t launch_chain_order(const uint8_t* chain_cls, uint32_t C, const int32_t* class_count,
                               int32_t* class_off, int32_t* class_fill, int32_t* n_long, int32_t* light_begin,
@@ -155,6 +157,53 @@ hipError_t launch_piece_waves(const PieceDesc* pieces, const uint8_t* mono, cons
 hipError_t launch_piece_heavy(const PieceDesc* pieces, const PieceLists& L, const uint8_t* mono,
                               const float* chain_t, uint32_t* scratch, int64_t n_entries, const FragArgs& A, int n_cu,
                               hipStream_t s);
+// What a frame clears before its second half, and the curve windows: first[b] = the curve that
+// holds entry b * window.  With a budget, the exact total decides here whether the frame runs.
+struct FrameInit {
+    struct Fill {
+        uint32_t* p;
+        int64_t n;             // words, at most mult * *n_dev + add of them when n_dev is set
+        const int32_t* n_dev;
+        int32_t mult, add;
+        uint32_t value;
+    } fill[6];
+    int n_fills;
+    const int32_t* offsets;    // scanned per-curve counts, C + 1
+    uint32_t C;
+    int32_t window;
+    int32_t* first;
+    int64_t n_first;
+    Budget budget;             // entries == 0: none
+};
+hipError_t launch_frame_init(const FrameInit& I, hipStream_t s);
+// The curve pass (k_curves.hip): frames below kChainFrame entries.
+// The intersection write and the fragment keys: one wave per window of `window`
+// entries takes the pieces that start there from the curve data to their keys (or sort words),
+// winding changes and bucket counts, without storing the entries unless A.inter is set.  Pieces
+// of more than kCurvePieceMax entries are queued in `big` for launch_big_pieces.
+// Frames of this many entries take the chain passes: they fill the chip with whole chains sorted by
+// length, which costs half the arithmetic of the curve pass (52.9 M entries: 1.8 ms against 3.4 ms),
+// but has their longest chain and seven launches as its span (0.73 M entries: 0.41 ms against 0.24
+// ms; 7.2 M: 0.63 ms against 0.52 ms).
+constexpr int64_t kChainFrame = (int64_t)1 << 23;
+constexpr int kCurveWindowMin = 64, kCurveWindowMax = 1024, kCurvePieceMax = 1024;
+struct CurveArgs {
+    const int32_t* offsets;
+    const float4* cuts;
+    const uint32_t* ncuts;
+    uint32_t C;
+    int64_t n;                 // entries, or their bound with n_dev
+    const int32_t* n_dev;
+    int32_t window;
+    const int32_t* first;
+    int32_t* big;              // [5 C] queue of piece slots 5 curve + piece
+    int32_t* big_count;        // zeroed
+    int32_t* split_count;      // zeroed: += chains solved by several lanes side by side
+    uint32_t* scratch;         // n words
+    float* chain_t;            // n values: parameters of pieces beyond LDS
+};
+hipError_t launch_curves(const CurveArgs& K, const FragArgs& A, hipStream_t s);
+hipError_t launch_big_pieces(const CurveArgs& K, const FragArgs& A, int n_cu, hipStream_t s);
 hipError_t launch_gen_fragment(const int2* inter, int64_t N, const uint32_t* cpos,
                                const uint32_t* ctype, const float* cweight, const uint32_t* cpath, const float2* tpos,
                                int w, int h, int32_t* key, int8_t* wn, uint32_t* epath,

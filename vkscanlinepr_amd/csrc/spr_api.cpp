@@ -125,7 +125,8 @@ struct spr_handle {
     spr_opts opts{};
     int device = 0;
     hipStream_t stream = nullptr;
-    hipStream_t stream2 = nullptr;  // the light chain solve and the pieces that need only it
+    hipStream_t stream2 = nullptr;  // the light chain solve and the pieces that need only it; oversized
+                                    // and short bands; the learned frame's prediction
     hipEvent_t ev_fork = nullptr, ev_light = nullptr, ev_small = nullptr, ev_join = nullptr;
     hipEvent_t ev_sfork = nullptr, ev_sjoin = nullptr;  // the short-band sort on the second stream
     hipEvent_t ev_pfork = nullptr, ev_pjoin = nullptr;  // the learned frame's prediction on the second stream
@@ -161,7 +162,7 @@ struct spr_handle {
     DBuf<float> chain_t;
     DBuf<spr::ChainDesc> chains;
     DBuf<spr::PieceDesc> pieces;
-    DBuf<int32_t> chain_order, heavy_list, lo_list, lo_cnt, wave_list;
+    DBuf<int32_t> chain_order, heavy_list, lo_list, lo_cnt, wave_list, win_first;
     DBuf<uint8_t> mono, chain_cls;
     int n_cu = 256;
     DBuf<int32_t> key;
@@ -227,7 +228,7 @@ struct spr_handle {
     // batch of documents (spr_load_batch): per-path canvas, per-document tables
     bool batch = false;
     uint32_t n_docs = 0;
-    int total_rows = 0, max_h = 0;
+    int total_rows = 0, max_w = 0, max_h = 0;
     size_t img_bytes = 0;
     std::vector<spr::DocDev> h_docs;
     DBuf<int2> pcanvas;
@@ -264,6 +265,10 @@ const spr::PaintArgs* paint_args(const spr_handle* H, spr::PaintArgs& pa) {
 
 namespace {
 
+// Counters of the curve pass (int32), after the chain passes' control words: queued big pieces,
+// chains solved by several lanes.
+enum { kCcBigPieces = spr::kCcWords, kCcSplit, kCcWords };
+
 // Per-frame zeroed control region, in 64-bit words.  Phase A is cleared at frame start (before
 // the host sync), phase B once N and the bucket count NB are known.
 struct ZeroLayout {
@@ -283,7 +288,7 @@ ZeroLayout zero_layout(uint32_t C, uint32_t Np, int64_t N, int64_t NB) {
     z.ctr = o; o += 4;                 // eight u32 counters of the phase-B scans
     z.totals = o; o += 2;              // int32 cells, spans, R, spare
     z.misc = o; o += 1;                // int32 error flag, big-band count
-    z.chainctl = o; o += (spr::kCcWords + 1) / 2;  // chain classes, offsets, counters (int32)
+    z.chainctl = o; o += (kCcWords + 1) / 2;  // counters of the curve pass (int32)
     z.st_hist = o; o += spr::scan_tiles(std::max<int64_t>(NB, 1));
     z.st_band = o; o += spr::scan_tiles(std::max<int64_t>(NB, 1));
     z.st_wind = o; o += (size_t)spr::max_bands_for(Np, N) + 1;  // statuses of the band-sum scan
@@ -335,6 +340,50 @@ void stage_mark(spr_handle* H, int idx) {
     if ((int)H->ev_stage.size() <= idx) return;
     SPR_HIP(hipEventRecord(H->ev_stage[idx], H->stream));
     H->n_marks = idx + 1;
+}
+
+// Entries per window of the curve pass.  A wave takes one window, and about 2,000 waves are
+// resident: windows shrink with the frame until each wave's crossings spread over its 64 lanes a
+// few at a time, so that a small frame ends after a few crossings, not after a window's worth.
+int32_t curve_window(const spr_handle* H, int64_t n) {
+    int64_t w = spr::kCurveWindowMax;
+    while (w > 2 * spr::kCurveWindowMin && n / w < 4096) w >>= 1;
+    w = w * 8 / H->chain_k;  // the tuned share
+    return (int32_t)std::min<int64_t>(std::max<int64_t>(w, spr::kCurveWindowMin), spr::kCurveWindowMax);
+}
+
+// Intersections and fragment keys of a frame below spr::kChainFrame entries (stage marks 4 and 6
+// are the caller's).
+void curve_pass(spr_handle* H, int32_t* d_cc, const spr::FragArgs& A, int64_t n, const int32_t* n_dev, int32_t window) {
+    const spr::CurveArgs K{H->counts.p, H->cuts.p, H->ncuts.p, H->C, n, n_dev, window, H->win_first.p, H->heavy_list.p,
+                           d_cc + kCcBigPieces, d_cc + kCcSplit, (uint32_t*)H->sbig.p, (float*)H->stmp.p};
+    SPR_HIP(spr::launch_curves(K, A, H->stream));
+    stage_mark(H, 5);
+    // a piece holds its start and at most the grid lines of each axis inside the canvas and one beyond
+    const int w = H->batch ? H->max_w : (int)H->w, h = H->batch ? H->max_h : (int)H->h;
+    if (1 + (w / 2 + 2) + (h / 2 + 2) > spr::kCurvePieceMax)
+        SPR_HIP(spr::launch_big_pieces(K, A, H->n_cu * H->merge_k / 8, H->stream));
+}
+
+// Buffers and descriptors of the chain passes.
+void chain_setup(spr_handle* H, int64_t n, int32_t* d_cc, const int2* pcanvas, const int32_t* over) {
+    const uint32_t C = H->C;
+    hipStream_t s = H->stream;
+    H->chain_t.ensure((size_t)std::max<int64_t>(n, 1));
+    H->chains.ensure((size_t)C * 10);
+    H->pieces.ensure((size_t)C * 5);
+    H->chain_order.ensure((size_t)C * 10);
+    H->lo_list.ensure((size_t)C * 5 + 64);
+    H->lo_cnt.ensure(((size_t)C * 5 + 63) / 64);
+    H->wave_list.ensure((size_t)C * 5);
+    H->chain_cls.ensure((size_t)C * 10);
+    H->mono.ensure((size_t)C * 10);
+    SPR_HIP(spr::launch_chain_prep(H->tpos.p, H->cpos.p, H->ctype.p, H->arcw(), H->cpath.p, H->visible.p, H->cuts.p,
+                                   H->ncuts.p, H->counts.p, C, (int)H->w, (int)H->h, H->chains.p, H->pieces.p,
+                                   H->chain_cls.p, d_cc, H->n_cu, s, over, pcanvas));
+    SPR_HIP(spr::launch_chain_order(H->chain_cls.p, C, d_cc, d_cc + spr::kCcOff, d_cc + spr::kCcFill,
+                                    d_cc + spr::kCcNLong, d_cc + spr::kCcLightBegin, d_cc + spr::kCcNLongLight,
+                                    H->chain_order.p, H->n_cu, s));
 }
 
 // Chain solve and piece kernels of one frame, on two streams: the heavy solve runs on the main
@@ -452,7 +501,6 @@ void run_frame(spr_handle* H, bool record_begin = true) {
     const size_t n1 = (size_t)std::max<int64_t>(N, 1), nb1 = (size_t)std::max<int64_t>(NB, 1);
     const int64_t max_bands = spr::max_bands_for(Np, N);
     H->inter.ensure(n1);
-    H->chain_t.ensure(n1);
     H->key.ensure(n1);
     H->wn.ensure(n1);
     H->epath.ensure(n1);
@@ -471,7 +519,20 @@ void run_frame(spr_handle* H, bool record_begin = true) {
     if (aa) { H->cell_first.ensure(2 * n1); H->cmask.ensure(2 * n1); H->chord.ensure(n1); }
     H->crec.ensure(2 * n1);
     H->image.ensure((size_t)4 * H->w * H->h);
-    SPR_HIP(spr::launch_fill_u32((uint32_t*)(H->zero.p + z.a_words), 2 * (int64_t)(z.total - z.a_words), 0u, s));
+    const bool gen = !H->inj && N > 0, by_chain = N >= spr::kChainFrame;
+    const int32_t window = curve_window(H, N);
+    spr::FrameInit init{};
+    init.fill[0] = {(uint32_t*)(H->zero.p + z.a_words), 2 * (int64_t)(z.total - z.a_words), nullptr, 0, 0, 0u};
+    init.n_fills = 1;
+    if (gen) {
+        H->heavy_list.ensure((size_t)C * 5);
+        if (!by_chain) {
+            H->win_first.ensure((size_t)ceil_div(N, window));
+            init.offsets = H->counts.p; init.C = C; init.window = window;
+            init.first = H->win_first.p; init.n_first = ceil_div(N, window);
+        }
+    }
+    SPR_HIP(spr::launch_frame_init(init, s));
     int32_t* d_totals = reinterpret_cast<int32_t*>(H->zero.p + z.totals);
     int32_t* d_err = reinterpret_cast<int32_t*>(H->zero.p + z.misc);
     int32_t* d_bigcount = d_err + 1;
@@ -480,40 +541,18 @@ void run_frame(spr_handle* H, bool record_begin = true) {
     int32_t* d_bsum = reinterpret_cast<int32_t*>(H->zero.p + z.bsum);
     int2* d_brec = reinterpret_cast<int2*>(H->zero.p + z.brec);
 
-    const bool gen = !H->inj && N > 0;
-    int32_t* d_cc = reinterpret_cast<int32_t*>(H->zero.p + z.chainctl);  // class counts
-    int32_t* d_cfill = d_cc + spr::kCcFill;
-    int32_t* d_coff = d_cc + spr::kCcOff;
-    int32_t* d_nlong = d_cc + spr::kCcNLong;
-    int32_t* d_work = d_cc + spr::kCcWork;
-    if (H->inj) {
-        SPR_HIP(hipMemcpyAsync(H->inter.p, H->inj_inter.data(), (size_t)N * 8, hipMemcpyHostToDevice, s));
-    } else if (gen) {
-        H->chains.ensure((size_t)C * 10);
-        H->pieces.ensure((size_t)C * 5);
-        H->chain_order.ensure((size_t)C * 10);
-        H->heavy_list.ensure((size_t)C * 5);
-        H->lo_list.ensure((size_t)C * 5 + 64);
-        H->lo_cnt.ensure(((size_t)C * 5 + 63) / 64);
-        H->wave_list.ensure((size_t)C * 5);
-        H->chain_cls.ensure((size_t)C * 10);
-        H->mono.ensure((size_t)C * 10);
-        SPR_HIP(spr::launch_chain_prep(H->tpos.p, H->cpos.p, H->ctype.p, H->arcw(), H->cpath.p, H->visible.p, H->cuts.p,
-                                       H->ncuts.p, H->counts.p, C, w, h, H->chains.p, H->pieces.p, H->chain_cls.p,
-                                       d_cc, H->n_cu, s));
-        SPR_HIP(spr::launch_chain_order(H->chain_cls.p, C, d_cc, d_coff, d_cfill, d_nlong, d_cc + spr::kCcLightBegin,
-                                        d_cc + spr::kCcNLongLight,
-                                        H->chain_order.p, H->n_cu, s));
-    }
+    int32_t* d_cc = reinterpret_cast<int32_t*>(H->zero.p + z.chainctl);
+    if (H->inj) SPR_HIP(hipMemcpyAsync(H->inter.p, H->inj_inter.data(), (size_t)N * 8, hipMemcpyHostToDevice, s));
+    if (gen && by_chain) chain_setup(H, N, d_cc, nullptr, nullptr);
     stage_mark(H, 4);
     if (gen) {
-        // chain solve, then piece merge and fragment keys in one pass
-        // narrow frames: the piece kernels store each entry's bucket (key) and sort word (epath)
+        // narrow frames: the curve pass stores each entry's bucket (key) and sort word (epath)
         const spr::FragArgs A{H->cpos.p, H->ctype.p, H->arcw(), H->cpath.p, H->tpos.p, w, h, nullptr,
                               H->key.p, H->wn.p, H->epath.p, H->bucket_base.p, H->prow.p, d_hist, d_err,
                               keep ? H->inter.p : nullptr, aa ? H->chord.p : nullptr,
                               narrow ? H->epath.p : nullptr};
-        solve_and_pieces(H, C, d_cc, A, (int64_t)n1, H->n_cu * H->chain_k / 8, H->n_cu * H->merge_k / 8);
+        if (by_chain) solve_and_pieces(H, C, d_cc, A, (int64_t)n1, H->n_cu * H->chain_k / 8, H->n_cu * H->merge_k / 8);
+        else curve_pass(H, d_cc, A, N, nullptr, window);
     } else {
         stage_mark(H, 5);
     }
@@ -606,9 +645,9 @@ void run_frame(spr_handle* H, bool record_begin = true) {
     S.p[kSumCells] = d_totals;
     S.p[kSumSpans] = d_totals + 1;
     S.p[kSumErr] = d_err;
-    S.p[kSumWaveChains] = gen ? d_nlong : nullptr;
-    S.p[kSumWaveChainsLight] = gen ? d_cc + spr::kCcNLongLight : nullptr;
-    S.p[kSumHeavyPieces] = gen ? d_cc + spr::kCcHeavyPieces : nullptr;
+    S.p[kSumWaveChains] = gen ? d_cc + (by_chain ? spr::kCcNLong : kCcSplit) : nullptr;
+    S.p[kSumWaveChainsLight] = gen && by_chain ? d_cc + spr::kCcNLongLight : nullptr;
+    S.p[kSumHeavyPieces] = gen ? d_cc + (by_chain ? spr::kCcHeavyPieces : kCcBigPieces) : nullptr;
     S.p[kSumLongBands] = reinterpret_cast<const int32_t*>(ctl_at(H, z.st_wind, z.ctr, 4).counter + 1);
     S.p[kSumBigBands] = d_bigcount;
     S.p[kSumTotal] = H->inj ? nullptr : H->counts.p + C;
@@ -650,7 +689,7 @@ LearnedLayout learned_layout(uint32_t C, uint32_t Np, int64_t nb_budget, int64_t
     z.totals = o; o += 2;       // int32 cells, spans, R, spare
     z.slots = o; o += 2;        // int32 sorted entries, bands, spare x2
     z.bound = o; o += 1;        // u64 upper bound of the intersections
-    z.chainctl = o; o += (spr::kCcWords + 1) / 2;
+    z.chainctl = o; o += (kCcWords + 1) / 2;
     z.st_count = o; o += spr::scan_tiles(std::max<uint32_t>(C, 1));
     z.st_arena = o; o += spr::scan_tiles(std::max<uint32_t>(Np, 1));
     z.st_pb = o; o += spr::scan_tiles(std::max<uint32_t>(Np, 1));
@@ -826,7 +865,7 @@ void run_learned_frame(spr_handle* H) {
         throw Fail{SPR_ERR_CAPACITY, "intersection budget exceeds 2^30"};
     const int64_t nl = std::max<int64_t>(H->lb_n, 1), nr = std::max<int64_t>(H->lb_r, 1);
     const int64_t max_bands = spr::max_bands_for(Np, nl);
-    H->inter.ensure(nl); H->chain_t.ensure(nl); H->key.ensure(nl); H->wn.ensure(nl); H->epath.ensure(nl);
+    H->inter.ensure(nl); H->key.ensure(nl); H->wn.ensure(nl); H->epath.ensure(nl);
     H->sbig.ensure(nl); H->stmp.ensure(nl); H->skey.ensure(nl);
     H->winding.ensure(nl + 1);
     H->bflag.ensure((size_t)nb_budget + 1);
@@ -847,40 +886,33 @@ void run_learned_frame(spr_handle* H) {
     H->brec_l.ensure((size_t)nb_budget + 1);
     // per-bucket tables: cleared up to the live bucket count (bucket_base[Np])
     const int32_t* d_nb = H->bucket_base.p + Np;
-    SPR_HIP(spr::launch_fill_u32_dev((uint32_t*)H->hist_l.p, nb_budget + 1, d_nb, 1, 1, 0u, s));
-    SPR_HIP(spr::launch_fill_u32_dev((uint32_t*)H->fill_l.p, nb_budget, d_nb, 1, 0, 0u, s));
-    SPR_HIP(spr::launch_fill_u32_dev((uint32_t*)H->bsum_l.p, max_bands, d_nb, 1, 0, 0u, s));  // bands <= buckets
-    SPR_HIP(spr::launch_fill_u32_dev((uint32_t*)H->brec_l.p, 2 * nb_budget, d_nb, 2, 0, 0u, s));
+    const int32_t window = curve_window(H, nl);
+    const bool by_chain = nl >= spr::kChainFrame;
+    spr::FrameInit init{};
+    init.fill[0] = {(uint32_t*)H->hist_l.p, nb_budget + 1, d_nb, 1, 1, 0u};
+    init.fill[1] = {(uint32_t*)H->fill_l.p, nb_budget, d_nb, 1, 0, 0u};
+    init.fill[2] = {(uint32_t*)H->bsum_l.p, max_bands, d_nb, 1, 0, 0u};  // bands <= buckets
+    init.fill[3] = {(uint32_t*)H->brec_l.p, 2 * nb_budget, d_nb, 2, 0, 0u};
+    init.n_fills = 4;
+    if (C) {
+        H->heavy_list.ensure((size_t)C * 5);
+        H->win_first.ensure((size_t)ceil_div(nl, window));
+        init.offsets = H->counts.p; init.C = C; init.window = window;
+        init.first = H->win_first.p; init.n_first = ceil_div(nl, window);
+        init.budget = {nl, d_live, d_over};
+    }
+    SPR_HIP(spr::launch_frame_init(init, s));
 
     // phase 2: the plain stages on device counts, within the budget
     int32_t* d_cc = reinterpret_cast<int32_t*>(H->zero.p + z.chainctl);
-    int32_t* d_cfill = d_cc + spr::kCcFill;
-    int32_t* d_coff = d_cc + spr::kCcOff;
-    int32_t* d_nlong = d_cc + spr::kCcNLong;
-    if (C) {
-        H->chains.ensure((size_t)C * 10);
-        H->pieces.ensure((size_t)C * 5);
-        H->chain_order.ensure((size_t)C * 10);
-        H->heavy_list.ensure((size_t)C * 5);
-        H->lo_list.ensure((size_t)C * 5 + 64);
-        H->lo_cnt.ensure(((size_t)C * 5 + 63) / 64);
-        H->wave_list.ensure((size_t)C * 5);
-        H->chain_cls.ensure((size_t)C * 10);
-        H->mono.ensure((size_t)C * 10);
-        const spr::Budget B{nl, d_live, d_over};
-        SPR_HIP(spr::launch_chain_prep(H->tpos.p, H->cpos.p, H->ctype.p, H->arcw(), H->cpath.p, H->visible.p, H->cuts.p,
-                                       H->ncuts.p, H->counts.p, C, w, h, H->chains.p, H->pieces.p, H->chain_cls.p,
-                                       d_cc, H->n_cu, s, &B, pcv));
-        SPR_HIP(spr::launch_chain_order(H->chain_cls.p, C, d_cc, d_coff, d_cfill, d_nlong, d_cc + spr::kCcLightBegin,
-                                        d_cc + spr::kCcNLongLight,
-                                        H->chain_order.p, H->n_cu, s));
-    }
+    if (C && by_chain) chain_setup(H, nl, d_cc, pcv, d_over);
     stage_mark(H, 4);
     if (C) {
         const spr::FragArgs A{H->cpos.p, H->ctype.p, H->arcw(), H->cpath.p, H->tpos.p, w, h, pcv,
                               H->key.p, H->wn.p, H->epath.p, H->bucket_base.p, H->prow.p, H->hist_l.p, d_err,
                               debug ? H->inter.p : nullptr, nullptr, narrow ? H->epath.p : nullptr};
-        solve_and_pieces(H, C, d_cc, A, nl, H->n_cu * H->chain_k / 8, H->n_cu * H->merge_k / 8);
+        if (by_chain) solve_and_pieces(H, C, d_cc, A, nl, H->n_cu * H->chain_k / 8, H->n_cu * H->merge_k / 8);
+        else curve_pass(H, d_cc, A, nl, d_live, window);
     } else {
         stage_mark(H, 5);
     }
@@ -967,9 +999,9 @@ void run_learned_frame(spr_handle* H) {
     S.p[kSumCells] = d_totals;
     S.p[kSumSpans] = d_totals + 1;
     S.p[kSumErr] = d_err;
-    S.p[kSumWaveChains] = C ? d_nlong : nullptr;
-    S.p[kSumWaveChainsLight] = C ? d_cc + spr::kCcNLongLight : nullptr;
-    S.p[kSumHeavyPieces] = C ? d_cc + spr::kCcHeavyPieces : nullptr;
+    S.p[kSumWaveChains] = C ? d_cc + (by_chain ? spr::kCcNLong : kCcSplit) : nullptr;
+    S.p[kSumWaveChainsLight] = C && by_chain ? d_cc + spr::kCcNLongLight : nullptr;
+    S.p[kSumHeavyPieces] = C ? d_cc + (by_chain ? spr::kCcHeavyPieces : kCcBigPieces) : nullptr;
     S.p[kSumLongBands] = reinterpret_cast<const int32_t*>(ticket + 1);
     S.p[kSumBigBands] = d_bigcount;
     S.p[kSumTotal] = H->counts.p + C;
@@ -1306,7 +1338,8 @@ int spr_destroy(spr_handle* H) {
     H->rule.release(); H->fill.release(); H->tpos.release(); H->visible.release(); H->cuts.release();
     H->ncuts.release(); H->counts.release(); H->seg.release(); H->inter.release();
     H->chain_t.release(); H->chains.release(); H->pieces.release(); H->chain_order.release();
-    H->heavy_list.release(); H->lo_list.release(); H->lo_cnt.release(); H->wave_list.release(); H->chain_cls.release(); H->mono.release(); H->key.release(); H->wn.release(); H->epath.release(); H->sorted.release();
+    H->heavy_list.release(); H->lo_list.release(); H->lo_cnt.release(); H->wave_list.release();
+    H->chain_cls.release(); H->mono.release(); H->win_first.release(); H->key.release(); H->wn.release(); H->epath.release(); H->sorted.release();
     H->sbig.release(); H->stmp.release(); H->skey.release(); H->sidx.release();
     H->winding.release(); H->flags.release(); H->records.release(); H->crec.release();
     H->cell_first.release(); H->cmask.release(); H->chord.release();
@@ -1667,7 +1700,7 @@ int spr_load_batch(spr_handle* H, const spr_scene* const* docs, const uint32_t* 
         std::vector<int2> pcv;
         std::vector<int32_t> first;
         size_t img = 0;
-        int rows = 0, max_h = 1;
+        int rows = 0, max_w = 1, max_h = 1;
         for (uint32_t d = 0; d < n_docs; ++d) {
             if (!docs[d]) throw Fail{SPR_ERR_INVALID, "null document"};
             const uint32_t w = widths[d], h = heights[d];
@@ -1704,6 +1737,7 @@ int spr_load_batch(spr_handle* H, const spr_scene* const* docs, const uint32_t* 
             dd[d].pad = 0;
             img += (size_t)4 * w * h;
             rows += (int)(h + 1) / 2;
+            max_w = std::max<int>(max_w, (int)w);
             max_h = std::max<int>(max_h, (int)h);
             for (uint32_t p = p_off; p < rule.size(); ++p) { pcv.push_back(make_int2((int)w, (int)h)); first.push_back((int32_t)p_off); }
         }
@@ -1727,6 +1761,7 @@ int spr_load_batch(spr_handle* H, const spr_scene* const* docs, const uint32_t* 
         H->n_docs = n_docs;
         H->h_docs = dd;
         H->total_rows = rows;
+        H->max_w = max_w;
         H->max_h = max_h;
         H->img_bytes = img;
         H->lb_dirty = true;
