@@ -19,8 +19,8 @@
 // classifying pass, by 256-thread workgroups that take them in chunks, the first chunk by
 // workgroup id and the rest from an atomic ticket (their cost varies with the band length, so
 // the work is handed out as it frees up, and a frame without long bands takes no ticket at all).
-// A band above 2048 entries is a single oversized (path, row) bucket; such bands are queued, and
-// each is then sorted by one workgroup with LDS chunk sorts followed by merge-path passes
+// A band above 2048 entries is a single oversized (path, row) bucket; in debug frames such bands are
+// queued, and each is then sorted by one workgroup with LDS chunk sorts followed by merge-path passes
 // through global memory, the last pass writing keys and winding numbers.
 //
 // Frames that export no stage sort the narrow 32-bit words of the scatter instead (bucket inside
@@ -33,7 +33,7 @@
 // sorted words and winding numbers still in registers: every flag of a band depends on its own entries
 // only (a band starts at a bucket, i.e. a new cell row), so each band writes its records at twice
 // its start, the record range of each of its buckets and its (cells, spans); the oversized bands
-// do the same from their sorted keys (k_emit_big_bands).  Debug frames write keys, indices and
+// get theirs from sums per cell column, without a sort (k_big_bands).  Debug frames write keys, indices and
 // winding numbers, and k_mark_emit (k_scan.hip) emits the records in the reference's order.
 #include <algorithm>
 
@@ -111,8 +111,6 @@ struct Unpacked {
 struct Wide {
     typedef u64 T;
     static constexpr T kPad = ~0ull;  // no word has 3 in its low two bits
-    int2 pr;
-    __device__ void band(const int2*, int64_t) {}
     __device__ int32_t key(T w) const { return (int32_t)((uint32_t)(w >> 32) ^ 0x80000000u); }
     __device__ void put(const Unpacked& o, int64_t i, T w) const {
         o.skey[i] = key(w);
@@ -126,14 +124,12 @@ struct Narrow {
     typedef uint32_t T;
     static constexpr T kPad = ~0u;
     int2 pr;
-    __device__ void band(const int2* band_pr, int64_t b) { pr = band_pr[b]; }
     __device__ int32_t key(T w) const {
         const int loc = (int)(w >> 17);
         const uint32_t x = ((w >> 2) & 0x7FFFu) + kNarrowX0;
         const int y = loc < pr.y ? 2 * (pr.x + loc) : 0;
         return loc == pr.y ? (int32_t)kSentinelKey : (int32_t)(((uint32_t)(y + 0x7FFF) << 16) | x);
     }
-    __device__ void put(const Unpacked& o, int64_t i, T w) const { o.skey[i] = key(w); }
 };
 template <class T>
 __device__ inline int32_t wn_of(T w) { return (int32_t)(w & 3u) - 1; }
@@ -167,80 +163,6 @@ __device__ inline BandPath band_path_of(const EmitArgs& E, int64_t band, int2 pr
     return b;
 }
 
-// Mark + emit of band entries [c0, c0 + m) of a band of n entries (mark_merged_fragment_and_
-// span.comp:48-120, gen_merged_fragment_and_span.comp:152-222), THREADS threads with kItems
-// consecutive entries each.  key(j) and wind(j) give entry j's key and winding number (j in
-// [0, n)).  A cell is an in-canvas entry whose key differs from the previous entry's (the
-// band's first entry follows another bucket, so its key differs); a span runs from the previous
-// entry of the same cell row to this one when the winding number fills.  Records go to
-// crec[r0 + carry + ...]; carry (records of earlier chunks) is advanced and the chunk's
-// (cells, spans) are added to cnt (thread 0).
-template <int THREADS, class KEY, class WIND>
-__device__ inline void emit_chunk(const EmitArgs& E, const BandPath& b, KEY key, WIND wind, int64_t c0, int m,
-                                  int64_t n, int32_t& carry, int2& cnt, int32_t* s_w) {
-    const int64_t j0 = c0 + (int64_t)threadIdx.x * kItems;
-    int32_t keys[kItems];
-    uint32_t cbits = 0, sbits = 0;
-    int32_t kprev = j0 > 0 && j0 - 1 < n ? key(j0 - 1) : 0;
-#pragma unroll
-    for (int k = 0; k < kItems; ++k) {
-        const int64_t j = j0 + k;
-        keys[k] = 0;
-        if (j >= c0 + m) continue;
-        const int32_t k1 = key(j);
-        keys[k] = k1;
-        const int x1 = key_x(k1), y1 = key_y(k1);
-        const bool in_canvas = !(x1 < 0 || y1 < 0 || x1 >= b.cw || y1 >= b.ch);
-        const bool cell = in_canvas && (j == 0 || kprev != k1);
-        bool span = false;
-        if (j > 0) {
-            const int32_t wn = (int32_t)((uint32_t)wind(j) - (uint32_t)b.wb);
-            const bool wf = (b.rule == 0u && wn != 0) || (b.rule == 1u && (wn & 1) != 0);
-            span = key_y(kprev) == y1 && key_x(kprev) + 2 < x1 && wf;
-        }
-        cbits |= (uint32_t)cell << k;
-        sbits |= (uint32_t)span << k;
-        kprev = k1;
-    }
-    // chunk scan of (cells | spans << 16): a chunk holds at most 2048 of each
-    int32_t tot;
-    const int32_t ex = block_exclusive_add<int32_t, THREADS / 64>(__popc(cbits) | (__popc(sbits) << 16), s_w, tot);
-    int64_t pos = b.r0 + carry + (ex & 0xFFFF) + (ex >> 16);
-    kprev = j0 > 0 && j0 - 1 < n ? key(j0 - 1) : 0;
-#pragma unroll
-    for (int k = 0; k < kItems; ++k) {
-        const int64_t j = j0 + k;
-        if (j >= c0 + m) continue;
-        const int32_t k1 = keys[k];
-        const int cell = (cbits >> k) & 1, span = (sbits >> k) & 1;
-        const int x1 = key_x(k1), y1 = key_y(k1);
-        if (cell) E.crec[pos] = (uint32_t)x1 | (2u << 16);
-        if (span) {
-            const int x0 = max(0, key_x(kprev) + 2);
-            E.crec[pos + cell] = (uint32_t)x0 | ((uint32_t)(x1 - x0) << 16);
-        }
-        // record range of this entry's (path, cell row) bucket, for the composite
-        if ((uint32_t)k1 != kSentinelKey && y1 >= 0 && y1 < b.ch) {
-            const int32_t kn = j + 1 < n ? (k + 1 < kItems ? keys[k + 1 < kItems ? k + 1 : k] : key(j + 1)) : 0;
-            const bool first = j == 0 || (kprev >> 16) != (k1 >> 16);
-            const bool last = j == n - 1 || (kn >> 16) != (k1 >> 16);
-            if (first || last) {
-                const int r = y1 >> 1;
-                const int loc = r == 0 ? b.pr.y + 1 : r - b.pr.x;
-                if (loc >= 0 && loc < b.pr.y + 2) {  // out of range only after a flagged bound error
-                    int2* br = &E.brec[b.bb + loc];
-                    if (first) br->x = (int32_t)pos;
-                    if (last) br->y = (int32_t)(pos + cell + span);
-                }
-            }
-        }
-        pos += cell + span;
-        kprev = k1;
-    }
-    carry += (tot & 0xFFFF) + (tot >> 16);
-    if (threadIdx.x == 0) { cnt.x += tot & 0xFFFF; cnt.y += tot >> 16; }
-}
-
 // Sorts n <= THREADS * kItems words from src with one workgroup of THREADS threads (buf: 2 x
 // kPadded words of LDS) into dst (sort words) or, when dst is null, unpacked into out at offset
 // o0 with winding numbers from the band's exclusive prefix `pre`.
@@ -248,8 +170,7 @@ template <class W, int THREADS>
 __device__ __forceinline__ void tile_sort(const W& wd, const typename W::T* __restrict__ src,
                                           typename W::T* __restrict__ dst, int n,
                                           typename W::T (*buf)[Tile<THREADS>::kPadded], const Unpacked& out,
-                                          int64_t o0, int32_t pre, int32_t* s_w, const EmitArgs& E,
-                                          bool emit, int64_t band) {
+                                          int64_t o0, int32_t pre, int32_t* s_w) {
     typedef typename W::T T;
     constexpr T kPad = W::kPad;
     int P2 = kItems;
@@ -332,18 +253,6 @@ __device__ __forceinline__ void tile_sort(const W& wd, const typename W::T* __re
         if (i < n) wl[i] = wadd(ex, w8[k]);
     }
     __syncthreads();
-    if (emit) {
-        // mark + emit from LDS: sorted words and winding numbers stay on chip
-        const BandPath b = band_path_of(E, band, wd.pr, o0);
-        const T* S = buf[cur];
-        int32_t carry = 0;
-        int2 cnt = make_int2(0, 0);
-        emit_chunk<THREADS>(E, b, [&](int64_t j) { return wd.key(S[pad((int)j)]); },
-                            [&](int64_t j) { return wl[j]; }, 0, n, n, carry, cnt, s_w);
-        if (tid == 0) E.band_cnt[band] = cnt;
-        __syncthreads();
-        return;
-    }
     for (int i = tid; i < n; i += THREADS) {
         wd.put(out, o0 + i, buf[cur][pad(i)]);
         out.winding[o0 + i] = wl[i];
@@ -596,8 +505,8 @@ __global__ __launch_bounds__(kClassifyThreads) void k_band_classify2(const int32
     const bool med = n > kSmallBandMax && n <= kMediumBandMax;
     const bool large = n > kMediumBandMax && n <= kWaveBandMax;
     if (n > kWaveBandMax) {
-        // a single oversized (path, row) bucket: queued with its exclusive prefix for the
-        // global-merge kernels, which may run beside the wave sorts
+        // a single oversized (path, row) bucket: queued with its exclusive prefix for
+        // k_big_bands, which may run beside the wave sorts
         const int32_t q = atomicAdd(big_count, 1);
         big_list[q] = (int32_t)t;
         big_excl[q] = bpre[t];
@@ -625,16 +534,13 @@ __global__ __launch_bounds__(kClassifyThreads) void k_band_classify2(const int32
 // CLS 0: every band of up to 512 words, one wave each (four per workgroup; the others are
 // skipped).  CLS 1: the listed bands of 513..1024 words (16 per lane).  CLS 2: the listed bands of
 // 1025..2048 words (32 per lane); k_band_classify2 queues the longer ones (single oversized
-// buckets) for the global-merge kernels.
+// buckets) for k_big_bands.
 template <int CLS>
 __global__ __launch_bounds__(256) void k_sort_bands_wave(const int32_t* __restrict__ band_start,
                                                          const int32_t* __restrict__ n_bands,
                                                          const uint32_t* __restrict__ src,
                                                          const int32_t* __restrict__ bpre,
                                                          const int2* __restrict__ band_pr,
-                                                         int32_t* __restrict__ big_list,
-                                                         int32_t* __restrict__ big_excl,
-                                                         int32_t* __restrict__ big_count,
                                                          const int32_t* __restrict__ list, int64_t cap,
                                                          const uint32_t* __restrict__ count, EmitArgs EA) {
     constexpr int RMAX = CLS == 0 ? 8 : (CLS == 1 ? 16 : 32);
@@ -677,13 +583,12 @@ __global__ __launch_bounds__(THREADS) void k_sort_bands(const int32_t* __restric
                                                         uint32_t* __restrict__ ticket,
                                                         int32_t* __restrict__ big_list,
                                                         int32_t* __restrict__ big_excl,
-                                                        int32_t* __restrict__ big_count,
-                                                        const int2* __restrict__ band_pr, EmitArgs E, bool emit) {
+                                                        int32_t* __restrict__ big_count) {
     constexpr int kSize = Tile<THREADS>::kSize;
     __shared__ typename W::T buf[2][Tile<THREADS>::kPadded];
     __shared__ int32_t s_w[Tile<THREADS>::kWaves], s_t;
     const int32_t nb = *n_bands;
-    if (BIG && !emit && blockIdx.x == 0 && threadIdx.x == 0) {
+    if (BIG && blockIdx.x == 0 && threadIdx.x == 0) {
         if (nb > 0) out.winding[band_start[nb]] = bpre[nb];  // the scan's total
         else out.winding[0] = 0;
     }
@@ -706,9 +611,7 @@ __global__ __launch_bounds__(THREADS) void k_sort_bands(const int32_t* __restric
                 continue;
             }
             W wd;
-            wd.band(band_pr, t);
-            tile_sort<W, THREADS>(wd, src + s, (typename W::T*)nullptr, (int)n, buf, out, s, bpre[t], s_w, E,
-                                  emit, t);
+            tile_sort<W, THREADS>(wd, src + s, (typename W::T*)nullptr, (int)n, buf, out, s, bpre[t], s_w);
         }
         // any order: only the hand-out of the chunks matters
         c = BIG ? (int64_t)gridDim.x + ordered_tile_id(ticket, &s_t) : c + gridDim.x;
@@ -724,8 +627,7 @@ __global__ __launch_bounds__(kBigThreads) void k_sort_big_bands(const int32_t* _
                                                              const int32_t* __restrict__ big_excl,
                                                              const int32_t* __restrict__ big_count,
                                                              typename W::T* __restrict__ scatter,
-                                                             typename W::T* __restrict__ a, Unpacked out,
-                                                             const int2* __restrict__ band_pr) {
+                                                             typename W::T* __restrict__ a, Unpacked out) {
     typedef typename W::T T;
     constexpr int kThreads = kBigThreads;
     __shared__ T buf[2][Tile<kThreads>::kPadded];
@@ -735,10 +637,9 @@ __global__ __launch_bounds__(kBigThreads) void k_sort_big_bands(const int32_t* _
         const int32_t band = big_list[q];
         const int64_t s = band_start[band], n = band_start[band + 1] - s;
         W wd;
-        wd.band(band_pr, band);
         for (int64_t c = 0; c < n; c += kSortTile) {
             const int m = (int)(n - c < kSortTile ? n - c : kSortTile);
-            tile_sort<W, kThreads>(wd, scatter + s + c, a + s + c, m, buf, out, 0, 0, s_w, EmitArgs{}, false, 0);
+            tile_sort<W, kThreads>(wd, scatter + s + c, a + s + c, m, buf, out, 0, 0, s_w);
         }
         __threadfence_block();
         __syncthreads();
@@ -796,28 +697,110 @@ __global__ __launch_bounds__(kBigThreads) void k_sort_big_bands(const int32_t* _
 
 namespace {
 
-// Mark + emit of each oversized band (one workgroup per band) from its sorted keys and winding
-// numbers, in chunks of one tile with the records carried across.
-__global__ __launch_bounds__(kBigThreads) void k_emit_big_bands(const int32_t* __restrict__ band_start,
-                                                                 const int32_t* __restrict__ big_list,
-                                                                 const int32_t* __restrict__ big_count,
-                                                                 const int32_t* __restrict__ skey,
-                                                                 const int32_t* __restrict__ winding,
-                                                                 const int2* __restrict__ band_pr, EmitArgs E) {
-    __shared__ int32_t s_w[Tile<kBigThreads>::kWaves];
+// The oversized bands of frames with emit, one workgroup each.  Such a band is one (path, cell
+// row) bucket, so its entries differ only in their cell column and need no sort: their winding
+// changes are summed per column in LDS (16 KiB for the widest canvas), and one scan over the
+// columns gives every cell's winding number, the cells and the spans.  The words are read once
+// and nothing but records is written; a merge sort of the band passed over it log2(n / 2048)
+// times through memory, on one compute unit.  The off-canvas bucket holds no cell: it has
+// no records, whatever its size.
+constexpr int kColThreads = 1024;
+constexpr int kCols = 8192 / 2 + 3;  // columns -1 .. (w & ~1) / 2 + 1 of the widest canvas
+__global__ __launch_bounds__(kColThreads) void k_big_bands(const int32_t* __restrict__ band_start,
+                                                           const int32_t* __restrict__ big_list,
+                                                           const int32_t* __restrict__ big_excl,
+                                                           const int32_t* __restrict__ big_count,
+                                                           const uint32_t* __restrict__ src,
+                                                           const int2* __restrict__ band_pr, EmitArgs E) {
+    __shared__ int32_t s_sum[kCols];
+    __shared__ uint32_t s_has[(kCols + 31) / 32];
+    __shared__ int32_t s_w[kColThreads / 64], s_last[kColThreads / 64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int32_t nbig = *big_count;
     for (int32_t q = blockIdx.x; q < nbig; q += gridDim.x) {
         const int32_t band = big_list[q];
-        const int64_t s = band_start[band], n = band_start[band + 1] - s;
-        const BandPath b = band_path_of(E, band, band_pr[band], s);
-        int32_t carry = 0;
-        int2 cnt = make_int2(0, 0);
-        for (int64_t c = 0; c < n; c += kSortTile) {
-            const int m = (int)(n - c < kSortTile ? n - c : kSortTile);
-            emit_chunk<kBigThreads>(E, b, [&](int64_t j) { return skey[s + j]; },
-                                    [&](int64_t j) { return winding[s + j]; }, c, m, n, carry, cnt, s_w);
+        const int64_t s = band_start[band];
+        const int32_t n = (int32_t)(band_start[band + 1] - s);
+        const int2 pr = band_pr[band];
+        const BandPath b = band_path_of(E, band, pr, s);
+        const uint32_t* w = src + s;
+        const int loc = (int)(w[0] >> 17);
+        if (loc == pr.y) {
+            if (tid == 0) E.band_cnt[band] = make_int2(0, 0);
+            continue;
         }
-        if (threadIdx.x == 0) E.band_cnt[band] = cnt;
+        for (int i = tid; i < kCols; i += kColThreads) s_sum[i] = 0;
+        for (int i = tid; i < (kCols + 31) / 32; i += kColThreads) s_has[i] = 0u;
+        __syncthreads();
+        for (int32_t i = tid; i < n; i += kColThreads) {
+            const uint32_t v = w[i];
+            const int col = min((int)((v >> 3) & 0x3FFFu), kCols - 1);
+            const int32_t wn = wn_of(v);
+            if (!((s_has[col >> 5] >> (col & 31)) & 1u)) atomicOr(&s_has[col >> 5], 1u << (col & 31));
+            if (wn) atomicAdd(&s_sum[col], wn);
+        }
+        __syncthreads();
+        // thread t owns columns t * per ..; what it needs of the columns before: their winding sum
+        // and the last one with an entry
+        constexpr int kPer = (kCols + kColThreads - 1) / kColThreads;
+        const int c0 = tid * kPer;
+        int32_t sum = 0, last = -1;
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            const int c = c0 + k;
+            if (c < kCols && ((s_has[c >> 5] >> (c & 31)) & 1u)) { sum = wadd(sum, s_sum[c]); last = c; }
+        }
+        int32_t tot;
+        int32_t run = wadd(big_excl[q], block_exclusive_add<int32_t, kColThreads / 64>(sum, s_w, tot));
+        int32_t prev = last;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int32_t u = __shfl_up(prev, o);
+            if (lane >= o) prev = max(prev, u);
+        }
+        if (lane == 63) s_last[wave] = prev;
+        prev = __shfl_up(prev, 1);
+        if (lane == 0) prev = -1;
+        __syncthreads();
+        for (int k = 0; k < wave; ++k) prev = max(prev, s_last[k]);
+        const int y = loc < pr.y ? 2 * (pr.x + loc) : 0;
+        uint32_t cells = 0, spans = 0;
+        int32_t from = prev;
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            const int c = c0 + k;
+            if (c >= kCols || !((s_has[c >> 5] >> (c & 31)) & 1u)) continue;
+            const int x = 2 * c - 2;
+            const int32_t wn = (int32_t)((uint32_t)run - (uint32_t)b.wb);
+            const bool fills = (b.rule == 0u && wn != 0) || (b.rule == 1u && (wn & 1) != 0);
+            if (x >= 0 && x < b.cw && y < b.ch) cells |= 1u << k;
+            if (from >= 0 && from + 1 < c && fills) spans |= 1u << k;
+            run = wadd(run, s_sum[c]);
+            from = c;
+        }
+        __syncthreads();  // s_w is used again
+        int32_t total;
+        int32_t ex = block_exclusive_add<int32_t, kColThreads / 64>(__popc(cells) | (__popc(spans) << 16), s_w, total);
+        int64_t pos = b.r0 + (ex & 0xFFFF) + (ex >> 16);
+        from = prev;
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            const int c = c0 + k;
+            if (c >= kCols || !((s_has[c >> 5] >> (c & 31)) & 1u)) continue;
+            const int x = 2 * c - 2;
+            if ((cells >> k) & 1u) E.crec[pos++] = (uint32_t)x | (2u << 16);
+            if ((spans >> k) & 1u) {
+                const int x0 = max(0, 2 * from);
+                E.crec[pos++] = (uint32_t)x0 | ((uint32_t)(x - x0) << 16);
+            }
+            from = c;
+        }
+        if (tid == 0) {
+            const int32_t nc = total & 0xFFFF, ns = total >> 16;
+            E.band_cnt[band] = make_int2(nc, ns);
+            if (y < b.ch && loc < pr.y + 2) E.brec[b.bb + loc] = make_int2((int32_t)b.r0, (int32_t)(b.r0 + nc + ns));
+        }
+        __syncthreads();  // the LDS is used again
     }
 }
 
@@ -858,13 +841,15 @@ unsigned class_grid(int64_t max_bands, int n_cu) {
     return (unsigned)(max_bands < g ? max_bands : g);
 }
 
-template <class W>
-hipError_t launch_classes(const int32_t* band_start, const int32_t* n_bands, int64_t max_bands,
-                          const typename W::T* src, const Unpacked& out, const int32_t* bpre, uint32_t* ticket,
-                          int32_t* big_list, int32_t* big_excl, int32_t* big_count, int n_cu, hipStream_t s,
-                          const int2* band_pr, const EmitArgs* emit, SideStream side) {
-    typedef typename W::T T;
-    const EmitArgs E = emit ? *emit : EmitArgs{};
+}  // namespace
+
+// The bands of frames without emit: wide words, the short bands beside the long ones.
+hipError_t launch_sort_bands(const int32_t* band_start, const int32_t* n_bands, int64_t max_bands,
+                             const unsigned long long* src, int32_t* skey, int32_t* sidx, int32_t* winding,
+                             int32_t* big_list, int32_t* big_excl, int32_t* big_count, const int32_t* bpre,
+                             uint32_t* ticket, int n_cu, hipStream_t s, SideStream side) {
+    if (max_bands <= 0) return hipSuccess;
+    const Unpacked out{skey, sidx, winding};
     int32_t* long_list = big_list + 2 * max_bands;
     // the short bands (no dependence on the long ones) on the second stream when there is one
     hipStream_t ss = s;
@@ -874,13 +859,12 @@ hipError_t launch_classes(const int32_t* band_start, const int32_t* n_bands, int
         if (e != hipSuccess) return e;
         ss = side.s2;
     }
-    k_sort_bands<W, 64, false><<<class_grid<T, 64>(max_bands, n_cu), 64, 0, ss>>>(
-        band_start, n_bands, src, out, bpre, nullptr, nullptr, nullptr, nullptr, nullptr, band_pr, E, emit != nullptr);
+    k_sort_bands<Wide, 64, false><<<class_grid<u64, 64>(max_bands, n_cu), 64, 0, ss>>>(
+        band_start, n_bands, src, out, bpre, nullptr, nullptr, nullptr, nullptr, nullptr);
     k_band_classify<<<(unsigned)((max_bands + kClassifyThreads - 1) / kClassifyThreads), kClassifyThreads, 0, s>>>(
         band_start, n_bands, long_list, ticket + 1);
-    k_sort_bands<W, 256, true><<<class_grid<T, 256>((max_bands + kChunk - 1) / kChunk, n_cu), 256, 0, s>>>(
-        band_start, n_bands, src, out, bpre, long_list, ticket, big_list, big_excl, big_count, band_pr, E,
-        emit != nullptr);
+    k_sort_bands<Wide, 256, true><<<class_grid<u64, 256>((max_bands + kChunk - 1) / kChunk, n_cu), 256, 0, s>>>(
+        band_start, n_bands, src, out, bpre, long_list, ticket, big_list, big_excl, big_count);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && side.s2) {
         e = hipEventRecord(side.join, side.s2);
@@ -889,39 +873,25 @@ hipError_t launch_classes(const int32_t* band_start, const int32_t* n_bands, int
     return e;
 }
 
-}  // namespace
-
-hipError_t launch_sort_bands(const int32_t* band_start, const int32_t* n_bands, int64_t max_bands,
-                             const unsigned long long* src, int32_t* skey, int32_t* sidx, int32_t* winding,
-                             int32_t* big_list, int32_t* big_excl, int32_t* big_count, const int32_t* bpre,
-                             uint32_t* ticket, int n_cu, hipStream_t s, const int2* band_pr,
-                             const EmitArgs* emit, SideStream side, int64_t n_entries, hipStream_t s_small) {
+// The bands of frames with emit (after launch_band_classify): one wave per band, four bands per
+// workgroup; the bands above 512 words (at most N / 513 of them) in later launches.
+hipError_t launch_sort_bands_emit(const int32_t* band_start, const int32_t* n_bands, int64_t max_bands,
+                                  const unsigned long long* src, const int32_t* big_list, const int32_t* bpre,
+                                  const uint32_t* ticket, const int2* band_pr, const EmitArgs& emit,
+                                  int64_t n_entries, hipStream_t s, hipStream_t s_small) {
     if (max_bands <= 0) return hipSuccess;
-    const Unpacked out{skey, sidx, winding};
-    if (band_pr) {
-        if (sidx) return hipErrorInvalidValue;  // narrow words hold no index
-        if (emit) {
-            // production frames (after launch_band_classify): one wave per band, four bands per
-            // workgroup; the bands above 512 words (at most N / 513 of them) in later launches
-            const uint32_t* w = reinterpret_cast<const uint32_t*>(src);
-            int32_t* lists = big_list + 2 * max_bands;  // 2 * max_bands slots: both lists of long bands
-            const int64_t cap = 2 * max_bands;
-            k_sort_bands_wave<0><<<(unsigned)((max_bands + 3) / 4), 256, 0, s_small ? s_small : s>>>(
-                band_start, n_bands, w, bpre, band_pr, big_list, big_excl, big_count, lists, cap, ticket + 1, *emit);
-            const int64_t max_med = std::min<int64_t>(max_bands, n_entries / (kSmallBandMax + 1) + 1);
-            k_sort_bands_wave<1><<<(unsigned)((max_med + 3) / 4), 256, 0, s>>>(
-                band_start, n_bands, w, bpre, band_pr, big_list, big_excl, big_count, lists, cap, ticket + 1, *emit);
-            const int64_t max_large = std::min<int64_t>(max_bands, n_entries / (kMediumBandMax + 1) + 1);
-            k_sort_bands_wave<2><<<(unsigned)((max_large + 3) / 4), 256, 0, s>>>(
-                band_start, n_bands, w, bpre, band_pr, big_list, big_excl, big_count, lists, cap, ticket + 1, *emit);
-            return hipGetLastError();
-        }
-        return launch_classes<Narrow>(band_start, n_bands, max_bands, reinterpret_cast<const uint32_t*>(src), out,
-                                      bpre, ticket, big_list, big_excl, big_count, n_cu, s, band_pr, emit, side);
-    }
-    if (emit) return hipErrorInvalidValue;  // wide words: the debug path keeps the separate mark + emit
-    return launch_classes<Wide>(band_start, n_bands, max_bands, src, out, bpre, ticket, big_list, big_excl,
-                                big_count, n_cu, s, nullptr, nullptr, side);
+    const uint32_t* w = reinterpret_cast<const uint32_t*>(src);
+    const int32_t* lists = big_list + 2 * max_bands;  // 2 * max_bands slots: both lists of long bands
+    const int64_t cap = 2 * max_bands;
+    k_sort_bands_wave<0><<<(unsigned)((max_bands + 3) / 4), 256, 0, s_small>>>(band_start, n_bands, w, bpre, band_pr,
+                                                                               lists, cap, ticket + 1, emit);
+    const int64_t max_med = std::min<int64_t>(max_bands, n_entries / (kSmallBandMax + 1) + 1);
+    k_sort_bands_wave<1><<<(unsigned)((max_med + 3) / 4), 256, 0, s>>>(band_start, n_bands, w, bpre, band_pr, lists,
+                                                                       cap, ticket + 1, emit);
+    const int64_t max_large = std::min<int64_t>(max_bands, n_entries / (kMediumBandMax + 1) + 1);
+    k_sort_bands_wave<2><<<(unsigned)((max_large + 3) / 4), 256, 0, s>>>(band_start, n_bands, w, bpre, band_pr, lists,
+                                                                         cap, ticket + 1, emit);
+    return hipGetLastError();
 }
 
 hipError_t launch_band_classify(const int32_t* band_start, const int32_t* n_bands, int64_t max_bands,
@@ -934,10 +904,11 @@ hipError_t launch_band_classify(const int32_t* band_start, const int32_t* n_band
     return hipGetLastError();
 }
 
-hipError_t launch_emit_big_bands(const int32_t* band_start, const int32_t* big_list, const int32_t* big_count,
-                                 const int32_t* skey, const int32_t* winding, const int2* band_pr,
-                                 const EmitArgs& emit, hipStream_t s) {
-    k_emit_big_bands<<<64, kBigThreads, 0, s>>>(band_start, big_list, big_count, skey, winding, band_pr, emit);
+hipError_t launch_big_bands(const int32_t* band_start, const int32_t* big_list, const int32_t* big_excl,
+                            const int32_t* big_count, const unsigned long long* src, const int2* band_pr,
+                            const EmitArgs& emit, int n_cu, hipStream_t s) {
+    k_big_bands<<<(unsigned)n_cu, kColThreads, 0, s>>>(band_start, big_list, big_excl, big_count,
+                                                       reinterpret_cast<const uint32_t*>(src), band_pr, emit);
     return hipGetLastError();
 }
 
@@ -948,18 +919,9 @@ hipError_t launch_band_totals(const int2* band_cnt, const int32_t* n_bands, int3
 
 hipError_t launch_sort_big_bands(const int32_t* band_start, const int32_t* big_list, const int32_t* big_excl,
                                  const int32_t* big_count, unsigned long long* scatter, unsigned long long* tmp,
-                                 int32_t* skey, int32_t* sidx, int32_t* winding, hipStream_t s,
-                                 const int2* band_pr) {
+                                 int32_t* skey, int32_t* sidx, int32_t* winding, hipStream_t s) {
     const Unpacked out{skey, sidx, winding};
-    if (band_pr) {
-        if (sidx) return hipErrorInvalidValue;
-        k_sort_big_bands<Narrow><<<64, kBigThreads, 0, s>>>(band_start, big_list, big_excl, big_count,
-                                                          reinterpret_cast<uint32_t*>(scatter),
-                                                          reinterpret_cast<uint32_t*>(tmp), out, band_pr);
-        return hipGetLastError();
-    }
-    k_sort_big_bands<Wide><<<64, kBigThreads, 0, s>>>(band_start, big_list, big_excl, big_count, scatter, tmp, out,
-                                                    nullptr);
+    k_sort_big_bands<Wide><<<64, kBigThreads, 0, s>>>(band_start, big_list, big_excl, big_count, scatter, tmp, out);
     return hipGetLastError();
 }
 

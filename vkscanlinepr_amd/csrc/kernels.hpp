@@ -269,23 +269,13 @@ struct EmitArgs {
     const int32_t* wbase; // per-path winding base of a batch, or null
     int w, h;
 };
-// The band sorts write the sorted keys, winding changes and (optionally) indices directly.
-// Sorts every band and writes keys, (debug) indices and winding numbers (the exclusive scan of
-// the sorted winding changes, total at winding[n]); bpre holds each band's exclusive prefix of
-// the winding changes (total at bpre[n_bands]).  Oversized bands are queued (with their
-// exclusive prefix) for launch_sort_big_bands.  big_list: 3 * max_bands int32.  ticket: two
-// zeroed u32 counters.  narrow (band_pr non-null): 32-bit words from the narrow scatter; sidx
-// must be null.
-// emit (narrow only, or null): mark + emit fused (EmitArgs); the bands then write no keys or
-// winding numbers, except the oversized ones, which launch_emit_big_bands reads back.  With
-// emit, launch_band_classify must run first: it lists the long bands for the wave sorts and
-// queues the oversized ones, so that launch_sort_big_bands and launch_emit_big_bands may run on
-// another stream beside the wave sorts.
+// Bands of frames without emit (wide words): writes keys, (debug) indices and winding numbers (the
+// exclusive scan of the sorted winding changes, total at winding[n]); bpre holds each band's
+// exclusive prefix of the winding changes (total at bpre[n_bands]).  Oversized bands are queued
+// (with their exclusive prefix) for launch_sort_big_bands.  big_list: 4 * max_bands int32.
+// ticket: two zeroed u32 counters.
 // side (optional): a second stream and two events; the short bands are then sorted there,
-// beside the long ones, and s waits for them before it returns.  n_entries: an upper bound of the
-// sorted entries (sizes the launch for the bands above 512 words of frames with emit).  s_small
-// (emit only, optional): the stream of the sort of the bands of up to 512 words, which the caller
-// forks from s after launch_band_classify and joins.
+// beside the long ones, and s waits for them before it returns.
 struct SideStream {
     hipStream_t s2;
     hipEvent_t fork, join;
@@ -293,25 +283,28 @@ struct SideStream {
 hipError_t launch_sort_bands(const int32_t* band_start, const int32_t* n_bands, int64_t max_bands,
                              const unsigned long long* src, int32_t* skey, int32_t* sidx, int32_t* winding,
                              int32_t* big_list, int32_t* big_excl, int32_t* big_count, const int32_t* bpre,
-                             uint32_t* ticket, int n_cu, hipStream_t s, const int2* band_pr = nullptr,
-                             const EmitArgs* emit = nullptr, SideStream side = {nullptr, nullptr, nullptr},
-                             int64_t n_entries = 0, hipStream_t s_small = nullptr);
-// Lists the bands of 513..1024 and 1025..2048 words (ticket[1..2] count them) and queues the
-// longer ones with their exclusive prefixes (big_count zeroed): the first launch of a sort with
-// emit.
+                             uint32_t* ticket, int n_cu, hipStream_t s,
+                             SideStream side = {nullptr, nullptr, nullptr});
+hipError_t launch_sort_big_bands(const int32_t* band_start, const int32_t* big_list, const int32_t* big_excl,
+                                 const int32_t* big_count, unsigned long long* scatter, unsigned long long* tmp,
+                                 int32_t* skey, int32_t* sidx, int32_t* winding, hipStream_t s);
+// Bands of frames with emit (narrow words; EmitArgs).  launch_band_classify comes first: it lists
+// the bands of 513..1024 and 1025..2048 words (ticket[1..2] count them) and queues the longer
+// ones with their exclusive prefixes (big_count zeroed).  launch_big_bands and the sort of the
+// bands of up to 512 words (s_small) may run on another stream, which the caller forks from s
+// after the classify pass and joins.  n_entries: an upper bound of the sorted entries.
 hipError_t launch_band_classify(const int32_t* band_start, const int32_t* n_bands, int64_t max_bands,
                                 const int32_t* bpre, int32_t* big_list, int32_t* big_excl, int32_t* big_count,
                                 uint32_t* ticket, hipStream_t s);
-// Mark + emit of the oversized bands from their sorted keys and winding numbers.
-hipError_t launch_emit_big_bands(const int32_t* band_start, const int32_t* big_list, const int32_t* big_count,
-                                 const int32_t* skey, const int32_t* winding, const int2* band_pr,
-                                 const EmitArgs& emit, hipStream_t s);
+hipError_t launch_sort_bands_emit(const int32_t* band_start, const int32_t* n_bands, int64_t max_bands,
+                                  const unsigned long long* src, const int32_t* big_list, const int32_t* bpre,
+                                  const uint32_t* ticket, const int2* band_pr, const EmitArgs& emit,
+                                  int64_t n_entries, hipStream_t s, hipStream_t s_small);
+hipError_t launch_big_bands(const int32_t* band_start, const int32_t* big_list, const int32_t* big_excl,
+                            const int32_t* big_count, const unsigned long long* src, const int2* band_pr,
+                            const EmitArgs& emit, int n_cu, hipStream_t s);
 // totals[0..2] (zeroed) += cells, spans, records: the sums of band_cnt over the bands.
 hipError_t launch_band_totals(const int2* band_cnt, const int32_t* n_bands, int32_t* totals, hipStream_t s);
-hipError_t launch_sort_big_bands(const int32_t* band_start, const int32_t* big_list, const int32_t* big_excl,
-                                 const int32_t* big_count, unsigned long long* scatter, unsigned long long* tmp,
-                                 int32_t* skey, int32_t* sidx, int32_t* winding, hipStream_t s,
-                                 const int2* band_pr = nullptr);
 
 // ---- winding / mark / emit (a10 scan, a11); also writes each (path, row) bucket's record range
 hipError_t launch_mark_emit(const int32_t* skey, const int32_t* winding, const uint32_t* epath,

@@ -594,15 +594,10 @@ void run_frame(spr_handle* H, bool record_begin = true) {
                 SPR_HIP(hipEventRecord(H->ev_sfork, s));
                 SPR_HIP(hipStreamWaitEvent(s2, H->ev_sfork, 0));
             }
-            SPR_HIP(spr::launch_sort_big_bands(H->band_start.p, H->big_list.p, H->big_list.p + max_bands, d_bigcount,
-                                               H->sbig.p, H->stmp.p, H->skey.p, nullptr, H->winding.p, s2,
-                                               H->band_pr.p));
-            SPR_HIP(spr::launch_emit_big_bands(H->band_start.p, H->big_list.p, d_bigcount, H->skey.p, H->winding.p,
-                                               H->band_pr.p, E, s2));
-            SPR_HIP(spr::launch_sort_bands(H->band_start.p, H->bflag.p + NB, max_bands, H->sbig.p, H->skey.p,
-                                           nullptr, H->winding.p, H->big_list.p, H->big_list.p + max_bands,
-                                           d_bigcount, d_bsum, ticket, H->n_cu, s, H->band_pr.p, &E,
-                                           side_for(H, N, Np), N, s2));
+            SPR_HIP(spr::launch_big_bands(H->band_start.p, H->big_list.p, H->big_list.p + max_bands, d_bigcount,
+                                          H->sbig.p, H->band_pr.p, E, H->n_cu, s2));
+            SPR_HIP(spr::launch_sort_bands_emit(H->band_start.p, H->bflag.p + NB, max_bands, H->sbig.p, H->big_list.p,
+                                                d_bsum, ticket, H->band_pr.p, E, N, s, s2));
             if (s2 != s) {
                 SPR_HIP(hipEventRecord(H->ev_sjoin, s2));  // after the short bands' sort on s2
                 SPR_HIP(hipStreamWaitEvent(s, H->ev_sjoin, 0));
@@ -612,10 +607,10 @@ void run_frame(spr_handle* H, bool record_begin = true) {
             SPR_HIP(spr::launch_sort_bands(H->band_start.p, H->bflag.p + NB, max_bands, H->sbig.p, H->skey.p,
                                            keep ? H->sidx.p : nullptr, H->winding.p, H->big_list.p,
                                            H->big_list.p + max_bands, d_bigcount, d_bsum, ticket, H->n_cu, s,
-                                           nullptr, nullptr, side_for(H, N, Np), N));
+                                           side_for(H, N, Np)));
             SPR_HIP(spr::launch_sort_big_bands(H->band_start.p, H->big_list.p, H->big_list.p + max_bands, d_bigcount,
                                                H->sbig.p, H->stmp.p, H->skey.p, keep ? H->sidx.p : nullptr,
-                                               H->winding.p, s, nullptr));
+                                               H->winding.p, s));
         }
     }
     stage_mark(H, 9);
@@ -952,15 +947,10 @@ void run_learned_frame(spr_handle* H) {
             SPR_HIP(hipEventRecord(H->ev_sfork, s));
             SPR_HIP(hipStreamWaitEvent(sb, H->ev_sfork, 0));
         }
-        SPR_HIP(spr::launch_sort_big_bands(H->band_start.p, H->big_list.p, H->big_list.p + max_bands, d_bigcount,
-                                           H->sbig.p, H->stmp.p, H->skey.p, nullptr, H->winding.p, sb,
-                                           H->band_pr.p));
-        SPR_HIP(spr::launch_emit_big_bands(H->band_start.p, H->big_list.p, d_bigcount, H->skey.p, H->winding.p,
-                                           H->band_pr.p, E, sb));
-        SPR_HIP(spr::launch_sort_bands(H->band_start.p, d_nbands, max_bands, H->sbig.p, H->skey.p, nullptr,
-                                       H->winding.p, H->big_list.p, H->big_list.p + max_bands, d_bigcount,
-                                       H->bsum_l.p, ticket, H->n_cu, s, H->band_pr.p, &E, side_for(H, nl, Np), nl,
-                                       sb));
+        SPR_HIP(spr::launch_big_bands(H->band_start.p, H->big_list.p, H->big_list.p + max_bands, d_bigcount,
+                                      H->sbig.p, H->band_pr.p, E, H->n_cu, sb));
+        SPR_HIP(spr::launch_sort_bands_emit(H->band_start.p, d_nbands, max_bands, H->sbig.p, H->big_list.p,
+                                            H->bsum_l.p, ticket, H->band_pr.p, E, nl, s, sb));
         if (sb != s) {
             SPR_HIP(hipEventRecord(H->ev_sjoin, sb));  // after the short bands' sort on sb
             SPR_HIP(hipStreamWaitEvent(s, H->ev_sjoin, 0));
@@ -970,10 +960,10 @@ void run_learned_frame(spr_handle* H) {
         SPR_HIP(spr::launch_sort_bands(H->band_start.p, d_nbands, max_bands, H->sbig.p, H->skey.p,
                                        debug ? H->sidx.p : nullptr, H->winding.p, H->big_list.p,
                                        H->big_list.p + max_bands, d_bigcount, H->bsum_l.p, ticket, H->n_cu, s,
-                                       nullptr, nullptr, side_for(H, nl, Np), nl));
+                                       side_for(H, nl, Np)));
         SPR_HIP(spr::launch_sort_big_bands(H->band_start.p, H->big_list.p, H->big_list.p + max_bands, d_bigcount,
                                            H->sbig.p, H->stmp.p, H->skey.p, debug ? H->sidx.p : nullptr,
-                                           H->winding.p, s, nullptr));
+                                           H->winding.p, s));
     }
     stage_mark(H, 9);
     if (H->batch && !narrow)
