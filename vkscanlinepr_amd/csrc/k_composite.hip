@@ -6,10 +6,11 @@
 // wins), and canvas row y lands on image row h-1-y.  All records sit on even rows, so the image
 // is a stack of independent two-pixel "cell rows".
 //
-// One workgroup owns one cell row, in column chunks of 4096; each thread keeps PIX consecutive
-// pixels of the chunk in registers (16; 8 in the anti-aliased variants, which keep both rows of a
-// cell row, in workgroups of 512 threads, so that they run as many waves per SIMD).  The per-column event words
-// live in LDS column-interleaved (column c at (c % PIX) * (4096 / PIX) + c / PIX), so the 64 lanes
+// One workgroup owns one chunk of CHUNK columns of one cell row; each thread keeps PIX consecutive
+// pixels of the chunk in registers.  The chunk follows the canvas (launch_composite): a canvas
+// row that fills a quarter of a chunk leaves three quarters of the threads without a pixel
+// and gives the others four times the pixels to fold one after another.  The per-column event words
+// live in LDS column-interleaved (column c at (c % PIX) * (CHUNK / PIX) + c / PIX), so the 64 lanes
 // of a wave touching "their" j-th column hit consecutive words instead of one bank.  The (path, row) bucket table gives each path's records on
 // this row as one contiguous range of non-overlapping compact records (x | width << 16) with one
 // colour.  Paths are taken in order, 64 at a time: a record toggles its path's bit at its first
@@ -23,7 +24,10 @@
 // Gradient paints (no reference counterpart: the reference draws solid colours only): a path
 // with a paint takes, at each covered pixel, the paint's colour at that pixel's centre, packed
 // like a solid fill, so the two rows of a cell row get their own colours; the variant that
-// evaluates them keeps a second row of pixels per thread.
+// evaluates them keeps a second row of pixels per thread.  An evaluation is some 150 dependent
+// operations per pixel and path, so this variant runs few pixels per thread (more waves), maps each
+// pixel centre back to the scene once for all its paths, and reads the batch's paints and stops
+// from LDS instead of through two dependent loads per evaluation.
 //
 // Anti-aliased coverage (src-over): a boundary cell record whose 64-sample mask (k_aa.hip) is not
 // full appends, at each of its two columns, an entry (path of the batch, covered samples of row y,
@@ -37,8 +41,7 @@ namespace spr {
 
 namespace {
 
-constexpr int kChunk = 4096;               // columns per pass (a workgroup of kChunk / PIX threads)
-constexpr int kPixOne = 16;                // pixels per thread of the variants that keep one row
+constexpr int kStops = 512;                // gradient stops of one batch in LDS
 constexpr int kBatch = 64;                 // paths per coverage mask
 constexpr int kAaSlots = 4;                // partial-coverage entries per column and batch
 constexpr int kList = 512;                 // paths listed before their batches are folded
@@ -46,10 +49,10 @@ constexpr int kListStep = 256;             // candidate paths examined per listi
 constexpr int kUnroll = 4;                 // records loaded per thread before applying
 typedef unsigned long long u64;
 
-// LDS slot of chunk column c (0 <= c < kChunk) with PIX consecutive pixels per thread: thread t's
-// column t * PIX + j sits at j * (kChunk / PIX) + t.
-template <int PIX>
-__device__ inline int ev_slot(int c) { return (c % PIX) * (kChunk / PIX) + c / PIX; }
+// LDS slot of chunk column c (0 <= c < CHUNK) with PIX consecutive pixels per thread: thread t's
+// column t * PIX + j sits at j * (CHUNK / PIX) + t.
+template <int PIX, int CHUNK>
+__device__ inline int ev_slot(int c) { return (c % PIX) * (CHUNK / PIX) + c / PIX; }
 
 __device__ inline u64 shfl_up_u64(u64 v, int d) {
     const uint32_t lo = (uint32_t)v, hi = (uint32_t)(v >> 32);
@@ -76,17 +79,19 @@ __device__ inline u64 block_exclusive_xor(u64 v, u64* lds) {
     return off ^ inc ^ v;
 }
 
-// A gradient's colour at the centre of canvas pixel (x, y), packed like a solid fill (channel
-// times 255 truncated, alpha times opacity, 0 when the alpha byte is 0).  Every float operation
-// is written out in order (the library is built without contraction).
-__device__ __forceinline__ uint32_t paint_color(const PaintArgs& pa, uint32_t pi, int x, int y) {
-    const float* h = pa.inv;
+// The scene point under the centre of canvas pixel (x, y); h: the inverse MVP's rows.
+__device__ __forceinline__ float2 scene_point(const float* h, int x, int y) {
     const float px = (float)x + 0.5f, py = (float)y + 0.5f;
     const float u = (h[0] * px + h[1] * py) + h[2];
     const float v = (h[3] * px + h[4] * py) + h[5];
     const float q = (h[6] * px + h[7] * py) + h[8];
-    const float sx = u / q, sy = v / q;
-    const Paint& g = pa.paints[pi];
+    return make_float2(u / q, v / q);
+}
+
+// A gradient's colour at scene point (sx, sy), packed like a solid fill (channel times 255
+// truncated, alpha times opacity, 0 when the alpha byte is 0).  st: the paint's stops.  Every
+// float operation is written out in order (the library is built without contraction).
+__device__ __forceinline__ uint32_t paint_color(const Paint& g, const float* st, float sx, float sy) {
     const float gx = (g.xform[0] * sx + g.xform[1] * sy) + g.xform[2];
     const float gy = (g.xform[3] * sx + g.xform[4] * sy) + g.xform[5];
     float t;
@@ -124,7 +129,6 @@ __device__ __forceinline__ uint32_t paint_color(const PaintArgs& pa, uint32_t pi
         }
         if (!(t == t)) t = 0.0f;
     }
-    const float* st = pa.stops + 5 * (size_t)g.first_stop;
     const uint32_t n = g.n_stops;
     float c[4];
     if (t <= st[0]) {
@@ -152,9 +156,12 @@ __device__ __forceinline__ uint32_t paint_color(const PaintArgs& pa, uint32_t pi
     return (out & 0xFF000000u) ? out : 0u;
 }
 
-// The colours of pixels (x, y) and (x, y + 1), the two rows of a cell row.
-__device__ __noinline__ uint2 paint_pair(const PaintArgs pa, uint32_t pi, int x, int y) {
-    return make_uint2(paint_color(pa, pi, x, y), paint_color(pa, pi, x, y + 1));
+// The colours of a pixel of each row of a cell row, from a paint and stops in memory (a paint
+// with more stops than LDS holds).
+__device__ __noinline__ uint2 paint_pair_far(const PaintArgs pa, uint32_t pi, float2 s0, float2 s1) {
+    const Paint g = pa.paints[pi];
+    const float* st = pa.stops + 5 * (size_t)g.first_stop;
+    return make_uint2(paint_color(g, st, s0.x, s0.y), paint_color(g, st, s1.x, s1.y));
 }
 
 // (r*a, g*a, b*a, a) of a packed colour, as the blend uses it.
@@ -175,8 +182,8 @@ __device__ inline void blend(float* d, const float4 sa) {
     d[3] = sa.w + d[3] * ia;
 }
 
-template <int COMPOSE, int GRAD, int AA, int PIX>
-__global__ __launch_bounds__(kChunk / PIX) __attribute__((amdgpu_waves_per_eu((AA && !GRAD) ? 4 : 1))) void k_composite(const uint32_t* __restrict__ records,
+template <int COMPOSE, int GRAD, int AA, int PIX, int CHUNK>
+__global__ __launch_bounds__(CHUNK / PIX) __attribute__((amdgpu_waves_per_eu((AA && !GRAD) ? 4 : 1))) void k_composite(const uint32_t* __restrict__ records,
                                                       const int2* __restrict__ brec,
                                                       const int32_t* __restrict__ bucket_base,
                                                       const int2* __restrict__ prow,
@@ -187,18 +194,21 @@ __global__ __launch_bounds__(kChunk / PIX) __attribute__((amdgpu_waves_per_eu((A
                                                       const PaintArgs pa,
                                                       const unsigned long long* __restrict__ cmask) {
     constexpr int TWO = (GRAD || AA) ? 1 : 0;            // the two rows of a cell row differ
-    constexpr int BLOCK = kChunk / PIX;                  // threads; each keeps PIX consecutive pixels
-    static_assert(PIX % 4 == 0 && BLOCK % 64 == 0 && BLOCK >= kListStep, "composite shape");
-    // partial coverage: entry k of column c at lslot[k * kChunk + ev_slot<PIX>(c)], q | n0 << 6 | n1 << 11;
+    constexpr int BLOCK = CHUNK / PIX;                   // threads; each keeps PIX consecutive pixels
+    static_assert(PIX % (AA ? 4 : 2) == 0 && BLOCK % 64 == 0 && BLOCK >= kListStep, "composite shape");
+    // partial coverage: entry k of column c at lslot[k * CHUNK + ev_slot<PIX, CHUNK>(c)], q | n0 << 6 | n1 << 11;
     // byte c of lcnt counts the column's entries (a thread's 16 columns in one 16-byte word)
-    __shared__ uint16_t lslot[AA ? kAaSlots * kChunk : 1];
-    __shared__ uint32_t lcnt[AA ? kChunk / 4 : 1];
+    __shared__ uint16_t lslot[AA ? kAaSlots * CHUNK : 1];
+    __shared__ uint32_t lcnt[AA ? CHUNK / 4 : 1];
     __shared__ int32_t lovf;
-    __shared__ u64 ev[kChunk];
+    __shared__ u64 ev[CHUNK];
     __shared__ int2 list[kList];
     __shared__ uint32_t lcol[kList];
     __shared__ uint32_t lpaint[GRAD ? kList : 1];  // each listed path's paint (kSolidPaint: its colour)
     __shared__ u64 lgrad;                          // the batch's paths that have a paint
+    __shared__ Paint lpnt[GRAD ? kBatch : 1];      // their paints (first_stop: the first in lstop, ~0: in memory)
+    __shared__ float lstop[GRAD ? 5 * kStops : 1];
+    __shared__ int32_t lfit;                       // paths of the batch whose stops fit in lstop
     __shared__ float4 lsa[kBatch];   // (r*a, g*a, b*a, a) of each path of the batch, as the blend uses them
     __shared__ int32_t wcount[BLOCK / 64];
     __shared__ int32_t bpre[kBatch + 1];
@@ -221,8 +231,10 @@ __global__ __launch_bounds__(kChunk / PIX) __attribute__((amdgpu_waves_per_eu((A
     const int y = 2 * r;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int xb = tid * PIX;  // first column of this thread inside the chunk
-    for (int c0 = 0; c0 < w; c0 += kChunk) {
-        const int cw = w - c0 < kChunk ? w - c0 : kChunk;
+    const int c0 = (int)blockIdx.y * CHUNK;
+    if (c0 >= w) return;  // a narrower document of a batch
+    {
+        const int cw = w - c0 < CHUNK ? w - c0 : CHUNK;
         uint32_t pix[PIX], pix1[TWO ? PIX : 1];  // rows y and, with paints or coverage, y + 1
         float acc[COMPOSE ? PIX : 1][4], acc1[(COMPOSE && TWO) ? PIX : 1][4];
 #pragma unroll
@@ -274,7 +286,7 @@ __global__ __launch_bounds__(kChunk / PIX) __attribute__((amdgpu_waves_per_eu((A
                 qn = n - q0 < kBatch ? n - q0 : kBatch;
             batch:
                 if constexpr (AA != 0) {
-                    for (int k = tid; k < kChunk / 4; k += BLOCK) lcnt[k] = 0u;
+                    for (int k = tid; k < CHUNK / 4; k += BLOCK) lcnt[k] = 0u;
                     if (tid == 0) lovf = 0;
                 }
                 // clear the event words; the batch's colours; its records as one flat index space
@@ -285,8 +297,32 @@ __global__ __launch_bounds__(kChunk / PIX) __attribute__((amdgpu_waves_per_eu((A
                         if (lane < qn) lsa[lane] = premul(lcol[q0 + lane]);
                     }
                     if constexpr (GRAD != 0) {
-                        const u64 gm = __ballot(lane < qn && lpaint[q0 + lane] != kSolidPaint);
+                        const uint32_t pi = lane < qn ? lpaint[q0 + lane] : kSolidPaint;
+                        const u64 gm = __ballot(pi != kSolidPaint);
                         if (lane == 0) lgrad = gm;
+                        Paint g;
+                        g.n_stops = 0;
+                        if (pi != kSolidPaint) g = pa.paints[pi];
+                        int upto = (int)min(g.n_stops, (uint32_t)kStops + 1u);
+#pragma unroll
+                        for (int d = 1; d < 64; d <<= 1) {
+                            const int u = __shfl_up(upto, d);
+                            if (lane >= d) upto += u;
+                        }
+                        // the paths up to the first whose stops no longer fit (that one alone, if
+                        // it is the first: its stops stay in memory)
+                        const u64 over = __ballot(upto > kStops);
+                        const int fit = max(1, over ? __ffsll((long long)over) - 1 : 64);
+                        if (lane == 0) lfit = fit;
+                        if (pi != kSolidPaint && lane < fit) {
+                            const float* src = pa.stops + 5 * (size_t)g.first_stop;
+                            const int at = upto - (int)g.n_stops;
+                            const bool near = upto <= kStops;
+                            if (near)
+                                for (uint32_t k = 0; k < 5u * g.n_stops; ++k) lstop[5 * at + (int)k] = src[k];
+                            g.first_stop = near ? (uint32_t)at : ~0u;
+                            lpnt[lane] = g;
+                        }
                     }
                     const int2 rg = lane < qn ? list[q0 + lane] : make_int2(0, 0);
                     int inc = rg.y - rg.x;
@@ -299,6 +335,7 @@ __global__ __launch_bounds__(kChunk / PIX) __attribute__((amdgpu_waves_per_eu((A
                     if (lane == 0) bpre[0] = 0;
                 }
                 __syncthreads();
+                if constexpr (GRAD != 0) qn = min(qn, lfit);
                 const int total = bpre[qn];
                 for (int f0 = tid; f0 < total; f0 += BLOCK * kUnroll) {
                     uint32_t rec[kUnroll];
@@ -328,8 +365,8 @@ __global__ __launch_bounds__(kChunk / PIX) __attribute__((amdgpu_waves_per_eu((A
                         xs = xs < 0 ? 0 : xs;
                         xe = xe > cw ? cw : xe;
                         if (xs < xe) {
-                            atomicXor(&ev[ev_slot<PIX>(xs)], bit);
-                            if (xe < cw) atomicXor(&ev[ev_slot<PIX>(xe)], bit);  // ends past the chunk change nothing
+                            atomicXor(&ev[ev_slot<PIX, CHUNK>(xs)], bit);
+                            if (xe < cw) atomicXor(&ev[ev_slot<PIX, CHUNK>(xe)], bit);  // ends past the chunk change nothing
                         }
                         if constexpr (AA != 0) {
                             const unsigned long long cm = cmask[ri[u]];
@@ -341,11 +378,11 @@ __global__ __launch_bounds__(kChunk / PIX) __attribute__((amdgpu_waves_per_eu((A
                                     if (col < 0 || col >= cw) continue;
                                     const uint32_t n0 = __popcll((cm >> (16 * px)) & 0xFFFFull);
                                     const uint32_t n1 = __popcll((cm >> (16 * (2 + px))) & 0xFFFFull);
-                                    const int sl = ev_slot<PIX>(col);
+                                    const int sl = ev_slot<PIX, CHUNK>(col);
                                     const uint32_t k = (atomicAdd(&lcnt[col >> 2], 1u << (8 * (col & 3))) >>
                                                         (8 * (col & 3))) & 0xFFu;
                                     if (k < (uint32_t)kAaSlots)
-                                        lslot[k * kChunk + sl] = (uint16_t)((uint32_t)qi[u] | (n0 << 6) | (n1 << 11));
+                                        lslot[k * CHUNK + sl] = (uint16_t)((uint32_t)qi[u] | (n0 << 6) | (n1 << 11));
                                     else
                                         lovf = 1;
                                 }
@@ -367,7 +404,7 @@ __global__ __launch_bounds__(kChunk / PIX) __attribute__((amdgpu_waves_per_eu((A
                 for (int j = 0; j < PIX; ++j) run ^= ev[j * BLOCK + tid];
                 u64 cov = block_exclusive_xor<BLOCK>(run, xlds);
                 const u64 gmask = GRAD ? lgrad : 0ull;
-                uint32_t cnt4[PIX / 4];  // AA: the partial-entry counts of the thread's columns, bytes
+                uint32_t cnt4[(PIX + 3) / 4];  // AA: the partial-entry counts of the thread's columns, bytes
 #pragma unroll
                 for (int k = 0; k < PIX / 4; ++k) cnt4[k] = AA ? lcnt[tid * (PIX / 4) + k] : 0u;
 #pragma unroll
@@ -375,7 +412,21 @@ __global__ __launch_bounds__(kChunk / PIX) __attribute__((amdgpu_waves_per_eu((A
                     cov ^= ev[j * BLOCK + tid];
                     u64 mm = cov;
                     if (mm == 0ull) continue;
-                    const int x = c0 + xb + j;  // the pixel's canvas column
+                    // the scene points of the pixel's centres, for its gradients
+                    float2 g0, g1;
+                    auto pair = [&](int k) -> uint2 {  // colours of path k of the batch
+                        const Paint& g = lpnt[k];
+                        if (g.first_stop == ~0u) return paint_pair_far(pa, lpaint[q0 + k], g0, g1);
+                        const float* st = lstop + 5 * g.first_stop;
+                        return make_uint2(paint_color(g, st, g0.x, g0.y), paint_color(g, st, g1.x, g1.y));
+                    };
+                    if constexpr (GRAD != 0) {
+                        if (mm & gmask) {
+                            const int x = c0 + xb + j;  // the pixel's canvas column
+                            g0 = scene_point(pa.inv, x, y);
+                            g1 = scene_point(pa.inv, x, y + 1);
+                        }
+                    }
                     // this pixel's partial-coverage entries (AA), and the paths they belong to
                     uint32_t pe[AA ? kAaSlots : 1];
                     uint32_t np = 0;
@@ -389,7 +440,7 @@ __global__ __launch_bounds__(kChunk / PIX) __attribute__((amdgpu_waves_per_eu((A
 #pragma unroll
                             for (int k = 0; k < kAaSlots; ++k) {
                                 if ((uint32_t)k < np) {
-                                    pe[k] = (uint32_t)lslot[k * kChunk + sl];
+                                    pe[k] = (uint32_t)lslot[k * CHUNK + sl];
                                     pm |= 1ull << (pe[k] & 63u);
                                 }
                             }
@@ -398,7 +449,7 @@ __global__ __launch_bounds__(kChunk / PIX) __attribute__((amdgpu_waves_per_eu((A
                     if constexpr (COMPOSE == 0) {
                         const int q = 63 - __clzll((long long)mm);
                         if (GRAD && ((gmask >> q) & 1ull)) {
-                            const uint2 pc = paint_pair(pa, lpaint[q0 + q], x, y);
+                            const uint2 pc = pair(q);
                             pix[j] = pc.x;
                             pix1[j] = pc.y;
                         } else {
@@ -418,7 +469,7 @@ __global__ __launch_bounds__(kChunk / PIX) __attribute__((amdgpu_waves_per_eu((A
                                 if constexpr (TWO != 0) {
                                     float4 s0 = L[q], s1 = L[q];
                                     if (GRAD && ((gmask >> (32 * hw + q)) & 1ull)) {
-                                        const uint2 pc = paint_pair(pa, lpaint[q0 + 32 * hw + q], x, y);
+                                        const uint2 pc = pair(32 * hw + q);
                                         s0 = premul(pc.x);
                                         s1 = premul(pc.y);
                                     }
@@ -470,7 +521,9 @@ __global__ __launch_bounds__(kChunk / PIX) __attribute__((amdgpu_waves_per_eu((A
                 if constexpr (TWO != 0) out[j] = yy == y ? pix[j] : pix1[j];
                 else out[j] = pix[j];
             }
-            if (xb + PIX <= cw && (((uintptr_t)(row + xb)) & 15u) == 0) {
+            if (PIX == 2 && xb + PIX <= cw && (((uintptr_t)(row + xb)) & 7u) == 0) {
+                *reinterpret_cast<uint2*>(row + xb) = make_uint2(out[0], out[1]);
+            } else if (PIX >= 4 && xb + PIX <= cw && (((uintptr_t)(row + xb)) & 15u) == 0) {
                 uint4* q = reinterpret_cast<uint4*>(row + xb);
 #pragma unroll
                 for (int k = 0; k < PIX / 4; ++k)
@@ -487,25 +540,39 @@ __global__ __launch_bounds__(kChunk / PIX) __attribute__((amdgpu_waves_per_eu((A
 
 }  // namespace
 
+// Chunk and pixels per thread by the widest row: the narrowest of 512, 1024 and 2048 columns in
+// workgroups of 256 threads that holds it, else 4096 columns at 16 pixels per thread (256 threads)
+// or, with coverage, 8 (512 threads: two rows of accumulators, 128 VGPRs, 4 waves per SIMD).  With
+// paints always 1024 columns at 4 per thread.
 hipError_t launch_composite(const uint32_t* records, const int2* brec, const int32_t* bucket_base,
                             const int2* prow, const uint32_t* fill, uint32_t Np, int w, int h, int compose,
                             uint8_t* image, hipStream_t s, int64_t rec_cap, const DocDev* docs, int n_docs,
                             int total_rows, const PaintArgs* paint, const unsigned long long* cmask) {
     const int rows = docs ? total_rows : (h + 1) / 2;
-    if (rows == 0 || (!docs && w == 0)) return hipSuccess;
+    if (rows == 0 || w == 0) return hipSuccess;
     if (cmask && !compose) return hipErrorInvalidValue;  // coverage needs the src-over blend
     const PaintArgs pa = paint ? *paint : PaintArgs{nullptr, nullptr, nullptr, nullptr};
-// pixels per thread: the coverage variants keep two rows of accumulators, so they run 8 per
-// thread in workgroups of 512 threads (without paints: at most 128 VGPRs, 4 waves per SIMD)
-#define SPR_COMPOSITE(C, G, A)                                                                              \
-    k_composite<C, G, A, (A) ? 8 : kPixOne><<<rows, kChunk / ((A) ? 8 : kPixOne), 0, s>>>(                    \
+#define SPR_COMPOSITE(C, G, A, PIX, CHUNK)                                                                      \
+    k_composite<C, G, A, PIX, CHUNK><<<dim3((unsigned)rows, (unsigned)((w + (CHUNK) - 1) / (CHUNK))), (CHUNK) / (PIX), 0, s>>>( \
         records, brec, bucket_base, prow, fill, Np, w, h, rec_cap, image, docs, n_docs, pa, cmask)
-    if (cmask) {
-        if (paint) SPR_COMPOSITE(1, 1, 1); else SPR_COMPOSITE(1, 0, 1);
+    if (paint) {
+        if (cmask) SPR_COMPOSITE(1, 1, 1, 4, 1024);
+        else if (compose) SPR_COMPOSITE(1, 1, 0, 4, 1024);
+        else SPR_COMPOSITE(0, 1, 0, 4, 1024);
+    } else if (cmask) {
+        if (w <= 1024) SPR_COMPOSITE(1, 0, 1, 4, 1024);
+        else if (w <= 2048) SPR_COMPOSITE(1, 0, 1, 8, 2048);
+        else SPR_COMPOSITE(1, 0, 1, 8, 4096);
     } else if (compose) {
-        if (paint) SPR_COMPOSITE(1, 1, 0); else SPR_COMPOSITE(1, 0, 0);
+        if (w <= 512) SPR_COMPOSITE(1, 0, 0, 2, 512);
+        else if (w <= 1024) SPR_COMPOSITE(1, 0, 0, 4, 1024);
+        else if (w <= 2048) SPR_COMPOSITE(1, 0, 0, 8, 2048);
+        else SPR_COMPOSITE(1, 0, 0, 16, 4096);
     } else {
-        if (paint) SPR_COMPOSITE(0, 1, 0); else SPR_COMPOSITE(0, 0, 0);
+        if (w <= 512) SPR_COMPOSITE(0, 0, 0, 2, 512);
+        else if (w <= 1024) SPR_COMPOSITE(0, 0, 0, 4, 1024);
+        else if (w <= 2048) SPR_COMPOSITE(0, 0, 0, 8, 2048);
+        else SPR_COMPOSITE(0, 0, 0, 16, 4096);
     }
 #undef SPR_COMPOSITE
     return hipGetLastError();

@@ -402,7 +402,7 @@ struct PaintArgs {
     const float* inv;            // 9 floats: inverse of the MVP's 2D projective part, rows
 };
 
-// ---- composite (a12).  paint (optional): per-pixel gradient colours for the paths that have one.
+// ---- composite (a12).  w: the canvas, the widest one of a batch.  paint (optional): per-pixel gradient colours for the paths that have one.
 // cmask (optional, src-over only): the records' sample coverage (launch_cell_cover).
 hipError_t launch_composite(const uint32_t* records, const int2* brec, const int32_t* bucket_base,
                             const int2* prow, const uint32_t* fill, uint32_t Np, int w, int h, int compose,

@@ -977,8 +977,8 @@ void run_learned_frame(spr_handle* H) {
                                       H->batch ? H->wbase.p : nullptr));
     stage_mark(H, 11);
     spr::PaintArgs pa;
-    SPR_HIP(spr::launch_composite(H->crec.p, H->brec_l.p, H->bucket_base.p, H->prow.p, H->fill.p, Np, w, h,
-                                  (int)H->opts.compose, H->image.p, s, rec_cap, H->batch ? H->docs.p : nullptr,
+    SPR_HIP(spr::launch_composite(H->crec.p, H->brec_l.p, H->bucket_base.p, H->prow.p, H->fill.p, Np,
+                                  H->batch ? H->max_w : w, h, (int)H->opts.compose, H->image.p, s, rec_cap, H->batch ? H->docs.p : nullptr,
                                   (int)H->n_docs, H->total_rows, paint_args(H, pa)));
     stage_mark(H, 12);
     if (!joined) SPR_HIP(hipStreamWaitEvent(s, H->ev_pjoin, 0));
