@@ -26,23 +26,6 @@ inline unsigned grid_for(int64_t n) {
     return (unsigned)(g < 1 ? 1 : g);
 }
 
-// Per-path bucket table from the path's cell-row bounds [lo, hi] (clamped to the canvas):
-// in-canvas rows r >= 1 get buckets first..first+nrows-1, then the off-canvas bucket, then row 0.
-__global__ void k_bucket_counts(const int32_t* __restrict__ row_lo, const int32_t* __restrict__ row_hi,
-                                uint32_t Np, int rmax, int32_t* __restrict__ nb, int2* __restrict__ prow,
-                                const int2* __restrict__ pcanvas) {
-    const uint32_t p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= Np) return;
-    if (pcanvas) rmax = (pcanvas[p].y - 1) / 2;
-    int lo = row_lo[p], hi = row_hi[p];
-    int first = lo < 1 ? 1 : lo;
-    int last = hi > rmax ? rmax : hi;
-    int nrows = last >= first ? last - first + 1 : 0;
-    if (lo > hi) { first = 1; nrows = 0; }  // no points
-    prow[p] = make_int2(first, nrows);
-    nb[p] = nrows + 2;
-}
-
 // Scatter into band order.  The wide sort word orders exactly like the reference's signed
 // (key, index) pair and carries the winding change in its two low bits.  The narrow word (used
 // when no stage is exported) drops the index: (bucket inside its path) << 17 | (x + 2) << 2 |
@@ -153,88 +136,222 @@ __global__ __launch_bounds__(kBlock) void k_bucket_scatter(const int32_t* __rest
     }
 }
 
-// Band starts: a band is a run of consecutive buckets of one path whose entries start in the
-// same 512-entry window (kBandWindowLog); a bucket of more than 512 entries is a band of its own.
-// Every band therefore holds at most 1024 entries (sorted by one wave, 16 per lane) unless it is a
-// single larger bucket.
-// One wave per path: the most recent non-empty bucket before each bucket is the nearest lane
-// below it in the ballot of non-empty buckets (or, for the chunk's first ones, the last
-// non-empty bucket of the earlier chunks), read with one shuffle.
-__global__ __launch_bounds__(kBlock) void k_band_flags(const int32_t* __restrict__ bucket_base, uint32_t Np,
-                                                       const int32_t* __restrict__ boff,
-                                                       int32_t* __restrict__ flag, int window_log) {
-    const uint32_t p = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (p >= Np) return;
-    const int32_t b0 = bucket_base[p], b1 = bucket_base[p + 1];
-    bool have = false;         // a non-empty bucket in an earlier chunk
-    int32_t cps = 0, cpz = 0;  // its start and size
-    for (int32_t c = b0; c < b1; c += 64) {
-        const int32_t b = c + lane;
-        int32_t o = 0, sz = 0;
-        if (b < b1) { o = boff[b]; sz = boff[b + 1] - o; }
-        const unsigned long long ne = __ballot(sz > 0);
-        const unsigned long long below = ne & ((1ull << lane) - 1ull);
-        const int src = below ? 63 - __clzll((long long)below) : lane;
-        const int32_t ps_l = __shfl(o, src), pz_l = __shfl(sz, src);
-        if (b < b1) {
-            int32_t f = 0;
-            if (sz > 0) {
-                const bool prev = below != 0ull || have;
-                if (!prev) {
-                    f = 1;
-                } else {
-                    const int32_t ps = below ? ps_l : cps, pz = below ? pz_l : cpz;
-                    const int32_t win = 1 << window_log;
-                    f = (o >> window_log) != (ps >> window_log) || pz > win || sz > win;
-                }
-            }
-            flag[b] = f;
-        }
-        if (ne) {
-            const int last = 63 - __clzll((long long)ne);
-            cps = __shfl(o, last);
-            cpz = __shfl(sz, last);
-            have = true;
-        }
+// What a run of buckets tells the buckets after it: its entries and the size of its last non-empty
+// bucket since the last path start (0: none since then), if it holds either.
+struct OpBands {
+    struct T {
+        uint32_t sum, last;
+        bool defined;
+    };
+    __device__ static T zero() { return {0u, 0u, false}; }
+    __device__ static T add(const T& a, const T& b) {  // b follows a
+        return {a.sum + b.sum, b.defined ? b.last : a.last, a.defined || b.defined};
     }
+    // sums and sizes are at most 2^30, a size with an entry after it less
+    __device__ static uint64_t encode(uint64_t st, const T& v) {
+        return (st << 62) | ((uint64_t)(v.defined ? 1u : 0u) << 61) | ((uint64_t)min(v.last, (1u << 30) - 1u) << 31) |
+               (v.sum & 0x7FFFFFFFu);
+    }
+    __device__ static uint64_t state(uint64_t w) { return w >> 62; }
+    __device__ static T value(uint64_t w) {
+        return {(uint32_t)(w & 0x7FFFFFFFu), (uint32_t)(w >> 31) & 0x3FFFFFFFu, ((w >> 61) & 1u) != 0};
+    }
+};
+
+__device__ inline OpBands::T shfl_up_bands(const OpBands::T& v, int d) {
+    return {(uint32_t)__shfl_up((int)v.sum, d), (uint32_t)__shfl_up((int)v.last, d), __shfl_up(v.defined ? 1 : 0, d) != 0};
 }
 
-// Band starts, and each band's path rows (of the path whose bucket range holds the band's first
-// bucket).
-__global__ void k_band_emit(const int32_t* __restrict__ flag_scan, const int32_t* __restrict__ boff,
-                            int32_t NB_max, int64_t N_max, int32_t* __restrict__ band_start,
-                            const int32_t* __restrict__ nb_dev, const int32_t* __restrict__ n_dev,
-                            const int32_t* __restrict__ bucket_base, uint32_t Np, const int2* __restrict__ prow,
-                            int2* __restrict__ band_pr, int32_t* __restrict__ band_path) {
-    const int32_t NB = nb_dev ? min(*nb_dev, NB_max) : NB_max;
-    const int64_t N = n_dev ? min((int64_t)*n_dev, N_max) : N_max;
-    // grid-stride over the live buckets (a launch for a bucket budget is capped)
-    for (int64_t b = (int64_t)blockIdx.x * kBlock + threadIdx.x; b < NB; b += (int64_t)gridDim.x * kBlock) {
-        if (flag_scan[b + 1] != flag_scan[b]) {
-            band_start[flag_scan[b]] = boff[b];
-            if (band_pr) {
-                uint32_t lo = 0, hi = Np;  // bucket_base[lo] <= b < bucket_base[hi]
-                while (hi - lo > 1) {
-                    const uint32_t mid = (lo + hi) >> 1;
-                    if (bucket_base[mid] <= b) lo = mid; else hi = mid;
+// The exclusive prefix of a tile by decoupled look-back, 64 predecessors at a time (first wave only);
+// as lookback() of scan_common.hpp for an operation that does not commute.
+__device__ inline OpBands::T lookback_bands(unsigned long long* status, int64_t tile, const OpBands::T& agg) {
+    const int lane = threadIdx.x & 63;
+    if (lane == 0) store_status(&status[tile], OpBands::encode(tile == 0 ? kStInclusive : kStAggregate, agg));
+    OpBands::T excl = OpBands::zero();
+    for (int64_t pred = tile - 1; pred >= 0;) {
+        const int64_t idx = pred - lane;
+        const unsigned long long st = idx >= 0 ? load_status(&status[idx]) : OpBands::encode(kStInclusive, OpBands::zero());
+        const uint64_t state = OpBands::state(st);
+        const unsigned long long inc_mask = __ballot(state == kStInclusive), bad_mask = __ballot(state == 0);
+        const int first_inc = inc_mask ? __ffsll((long long)inc_mask) - 1 : 64;
+        const unsigned long long upto = first_inc >= 63 ? ~0ull : ((2ull << first_inc) - 1ull);
+        if (bad_mask & upto) {
+            __builtin_amdgcn_s_sleep(1);
+            continue;
+        }
+        // lane 0 holds the nearest predecessor: combine from the highest lane down
+        OpBands::T v = lane <= first_inc ? OpBands::value(st) : OpBands::zero();
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const OpBands::T u = {(uint32_t)__shfl_down((int)v.sum, o), (uint32_t)__shfl_down((int)v.last, o),
+                                  __shfl_down(v.defined ? 1 : 0, o) != 0};
+            if (lane + o < 64) v = OpBands::add(u, v);
+        }
+        const OpBands::T all = {(uint32_t)__shfl((int)v.sum, 0), (uint32_t)__shfl((int)v.last, 0),
+                                __shfl(v.defined ? 1 : 0, 0) != 0};
+        excl = OpBands::add(all, excl);
+        if (first_inc < 64) break;
+        pred -= 64;
+    }
+    if (lane == 0 && tile > 0) store_status(&status[tile], OpBands::encode(kStInclusive, OpBands::add(excl, agg)));
+    return excl;
+}
+
+// Bucket offsets and bands in one pass over the bucket counts (in place: `hist` becomes the
+// exclusive offsets, total at [NB]).  A band is a run of consecutive buckets of one path whose
+// entries start in the same 512-entry window (kBandWindowLog); a bucket of more than 512 entries is
+// a band of its own.  Every band therefore holds at most 1024 entries (sorted by one wave, 16 per
+// lane) unless it is a single larger bucket.  A bucket starts a band when it is not empty and the
+// last non-empty bucket of its path before it started in another window, or either exceeds the
+// window, or there is none; that bucket ends where this one starts, so its size is all that the
+// look-back has to carry besides the offset.  A second look-back numbers the bands: flag_scan[b] =
+// bands before bucket b (total at [NB]), and each band's start, path and path rows are written.
+constexpr int kBandItems = 8, kBandTile = kBlock * kBandItems;
+constexpr int kBandPaths = kBandTile / 2 + 2;  // paths of a tile at most: a path owns two buckets or more
+static_assert(kBandTile == kBucketBandTile, "status arrays of the band pass");
+__global__ __launch_bounds__(kBlock) void k_bands(const BandArgs K) {
+    __shared__ int32_t s_base[kBandPaths];
+    __shared__ int32_t s_w[kBlock / 64], s_tile, s_p0;
+    __shared__ uint32_t s_sum[kBlock / 64], s_last[kBlock / 64];
+    __shared__ bool s_def[kBlock / 64];
+    const int32_t NB = K.nb_dev ? min(*K.nb_dev, K.NB) : K.NB;
+    if ((int64_t)blockIdx.x * kBandTile >= (NB > 0 ? NB : 1)) return;  // past the live buckets: no ticket
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t tile = ordered_tile_id(K.counter, &s_tile);
+    const int64_t b0 = tile * kBandTile;
+    // the paths of the tile's buckets: the path that holds b0, by a 64-way search of the first wave
+    if (wave == 0) {
+        int64_t lo = 0, hi = K.Np;  // bucket_base[lo] <= b0 < bucket_base[hi]
+        while (hi - lo > 1) {
+            const int64_t step = (hi - lo + 63) / 64;
+            const int64_t at = min(lo + (lane + 1) * step, hi);
+            const unsigned long long above = __ballot(at >= (int64_t)K.Np || (int64_t)K.bucket_base[at] > b0);
+            const int f = above ? __ffsll((long long)above) - 1 : 63;
+            const int64_t base = lo;
+            hi = min(base + (f + 1) * step, hi);
+            lo = base + f * step;
+        }
+        if (lane == 0) s_p0 = (int32_t)lo;
+    }
+    __syncthreads();
+    const int32_t p0 = s_p0;
+    for (int i = tid; i < kBandPaths; i += kBlock)
+        s_base[i] = p0 + i <= (int32_t)K.Np ? K.bucket_base[p0 + i] : 0x7FFFFFFF;
+    __syncthreads();
+    // thread t owns kBandItems consecutive buckets
+    const int64_t my = b0 + (int64_t)tid * kBandItems;
+    int pl = 0;  // path (local) of bucket my: s_base[pl] <= my < s_base[pl + 1]
+    {
+        int hi = kBandPaths - 1;
+        while (hi - pl > 1) {
+            const int mid = (pl + hi) >> 1;
+            if ((int64_t)s_base[mid] <= my) pl = mid; else hi = mid;
+        }
+    }
+    int32_t sz[kBandItems];
+#pragma unroll
+    for (int k = 0; k < kBandItems; ++k) sz[k] = my + k < NB ? K.hist[my + k] : 0;
+    OpBands::T agg = OpBands::zero();
+    {
+        int q = pl;
+#pragma unroll
+        for (int k = 0; k < kBandItems; ++k) {
+            while (q + 1 < kBandPaths && (int64_t)s_base[q + 1] <= my + k) ++q;
+            if ((int64_t)s_base[q] == my + k) { agg.last = 0; agg.defined = true; }
+            if (sz[k] > 0) { agg.last = (uint32_t)sz[k]; agg.defined = true; }
+            agg.sum += (uint32_t)sz[k];
+        }
+    }
+    OpBands::T inc = agg;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const OpBands::T u = shfl_up_bands(inc, o);
+        if (lane >= o) inc = OpBands::add(u, inc);
+    }
+    if (lane == 63) { s_sum[wave] = inc.sum; s_last[wave] = inc.last; s_def[wave] = inc.defined; }
+    __syncthreads();
+    OpBands::T before = OpBands::zero(), total = OpBands::zero();
+#pragma unroll
+    for (int k = 0; k < kBlock / 64; ++k) {
+        const OpBands::T x = {s_sum[k], s_last[k], s_def[k]};
+        if (k < wave) before = OpBands::add(before, x);
+        total = OpBands::add(total, x);
+    }
+    __syncthreads();
+    if (wave == 0) {
+        const OpBands::T pre = lookback_bands(K.status, tile, total);
+        if (lane == 0) { s_sum[0] = pre.sum; s_last[0] = pre.last; s_def[0] = pre.defined; }
+    }
+    __syncthreads();
+    const OpBands::T tile_pre = {s_sum[0], s_last[0], s_def[0]};
+    OpBands::T ex = shfl_up_bands(inc, 1);
+    if (lane == 0) ex = OpBands::zero();
+    ex = OpBands::add(tile_pre, OpBands::add(before, ex));
+    // flags
+    const int32_t win = 1 << K.window_log;
+    uint32_t flags = 0;
+    {
+        int32_t o = (int32_t)ex.sum, last = (int32_t)ex.last;
+        int q = pl;
+#pragma unroll
+        for (int k = 0; k < kBandItems; ++k) {
+            while (q + 1 < kBandPaths && (int64_t)s_base[q + 1] <= my + k) ++q;
+            if ((int64_t)s_base[q] == my + k) last = 0;
+            if (sz[k] > 0) {
+                const bool f = last == 0 || (o >> K.window_log) != ((o - last) >> K.window_log) || last > win || sz[k] > win;
+                flags |= f ? 1u << k : 0u;
+                last = sz[k];
+            }
+            o += sz[k];
+        }
+    }
+    const int32_t mine = __popc(flags);
+    const int32_t binc = wave_inclusive_add(mine);
+    if (lane == 63) s_w[wave] = binc;
+    __syncthreads();
+    int32_t bbefore = 0, btotal = 0;
+#pragma unroll
+    for (int k = 0; k < kBlock / 64; ++k) {
+        if (k < wave) bbefore += s_w[k];
+        btotal += s_w[k];
+    }
+    __syncthreads();
+    if (wave == 0) {
+        const int32_t pre = lookback<OpI32>(K.status2, tile, btotal);
+        if (lane == 0) s_w[0] = pre;
+    }
+    __syncthreads();
+    int32_t band = s_w[0] + bbefore + binc - mine;
+    {
+        int32_t o = (int32_t)ex.sum;
+        int q = pl;
+#pragma unroll
+        for (int k = 0; k < kBandItems; ++k) {
+            if (my + k >= NB) break;
+            while (q + 1 < kBandPaths && (int64_t)s_base[q + 1] <= my + k) ++q;
+            K.hist[my + k] = o;
+            K.flag_scan[my + k] = band;
+            if ((flags >> k) & 1u) {
+                K.band_start[band] = o;
+                if (K.band_pr) {
+                    K.band_pr[band] = K.prow[p0 + q];
+                    K.band_path[band] = p0 + q;
                 }
-                band_pr[flag_scan[b]] = prow[lo];
-                if (band_path) band_path[flag_scan[b]] = (int32_t)lo;
+                ++band;
+            }
+            o += sz[k];
+            if (my + k == NB - 1) {
+                K.hist[NB] = o;
+                K.flag_scan[NB] = band;
+                K.band_start[band] = o;
+                if (K.n_sorted) *K.n_sorted = o;
+                if (K.n_bands) *K.n_bands = band;
             }
         }
-        if (b == NB - 1) band_start[flag_scan[NB]] = (int32_t)N;
     }
 }
 
 }  // namespace
-
-hipError_t launch_bucket_counts(const int32_t* row_lo, const int32_t* row_hi, uint32_t Np, int rmax,
-                                int32_t* nb, int2* prow, hipStream_t s, const int2* pcanvas) {
-    if (Np == 0) return hipSuccess;
-    k_bucket_counts<<<grid_for(Np), kBlock, 0, s>>>(row_lo, row_hi, Np, rmax, nb, prow, pcanvas);
-    return hipGetLastError();
-}
 
 hipError_t launch_bucket_scatter(const int32_t* key, const int8_t* wn, const uint32_t* epath, int64_t N,
                                  const int32_t* bucket_base, const int2* prow, const int32_t* flag_scan,
@@ -257,23 +374,10 @@ hipError_t launch_bucket_scatter(const int32_t* key, const int8_t* wn, const uin
     return hipGetLastError();
 }
 
-hipError_t launch_band_flags(const int32_t* bucket_base, uint32_t Np, const int32_t* boff, int32_t* flag,
-                             hipStream_t s, int window_log) {
-    if (Np == 0) return hipSuccess;
-    if (window_log < kBandWindowLog || window_log > 10) return hipErrorInvalidValue;  // bands <= max_bands_for
-    k_band_flags<<<(Np + 3) / 4, kBlock, 0, s>>>(bucket_base, Np, boff, flag, window_log);
-    return hipGetLastError();
-}
-
-hipError_t launch_band_emit(const int32_t* flag_scan, const int32_t* boff, int32_t NB, int64_t N,
-                            int32_t* band_start, hipStream_t s, const int32_t* nb_dev, const int32_t* n_dev,
-                            const int32_t* bucket_base, uint32_t Np, const int2* prow, int2* band_pr,
-                            int32_t* band_path) {
-    if (NB == 0) return hipSuccess;
-    unsigned g = grid_for(NB);
-    if (g > 2048u) g = 2048u;  // the kernel strides over the live buckets
-    k_band_emit<<<g, kBlock, 0, s>>>(flag_scan, boff, NB, N, band_start, nb_dev, n_dev, bucket_base, Np, prow,
-                                     band_pr, band_path);
+hipError_t launch_bands(const BandArgs& K, hipStream_t s) {
+    if (K.Np == 0 || K.NB == 0) return hipSuccess;
+    if (K.window_log < kBandWindowLog || K.window_log > 10) return hipErrorInvalidValue;  // bands <= max_bands_for
+    k_bands<<<(unsigned)((K.NB + kBandTile - 1) / kBandTile), kBlock, 0, s>>>(K);
     return hipGetLastError();
 }
 

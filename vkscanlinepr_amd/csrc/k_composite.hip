@@ -36,6 +36,7 @@
 // redone with half as many paths (kAaSlots paths can never overflow).
 #include "device_common.hpp"
 #include "kernels.hpp"
+#include "scan_common.hpp"
 
 namespace spr {
 
@@ -182,6 +183,45 @@ __device__ inline void blend(float* d, const float4 sa) {
     d[3] = sa.w + d[3] * ia;
 }
 
+// The first workgroups of the launch: the cells and spans of the bands summed into totals, and, by the
+// last of them to end, the frame's counters gathered into host memory.  (On their own the two were
+// a launch each, and a copy.)
+template <int BLOCK>
+__device__ inline void tally(const TallyArgs& T) {
+    __shared__ int32_t s_c[BLOCK / 64], s_s[BLOCK / 64];
+    __shared__ uint32_t s_rank;
+    const int tid = threadIdx.x;
+    if (T.band_cnt) {
+        const int32_t nb = *T.n_bands;
+        int32_t c = 0, sp = 0;
+        for (int32_t t = (int32_t)blockIdx.x * BLOCK + tid; t < nb; t += T.blocks * BLOCK) {
+            const int2 v = T.band_cnt[t];
+            c += v.x;
+            sp += v.y;
+        }
+        c = wave_sum(c);
+        sp = wave_sum(sp);
+        if ((tid & 63) == 0) { s_c[tid >> 6] = c; s_s[tid >> 6] = sp; }
+        __syncthreads();
+        if (tid == 0) {
+            int32_t tc = 0, ts = 0;
+            for (int k = 0; k < BLOCK / 64; ++k) { tc += s_c[k]; ts += s_s[k]; }
+            if (tc) atomicAdd(&T.totals[0], tc);
+            if (ts) atomicAdd(&T.totals[1], ts);
+            if (tc + ts) atomicAdd(&T.totals[2], tc + ts);
+        }
+    }
+    if (tid == 0) {
+        __threadfence();
+        s_rank = atomicAdd(T.done, 1u);
+    }
+    __syncthreads();
+    if (s_rank != (uint32_t)T.blocks - 1u || tid >= T.src.n) return;
+    const int32_t* p = T.src.p[tid];
+    const int32_t v = p ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    __hip_atomic_store(&T.out[tid], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 template <int COMPOSE, int GRAD, int AA, int PIX, int CHUNK>
 __global__ __launch_bounds__(CHUNK / PIX) __attribute__((amdgpu_waves_per_eu((AA && !GRAD) ? 4 : 1))) void k_composite(const uint32_t* __restrict__ records,
                                                       const int2* __restrict__ brec,
@@ -192,7 +232,8 @@ __global__ __launch_bounds__(CHUNK / PIX) __attribute__((amdgpu_waves_per_eu((AA
                                                       uint8_t* __restrict__ image,
                                                       const DocDev* __restrict__ docs, int n_docs,
                                                       const PaintArgs pa,
-                                                      const unsigned long long* __restrict__ cmask) {
+                                                      const unsigned long long* __restrict__ cmask,
+                                                      const TallyArgs T) {
     constexpr int TWO = (GRAD || AA) ? 1 : 0;            // the two rows of a cell row differ
     constexpr int BLOCK = CHUNK / PIX;                   // threads; each keeps PIX consecutive pixels
     static_assert(PIX % (AA ? 4 : 2) == 0 && BLOCK % 64 == 0 && BLOCK >= kListStep, "composite shape");
@@ -213,7 +254,11 @@ __global__ __launch_bounds__(CHUNK / PIX) __attribute__((amdgpu_waves_per_eu((AA
     __shared__ int32_t wcount[BLOCK / 64];
     __shared__ int32_t bpre[kBatch + 1];
     __shared__ u64 xlds[BLOCK / 64];
-    int r = blockIdx.x;
+    if ((int)blockIdx.x < T.blocks) {
+        if (blockIdx.y == 0) tally<BLOCK>(T);
+        return;
+    }
+    int r = (int)blockIdx.x - T.blocks;
     uint32_t pbeg = 0, pend = Np;
     if (docs) {
         // batch: find this cell row's document (documents are numbered by first row)
@@ -547,14 +592,17 @@ __global__ __launch_bounds__(CHUNK / PIX) __attribute__((amdgpu_waves_per_eu((AA
 hipError_t launch_composite(const uint32_t* records, const int2* brec, const int32_t* bucket_base,
                             const int2* prow, const uint32_t* fill, uint32_t Np, int w, int h, int compose,
                             uint8_t* image, hipStream_t s, int64_t rec_cap, const DocDev* docs, int n_docs,
-                            int total_rows, const PaintArgs* paint, const unsigned long long* cmask) {
-    const int rows = docs ? total_rows : (h + 1) / 2;
-    if (rows == 0 || w == 0) return hipSuccess;
+                            int total_rows, const PaintArgs* paint, const unsigned long long* cmask, const TallyArgs* tally) {
+    const TallyArgs T = tally ? *tally : TallyArgs{};
+    int rows = docs ? total_rows : (h + 1) / 2;
+    if (w == 0) rows = 0;
+    if (rows + T.blocks == 0) return hipSuccess;
+    if (rows == 0) w = 1;  // the tally alone
     if (cmask && !compose) return hipErrorInvalidValue;  // coverage needs the src-over blend
     const PaintArgs pa = paint ? *paint : PaintArgs{nullptr, nullptr, nullptr, nullptr};
 #define SPR_COMPOSITE(C, G, A, PIX, CHUNK)                                                                      \
-    k_composite<C, G, A, PIX, CHUNK><<<dim3((unsigned)rows, (unsigned)((w + (CHUNK) - 1) / (CHUNK))), (CHUNK) / (PIX), 0, s>>>( \
-        records, brec, bucket_base, prow, fill, Np, w, h, rec_cap, image, docs, n_docs, pa, cmask)
+    k_composite<C, G, A, PIX, CHUNK><<<dim3((unsigned)(rows + T.blocks), (unsigned)((w + (CHUNK) - 1) / (CHUNK))), (CHUNK) / (PIX), 0, s>>>( \
+        records, brec, bucket_base, prow, fill, Np, w, h, rec_cap, image, docs, n_docs, pa, cmask, T)
     if (paint) {
         if (cmask) SPR_COMPOSITE(1, 1, 1, 4, 1024);
         else if (compose) SPR_COMPOSITE(1, 1, 0, 4, 1024);

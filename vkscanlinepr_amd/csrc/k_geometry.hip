@@ -2,6 +2,7 @@
 // (gfx950).  The intersection write between count and keys lives in k_curves.hip.
 #include "device_common.hpp"
 #include "kernels.hpp"
+#include "scan_common.hpp"
 
 namespace spr {
 
@@ -15,21 +16,6 @@ inline unsigned grid_for(int64_t n, int block = kBlock) {
 }
 
 __global__ void k_fill_u32(uint32_t* __restrict__ p, int64_t n, uint32_t v) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        p[i] = v;
-}
-
-// Frame summary: dst[i] = *src.p[i] (0 for a null source), one lane per value, so that one
-// device-to-host copy returns every counter of the frame.
-__global__ void k_gather_summary(SummarySrc src, int32_t* __restrict__ dst) {
-    const int i = threadIdx.x;
-    if (i < src.n) dst[i] = src.p[i] ? *src.p[i] : 0;
-}
-
-// Fill of min(n_max, mult * *n_dev + add) words (a count known only on the device).
-__global__ void k_fill_u32_dev(uint32_t* __restrict__ p, int64_t n_max, const int32_t* __restrict__ n_dev,
-                               int64_t mult, int64_t add, uint32_t v) {
-    const int64_t n = min(n_max, mult * (int64_t)*n_dev + add);
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         p[i] = v;
 }
@@ -123,56 +109,107 @@ __global__ __launch_bounds__(kBlock) void k_transform(const float2* __restrict__
     }
 }
 
-// make_intersection_0.comp:226-411: monotone cuts, cut cache, per-curve intersection count.
-__global__ __launch_bounds__(kBlock) void k_count(const float2* __restrict__ tpos,
-                                                  const uint32_t* __restrict__ cpos,
-                                                  const uint32_t* __restrict__ ctype,
-                                                  const float* __restrict__ cweight,
-                                                  const uint32_t* __restrict__ cpath,
-                                                  const int32_t* __restrict__ visible, uint32_t C,
-                                                  int w, int h, float4* __restrict__ cuts,
-                                                  uint32_t* __restrict__ ncuts,
-                                                  int32_t* __restrict__ counts,
-                                                  const int2* __restrict__ pcanvas) {
-    const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
-    if (c >= C) return;
-    const uint32_t path = cpath[c];
-    if (pcanvas) { w = pcanvas[path].x; h = pcanvas[path].y; }  // a batch: the path's document canvas
-    const CurvePts cv = load_curve(tpos, cpos[c], ctype[c], cweight, c);
-    const bool vis = visible_mask(visible[path]);
-    float q[4];
-    const uint32_t n = monotone_cuts(cv, vis, q);
-    cuts[c] = make_float4(q[0], q[1], q[2], q[3]);
-    ncuts[c] = n;
-    int32_t cnt = 0;
-    if (vis) {
-        float p0x = cv.x[0], p0y = cv.y[0];
+// Exclusive scan of one value per thread over the tiles of a launch (256 values a tile), with the
+// decoupled look-back of the tile's first wave.  Returns the thread's exclusive prefix; `upto`
+// receives the prefix after the tile.
+__device__ inline int32_t tile_scan(int32_t v, int64_t tile, unsigned long long* status, int32_t* s_w, int32_t& upto) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int32_t inc = wave_inclusive_add(v);
+    if (lane == 63) s_w[wave] = inc;
+    __syncthreads();
+    int32_t before = 0, total = 0;
 #pragma unroll
-        for (uint32_t k = 0; k < 5; ++k) {
-            if (k > n) break;
-            const float t = k < n ? q[k] : 1.0f;
-            const float p1x = cv.ex(t), p1y = cv.ey(t);
-            cnt += piece_count(p0x, p0y, p1x, p1y, w, h);
-            p0x = p1x; p0y = p1y;
-        }
+    for (int k = 0; k < kBlock / 64; ++k) {
+        const int32_t x = s_w[k];
+        if (k < wave) before = wadd(before, x);
+        total = wadd(total, x);
     }
-    counts[c] = cnt;
+    __syncthreads();
+    if (wave == 0) {
+        const int32_t pre = lookback<OpI32>(status, tile, total);
+        if (lane == 0) s_w[0] = pre;
+    }
+    __syncthreads();
+    const int32_t pre = s_w[0];
+    upto = wadd(pre, total);
+    return wadd(pre, wadd(before, (int32_t)((uint32_t)inc - (uint32_t)v)));
 }
 
-// Per-path segment starts: seg[p] = entries of all curves of paths < p (the sort segments of
-// gen_fragment.comp:227-244, derived from the curve offsets instead of entry boundaries).
-__global__ void k_path_segments(const uint32_t* __restrict__ cpath, uint32_t C,
-                                const int32_t* __restrict__ offsets, uint32_t Np,
-                                int32_t* __restrict__ seg) {
-    const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
-    if (c >= C) return;
-    const uint32_t p = cpath[c];
-    const uint32_t lo = c == 0 ? 0u : cpath[c - 1] + 1u;
-    const int32_t off = offsets[c];
-    for (uint32_t j = lo; j <= p; ++j) seg[j] = off;
-    if (c == C - 1) {
-        const int32_t total = offsets[C];
-        for (uint32_t j = p + 1; j <= Np; ++j) seg[j] = total;
+// make_intersection_0.comp:226-411 and the scans after it in one launch: the last K.curve_tiles
+// workgroups take 256 curves each (monotone cuts, cut cache, intersection count and its exclusive
+// scan, total at counts[C]; where each path's entries start, the sort segments of
+// gen_fragment.comp:227-244, falls out of it), the first K.path_tiles 256 paths each (their bucket rows from the row
+// bounds, and the exclusive scan of the bucket counts, total at bucket_base[Np]).  A count takes
+// microseconds and a scan by itself little but its launch, so the tiles' look-backs hide behind
+// the counting of the tiles after them.  The totals also go to host memory when the host waits
+// for them.  What bounds a small frame's prefix is its launches (about 4.5 us each, back to back, and
+// 8 us for a copy and its wait): with this kernel in the place of five launches and two copies, and
+// its fills in one launch instead of four, the 512 x 512 sketch's frame went from 375 us to 345 us.
+__global__ __launch_bounds__(kBlock) void k_count(const CountArgs K) {
+    __shared__ int32_t s_w[kBlock / 64], s_tile;
+    int32_t upto;
+    if ((int)blockIdx.x < K.path_tiles) {
+        // in-canvas rows r >= 1 get buckets first..first+nrows-1, then the off-canvas bucket, then row 0
+        const int64_t tile = ordered_tile_id(K.path_counter, &s_tile);
+        const int64_t p = tile * kBlock + threadIdx.x;
+        int32_t n = 0;
+        if (p < (int64_t)K.Np) {
+            const int rmax = K.pcanvas ? (K.pcanvas[p].y - 1) / 2 : K.rmax;
+            const int lo = K.row_lo[p], hi = K.row_hi[p];
+            int first = lo < 1 ? 1 : lo;
+            const int last = hi > rmax ? rmax : hi;
+            int nrows = last >= first ? last - first + 1 : 0;
+            if (lo > hi) { first = 1; nrows = 0; }  // no points
+            K.prow[p] = make_int2(first, nrows);
+            n = nrows + 2;
+        }
+        const int32_t at = tile_scan(n, tile, K.path_status, s_w, upto);
+        if (p < (int64_t)K.Np) K.bucket_base[p] = at;
+        if (tile == K.path_tiles - 1 && threadIdx.x == 0) {
+            K.bucket_base[K.Np] = upto;
+            if (K.host) __hip_atomic_store(&K.host[1], upto, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        return;
+    }
+    const int64_t tile = ordered_tile_id(K.curve_counter, &s_tile);
+    const int64_t c = tile * kBlock + threadIdx.x;
+    int32_t cnt = 0;
+    if (c < (int64_t)K.C) {
+        const uint32_t path = K.cpath[c];
+        int w = K.w, h = K.h;
+        if (K.pcanvas) { w = K.pcanvas[path].x; h = K.pcanvas[path].y; }  // a batch: the path's document canvas
+        const CurvePts cv = load_curve(K.tpos, K.cpos[c], K.ctype[c], K.cweight, (uint32_t)c);
+        const bool vis = visible_mask(K.visible[path]);
+        float q[4];
+        const uint32_t n = monotone_cuts(cv, vis, q);
+        K.cuts[c] = make_float4(q[0], q[1], q[2], q[3]);
+        K.ncuts[c] = n;
+        if (vis) {
+            float p0x = cv.x[0], p0y = cv.y[0];
+#pragma unroll
+            for (uint32_t k = 0; k < 5; ++k) {
+                if (k > n) break;
+                const float t = k < n ? q[k < 4 ? k : 3] : 1.0f;
+                const float p1x = cv.ex(t), p1y = cv.ey(t);
+                cnt += piece_count(p0x, p0y, p1x, p1y, w, h);
+                p0x = p1x; p0y = p1y;
+            }
+        }
+    }
+    const int32_t at = tile_scan(cnt, tile, K.curve_status, s_w, upto);
+    if (c < (int64_t)K.C) {
+        K.counts[c] = at;
+        if (K.seg) {
+            // the paths that start with this curve (and the empty ones before them)
+            const uint32_t path = K.cpath[c];
+            for (uint32_t j = c == 0 ? 0u : K.cpath[c - 1] + 1u; j <= path; ++j) K.seg[j] = at;
+            if (c == (int64_t)K.C - 1)
+                for (uint32_t j = path + 1; j <= K.Np; ++j) K.seg[j] = upto;
+        }
+    }
+    if (tile == K.curve_tiles - 1 && threadIdx.x == 0) {
+        K.counts[K.C] = upto;
+        if (K.host) __hip_atomic_store(&K.host[0], upto, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -256,21 +293,6 @@ __global__ __launch_bounds__(kBlock) void k_gen_fragment(const int2* __restrict_
 
 }  // namespace
 
-hipError_t launch_fill_u32_dev(uint32_t* p, int64_t n_max, const int32_t* n_dev, int64_t mult, int64_t add,
-                               uint32_t v, hipStream_t s) {
-    if (n_max <= 0) return hipSuccess;
-    int64_t g = (n_max + kBlock - 1) / kBlock;
-    if (g > 4096) g = 4096;
-    k_fill_u32_dev<<<(unsigned)g, kBlock, 0, s>>>(p, n_max, n_dev, mult, add, v);
-    return hipGetLastError();
-}
-
-hipError_t launch_gather_summary(const SummarySrc& src, int32_t* dst, hipStream_t s) {
-    if (src.n <= 0 || src.n > kSummaryMax) return hipErrorInvalidValue;
-    k_gather_summary<<<1, 64, 0, s>>>(src, dst);
-    return hipGetLastError();
-}
-
 hipError_t launch_frame_init(const FrameInit& I, hipStream_t s) {
     int64_t n = I.C;
     for (int k = 0; k < I.n_fills; ++k) n = n > I.fill[k].n ? n : I.fill[k].n;
@@ -297,19 +319,8 @@ hipError_t launch_transform(const float2* pos, const uint32_t* pos_path, uint32_
     return hipGetLastError();
 }
 
-hipError_t launch_count(const float2* tpos, const uint32_t* cpos, const uint32_t* ctype,
-                        const float* cweight, const uint32_t* cpath, const int32_t* visible, uint32_t C, int w, int h,
-                        float4* cuts, uint32_t* ncuts, int32_t* counts, hipStream_t s, const int2* pcanvas) {
-    if (C == 0) return hipSuccess;
-    k_count<<<grid_for(C), kBlock, 0, s>>>(tpos, cpos, ctype, cweight, cpath, visible, C, w, h, cuts, ncuts, counts,
-                                           pcanvas);
-    return hipGetLastError();
-}
-
-hipError_t launch_path_segments(const uint32_t* cpath, uint32_t C, const int32_t* offsets,
-                                uint32_t Np, int32_t* seg, hipStream_t s) {
-    if (C == 0) return launch_fill_u32((uint32_t*)seg, (int64_t)Np + 1, 0u, s);
-    k_path_segments<<<grid_for(C), kBlock, 0, s>>>(cpath, C, offsets, Np, seg);
+hipError_t launch_count(const CountArgs& K, hipStream_t s) {
+    k_count<<<(unsigned)(K.path_tiles + K.curve_tiles), kBlock, 0, s>>>(K);
     return hipGetLastError();
 }
 

@@ -366,12 +366,13 @@ __global__ void k_doc_winding_base(const int32_t* __restrict__ winding, const in
 // Winding number at each document's first sorted entry from the bands: that position is a band
 // start (a path's first non-empty bucket starts a band) or the end, whose prefix is the total.
 __global__ void k_doc_winding_base_bands(const int32_t* __restrict__ band_start, const int32_t* __restrict__ bpre,
-                                         const int32_t* __restrict__ n_bands, const int32_t* __restrict__ sstart,
+                                         const int32_t* __restrict__ n_bands, const int32_t* __restrict__ boff,
+                                         const int32_t* __restrict__ bucket_base,
                                          const int32_t* __restrict__ doc_first_path, uint32_t Np,
                                          int32_t* __restrict__ wbase) {
     const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= Np) return;
-    const int32_t pos = sstart[doc_first_path[p]];
+    const int32_t pos = boff[bucket_base[doc_first_path[p]]];
     int32_t lo = 0, hi = *n_bands;  // band_start[lo] <= pos < band_start[hi], band_start[n_bands] = end
     while (hi - lo > 1) {
         const int32_t mid = (lo + hi) >> 1;
@@ -425,10 +426,11 @@ hipError_t launch_doc_winding_base(const int32_t* winding, const int32_t* sstart
 }
 
 hipError_t launch_doc_winding_base_bands(const int32_t* band_start, const int32_t* bpre, const int32_t* n_bands,
-                                         const int32_t* sstart, const int32_t* doc_first_path, uint32_t Np,
-                                         int32_t* wbase, hipStream_t s) {
+                                         const int32_t* boff, const int32_t* bucket_base,
+                                         const int32_t* doc_first_path, uint32_t Np, int32_t* wbase, hipStream_t s) {
     if (Np == 0) return hipSuccess;
-    k_doc_winding_base_bands<<<blocks(Np), 256, 0, s>>>(band_start, bpre, n_bands, sstart, doc_first_path, Np, wbase);
+    k_doc_winding_base_bands<<<blocks(Np), 256, 0, s>>>(band_start, bpre, n_bands, boff, bucket_base,
+                                                       doc_first_path, Np, wbase);
     return hipGetLastError();
 }
 

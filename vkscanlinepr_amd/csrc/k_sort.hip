@@ -487,20 +487,37 @@ __device__ __forceinline__ void wave_band(const uint32_t* __restrict__ src, int 
     if (lane == 63) EA.band_cnt[band] = make_int2(inc & 0xFFFF, inc >> 16);
 }
 
-// Bands above 512 words in two lists: up to 1024 words from the front of `list`, longer ones (single
-// buckets) from the back (list holds `cap` slots); counts in count[0] and count[1].  One atomic per
-// list per 1024-thread block.
+// The bands' exclusive prefixes of the winding changes (`bsum` in place, total at [n_bands]) by one
+// look-back scan, and the bands above 512 words in two lists: up to 1024 words from the front of
+// `list`, longer ones (single buckets) from the back (list holds `cap` slots); counts in count[0]
+// and count[1].  One atomic per list per 1024-thread block.
 __global__ __launch_bounds__(kClassifyThreads) void k_band_classify2(const int32_t* __restrict__ band_start,
                                                                      const int32_t* __restrict__ n_bands,
                                                                      int32_t* __restrict__ list, int64_t cap,
                                                                      uint32_t* __restrict__ count,
-                                                                     const int32_t* __restrict__ bpre,
+                                                                     int32_t* __restrict__ bsum,
+                                                                     unsigned long long* __restrict__ status,
+                                                                     uint32_t* __restrict__ counter,
                                                                      int32_t* __restrict__ big_list,
                                                                      int32_t* __restrict__ big_excl,
                                                                      int32_t* __restrict__ big_count) {
     __shared__ uint32_t s_n[2][kClassifyThreads / 64], s_base[2];
-    const int64_t t = (int64_t)blockIdx.x * kClassifyThreads + threadIdx.x;
+    __shared__ int32_t s_w[kClassifyThreads / 64], s_pre, s_tile;
     const int32_t nb = *n_bands;
+    if ((int64_t)blockIdx.x * kClassifyThreads >= (nb > 0 ? nb : 1)) return;  // past the live bands: no ticket
+    const int64_t tile = ordered_tile_id(counter, &s_tile);
+    const int64_t t = tile * kClassifyThreads + threadIdx.x;
+    const int32_t sum = t < nb ? bsum[t] : 0;
+    int32_t total;
+    int32_t excl = block_exclusive_add<int32_t, kClassifyThreads / 64>(sum, s_w, total);
+    if (threadIdx.x < 64) {
+        const int32_t pre = lookback<OpI32>(status, tile, total);
+        if (threadIdx.x == 0) s_pre = pre;
+    }
+    __syncthreads();
+    excl = wadd(s_pre, excl);
+    if (t < nb) bsum[t] = excl;
+    if (t == nb - 1 || (nb == 0 && t == 0)) bsum[nb] = wadd(excl, sum);
     const int32_t n = t < nb ? band_start[t + 1] - band_start[t] : 0;
     const bool med = n > kSmallBandMax && n <= kMediumBandMax;
     const bool large = n > kMediumBandMax && n <= kWaveBandMax;
@@ -509,7 +526,7 @@ __global__ __launch_bounds__(kClassifyThreads) void k_band_classify2(const int32
         // k_big_bands, which may run beside the wave sorts
         const int32_t q = atomicAdd(big_count, 1);
         big_list[q] = (int32_t)t;
-        big_excl[q] = bpre[t];
+        big_excl[q] = excl;
     }
     const unsigned long long mm = __ballot(med), ml = __ballot(large);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -804,33 +821,6 @@ __global__ __launch_bounds__(kColThreads) void k_big_bands(const int32_t* __rest
     }
 }
 
-// totals (zeroed) += (cells, spans, records) summed over the bands' counts: a grid-stride
-// loop, one sum per block, three atomics per block.
-constexpr int kTotBlocks = 64, kTotThreads = 256;
-__global__ __launch_bounds__(kTotThreads) void k_band_totals(const int2* __restrict__ band_cnt,
-                                                             const int32_t* __restrict__ n_bands,
-                                                             int32_t* __restrict__ totals) {
-    __shared__ int32_t s_c[kTotThreads / 64], s_s[kTotThreads / 64];
-    const int32_t nb = *n_bands;
-    int32_t c = 0, sp = 0;
-    for (int32_t t = blockIdx.x * kTotThreads + threadIdx.x; t < nb; t += kTotBlocks * kTotThreads) {
-        const int2 v = band_cnt[t];
-        c += v.x;
-        sp += v.y;
-    }
-    c = wave_sum(c);
-    sp = wave_sum(sp);
-    if ((threadIdx.x & 63) == 0) { s_c[threadIdx.x >> 6] = c; s_s[threadIdx.x >> 6] = sp; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int32_t tc = 0, ts = 0;
-        for (int k = 0; k < kTotThreads / 64; ++k) { tc += s_c[k]; ts += s_s[k]; }
-        if (tc) atomicAdd(&totals[0], tc);
-        if (ts) atomicAdd(&totals[1], ts);
-        if (tc + ts) atomicAdd(&totals[2], tc + ts);
-    }
-}
-
 // Workgroups per CU for a class: as many as the CU's 32 wave slots and 160 KiB of LDS allow.
 template <class T, int THREADS>
 unsigned class_grid(int64_t max_bands, int n_cu) {
@@ -895,12 +885,13 @@ hipError_t launch_sort_bands_emit(const int32_t* band_start, const int32_t* n_ba
 }
 
 hipError_t launch_band_classify(const int32_t* band_start, const int32_t* n_bands, int64_t max_bands,
-                                const int32_t* bpre, int32_t* big_list, int32_t* big_excl, int32_t* big_count,
-                                uint32_t* ticket, hipStream_t s) {
+                                int32_t* bsum, ScanCtl ctl, int32_t* big_list, int32_t* big_excl,
+                                int32_t* big_count, uint32_t* ticket, hipStream_t s) {
     if (max_bands <= 0) return hipSuccess;
     int32_t* lists = big_list + 2 * max_bands;
     k_band_classify2<<<(unsigned)((max_bands + kClassifyThreads - 1) / kClassifyThreads), kClassifyThreads, 0, s>>>(
-        band_start, n_bands, lists, 2 * max_bands, ticket + 1, bpre, big_list, big_excl, big_count);
+        band_start, n_bands, lists, 2 * max_bands, ticket + 1, bsum, ctl.status, ctl.counter, big_list, big_excl,
+        big_count);
     return hipGetLastError();
 }
 
@@ -909,11 +900,6 @@ hipError_t launch_big_bands(const int32_t* band_start, const int32_t* big_list, 
                             const EmitArgs& emit, int n_cu, hipStream_t s) {
     k_big_bands<<<(unsigned)n_cu, kColThreads, 0, s>>>(band_start, big_list, big_excl, big_count,
                                                        reinterpret_cast<const uint32_t*>(src), band_pr, emit);
-    return hipGetLastError();
-}
-
-hipError_t launch_band_totals(const int2* band_cnt, const int32_t* n_bands, int32_t* totals, hipStream_t s) {
-    k_band_totals<<<kTotBlocks, kTotThreads, 0, s>>>(band_cnt, n_bands, totals);
     return hipGetLastError();
 }
 

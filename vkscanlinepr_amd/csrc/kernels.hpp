@@ -27,28 +27,51 @@ inline int64_t scan_tiles(int64_t n) { return (n + kScanTile - 1) / kScanTile; }
 
 // ---- control
 hipError_t launch_fill_u32(uint32_t* p, int64_t n, uint32_t v, hipStream_t s);
-hipError_t launch_fill_u32_dev(uint32_t* p, int64_t n_max, const int32_t* n_dev, int64_t mult, int64_t add,
-                               uint32_t v, hipStream_t s);
-// One device-to-host copy per frame: the frame's counters gathered from wherever the kernels
-// left them into one contiguous int32 array.
+// The frame's counters, gathered from wherever the kernels left them.
 constexpr int kSummaryMax = 24;
 struct SummarySrc {
-    const int32_t* p[kSummaryMax];
+    const int32_t* p[kSummaryMax];  // null: 0
     int n;
 };
-hipError_t launch_gather_summary(const SummarySrc& src, int32_t* dst, hipStream_t s);
 
 // ---- geometry (a3, a4, a7, a8)
 // mvp_dev (optional): the matrix read from device memory instead of m.
 hipError_t launch_transform(const float2* pos, const uint32_t* pos_path, uint32_t P, const Mvp& m,
                             int w, int h, float2* tpos, int32_t* visible, int32_t* row_lo, int32_t* row_hi,
                             hipStream_t s, const int2* pcanvas = nullptr, const float* mvp_dev = nullptr);
-hipError_t launch_count(const float2* tpos, const uint32_t* cpos, const uint32_t* ctype,
-                        const float* cweight, const uint32_t* cpath, const int32_t* visible, uint32_t C, int w, int h,
-                        float4* cuts, uint32_t* ncuts, int32_t* counts, hipStream_t s,
-                        const int2* pcanvas = nullptr);
-hipError_t launch_path_segments(const uint32_t* cpath, uint32_t C, const int32_t* offsets,
-                                uint32_t Np, int32_t* seg, hipStream_t s);
+// Count pass with the exclusive scans of the per-curve counts and of the paths' bucket counts.
+// Statuses and counters zeroed; tiles of kCountTile curves or paths, at least one of each.
+constexpr int kCountTile = 256;
+inline int count_tiles(int64_t n) { return (int)(n > 0 ? (n + kCountTile - 1) / kCountTile : 1); }
+struct CountArgs {
+    const float2* tpos;
+    const uint32_t* cpos;
+    const uint32_t* ctype;
+    const float* cweight;
+    const uint32_t* cpath;
+    const int32_t* visible;
+    uint32_t C;
+    int w, h;
+    float4* cuts;
+    uint32_t* ncuts;
+    int32_t* counts;            // [C + 1]
+    int32_t* seg;               // [Np + 1] entries of all curves of paths < p, or null
+    int curve_tiles;
+    unsigned long long* curve_status;
+    uint32_t* curve_counter;
+    const int32_t* row_lo;
+    const int32_t* row_hi;
+    uint32_t Np;
+    int rmax;
+    int32_t* bucket_base;       // [Np + 1]
+    int2* prow;
+    int path_tiles;
+    unsigned long long* path_status;
+    uint32_t* path_counter;
+    const int2* pcanvas;        // per-path canvas of a batch, or null
+    int32_t* host;              // the two totals in host memory, or null
+};
+hipError_t launch_count(const CountArgs& K, hipStream_t s);
 hipError_t launch_segment_stats(const int32_t* seg, uint32_t Np, int32_t* max_len, hipStream_t s);
 // One (curve, piece, axis) chain of dependent crossing solves, and one monotone piece.
 struct ChainDesc {
@@ -231,8 +254,6 @@ constexpr int kBandWindowLog = 9;
 inline int64_t max_bands_for(uint32_t Np, int64_t n_entries) {
     return (int64_t)Np + 3 * (n_entries >> kBandWindowLog) + 2;
 }
-hipError_t launch_bucket_counts(const int32_t* row_lo, const int32_t* row_hi, uint32_t Np, int rmax,
-                                int32_t* nb, int2* prow, hipStream_t s, const int2* pcanvas = nullptr);
 // narrow: 32-bit sort words (first half of `out`) without the entry index, for frames that
 // export no stage and whose canvases are narrower than kNarrowMaxW.
 constexpr uint32_t kNarrowX0 = 0x7FFDu;   // x field of the leftmost key (x = -2)
@@ -245,15 +266,29 @@ hipError_t launch_bucket_scatter(const int32_t* key, const int8_t* wn, const uin
                                  const int32_t* band_start, int32_t* fill, int32_t* bsum, unsigned long long* out,
                                  int32_t* err, hipStream_t s, const int32_t* n_dev = nullptr, bool narrow = false,
                                  bool packed = false);
-// window_log: bands start in 2^window_log-entry windows (9 = kBandWindowLog or 10; tuned).
-hipError_t launch_band_flags(const int32_t* bucket_base, uint32_t Np, const int32_t* boff, int32_t* flag,
-                             hipStream_t s, int window_log = kBandWindowLog);
-// band_pr (or null): each band's path rows (prow of its path), for the narrow sort.
-// band_path (with band_pr): each band's path.
-hipError_t launch_band_emit(const int32_t* flag_scan, const int32_t* boff, int32_t NB, int64_t N,
-                            int32_t* band_start, hipStream_t s, const int32_t* nb_dev = nullptr,
-                            const int32_t* n_dev = nullptr, const int32_t* bucket_base = nullptr, uint32_t Np = 0,
-                            const int2* prow = nullptr, int2* band_pr = nullptr, int32_t* band_path = nullptr);
+// Bucket offsets and bands from the bucket counts.  Statuses and counter zeroed, one status of each
+// kind per kBucketBandTile buckets.
+constexpr int kBucketBandTile = 2048;
+inline int64_t bucket_band_tiles(int64_t nb) { return nb > 0 ? (nb + kBucketBandTile - 1) / kBucketBandTile : 1; }
+struct BandArgs {
+    int32_t* hist;              // [NB + 1] counts in, exclusive offsets out
+    int32_t NB;                 // buckets, or their bound with nb_dev
+    const int32_t* nb_dev;
+    const int32_t* bucket_base;
+    uint32_t Np;
+    const int2* prow;
+    int window_log;             // bands start in 2^window_log-entry windows (9 = kBandWindowLog or 10; tuned)
+    int32_t* flag_scan;         // [NB + 1] bands before each bucket
+    int32_t* band_start;        // [bands + 1]
+    int2* band_pr;              // each band's path rows (prow of its path) and path, for the narrow
+    int32_t* band_path;         // sort, or null
+    int32_t* n_sorted;          // entries and bands, or null
+    int32_t* n_bands;
+    unsigned long long* status;
+    unsigned long long* status2;
+    uint32_t* counter;
+};
+hipError_t launch_bands(const BandArgs& K, hipStream_t s);
 // Mark + emit fused into the narrow band sort (frames that export no stage): each band flags its
 // cells and spans (every flag depends only on the band's own entries: bands split at (path, row)
 // bucket boundaries), writes its compact records at [2 * band_start, ...) of crec, the record
@@ -288,14 +323,15 @@ hipError_t launch_sort_bands(const int32_t* band_start, const int32_t* n_bands, 
 hipError_t launch_sort_big_bands(const int32_t* band_start, const int32_t* big_list, const int32_t* big_excl,
                                  const int32_t* big_count, unsigned long long* scatter, unsigned long long* tmp,
                                  int32_t* skey, int32_t* sidx, int32_t* winding, hipStream_t s);
-// Bands of frames with emit (narrow words; EmitArgs).  launch_band_classify comes first: it lists
-// the bands of 513..1024 and 1025..2048 words (ticket[1..2] count them) and queues the longer
-// ones with their exclusive prefixes (big_count zeroed).  launch_big_bands and the sort of the
+// Bands of frames with emit (narrow words; EmitArgs).  launch_band_classify comes first: it scans the
+// bands' sums of winding changes in place, lists the bands of 513..1024 and 1025..2048 words
+// (ticket[1..2] count them) and queues the longer ones with their exclusive prefixes (big_count
+// zeroed).  launch_big_bands and the sort of the
 // bands of up to 512 words (s_small) may run on another stream, which the caller forks from s
 // after the classify pass and joins.  n_entries: an upper bound of the sorted entries.
 hipError_t launch_band_classify(const int32_t* band_start, const int32_t* n_bands, int64_t max_bands,
-                                const int32_t* bpre, int32_t* big_list, int32_t* big_excl, int32_t* big_count,
-                                uint32_t* ticket, hipStream_t s);
+                                int32_t* bsum, ScanCtl ctl, int32_t* big_list, int32_t* big_excl,
+                                int32_t* big_count, uint32_t* ticket, hipStream_t s);
 hipError_t launch_sort_bands_emit(const int32_t* band_start, const int32_t* n_bands, int64_t max_bands,
                                   const unsigned long long* src, const int32_t* big_list, const int32_t* bpre,
                                   const uint32_t* ticket, const int2* band_pr, const EmitArgs& emit,
@@ -303,9 +339,6 @@ hipError_t launch_sort_bands_emit(const int32_t* band_start, const int32_t* n_ba
 hipError_t launch_big_bands(const int32_t* band_start, const int32_t* big_list, const int32_t* big_excl,
                             const int32_t* big_count, const unsigned long long* src, const int2* band_pr,
                             const EmitArgs& emit, int n_cu, hipStream_t s);
-// totals[0..2] (zeroed) += cells, spans, records: the sums of band_cnt over the bands.
-hipError_t launch_band_totals(const int2* band_cnt, const int32_t* n_bands, int32_t* totals, hipStream_t s);
-
 // ---- winding / mark / emit (a10 scan, a11); also writes each (path, row) bucket's record range
 hipError_t launch_mark_emit(const int32_t* skey, const int32_t* winding, const uint32_t* epath,
                             const uint32_t* rule, const uint32_t* fill, int64_t N, int w, int h,
@@ -384,8 +417,8 @@ struct DocDev {
 // The same from the bands' exclusive prefixes (bpre, total at [n_bands]), before the band sort:
 // every sorted path start is a band start or the end.
 hipError_t launch_doc_winding_base_bands(const int32_t* band_start, const int32_t* bpre, const int32_t* n_bands,
-                                         const int32_t* sstart, const int32_t* doc_first_path, uint32_t Np,
-                                         int32_t* wbase, hipStream_t s);
+                                         const int32_t* boff, const int32_t* bucket_base,
+                                         const int32_t* doc_first_path, uint32_t Np, int32_t* wbase, hipStream_t s);
 hipError_t launch_doc_winding_base(const int32_t* winding, const int32_t* sstart, const int32_t* doc_first_path,
                                    uint32_t Np, int32_t* wbase, hipStream_t s);
 
@@ -402,12 +435,24 @@ struct PaintArgs {
     const float* inv;            // 9 floats: inverse of the MVP's 2D projective part, rows
 };
 
+// What the frame reports: totals[0..2] (zeroed) += cells, spans, records over band_cnt (null: the
+// totals are there already), then src into host memory.  done: one zeroed u32.
+struct TallyArgs {
+    const int2* band_cnt;
+    const int32_t* n_bands;
+    int32_t* totals;
+    uint32_t* done;
+    SummarySrc src;
+    int32_t* out;
+    int blocks;                 // workgroups; 0: no tally
+};
+
 // ---- composite (a12).  w: the canvas, the widest one of a batch.  paint (optional): per-pixel gradient colours for the paths that have one.
 // cmask (optional, src-over only): the records' sample coverage (launch_cell_cover).
 hipError_t launch_composite(const uint32_t* records, const int2* brec, const int32_t* bucket_base,
                             const int2* prow, const uint32_t* fill, uint32_t Np, int w, int h, int compose,
                             uint8_t* image, hipStream_t s, int64_t rec_cap, const DocDev* docs = nullptr,
                             int n_docs = 0, int total_rows = 0, const PaintArgs* paint = nullptr,
-                            const unsigned long long* cmask = nullptr);
+                            const unsigned long long* cmask = nullptr, const TallyArgs* tally = nullptr);
 
 }  // namespace spr

@@ -186,7 +186,6 @@ struct spr_handle {
                                     // [16, 16 + kSummaryMax) the last frame's summary, [48, 73) the
                                     // MVP rows and the inverse of its 2D projective part, [73, 75)
                                     // the prediction's skip flag and arena count
-    DBuf<int32_t> summary;          // the frame summary on the device, copied to h_pinned + 16
     DBuf<unsigned long long> scan_ws;  // spr_scan_i32: tile statuses and the tile counter
     int32_t sum(int k) const { return h_pinned[16 + k]; }
     float* mvp_pinned() const { return reinterpret_cast<float*>(h_pinned + 48); }  // [48, 64): the MVP rows
@@ -281,16 +280,16 @@ struct ZeroLayout {
 ZeroLayout zero_layout(uint32_t C, uint32_t Np, int64_t N, int64_t NB) {
     ZeroLayout z;
     size_t o = 0;
-    z.ctr_a = o; o += 1;               // two u32 counters of the phase-A scans
-    z.st_count = o; o += spr::scan_tiles(std::max<int64_t>(C, 1));
-    z.st_pbase = o; o += spr::scan_tiles(std::max<uint32_t>(Np, 1));
+    z.ctr_a = o; o += 1;               // two u32 counters of the count pass's scans
+    z.st_count = o; o += (size_t)spr::count_tiles(C);
+    z.st_pbase = o; o += (size_t)spr::count_tiles(Np);
     z.a_words = o;
     z.ctr = o; o += 4;                 // eight u32 counters of the phase-B scans
-    z.totals = o; o += 2;              // int32 cells, spans, R, spare
+    z.totals = o; o += 2;              // int32 cells, spans, R, ended tally workgroups
     z.misc = o; o += 1;                // int32 error flag, big-band count
     z.chainctl = o; o += (kCcWords + 1) / 2;  // counters of the curve pass (int32)
-    z.st_hist = o; o += spr::scan_tiles(std::max<int64_t>(NB, 1));
-    z.st_band = o; o += spr::scan_tiles(std::max<int64_t>(NB, 1));
+    z.st_hist = o; o += (size_t)spr::bucket_band_tiles(NB);
+    z.st_band = o; o += (size_t)spr::bucket_band_tiles(NB);
     z.st_wind = o; o += (size_t)spr::max_bands_for(Np, N) + 1;  // statuses of the band-sum scan
     z.st_mark = o; o += spr::scan_tiles(std::max<int64_t>(N, 1));
     z.hist = o; o += (size_t)(NB + 2 + 1) / 2;  // NB+1 int32 (scanned in place)
@@ -329,10 +328,13 @@ spr::ScanCtl ctl_at(spr_handle* H, size_t st, size_t ctr_word, int counter) {
     return c;
 }
 
-// Gathers the frame's counters and starts their copy to the host (read once the stream is idle).
-void finish_summary(spr_handle* H, const spr::SummarySrc& S, hipStream_t s) {
-    SPR_HIP(spr::launch_gather_summary(S, H->summary.p, s));
-    SPR_HIP(hipMemcpyAsync(H->h_pinned + 16, H->summary.p, (size_t)S.n * 4, hipMemcpyDeviceToHost, s));
+// What the frame reports, summed and gathered by the composite's first workgroups: band_cnt is null
+// where mark + emit has left the totals already.  A workgroup of the tally reads about 1024 bands.
+spr::TallyArgs tally_args(spr_handle* H, const int2* band_cnt, const int32_t* n_bands, int64_t max_bands,
+                          int32_t* totals, const spr::SummarySrc& S) {
+    const int64_t blocks = band_cnt ? std::min<int64_t>(std::max<int64_t>(max_bands / 1024, 1), 64) : 1;
+    return spr::TallyArgs{band_cnt, n_bands, totals, reinterpret_cast<uint32_t*>(totals + 3), S, H->h_pinned + 16,
+                          (int)blocks};
 }
 
 void stage_mark(spr_handle* H, int idx) {
@@ -340,6 +342,26 @@ void stage_mark(spr_handle* H, int idx) {
     if ((int)H->ev_stage.size() <= idx) return;
     SPR_HIP(hipEventRecord(H->ev_stage[idx], H->stream));
     H->n_marks = idx + 1;
+}
+
+// Clears what the transform and the count pass start from, in one launch.
+void clear_prefix(spr_handle* H, int64_t control_words) {
+    spr::FrameInit init{};
+    init.fill[0] = {(uint32_t*)H->zero.p, control_words, nullptr, 0, 0, 0u};
+    init.fill[1] = {(uint32_t*)H->visible.p, H->Np, nullptr, 0, 0, 0u};
+    init.fill[2] = {(uint32_t*)H->row_lo.p, H->Np, nullptr, 0, 0, 0x7FFFFFFFu};
+    init.fill[3] = {(uint32_t*)H->row_hi.p, H->Np, nullptr, 0, 0, 0x80000000u};
+    init.n_fills = 4;
+    SPR_HIP(spr::launch_frame_init(init, H->stream));
+}
+
+// The count pass's arguments; counts, bucket bases and segments are scanned by the same launch.
+spr::CountArgs count_args(spr_handle* H, int rmax, spr::ScanCtl curves, spr::ScanCtl paths, const int2* pcanvas,
+                          int32_t* seg, int32_t* host) {
+    return spr::CountArgs{H->tpos.p, H->cpos.p, H->ctype.p, H->arcw(), H->cpath.p, H->visible.p, H->C, (int)H->w,
+                          (int)H->h, H->cuts.p, H->ncuts.p, H->counts.p, seg, spr::count_tiles(H->C), curves.status,
+                          curves.counter, H->row_lo.p, H->row_hi.p, H->Np, rmax, H->bucket_base.p, H->prow.p,
+                          spr::count_tiles(H->Np), paths.status, paths.counter, pcanvas, host};
 }
 
 // Entries per window of the curve pass.  A wave takes one window, and about 2,000 waves are
@@ -452,25 +474,18 @@ void run_frame(spr_handle* H, bool record_begin = true) {
     H->ncuts.ensure(std::max<uint32_t>(C, 1));
     H->counts.ensure((size_t)C + 1);
     H->seg.ensure((size_t)Np + 1);
-    SPR_HIP(spr::launch_fill_u32((uint32_t*)H->zero.p, 2 * (int64_t)za.a_words, 0u, s));
-    SPR_HIP(spr::launch_fill_u32((uint32_t*)H->visible.p, Np, 0u, s));
-    SPR_HIP(spr::launch_fill_u32((uint32_t*)H->row_lo.p, Np, 0x7FFFFFFFu, s));
-    SPR_HIP(spr::launch_fill_u32((uint32_t*)H->row_hi.p, Np, 0x80000000u, s));
+    clear_prefix(H, 2 * (int64_t)za.a_words);
     if (H->has_paint) SPR_HIP(hipMemcpyAsync(H->mvp_dev.p, H->mvp_pinned(), kMvpBytes, hipMemcpyHostToDevice, s));
     SPR_HIP(spr::launch_transform(H->pos.p, H->pos_path.p, P, H->mvp, w, h, H->tpos.p, H->visible.p,
                                   H->row_lo.p, H->row_hi.p, s));
     stage_mark(H, 1);
-    SPR_HIP(spr::launch_count(H->tpos.p, H->cpos.p, H->ctype.p, H->arcw(), H->cpath.p, H->visible.p, C, w, h,
-                              H->cuts.p, H->ncuts.p, H->counts.p, s));
+    // the two totals go straight to pinned memory
+    SPR_HIP(spr::launch_count(count_args(H, (h - 1) / 2, ctl_at(H, za.st_count, za.ctr_a, 0),
+                                         ctl_at(H, za.st_pbase, za.ctr_a, 1), nullptr, H->inj ? nullptr : H->seg.p,
+                                         H->h_pinned), s));
     stage_mark(H, 2);
-    SPR_HIP(spr::launch_scan_i32(H->counts.p, H->counts.p, C, ctl_at(H, za.st_count, za.ctr_a, 0), s));
-    SPR_HIP(spr::launch_bucket_counts(H->row_lo.p, H->row_hi.p, Np, (h - 1) / 2, H->bucket_base.p, H->prow.p, s));
-    SPR_HIP(spr::launch_scan_i32(H->bucket_base.p, H->bucket_base.p, Np, ctl_at(H, za.st_pbase, za.ctr_a, 1), s));
     int64_t N = 0;
-    if (!H->inj) {
-        SPR_HIP(spr::launch_path_segments(H->cpath.p, C, H->counts.p, Np, H->seg.p, s));
-        SPR_HIP(hipMemcpyAsync(H->h_pinned, H->counts.p + C, 4, hipMemcpyDeviceToHost, s));
-    } else {
+    if (H->inj) {
         N = (int64_t)H->inj_inter.size() / 2;
         std::vector<int32_t> hseg((size_t)Np + 1, 0);
         for (int64_t i = 0; i < N; ++i) {
@@ -485,7 +500,6 @@ void run_frame(spr_handle* H, bool record_begin = true) {
         }
         SPR_HIP(hipMemcpyAsync(H->seg.p, hseg.data(), hseg.size() * 4, hipMemcpyHostToDevice, s));
     }
-    SPR_HIP(hipMemcpyAsync(H->h_pinned + 1, H->bucket_base.p + Np, 4, hipMemcpyDeviceToHost, s));
     // ---- HOST SYNC: the count-then-write readback (scanline_rasterizer.cpp:355-356)
     SPR_HIP(hipStreamSynchronize(s));
     if (!H->inj) N = H->h_pinned[0];
@@ -564,17 +578,18 @@ void run_frame(spr_handle* H, bool record_begin = true) {
     stage_mark(H, 7);
     // ---- sort: bucket offsets, bands, scatter into band order, band sort in LDS
     if (N > 0) {
-        SPR_HIP(spr::launch_scan_i32(d_hist, d_hist, NB, ctl_at(H, z.st_hist, z.ctr, 0), s));
-        SPR_HIP(spr::launch_band_flags(H->bucket_base.p, Np, d_hist, H->bflag.p, s, H->band_window));
-        SPR_HIP(spr::launch_scan_i32(H->bflag.p, H->bflag.p, NB, ctl_at(H, z.st_band, z.ctr, 1), s));
-        SPR_HIP(spr::launch_band_emit(H->bflag.p, d_hist, (int32_t)NB, N, H->band_start.p, s, nullptr, nullptr,
-                                      H->bucket_base.p, Np, H->prow.p, narrow ? H->band_pr.p : nullptr,
-                                      narrow ? H->band_path.p : nullptr));
+        SPR_HIP(spr::launch_bands(spr::BandArgs{d_hist, (int32_t)NB, nullptr, H->bucket_base.p, Np, H->prow.p,
+                                                H->band_window, H->bflag.p, H->band_start.p,
+                                                narrow ? H->band_pr.p : nullptr, narrow ? H->band_path.p : nullptr,
+                                                nullptr, nullptr, H->zero.p + z.st_hist, H->zero.p + z.st_band,
+                                                ctl_at(H, z.st_hist, z.ctr, 0).counter}, s));
         SPR_HIP(spr::launch_bucket_scatter(H->key.p, H->wn.p, H->epath.p, N, H->bucket_base.p, H->prow.p,
                                            H->bflag.p, H->band_start.p, d_fill, d_bsum, H->sbig.p, d_err, s, nullptr,
                                            narrow, narrow && gen));
-        // each band's exclusive prefix of the winding changes (total at [n_bands])
-        SPR_HIP(spr::launch_scan_i32(d_bsum, d_bsum, max_bands, ctl_at(H, z.st_wind, z.ctr, 2), s, H->bflag.p + NB));
+        // each band's exclusive prefix of the winding changes (total at [n_bands]); narrow frames scan
+        // them as they classify the bands
+        if (!narrow)
+            SPR_HIP(spr::launch_scan_i32(d_bsum, d_bsum, max_bands, ctl_at(H, z.st_wind, z.ctr, 2), s, H->bflag.p + NB));
     }
     stage_mark(H, 8);
     // narrow frames fuse mark + emit into the band sort: records of band t at [2 * start, ...)
@@ -588,7 +603,8 @@ void run_frame(spr_handle* H, bool record_begin = true) {
             // the oversized bands (queued by the classify pass) are sorted and emitted on the second
             // stream, followed there by the bands of up to 512 words, beside the longer bands
             hipStream_t s2 = big_band_stream(H, N, Np);
-            SPR_HIP(spr::launch_band_classify(H->band_start.p, H->bflag.p + NB, max_bands, d_bsum, H->big_list.p,
+            SPR_HIP(spr::launch_band_classify(H->band_start.p, H->bflag.p + NB, max_bands, d_bsum,
+                                              ctl_at(H, z.st_wind, z.ctr, 2), H->big_list.p,
                                               H->big_list.p + max_bands, d_bigcount, ticket, s));
             if (s2 != s) {
                 SPR_HIP(hipEventRecord(H->ev_sfork, s));
@@ -602,7 +618,6 @@ void run_frame(spr_handle* H, bool record_begin = true) {
                 SPR_HIP(hipEventRecord(H->ev_sjoin, s2));  // after the short bands' sort on s2
                 SPR_HIP(hipStreamWaitEvent(s, H->ev_sjoin, 0));
             }
-            SPR_HIP(spr::launch_band_totals(H->band_cnt.p, H->bflag.p + NB, d_totals, s));
         } else {
             SPR_HIP(spr::launch_sort_bands(H->band_start.p, H->bflag.p + NB, max_bands, H->sbig.p, H->skey.p,
                                            keep ? H->sidx.p : nullptr, H->winding.p, H->big_list.p,
@@ -629,12 +644,7 @@ void run_frame(spr_handle* H, bool record_begin = true) {
     H->last_fused = narrow;
     H->last_packed = narrow && gen;
     stage_mark(H, 11);
-    // ---- composite
-    spr::PaintArgs pa;
-    SPR_HIP(spr::launch_composite(H->crec.p, d_brec, H->bucket_base.p, H->prow.p, H->fill.p, Np, w, h,
-                                  (int)H->opts.compose, H->image.p, s, (int64_t)(2 * n1), nullptr, 0, 0,
-                                  paint_args(H, pa), aa ? H->cmask.p : nullptr));
-    stage_mark(H, 12);
+    // ---- composite, and what the frame reports
     spr::SummarySrc S{};
     S.n = kSumCount;
     S.p[kSumCells] = d_totals;
@@ -646,7 +656,13 @@ void run_frame(spr_handle* H, bool record_begin = true) {
     S.p[kSumLongBands] = reinterpret_cast<const int32_t*>(ctl_at(H, z.st_wind, z.ctr, 4).counter + 1);
     S.p[kSumBigBands] = d_bigcount;
     S.p[kSumTotal] = H->inj ? nullptr : H->counts.p + C;
-    finish_summary(H, S, s);
+    const spr::TallyArgs T = tally_args(H, N > 0 && narrow ? H->band_cnt.p : nullptr, H->bflag.p + NB, max_bands,
+                                        d_totals, S);
+    spr::PaintArgs pa;
+    SPR_HIP(spr::launch_composite(H->crec.p, d_brec, H->bucket_base.p, H->prow.p, H->fill.p, Np, w, h,
+                                  (int)H->opts.compose, H->image.p, s, (int64_t)(2 * n1), nullptr, 0, 0,
+                                  paint_args(H, pa), aa ? H->cmask.p : nullptr, &T));
+    stage_mark(H, 12);
     SPR_HIP(hipEventRecord(H->ev_end, s));
     H->frame_done = true;
 }
@@ -681,15 +697,15 @@ LearnedLayout learned_layout(uint32_t C, uint32_t Np, int64_t nb_budget, int64_t
     z.ctl = o; o += 2;          // int32 live entries, over-budget flag, overflowing paths, spare
     z.misc = o; o += 1;         // int32 error flags, big-band count
     z.capr = o; o += 1;         // int32 predicted record total, spare
-    z.totals = o; o += 2;       // int32 cells, spans, R, spare
+    z.totals = o; o += 2;       // int32 cells, spans, R, ended tally workgroups
     z.slots = o; o += 2;        // int32 sorted entries, bands, spare x2
     z.bound = o; o += 1;        // u64 upper bound of the intersections
     z.chainctl = o; o += (kCcWords + 1) / 2;
-    z.st_count = o; o += spr::scan_tiles(std::max<uint32_t>(C, 1));
+    z.st_count = o; o += (size_t)spr::count_tiles(C);
     z.st_arena = o; o += spr::scan_tiles(std::max<uint32_t>(Np, 1));
-    z.st_pb = o; o += spr::scan_tiles(std::max<uint32_t>(Np, 1));
-    z.st_hist = o; o += spr::scan_tiles(std::max<int64_t>(nb_budget, 1));
-    z.st_band = o; o += spr::scan_tiles(std::max<int64_t>(nb_budget, 1));
+    z.st_pb = o; o += (size_t)spr::count_tiles(Np);
+    z.st_hist = o; o += (size_t)spr::bucket_band_tiles(nb_budget);
+    z.st_band = o; o += (size_t)spr::bucket_band_tiles(nb_budget);
     z.st_wind = o; o += (size_t)spr::max_bands_for(Np, std::max<int64_t>(n_budget, 1)) + 1;  // band-sum scan
     z.st_mark = o; o += spr::scan_tiles(std::max<int64_t>(n_budget, 1));
     z.total = o;
@@ -772,10 +788,7 @@ void run_learned_frame(spr_handle* H) {
     // phase 1: transform; the prediction on the second stream, the exact count on the first
     LearnedLayout z = learned_layout(C, Np, nb_budget, std::max<int64_t>(H->lb_n, 1));
     H->zero.ensure(z.total);
-    SPR_HIP(spr::launch_fill_u32((uint32_t*)H->zero.p, 2 * (int64_t)z.total, 0u, s));
-    SPR_HIP(spr::launch_fill_u32((uint32_t*)H->visible.p, Np, 0u, s));
-    SPR_HIP(spr::launch_fill_u32((uint32_t*)H->row_lo.p, Np, 0x7FFFFFFFu, s));
-    SPR_HIP(spr::launch_fill_u32((uint32_t*)H->row_hi.p, Np, 0x80000000u, s));
+    clear_prefix(H, 2 * (int64_t)z.total);
     // the prediction is a function of the scene, the MVP and the model: it runs after a change of
     // one of them and is otherwise left out (its outputs still hold); a captured frame with it
     // reads the same decision from the pinned words at every replay
@@ -808,11 +821,9 @@ void run_learned_frame(spr_handle* H) {
         SPR_HIP(spr::launch_scan_i32(H->arena.p, H->arena.p, Np, ctl_at(H, z.st_arena, z.counters, kLcArena), s2,
                                      d_arena_n));
     }
-    SPR_HIP(spr::launch_count(H->tpos.p, H->cpos.p, H->ctype.p, H->arcw(), H->cpath.p, H->visible.p, C, w, h, H->cuts.p,
-                              H->ncuts.p, H->counts.p, s, pcv));
+    SPR_HIP(spr::launch_count(count_args(H, rmax, ctl_at(H, z.st_count, z.counters, kLcCount),
+                                         ctl_at(H, z.st_pb, z.counters, kLcBucketBase), pcv, H->seg.p, nullptr), s));
     stage_mark(H, 2);
-    SPR_HIP(spr::launch_scan_i32(H->counts.p, H->counts.p, C, ctl_at(H, z.st_count, z.counters, kLcCount), s));
-    SPR_HIP(spr::launch_path_segments(H->cpath.p, C, H->counts.p, Np, H->seg.p, s));
     // the prediction's paths that overflowed their capacity (statistics only): on the second stream
     // once the per-path counts exist, unless this frame reads the prediction back (and re-lays the
     // control region), in which case they are counted at its end
@@ -824,9 +835,6 @@ void run_learned_frame(spr_handle* H) {
                                           reinterpret_cast<int32_t*>(H->zero.p + z.ctl) + 2, s2, d_skip));
     }
     if (s2 != s) SPR_HIP(hipEventRecord(H->ev_pjoin, s2));
-    SPR_HIP(spr::launch_bucket_counts(H->row_lo.p, H->row_hi.p, Np, rmax, H->bucket_base.p, H->prow.p, s, pcv));
-    SPR_HIP(spr::launch_scan_i32(H->bucket_base.p, H->bucket_base.p, Np, ctl_at(H, z.st_pb, z.counters, kLcBucketBase),
-                                 s));
     bool joined = s2 == s;
     if (H->need_prediction && !use_model) H->need_prediction = false;  // a batch without a model: no prediction
     if (H->need_prediction) {
@@ -913,26 +921,20 @@ void run_learned_frame(spr_handle* H) {
     }
     stage_mark(H, 6);
     stage_mark(H, 7);
-    SPR_HIP(spr::launch_scan_i32(H->hist_l.p, H->hist_l.p, nb_budget, ctl_at(H, z.st_hist, z.counters, kLcHist), s,
-                                 d_nb, d_nsorted));
-    SPR_HIP(spr::launch_band_flags(H->bucket_base.p, Np, H->hist_l.p, H->bflag.p, s, H->band_window));
-    SPR_HIP(spr::launch_scan_i32(H->bflag.p, H->bflag.p, nb_budget, ctl_at(H, z.st_band, z.counters, kLcBandFlags),
-                                 s, d_nb, d_nbands));
-    SPR_HIP(spr::launch_band_emit(H->bflag.p, H->hist_l.p, (int32_t)nb_budget, nl, H->band_start.p, s, d_nb,
-                                  d_nsorted, H->bucket_base.p, Np, H->prow.p, narrow ? H->band_pr.p : nullptr,
-                                  narrow ? H->band_path.p : nullptr));
+    SPR_HIP(spr::launch_bands(spr::BandArgs{H->hist_l.p, (int32_t)nb_budget, d_nb, H->bucket_base.p, Np, H->prow.p,
+                                            H->band_window, H->bflag.p, H->band_start.p,
+                                            narrow ? H->band_pr.p : nullptr, narrow ? H->band_path.p : nullptr,
+                                            d_nsorted, d_nbands, H->zero.p + z.st_hist, H->zero.p + z.st_band,
+                                            ctl_at(H, z.st_hist, z.counters, kLcHist).counter}, s));
     SPR_HIP(spr::launch_bucket_scatter(H->key.p, H->wn.p, H->epath.p, nl, H->bucket_base.p, H->prow.p,
                                        H->bflag.p, H->band_start.p, H->fill_l.p, H->bsum_l.p, H->sbig.p, d_err, s,
                                        d_live, narrow, narrow));
-    SPR_HIP(spr::launch_scan_i32(H->bsum_l.p, H->bsum_l.p, max_bands, ctl_at(H, z.st_wind, z.counters, kLcBandSums),
-                                 s, d_nbands));
-    // the sorted start of each path: read by the documents' winding bases and the separate mark + emit
-    if (H->batch || !narrow) SPR_HIP(spr::launch_sorted_starts(H->hist_l.p, H->bucket_base.p, Np, H->sstart.p, s));
-    // documents of a batch scan their winding numbers from their own first entry: with the fused
-    // mark + emit that base comes from the band prefixes, before the sort
-    if (H->batch && narrow)
-        SPR_HIP(spr::launch_doc_winding_base_bands(H->band_start.p, H->bsum_l.p, d_nbands, H->sstart.p,
-                                                   H->doc_first.p, Np, H->wbase.p, s));
+    if (!narrow) {
+        SPR_HIP(spr::launch_scan_i32(H->bsum_l.p, H->bsum_l.p, max_bands,
+                                     ctl_at(H, z.st_wind, z.counters, kLcBandSums), s, d_nbands));
+        // the sorted start of each path, for the documents' winding bases and the separate mark + emit
+        SPR_HIP(spr::launch_sorted_starts(H->hist_l.p, H->bucket_base.p, Np, H->sstart.p, s));
+    }
     stage_mark(H, 8);
     const spr::EmitArgs E{H->crec.p, H->brec_l.p, H->band_cnt.p, H->band_path.p, H->bucket_base.p, H->rule.p,
                           pcv, H->batch ? H->wbase.p : nullptr, w, h};
@@ -941,8 +943,14 @@ void run_learned_frame(spr_handle* H) {
         // the oversized bands (queued by the classify pass) are sorted and emitted on the second
         // stream, followed there by the bands of up to 512 words, beside the longer bands
         hipStream_t sb = big_band_stream(H, nl, Np);
-        SPR_HIP(spr::launch_band_classify(H->band_start.p, d_nbands, max_bands, H->bsum_l.p, H->big_list.p,
+        SPR_HIP(spr::launch_band_classify(H->band_start.p, d_nbands, max_bands, H->bsum_l.p,
+                                          ctl_at(H, z.st_wind, z.counters, kLcBandSums), H->big_list.p,
                                           H->big_list.p + max_bands, d_bigcount, ticket, s));
+        // documents of a batch scan their winding numbers from their own first entry: that base comes
+        // from the band prefixes, before the sort
+        if (H->batch)
+            SPR_HIP(spr::launch_doc_winding_base_bands(H->band_start.p, H->bsum_l.p, d_nbands, H->hist_l.p,
+                                                       H->bucket_base.p, H->doc_first.p, Np, H->wbase.p, s));
         if (sb != s) {
             SPR_HIP(hipEventRecord(H->ev_sfork, s));
             SPR_HIP(hipStreamWaitEvent(sb, H->ev_sfork, 0));
@@ -955,7 +963,6 @@ void run_learned_frame(spr_handle* H) {
             SPR_HIP(hipEventRecord(H->ev_sjoin, sb));  // after the short bands' sort on sb
             SPR_HIP(hipStreamWaitEvent(s, H->ev_sjoin, 0));
         }
-        SPR_HIP(spr::launch_band_totals(H->band_cnt.p, d_nbands, d_totals, s));
     } else {
         SPR_HIP(spr::launch_sort_bands(H->band_start.p, d_nbands, max_bands, H->sbig.p, H->skey.p,
                                        debug ? H->sidx.p : nullptr, H->winding.p, H->big_list.p,
@@ -976,11 +983,6 @@ void run_learned_frame(spr_handle* H) {
                                       H->brec_l.p, s, d_nsorted, H->sstart.p, Np, nr, d_err, pcv,
                                       H->batch ? H->wbase.p : nullptr));
     stage_mark(H, 11);
-    spr::PaintArgs pa;
-    SPR_HIP(spr::launch_composite(H->crec.p, H->brec_l.p, H->bucket_base.p, H->prow.p, H->fill.p, Np,
-                                  H->batch ? H->max_w : w, h, (int)H->opts.compose, H->image.p, s, rec_cap, H->batch ? H->docs.p : nullptr,
-                                  (int)H->n_docs, H->total_rows, paint_args(H, pa)));
-    stage_mark(H, 12);
     if (!joined) SPR_HIP(hipStreamWaitEvent(s, H->ev_pjoin, 0));
     if (use_model && predict && !ovf_side)
         SPR_HIP(spr::launch_path_overflow(H->seg.p, H->capn.p, H->visible.p, Np, d_novf, s, d_skip));
@@ -1001,7 +1003,12 @@ void run_learned_frame(spr_handle* H) {
     S.p[kSumArena] = H->arena.p + Np;
     S.p[kSumSorted] = d_nsorted;
     S.p[kSumCapR] = d_capr;
-    finish_summary(H, S, s);
+    const spr::TallyArgs T = tally_args(H, narrow ? H->band_cnt.p : nullptr, d_nbands, max_bands, d_totals, S);
+    spr::PaintArgs pa;
+    SPR_HIP(spr::launch_composite(H->crec.p, H->brec_l.p, H->bucket_base.p, H->prow.p, H->fill.p, Np,
+                                  H->batch ? H->max_w : w, h, (int)H->opts.compose, H->image.p, s, rec_cap, H->batch ? H->docs.p : nullptr,
+                                  (int)H->n_docs, H->total_rows, paint_args(H, pa), nullptr, &T));
+    stage_mark(H, 12);
     if (H->capturing) return;
     SPR_HIP(hipEventRecord(H->ev_end, s));
     learned_finish(H);
@@ -1307,7 +1314,6 @@ int spr_create(uint32_t width, uint32_t height, const spr_opts* opts, spr_handle
         for (auto& e : H->ev_stage) SPR_HIP(hipEventCreate(&e));
         SPR_HIP(hipHostMalloc((void**)&H->h_pinned, 512, hipHostMallocDefault));
         std::memset(H->h_pinned, 0, 512);
-        H->summary.ensure(spr::kSummaryMax);
         H->mvp_dev.ensure(32);  // before any capture: a frame never allocates it
         const float id[16] = {1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1};
         std::memcpy(H->mvp.m, id, sizeof(id));
@@ -1341,7 +1347,6 @@ int spr_destroy(spr_handle* H) {
     H->pcurve.release(); H->feat.release(); H->pred.release(); H->train_feat.release(); H->train_tgt.release();
     H->arena.release(); H->capn.release(); H->sstart.release();
     H->hist_l.release(); H->fill_l.release(); H->bsum_l.release(); H->brec_l.release(); H->pbound.release();
-    H->summary.release();
     H->scan_ws.release();
     H->inj_rec.release();
     H->mvp_dev.release();
