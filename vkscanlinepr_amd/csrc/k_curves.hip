@@ -8,12 +8,12 @@
 // (ties to x, :338) followed by its equal-t OR-merge (:361-375).  This file keeps every float
 // operation of the reference and only changes who computes what.
 //
-// The entries of a frame are cut into windows, and one wave takes the pieces whose first entry
+// The entries of a frame are cut into windows, and one workgroup takes the pieces whose first entry
 // lies in its window, whole, from the curve data to the fragment keys:
 //
-//  1. One lane per curve walks its pieces (their grid ranges, flagged end parameters and places)
+//  1. One lane per curve, of one wave, walks its pieces (their grid ranges, flagged end parameters and places)
 //     into a table in LDS.
-//  2. The chains are cut into segments of a few crossings, one lane each.  A chain carries only
+//  2. The chains are cut into segments of a few crossings, one thread each.  A chain carries only
 //     one value from crossing to crossing, the last parameter with its two low bits replaced, so
 //     a segment that guesses that value right computes exactly the chain's results.  It guesses by
 //     solving the crossings before it, the first of them from the piece's start: a bisection
@@ -48,22 +48,24 @@ namespace {
 
 constexpr int kBigPiece = kCurvePieceMax;       // longer pieces take a workgroup
 constexpr int kCap = kCurveWindowMax + kBigPiece;  // LDS slots: a window plus its last piece's overhang
-constexpr int kLanes = 64;                      // curves of a batch
+constexpr int kLanes = 64;                      // curves of a batch: one wave walks them
+constexpr int kThreads = 256;                   // of a window
+constexpr int kWaves = kThreads / 64;
 constexpr int kSlots = 5 * kLanes;              // piece slots: piece k of lane l's curve at 5 l + k
-constexpr int kPerLane = kBigPiece / kLanes;    // merged slots per lane and step
+constexpr int kPerLane = kBigPiece / kThreads;  // merged slots per thread and step
 constexpr int kBigThreads = 256;
 constexpr int kStage = 4096;                    // big pieces up to this many entries stay in LDS
 // Crossings solved before a segment to guess its start, the least length of a segment, and the
 // segments that a batch is cut into (besides one per chain).
-constexpr int kWarm = 4, kWarm8 = 8, kWarm16 = 16, kSegMin = 4, kSegTarget = 56;
-constexpr int kSegs = 768;
+constexpr int kWarm = 4, kWarm8 = 8, kWarm16 = 16, kSegMin = 4, kSegTarget = 112;
+constexpr int kSegs = 832;
 // chains are 2 * 320; the segments after a chain's first hold X / kSegTarget or more of the
 // batch's X crossings in all but one of a chain, and only chains of 1.5 of them have any
 static_assert(2 * kSlots + kSegTarget + (2 * kSegTarget) / 3 <= kSegs, "segment list");
 static_assert(2 * kSlots <= 1024, "chain numbers of 10 bits");
 constexpr uint32_t kNoPiece = 0xFFFFu;          // slot field of an empty piece slot
 static_assert(kFrag == 2, "piece records keep only the sign of the grid step");
-static_assert(kCap <= 2048 && kBigPiece % kLanes == 0, "slots of a batch");
+static_assert(kCap <= 2048 && kBigPiece % kThreads == 0, "slots of a batch");
 
 // Bits of a piece record's second word above ny.
 constexpr uint32_t kPwX = 1u << 22, kPwY = 1u << 23;            // grid step -2 on x, y
@@ -322,7 +324,9 @@ struct CurveBatch {
     unsigned long long starts[kCap / 64];  // bit per entry slot: a piece starts there
     uint16_t starts_before[kCap / 64];
     uint16_t head[2 * kSlots];           // length of each chain's first segment
-    uint32_t seg[kSegs];                 // chain | segment << 10 | crossings to guess its start from << 16
+    uint32_t seg[kSegs];                 // chain | segment << 10 | crossings to guess its start from << 20
+    int n_segs;
+    int n_pieces, longest, n_slots, crossings;  // of the batch
 };
 
 // The piece that entry slot e lies in or after, -1 before the first.
@@ -339,9 +343,9 @@ __device__ inline int piece_of(const CurveBatch& B, int e) {
 // goes both ways is merged by the sequential walk, through scratch.
 __device__ inline void merge_slots(CurveBatch& B, int s0, int s1, int longest, bool any_falls,
                                    uint32_t* __restrict__ scratch) {
-    const int lane = threadIdx.x & 63;
+    const int tid = threadIdx.x;
     if (any_falls) {
-        for (int p = lane; p < kSlots; p += kLanes) {
+        for (int p = tid; p < kSlots; p += kThreads) {
             const uint32_t w0 = B.pa[p].x, w1 = B.pa[p].y;
             const int base = (int)(w0 & 0xFFFFu), nx = (int)(w0 >> 16), ny = (int)(w1 & 0xFFFFu);
             if (base < s0 || base >= s1 || (w1 & (kPwFalls | kPwRises)) != (kPwFalls | kPwRises)) continue;
@@ -359,16 +363,16 @@ __device__ inline void merge_slots(CurveBatch& B, int s0, int s1, int longest, b
             }
         }
         __threadfence_block();
-        wave_sync();
+        __syncthreads();
     }
     float v[kPerLane];
     int from[kPerLane], len[kPerLane], rank[kPerLane], dest[kPerLane];
     uint32_t le = 0;  // bit j: rank counts equal values too
 #pragma unroll
     for (int j = 0; j < kPerLane; ++j) {
-        const int e = s0 + lane + kLanes * j;
+        const int e = s0 + tid + kThreads * j;
         v[j] = 0.0f; from[j] = 0; len[j] = 0; rank[j] = 0; dest[j] = -1;
-        if (s0 + kLanes * j >= s1) continue;
+        if (s0 + kThreads * j >= s1) continue;
         if (e < s1) {
             const int p = piece_of(B, e);
             if (p < 0) continue;
@@ -404,7 +408,7 @@ __device__ inline void merge_slots(CurveBatch& B, int s0, int s1, int longest, b
     for (int bit = longest ? 1 << (31 - __clz(longest)) : 0; bit; bit >>= 1) {
 #pragma unroll
         for (int j = 0; j < kPerLane; ++j) {
-            if (s0 + kLanes * j >= s1) continue;
+            if (s0 + kThreads * j >= s1) continue;
             const int r = rank[j] + bit;
             if (r <= len[j]) {
                 const float x = B.v[from[j] + r - 1];
@@ -412,11 +416,11 @@ __device__ inline void merge_slots(CurveBatch& B, int s0, int s1, int longest, b
             }
         }
     }
-    wave_sync();
+    __syncthreads();
 #pragma unroll
     for (int j = 0; j < kPerLane; ++j)
         if (dest[j] >= 0) B.v[dest[j] + rank[j]] = v[j];
-    wave_sync();
+    __syncthreads();
 }
 
 // An entry without a segment: the off-canvas cell, no winding change.
@@ -474,10 +478,18 @@ __device__ inline void seg_range(const CurveBatch& B, int ch, int j, int n, int 
     }
 }
 
-// One wave per window of K.window entries.  first[b] is the curve that holds entry b * window.
-__global__ __launch_bounds__(kLanes) void k_curves(const CurveArgs K, const FragArgs A) {
+// One workgroup per window of K.window entries.  first[b] is the curve that holds entry b * window.
+// Its span is latency (loads behind each other, chains of dependent solves, LDS searches), so the
+// waves that fit a CU decide its rate: one wave a window left 6 waves on a CU (23 KB of LDS each,
+// 160 VGPRs); four waves to the same LDS put 24 there (6 per SIMD, at most 80 VGPRs).  Four waves
+// also take a window of 1024 entries in about the time that one took 128, with a quarter of
+// the speculative solves per entry.  Frames in turn on three handles, us a frame, one wave and four:
+// 0.8 M entries on a few long curves 203 -> 134, 1.9 M on 20,000 glyphs 299 -> 261.  Two waves a
+// window: 138, 255; four to five per SIMD (96 to 128 VGPRs): 2 to 15% slower.
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6)))
+void k_curves(const CurveArgs K, const FragArgs A) {
     __shared__ CurveBatch B;
-    const int lane = threadIdx.x & 63;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t total = K.n_dev ? min((int64_t)*K.n_dev, K.n) : K.n;
     const int64_t wb64 = (int64_t)blockIdx.x * K.window;
     if (wb64 >= total) return;
@@ -509,86 +521,95 @@ __global__ __launch_bounds__(kLanes) void k_curves(const CurveArgs K, const Frag
         }
         const int bb0 = max(wb, bo);  // the entry of slot 0
         const bool mine = o0 < wend && o1 > o0 && o1 > wb;
-        if (lane < kCap / 64) B.starts[lane] = 0ull;
+        if (wave == 0) {
+            if (lane < kCap / 64) B.starts[lane] = 0ull;
 #pragma unroll
-        for (int k = 0; k < 5; ++k) { B.pa[5 * lane + k].x = kNoPiece; B.pa[5 * lane + k].y = 0u; }
-        wave_sync();
-        int np = 0, x_lane = 0, longest = 0, n_slots = 0;
-        if (mine) {
-            const uint32_t path = A.cpath[c];
-            int w = A.w, h = A.h;
-            if (A.pcanvas) { const int2 cw = A.pcanvas[path]; w = cw.x; h = cw.y; }
-            const uint32_t type = A.ctype[c];
-            const CurvePts cv = load_curve(A.tpos, A.cpos[c], type, A.cweight, (uint32_t)c);
-            const int2 pr = A.prow[path];
-            const int bb = A.bucket_base[path];
-            B.cx[lane] = make_float4(cv.x[0], cv.x[1], cv.x[2], cv.x[3]);
-            B.cy[lane] = make_float4(cv.y[0], cv.y[1], cv.y[2], cv.y[3]);
-            B.cm[lane] = make_int4(bb, pr.x, pr.y, (int)path);
-            B.canvas[lane] = make_int2(w, h);
-            int written = o0, prev = -1;  // prev: the piece before, when it is in the batch
-            bool needs = false;           // a piece of the batch ends at the first entry of one outside
-            PieceGeom after;
-            after.nx = after.ny = 0; after.t0 = after.t1 = after.x0 = 0.0f;
-            int needs_at = 0;
-            walk_pieces(cv, K.cuts[c], K.ncuts[c], o0, o1, w, h, [&](int k, const PieceGeom& g) {
-                if (!g.ok) { prev = -1; return; }
-                written = g.base + g.n();
-                const bool starts = g.base >= wb && g.base < wend;
-                const bool in = starts && g.n() <= kBigPiece;
-                const int at = 5 * lane + k;
-                if (prev >= 0) {
-                    if (in) B.tend[prev] = -1.0f;
-                    else { needs = true; needs_at = prev; after = g; }
-                }
-                prev = in ? at : -1;
-                if (starts && !in) K.big[atomicAdd(K.big_count, 1)] = (int32_t)(5 * c + k);
-                if (in) {
-                    const int rel = g.base - bb0;
-                    // a grid line is only meaningful (and then in [0, 16386]) on an axis with crossings
-                    B.pa[at] = make_uint4((uint32_t)rel | ((uint32_t)g.nx << 16),
-                                          (uint32_t)g.ny | ((uint32_t)lane << 16) | (g.xneg ? kPwX : 0u) |
-                                              (g.yneg ? kPwY : 0u) | (type_code(type) << kPwType),
-                                          (g.nx ? (uint32_t)(int)g.x0 : 0u) | ((g.ny ? (uint32_t)(int)g.y0 : 0u) << 16),
-                                          fbits(g.t1));
-                    B.tend[at] = 1.0f;
-                    B.v[rel] = g.t0;
-                    atomicOr(&B.starts[rel >> 6], 1ull << (rel & 63));
-                    ++np;
-                    x_lane += g.nx + g.ny;
-                    longest = max(longest, max(g.nx, g.ny));
-                    n_slots = rel + g.n();
-                }
-            });
-            // counted but not written (the passes round differently only far outside any canvas)
-            if (o0 >= wb)
-                for (int i = written; i < o1; ++i) store_gap(A, i, (int)c, path, (uint32_t)bb, pr);
-            if (needs) B.tend[needs_at] = first_entry_t(cv, after);
-        }
-        const int before = wave_inclusive_add(np);
-        if (__builtin_amdgcn_readlane(before, 63) == 0) continue;
+            for (int k = 0; k < 5; ++k) { B.pa[5 * lane + k].x = kNoPiece; B.pa[5 * lane + k].y = 0u; }
+            wave_sync();
+            int np = 0, x_lane = 0, longest = 0, n_slots = 0;
+            uint32_t in_set = 0;  // bit k: piece k of the lane's curve is in the batch
+            if (mine) {
+                const uint32_t path = A.cpath[c];
+                int w = A.w, h = A.h;
+                if (A.pcanvas) { const int2 cw = A.pcanvas[path]; w = cw.x; h = cw.y; }
+                const uint32_t type = A.ctype[c];
+                const CurvePts cv = load_curve(A.tpos, A.cpos[c], type, A.cweight, (uint32_t)c);
+                const int2 pr = A.prow[path];
+                const int bb = A.bucket_base[path];
+                B.cx[lane] = make_float4(cv.x[0], cv.x[1], cv.x[2], cv.x[3]);
+                B.cy[lane] = make_float4(cv.y[0], cv.y[1], cv.y[2], cv.y[3]);
+                B.cm[lane] = make_int4(bb, pr.x, pr.y, (int)path);
+                B.canvas[lane] = make_int2(w, h);
+                int written = o0, prev = -1;  // prev: the piece before, when it is in the batch
+                bool needs = false;           // a piece of the batch ends at the first entry of one outside
+                PieceGeom after;
+                after.nx = after.ny = 0; after.t0 = after.t1 = after.x0 = 0.0f;
+                int needs_at = 0;
+                walk_pieces(cv, K.cuts[c], K.ncuts[c], o0, o1, w, h, [&](int k, const PieceGeom& g) {
+                    if (!g.ok) { prev = -1; return; }
+                    written = g.base + g.n();
+                    const bool starts = g.base >= wb && g.base < wend;
+                    const bool in = starts && g.n() <= kBigPiece;
+                    const int at = 5 * lane + k;
+                    if (prev >= 0) {
+                        if (in) B.tend[prev] = -1.0f;
+                        else { needs = true; needs_at = prev; after = g; }
+                    }
+                    prev = in ? at : -1;
+                    if (starts && !in) K.big[atomicAdd(K.big_count, 1)] = (int32_t)(5 * c + k);
+                    if (in) {
+                        const int rel = g.base - bb0;
+                        // a grid line is only meaningful (and then in [0, 16386]) on an axis with crossings
+                        B.pa[at] = make_uint4((uint32_t)rel | ((uint32_t)g.nx << 16),
+                                              (uint32_t)g.ny | ((uint32_t)lane << 16) | (g.xneg ? kPwX : 0u) |
+                                                  (g.yneg ? kPwY : 0u) | (type_code(type) << kPwType),
+                                              (g.nx ? (uint32_t)(int)g.x0 : 0u) | ((g.ny ? (uint32_t)(int)g.y0 : 0u) << 16),
+                                              fbits(g.t1));
+                        B.tend[at] = 1.0f;
+                        B.v[rel] = g.t0;
+                        atomicOr(&B.starts[rel >> 6], 1ull << (rel & 63));
+                        ++np;
+                        in_set |= 1u << k;
+                        x_lane += g.nx + g.ny;
+                        longest = max(longest, max(g.nx, g.ny));
+                        n_slots = rel + g.n();
+                    }
+                });
+                // counted but not written (the passes round differently only far outside any canvas)
+                if (o0 >= wb)
+                    for (int i = written; i < o1; ++i) store_gap(A, i, (int)c, path, (uint32_t)bb, pr);
+                if (needs) B.tend[needs_at] = first_entry_t(cv, after);
+            }
+            const int before = wave_inclusive_add(np);
+            const int x_upto = wave_inclusive_add(x_lane);
+            int rank = before - np;
+            for (; in_set; in_set &= in_set - 1) B.by_rank[rank++] = (uint16_t)(5 * lane + __ffs((int)in_set) - 1);
 #pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) {
-            longest = max(longest, __shfl_xor(longest, o));
-            n_slots = max(n_slots, __shfl_xor(n_slots, o));
+            for (int o = 32; o >= 1; o >>= 1) {
+                longest = max(longest, __shfl_xor(longest, o));
+                n_slots = max(n_slots, __shfl_xor(n_slots, o));
+            }
+            wave_sync();
+            const int here = lane < kCap / 64 ? (int)__popcll(B.starts[lane]) : 0;
+            const int upto = wave_inclusive_add(here);
+            if (lane < kCap / 64) B.starts_before[lane] = (uint16_t)(upto - here);
+            if (lane == 63) {
+                B.n_pieces = before; B.crossings = x_upto; B.longest = longest; B.n_slots = n_slots;
+                B.n_segs = 0;
+            }
         }
-        longest = __builtin_amdgcn_readfirstlane(longest);
-        n_slots = __builtin_amdgcn_readfirstlane(n_slots);
-        const int crossings = __builtin_amdgcn_readlane(wave_inclusive_add(x_lane), 63);
-        wave_sync();
-        const int here = lane < kCap / 64 ? (int)__popcll(B.starts[lane]) : 0;
-        const int upto = wave_inclusive_add(here);
-        if (lane < kCap / 64) B.starts_before[lane] = (uint16_t)(upto - here);
+        __syncthreads();
+        if (B.n_pieces == 0) { __syncthreads(); continue; }
+        const int longest = __builtin_amdgcn_readfirstlane(B.longest), n_slots = __builtin_amdgcn_readfirstlane(B.n_slots);
+        const int crossings = __builtin_amdgcn_readfirstlane(B.crossings);
 
-        // ---- segments, listed chain by chain
+        // ---- segments: those of a chain side by side in the list and in order, the chains in any
         const int len = max(kSegMin, (crossings + kSegTarget - 1) / kSegTarget);
-        int n_segs = 0, rank = before - np;
 #pragma unroll 1
-        for (int i = 0; i < 10; ++i) {
-            const int ch = 10 * lane + i, p = ch >> 1;
-            if ((B.pa[p].x & 0xFFFFu) == kNoPiece) continue;
-            if (!(i & 1)) B.by_rank[rank++] = (uint16_t)p;
+        for (int ch = tid; ch < 2 * kSlots; ch += kThreads) {
+            if ((B.pa[ch >> 1].x & 0xFFFFu) == kNoPiece) continue;
             const ChainRef r = chain_of(B, ch);
+            if (r.n == 0) continue;
             int head = r.n;
             if (r.n > len + len / 2) {
                 head = len;
@@ -597,67 +618,57 @@ __global__ __launch_bounds__(kLanes) void k_curves(const CurveArgs K, const Frag
                 if (r.n - head < len / 2) head = r.n;
             }
             B.head[ch] = (uint16_t)head;
-            n_segs += (head ? 1 : 0) + seg_rest(r.n, head, len);
-            n_split += head < r.n ? 1 : 0;
-        }
-        const int segs_upto = wave_inclusive_add(n_segs);
-        const int S = __builtin_amdgcn_readlane(segs_upto, 63);
-        int at = segs_upto - n_segs;
-#pragma unroll 1
-        for (int i = 0; i < 10; ++i) {
-            const int ch = 10 * lane + i;
-            if ((B.pa[ch >> 1].x & 0xFFFFu) == kNoPiece) continue;
-            const ChainRef r = chain_of(B, ch);
-            const int head = B.head[ch];
-            if (head) B.seg[at++] = (uint32_t)ch;
+            const int m = seg_rest(r.n, head, len);
+            int at = atomicAdd(&B.n_segs, 1 + m);
+            B.seg[at++] = (uint32_t)ch;
             if (head >= r.n) continue;
+            ++n_split;
             int k8 = 0, k16 = 0;
             if (r.type != kLine) {
                 k8 = crossings_before(r.type, r.a, r.line0, r.neg, r.t0, 0.125f * r.t1, r.n);
                 if (k8) k16 = crossings_before(r.type, r.a, r.line0, r.neg, r.t0, 0.0625f * r.t1, r.n);
             }
-            const int m = seg_rest(r.n, head, len);
             for (int j = 0; j < m; ++j) {
                 const int i0 = head + seg_begin(r.n - head, m, j);
                 const int warm = i0 >= k8 ? kWarm : (i0 >= k16 ? kWarm8 : kWarm16);
-                B.seg[at++] = (uint32_t)ch | ((uint32_t)(j + 1) << 10) | ((uint32_t)warm << 16);
+                B.seg[at++] = (uint32_t)ch | ((uint32_t)(j + 1) << 10) | ((uint32_t)warm << 20);
             }
         }
-        wave_sync();
+        __syncthreads();
+        const int S = __builtin_amdgcn_readfirstlane(B.n_segs);
 
         // ---- the crossings, one segment per lane
-        for (int s0 = 0; s0 < S; s0 += kLanes) {
-            const bool on = s0 + lane < S;
-            const uint32_t e = B.seg[on ? s0 + lane : s0];
+        for (int s0 = 0; s0 < S; s0 += kThreads) {
+            const bool on = s0 + tid < S;
+            const uint32_t e = B.seg[on ? s0 + tid : s0];
             const int ch = (int)(e & 1023u);
             const ChainRef r = chain_of(B, ch);
             int i0, i1;
-            seg_range(B, ch, (int)((e >> 10) & 63u), r.n, len, i0, i1);
+            seg_range(B, ch, (int)((e >> 10) & 1023u), r.n, len, i0, i1);
             float* vs = B.v + r.at;
             // solve, then the guesses against what the segments before ended on: a segment whose
             // guess was off is solved again from there
             float g = r.t0, start = r.t0;
-            int k0 = max(0, i0 - (int)(e >> 16));
+            int k0 = max(0, i0 - (int)(e >> 20));
             bool run = on, redo = false;
             for (;;) {
                 if (run) {
                     const float got = solve_run_any(r.type, r.a, r.line0, r.neg, r.side, r.t1, k0, i0, i1, start, redo, vs);
                     if (!redo) g = got;
                 }
-                wave_sync();
+                __syncthreads();
                 const float is = on && i0 > 0 ? vs[i0 - 1] : g;
                 run = fbits(is) != fbits(g);
-                if (!__any(run)) break;
+                if (!__syncthreads_or(run ? 1 : 0)) break;
                 g = start = is;
                 k0 = i0;
                 redo = true;
-                wave_sync();
             }
         }
 
         // ---- the order of each piece's sequences, then the merge
         bool falls = false;
-        for (int e = lane; e < n_slots; e += kLanes) {
+        for (int e = tid; e < n_slots; e += kThreads) {
             const int p = piece_of(B, e);
             if (p < 0) continue;
             const int base = (int)(B.pa[p].x & 0xFFFFu), nx = (int)(B.pa[p].x >> 16), ny = (int)(B.pa[p].y & 0xFFFFu);
@@ -668,10 +679,9 @@ __global__ __launch_bounds__(kLanes) void k_curves(const CurveArgs K, const Frag
             const float prev = idx == 1 + nx ? B.v[base] : (idx == 1 && ny > 0 ? v : B.v[e - 1]);
             if (!(v >= prev)) { falls = true; atomicOr(&B.pa[p].y, kPwFalls); }
         }
-        const bool any_falls = __any(falls);
-        wave_sync();
+        const bool any_falls = __syncthreads_or(falls ? 1 : 0) != 0;
         if (any_falls) {
-            for (int e = lane; e < n_slots; e += kLanes) {
+            for (int e = tid; e < n_slots; e += kThreads) {
                 const int p = piece_of(B, e);
                 if (p < 0) continue;
                 const uint32_t w1 = B.pa[p].y;
@@ -683,7 +693,7 @@ __global__ __launch_bounds__(kLanes) void k_curves(const CurveArgs K, const Frag
                 const float prev = idx == 1 + nx ? B.v[base] : (idx == 1 && ny > 0 ? v : B.v[e - 1]);
                 if (!(v <= prev)) atomicOr(&B.pa[p].y, kPwRises);
             }
-            wave_sync();
+            __syncthreads();
         }
         for (int s0 = 0; s0 < n_slots;) {
             int s1 = n_slots;
@@ -715,7 +725,7 @@ __global__ __launch_bounds__(kLanes) void k_curves(const CurveArgs K, const Frag
 
         // ---- fragments: lane l evaluates the point of slot e0 + l; a slot's segment runs to the
         // next slot's point, so 64 points serve 63 slots
-        for (int e0 = 0; e0 < n_slots; e0 += 63) {
+        for (int e0 = 63 * wave; e0 < n_slots; e0 += 63 * kWaves) {
             const int e = e0 + lane;
             const int p = e < n_slots ? piece_of(B, e) : -1;
             const uint32_t w0 = B.pa[max(p, 0)].x, w1 = B.pa[max(p, 0)].y;
@@ -754,7 +764,7 @@ __global__ __launch_bounds__(kLanes) void k_curves(const CurveArgs K, const Frag
             }
             wave_count(A.hist, bucket, valid);
         }
-        wave_sync();  // the LDS is used again
+        __syncthreads();  // the LDS is used again
     }
     n_split = wave_sum(n_split);
     if (lane == 0 && n_split) atomicAdd(K.split_count, n_split);
@@ -876,7 +886,7 @@ hipError_t launch_curves(const CurveArgs& K, const FragArgs& A, hipStream_t s) {
     if (K.C == 0 || K.n == 0) return hipSuccess;
     if (K.window < kCurveWindowMin || K.window > kCurveWindowMax) return hipErrorInvalidValue;
     const int64_t g = (K.n + K.window - 1) / K.window;
-    k_curves<<<(unsigned)g, kLanes, 0, s>>>(K, A);
+    k_curves<<<(unsigned)g, kThreads, 0, s>>>(K, A);
     return hipGetLastError();
 }
 

@@ -200,14 +200,14 @@ struct FrameInit {
 };
 hipError_t launch_frame_init(const FrameInit& I, hipStream_t s);
 // The curve pass (k_curves.hip): frames below kChainFrame entries.
-// The intersection write and the fragment keys: one wave per window of `window`
+// The intersection write and the fragment keys: one workgroup per window of `window`
 // entries takes the pieces that start there from the curve data to their keys (or sort words),
 // winding changes and bucket counts, without storing the entries unless A.inter is set.  Pieces
 // of more than kCurvePieceMax entries are queued in `big` for launch_big_pieces.
 // Frames of this many entries take the chain passes: they fill the chip with whole chains sorted by
-// length, which costs half the arithmetic of the curve pass (52.9 M entries: 1.8 ms against 3.4 ms),
-// but has their longest chain and seven launches as its span (0.73 M entries: 0.41 ms against 0.24
-// ms; 7.2 M: 0.63 ms against 0.52 ms).
+// length, which costs half the arithmetic of the curve pass, but has their longest chain and seven
+// launches as its span.  ms a frame alone, by chains and by curves: 6.2 M entries 1.00 and 0.85,
+// 12.0 M 1.22 and 1.54, 24.7 M 1.85 and 2.65, 48.7 M 2.99 and 5.26.
 constexpr int64_t kChainFrame = (int64_t)1 << 23;
 constexpr int kCurveWindowMin = 64, kCurveWindowMax = 1024, kCurvePieceMax = 1024;
 struct CurveArgs {

@@ -212,6 +212,7 @@ struct spr_handle {
     DBuf<int32_t> arena, capn, sstart, hist_l, fill_l, bsum_l, pbound;
     DBuf<int2> brec_l;
     int64_t lb_n = 0, lb_r = 0;                     // learned frame budgets (entries, records)
+    int64_t total_seen = 0, route_n = 0;            // most entries a learned frame of the scene had; what chose the route
     bool need_prediction = true;                    // scene or model changed: read the prediction back
     bool lb_dirty = true;                           // scene, MVP, model or margin changed: the graph is stale
     int64_t n_live = 0;                             // entries of the last learned frame
@@ -364,12 +365,14 @@ spr::CountArgs count_args(spr_handle* H, int rmax, spr::ScanCtl curves, spr::Sca
                           spr::count_tiles(H->Np), paths.status, paths.counter, pcanvas, host};
 }
 
-// Entries per window of the curve pass.  A wave takes one window, and about 2,000 waves are
-// resident: windows shrink with the frame until each wave's crossings spread over its 64 lanes a
-// few at a time, so that a small frame ends after a few crossings, not after a window's worth.
+// Entries per window of the curve pass.  A workgroup takes one window, and 1,536 workgroups are
+// resident.  The larger the window, the fewer crossings are solved only to guess a segment's start,
+// so windows shrink only where the frame would leave CUs without two.  us a frame alone, windows of
+// 256, 512 and 1024: 0.15 M entries 529, 529, 562; 0.8 M 412, 348, 331; 1.9 M 427, 405, 424 (and
+// 304, 274, 261 with frames of other handles beside it).
 int32_t curve_window(const spr_handle* H, int64_t n) {
     int64_t w = spr::kCurveWindowMax;
-    while (w > 2 * spr::kCurveWindowMin && n / w < 4096) w >>= 1;
+    while (w > 4 * spr::kCurveWindowMin && n / w < 512) w >>= 1;
     w = w * 8 / H->chain_k;  // the tuned share
     return (int32_t)std::min<int64_t>(std::max<int64_t>(w, spr::kCurveWindowMin), spr::kCurveWindowMax);
 }
@@ -889,8 +892,13 @@ void run_learned_frame(spr_handle* H) {
     H->brec_l.ensure((size_t)nb_budget + 1);
     // per-bucket tables: cleared up to the live bucket count (bucket_base[Np])
     const int32_t* d_nb = H->bucket_base.p + Np;
-    const int32_t window = curve_window(H, nl);
-    const bool by_chain = nl >= spr::kChainFrame;
+    // The pass and its windows follow what the scene's frames needed so far, not the budget, which
+    // the prediction (or a batch's proven bound) can put far above it: a 6.2 M entry pan at 1920x1080
+    // on a budget above 2^24 took 1007 us by chains, 925 by curves.  A captured frame takes the route
+    // of the eager one before it, whose buffers are there.
+    if (!H->capturing) H->route_n = H->total_seen > 0 ? std::min(H->total_seen, nl) : nl;
+    const int32_t window = curve_window(H, H->route_n);
+    const bool by_chain = H->route_n >= spr::kChainFrame;
     spr::FrameInit init{};
     init.fill[0] = {(uint32_t*)H->hist_l.p, nb_budget + 1, d_nb, 1, 1, 0u};
     init.fill[1] = {(uint32_t*)H->fill_l.p, nb_budget, d_nb, 1, 0, 0u};
@@ -1022,6 +1030,7 @@ void learned_finish(spr_handle* H) {
     const int64_t caps = std::max<int32_t>(H->sum(kSumArena), 0);
     const int64_t total = H->sum(kSumTotal);
     const int64_t overflow_paths = H->sum(kSumOverflow);
+    H->total_seen = std::max(H->total_seen, total);
     H->frame_done = true;
     H->last_learned = true;
     H->last_fallback = false;
@@ -1264,6 +1273,7 @@ void load_arrays(spr_handle* H, const float* pos, const uint32_t* pos_path, uint
     H->frame_done = false;
     H->inj = false;
     H->inj_inter.clear();
+    H->total_seen = 0;
     H->lb_dirty = true;
     H->need_prediction = true;
     H->batch = false;
@@ -1759,6 +1769,7 @@ int spr_load_batch(spr_handle* H, const spr_scene* const* docs, const uint32_t* 
         H->max_w = max_w;
         H->max_h = max_h;
         H->img_bytes = img;
+        H->total_seen = 0;
         H->lb_dirty = true;
         H->need_prediction = true;
     });
