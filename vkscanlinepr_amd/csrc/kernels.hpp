@@ -199,6 +199,12 @@ struct FrameInit {
     Budget budget;             // entries == 0: none
 };
 hipError_t launch_frame_init(const FrameInit& I, hipStream_t s);
+// Device image to pinned host memory (k_readback.hip): bytes (whole pixels) from src to dst, in chunks of
+// kReadChunk; arrived[c] becomes mark when chunk c is there.
+constexpr int kReadChunk = 32768;
+hipError_t launch_read_out(const uint8_t* src, uint8_t* dst, int64_t bytes, uint32_t* arrived, uint32_t mark,
+                           hipStream_t s);
+
 // The curve pass (k_curves.hip): frames below kChainFrame entries.
 // The intersection write and the fragment keys: one workgroup per window of `window`
 // entries takes the pieces that start there from the curve data to their keys (or sort words),
