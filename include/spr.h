@@ -78,11 +78,9 @@ typedef struct spr_stats {
     int64_t learned_fallbacks; /* LEARNED: frames whose exact total exceeded the allocation and were
                                   rendered with the plain method (the allocation then grows) */
     /* Which kernel routes the last frame took (each route has its own kernel or mode): */
-    int64_t n_wave_chains;     /* crossing chains that the lanes of a wave share.  Frames of 2^23
-                                  intersections and more: chains solved by a whole wave each (896
-                                  or more crossings, and each launch's costliest classes while they
-                                  hold at most 512); smaller frames: chains cut into segments that
-                                  are solved side by side */
+    int64_t n_wave_chains;     /* crossing chains that several lanes share, cut into segments that are
+                                  solved side by side (frames of 2^23 intersections and more: the
+                                  chains of 256 or more crossings) */
     int64_t n_heavy_pieces;    /* monotone pieces merged by a 256-thread workgroup each (more than
                                   1024 entries, or, in frames of 2^23 intersections and more, whose
                                   last segment waits on a chain of 256 or more crossings of the

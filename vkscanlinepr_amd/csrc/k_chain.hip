@@ -12,14 +12,14 @@
 //     slot and per non-empty chain; chains are counted in length classes
 //     (quarter octaves for cubic chains, so that the 64 chains of one wave have similar lengths).
 //  2. k_chain_order: chains are laid out costliest class first (longest-processing-time order).
-//  3. k_chain_solve: a persistent kernel.  Waves first take the long cubic chains, one chain per
-//     wave: the 64 lanes evaluate the 63 midpoints of the next 6 bisection levels at once (lane l
-//     is node l of the decision tree and recomputes exactly the midpoints on its path), a ballot
-//     resolves the path in scalar registers, and 4 rounds give the reference's 24 iterations.
-//     Then waves take the remaining chains 64 at a time, one chain per lane, in descending
-//     length.  The first item of every wave is its global wave index (the first waves of a
-//     launch sit on distinct SIMDs, so the costliest items do not share one), later items come
-//     from an atomic counter; issue priority follows the item's cost.
+//  3. The solves: persistent kernels.  k_chain_solve takes the chains below 256 crossings 64 at a time,
+//     one chain per lane, in descending length.  k_chain_segments takes the longer ones, several
+//     lanes per chain: each lane solves a segment from a guess of the value before it, and the
+//     segments whose guess was off are solved again from the true one, so that the results are the
+//     sequential chain's (the reasons stand in k_curves.hip).  The first item of every wave is its
+//     global wave index (the first waves of a launch sit on distinct SIMDs, so the costliest items
+//     do not share one), later items come from an atomic counter; issue priority follows the item's
+//     cost.
 //  4. k_piece_small: one lane per piece slot.  A piece of at most 32 entries is merged by its
 //     lane with the reference's sequential walk, OR-merged and turned into fragment keys,
 //     winding changes and bucket counts (gen_fragment: the segment from an entry to the next one
@@ -40,23 +40,12 @@ namespace spr {
 namespace {
 
 constexpr int kBlock = 256;
-// cubic chains of class 4 * 9 + 3 and up (896+ crossings) get a whole wave: a lane-solved chain of
-// 900-1023 crossings outlasted the longest wave-solved chains
-constexpr int kWaveClass = 4 * 9 + 3;
-// below that, each launch also wave-solves its costliest cubic classes while they hold at most
-// kWaveBudget chains in all and at least 2^5 crossings each: in a scene with few long chains
-// (a 64-path scene, a glyph page) those chains alone set the launch's span, and a wave takes
-// 0.64 us per crossing against about 1.2 us for a lane
-constexpr int kWaveBudget = 512;
-constexpr int kWaveMinClass = 4 * 5;
 constexpr int kStage = 4096;       // piece values staged in LDS by the merging wave
 constexpr int kClasses = kChainClasses;  // 0..63: cubic chains (4 per octave), 64..79: line chains
-constexpr int kRounds = 4, kLevels = 6;  // wave solve: 4 rounds of 6 bisection levels
 // first heavy cubic class: a quarter-octave class 4*l + sub holds lengths >= 2^l (l = 8: 256)
 constexpr int kHeavyClass = 4 * 8;
 static_assert(kHeavyCrossings == 1 << 8, "heavy class boundary");
 static_assert(kFrag == 2, "chain descriptors keep only the sign of the grid step");
-static_assert(kRounds * kLevels == kCubicIters, "wave solve must run the reference's iterations");
 
 inline unsigned grid_for(int64_t n) {
     int64_t g = (n + kBlock - 1) / kBlock;
@@ -164,22 +153,19 @@ __global__ __launch_bounds__(kBlock) void k_chain_prep(
 
 // Class order: by estimated cost in quarter octaves, costliest first (a line crossing costs
 // about 2^-6 of a cubic one), cubic before line on ties.  Cost key: cubic class c -> 2(c+24)+1,
-// line class 64+l -> 8l; the keys are distinct.  The cubic classes from kWaveClass up
-// come first: the wave-solved chains.
+// line class 64+l -> 8l; the keys are distinct.
 __device__ inline int class_cost_key(int c) { return c < 64 ? 2 * (c + 24) + 1 : 8 * (c - 64); }
 
 // Chains in class order: each workgroup computes the class offsets (a class's offset is the
-// number of chains in the classes of higher cost key; the keys are distinct, and the wave-solved
-// classes and the heavy ones come first, so their totals are also the ends of those groups;
-// workgroup 0 stores them for the solve), owns a contiguous range of chain slots, counts its
+// number of chains in the classes of higher cost key; the keys are distinct, and the heavy classes
+// come first, so their total is also the end of that group; workgroup 0 stores them for the solve), owns a contiguous range of chain slots, counts its
 // chains per class (from the one-byte classes written by k_chain_prep), takes one block of places
 // per class with a single atomic, then writes the chain indices.
 __global__ __launch_bounds__(kBlock) void k_chain_order(const uint8_t* __restrict__ chain_cls, int64_t n_slots,
                                                         const int32_t* __restrict__ class_count,
                                                         int32_t* __restrict__ class_fill,
-                                                        int32_t* __restrict__ class_off, int32_t* __restrict__ n_long,
+                                                        int32_t* __restrict__ class_off,
                                                         int32_t* __restrict__ light_begin,
-                                                        int32_t* __restrict__ n_long_light,
                                                         int32_t* __restrict__ order) {
     __shared__ int32_t cnt[kClasses], base[kClasses], off[kClasses], total[kClasses];
     if (threadIdx.x < kClasses) {
@@ -194,26 +180,14 @@ __global__ __launch_bounds__(kBlock) void k_chain_order(const uint8_t* __restric
         off[threadIdx.x] = o;
         if (blockIdx.x == 0) class_off[threadIdx.x] = o;
     } else if (blockIdx.x == 0 && threadIdx.x == kClasses) {
-        int32_t all = 0, nl = 0, lb = 0;
+        int32_t all = 0, lb = 0;
         for (int d = 0; d < kClasses; ++d) {
             all += total[d];
-            if (d < 64 && d >= kWaveClass) nl += total[d];
+            // the heavy range holds cubic classes only (every line key is below theirs)
             if (d < 64 && d >= kHeavyClass) lb += total[d];
         }
-        // the heavy launch's range holds cubic classes only (every line key is below theirs)
-        for (int c = kWaveClass - 1; c >= kHeavyClass && nl + total[c] <= kWaveBudget; --c) nl += total[c];
-        // the light launch's range in key order: cubic class c comes right after line class
-        // (c + 25) / 4 when (c + 25) % 4 == 0 (key 8l = 2c + 50); wave items stop at a line class
-        int32_t nll = 0;
-        for (int c = kHeavyClass - 1; c >= kWaveMinClass; --c) {
-            if ((c + 25) % 4 == 0 && total[64 + (c + 25) / 4] > 0) break;
-            if (nll + total[c] > kWaveBudget) break;
-            nll += total[c];
-        }
         class_off[kClasses] = all;
-        *n_long = nl;
         *light_begin = lb;
-        *n_long_light = nll;
     }
     const int64_t per = ((n_slots + gridDim.x - 1) / gridDim.x + kBlock - 1) / kBlock * kBlock;
     const int64_t b0 = (int64_t)blockIdx.x * per, b1 = b0 + per < n_slots ? b0 + per : n_slots;
@@ -298,163 +272,22 @@ __device__ inline void solve_chain_lane(const ChainDesc& d, const CurveAxis& a, 
     else solve_chain_lane_t<kArc>(d, a, out, mono, stage);
 }
 
-// Cubic chain solved by one wave: 4 rounds of a 6-level speculative bisection per crossing.
-// Lane l (1..63) is node l of the round's decision tree: its depth is floor(log2 l) and the bits
-// of l below the leading one are its path (1 = right).  Each lane halves the round's interval
-// along its own path, exactly as the sequential bisection would, and evaluates the midpoint of
-// its node; the ballot D of "same sign as at t_min" fixes the path taken through the tree.  A
-// depth-5 node (lanes 32..63) lies on that path when D holds, at its five ancestors, the turns
-// that lead to it: one masked compare per lane and a second ballot name the node, whose
-// interval, midpoint and value are then read from its lane.
-struct WaveTree {
-    bool on[kLevels - 1], go_right[kLevels - 1];
-    unsigned long long anc_mask, anc_turn;
-};
-
-__device__ inline WaveTree wave_tree(int lane) {
-    WaveTree W;
-    const int depth = lane ? 31 - __clz(lane) : 0;
-    W.anc_mask = 0ull;
-    W.anc_turn = 1ull;  // inner nodes never match
-#pragma unroll
-    for (int lev = 0; lev < kLevels - 1; ++lev) {
-        W.on[lev] = lev < depth;
-        W.go_right[lev] = W.on[lev] && ((lane >> (depth - 1 - lev)) & 1);
-    }
-    if (depth == kLevels - 1) {
-        W.anc_turn = 0ull;
-#pragma unroll
-        for (int lev = 0; lev < kLevels - 1; ++lev) {
-            const int anc = lane >> (kLevels - 1 - lev);  // ancestor at depth lev
-            W.anc_mask |= 1ull << anc;
-            W.anc_turn |= (unsigned long long)((lane >> (kLevels - 2 - lev)) & 1) << anc;
-        }
-    }
-    return W;
-}
-
-// The 24 levels of one crossing's bisection on [lo, hi]: tm and vtm of the last level.  A node
-// turns right where the sign of v - c is s0 (MODE 0), or, with every value finite, where v < c
-// for a start below the line (MODE 1) or v >= c for a start above it (MODE 2).
-template <uint32_t T, int MODE>
-__device__ __forceinline__ void wave_bisect(const CurveAxis& a, float c, float lo, float hi, uint32_t s0,
-                                            const WaveTree& W, float& tm, float& vtm) {
-#pragma unroll
-    for (int round = 0; round < kRounds; ++round) {
-        float llo = lo, lhi = hi;
-#pragma unroll
-        for (int lev = 0; lev < kLevels - 1; ++lev) {
-            const float mid = (llo + lhi) * 0.5f;
-            llo = W.go_right[lev] ? mid : llo;
-            lhi = (W.on[lev] && !W.go_right[lev]) ? mid : lhi;
-        }
-        const float mym = (llo + lhi) * 0.5f;
-        const float myv = eval_axis(T, mym, a.c[0], a.c[1], a.c[2], a.c[3]);
-        // lane 0 is no node: its bit is never read
-        const bool right = MODE == 1 ? myv < c : (MODE == 2 ? !(myv < c) : (fbits(myv - c) & 0x80000000u) == s0);
-        // the interval this node leaves for the next round
-        const float nlo = right ? mym : llo, nhi = right ? lhi : mym;
-        const unsigned long long D = __ballot(right);
-        const unsigned long long P = __ballot((D & W.anc_mask) == W.anc_turn);
-        const int node = __builtin_amdgcn_readfirstlane(__builtin_ctzll(P));
-        lo = bitsf((uint32_t)__builtin_amdgcn_readlane((int)fbits(nlo), node));
-        hi = bitsf((uint32_t)__builtin_amdgcn_readlane((int)fbits(nhi), node));
-        if (round == kRounds - 1) {
-            tm = bitsf((uint32_t)__builtin_amdgcn_readlane((int)fbits(mym), node));
-            vtm = bitsf((uint32_t)__builtin_amdgcn_readlane((int)fbits(myv), node));
-        }
-    }
-}
-
-// DIRECT (every control value finite and below 2^17 in magnitude): a crossing whose start lies
-// on the side the chain comes from takes the single-compare rounds, and a crossing after one
-// that did not fall back starts there without evaluating at t_min (see bisect_below).
-template <uint32_t T, bool DIRECT>
-__device__ inline void solve_chain_wave_t(const ChainDesc& d, const CurveAxis& a, float* __restrict__ out,
-                                          uint8_t* __restrict__ mono) {
-    const int lane = threadIdx.x & 63;
-    const WaveTree W = wave_tree(lane);
-    const uint32_t side = (uint32_t)chain_side(d);
-    const bool neg = chain_step(d) < 0.0f;
-    float tprev = d.t0, line = d.line0;
-    bool up = true, down = true;
-    float kept = 0.0f;
-    bool known = false;  // this crossing starts on the side the chain comes from
-    for (int k = 0; k < d.n; ++k) {
-        const float c = line;
-        const float t_min = tprev;
-        const bool fb = DIRECT && fast_bracket(t_min, d.t1);
-        bool run = true, from = true;
-        uint32_t s0 = neg ? 0u : 0x80000000u;
-        if (!(fb && known)) {
-            // the same value in every lane: uniform branches below
-            const float vt0 = eval_axis(T, t_min, a.c[0], a.c[1], a.c[2], a.c[3]);
-            run = __builtin_amdgcn_readfirstlane(vt0 != c ? 1 : 0) != 0;
-            from = __builtin_amdgcn_readfirstlane((neg ? vt0 > c : vt0 < c) ? 1 : 0) != 0;
-            s0 = fbits(vt0 - c) & 0x80000000u;
-        }
-        float ts = t_min;
-        known = fb;  // a start on the line itself is a crossing with no fallback
-        if (run) {
-            float tm = t_min, vtm = 0.0f;
-            if (DIRECT && from && !neg) wave_bisect<T, DIRECT ? 1 : 0>(a, c, t_min, d.t1, s0, W, tm, vtm);
-            else if (DIRECT && from) wave_bisect<T, DIRECT ? 2 : 0>(a, c, t_min, d.t1, s0, W, tm, vtm);
-            else wave_bisect<T, 0>(a, c, t_min, d.t1, s0, W, tm, vtm);
-            const bool fell = fabsf(vtm - c) > 1.0f;
-            ts = fell ? t_min : tm;
-            known = fb && from && !fell;
-        }
-        const float v = bitsf((fbits(ts) & 0xFFFFFFFCu) | side);
-        // lane k % 64 keeps value k; 64 values are stored at once (coalesced)
-        if (lane == (k & 63)) kept = v;
-        if ((k & 63) == 63 || k == d.n - 1) {
-            if (lane <= (k & 63)) out[k - (k & 63) + lane] = kept;
-        }
-        if (k > 0 || side) { up = up && v >= tprev; down = down && v <= tprev; }
-        tprev = v;
-        line += chain_step(d);
-    }
-    if (lane == 0) *mono = (up ? 1 : 0) | (down ? 2 : 0);
-}
-
-// Wave-solved chains are never lines (line chains take the lane classes).
-__device__ inline void solve_chain_wave(const ChainDesc& d, const CurveAxis& a, float* __restrict__ out,
-                                        uint8_t* __restrict__ mono) {
-    const uint32_t type = (uint32_t)d.type;
-    const bool direct = fast_axis(type, a);
-    if (type == kCubic) {
-        if (direct) solve_chain_wave_t<kCubic, true>(d, a, out, mono);
-        else solve_chain_wave_t<kCubic, false>(d, a, out, mono);
-    } else if (type == kQuad) {
-        if (direct) solve_chain_wave_t<kQuad, true>(d, a, out, mono);
-        else solve_chain_wave_t<kQuad, false>(d, a, out, mono);
-    } else {
-        solve_chain_wave_t<kArc, false>(d, a, out, mono);
-    }
-}
-
+// The chains below kHeavyCrossings, [*light_begin, total) in class order, 64 at a time, one per lane.
 __global__ __launch_bounds__(kBlock) void k_chain_solve(const float2* __restrict__ tpos,
                                                         const uint32_t* __restrict__ cpos,
                                                         const float* __restrict__ cweight,
                                                         const ChainDesc* __restrict__ chains,
                                                         const int32_t* __restrict__ order,
                                                         const int32_t* __restrict__ class_off,
-                                                        const int32_t* __restrict__ n_long,
-                                                        const int32_t* __restrict__ light_begin, int heavy,
+                                                        const int32_t* __restrict__ light_begin,
                                                         int32_t* __restrict__ work,
                                                         float* __restrict__ chain_t,
                                                         uint8_t* __restrict__ mono) {
     __shared__ float s_stage[16 * kBlock];
     float* stage = s_stage + threadIdx.x;
     const int lane = threadIdx.x & 63;
-    const int32_t total = class_off[kClasses];
-    const int32_t lb = *light_begin;
-    // the launch's chains [r0, r1) in class order (heavy: [0, lb), light: [lb, total)): wave items
-    // on the first nl, lane items on the rest
-    const int32_t r0 = heavy ? 0 : lb, r1 = heavy ? lb : total;
-    const int32_t nl = *n_long;
-    const int32_t lane0 = r0 + nl, lane1 = r1;
-    const int32_t items = nl + (lane1 - lane0 + 63) / 64;
+    const int32_t lane0 = *light_begin, lane1 = class_off[kClasses];
+    const int32_t items = (lane1 - lane0 + 63) / 64;
     const int32_t n_waves = (int32_t)gridDim.x * (kBlock / 64);
     int32_t item = (int32_t)blockIdx.x * (kBlock / 64) + (int32_t)(threadIdx.x >> 6);
     // the wave's next item is taken one item ahead, so that the atomic's round trip overlaps the
@@ -462,36 +295,195 @@ __global__ __launch_bounds__(kBlock) void k_chain_solve(const float2* __restrict
     int32_t next = 0;
     if (lane == 0 && item < items) next = n_waves + atomicAdd(work, 1);
     while (item < items) {
-        if (item < nl) {
-            __builtin_amdgcn_s_setprio(3);
-            const int32_t ci = order[r0 + item];
-            const ChainDesc d = chains[ci];
-            const CurveAxis a = load_axis(tpos, cpos, cweight, d);
-            solve_chain_wave(d, a, chain_t + d.out, mono + ci);
-            __builtin_amdgcn_s_setprio(0);
-        } else {
-            const int32_t k = lane0 + (item - nl) * 64 + lane;
-            ChainDesc d;
-            d.n = 0; d.type = (int16_t)kLine;
-            int32_t ci = 0;
-            if (k < lane1) {
-                ci = order[k];
-                d = chains[ci];
-            }
-            // issue priority follows the cost of the wave's chains, read from lane 0's (the item's
-            // first chain: the longest run first and must not be starved by the short ones)
-            const int n0 = __builtin_amdgcn_readfirstlane(d.n);
-            const int b0 = __builtin_amdgcn_readfirstlane(d.type != (int16_t)kLine ? 1 : 0);
-            const int oct = class_cost_octave(chain_class(n0, b0 != 0));
-            if (oct >= 8) __builtin_amdgcn_s_setprio(3);
-            else if (oct >= 6) __builtin_amdgcn_s_setprio(2);
-            else if (oct >= 4) __builtin_amdgcn_s_setprio(1);
-            if (k < lane1) {
-                const CurveAxis a = load_axis(tpos, cpos, cweight, d);
-                solve_chain_lane(d, a, chain_t + d.out, mono + ci, stage);
-            }
-            __builtin_amdgcn_s_setprio(0);
+        const int32_t k = lane0 + item * 64 + lane;
+        ChainDesc d;
+        d.n = 0; d.type = (int16_t)kLine;
+        int32_t ci = 0;
+        if (k < lane1) {
+            ci = order[k];
+            d = chains[ci];
         }
+        // issue priority follows the cost of the wave's chains, read from lane 0's (the item's
+        // first chain: the longest run first and must not be starved by the short ones)
+        const int n0 = __builtin_amdgcn_readfirstlane(d.n);
+        const int b0 = __builtin_amdgcn_readfirstlane(d.type != (int16_t)kLine ? 1 : 0);
+        const int oct = class_cost_octave(chain_class(n0, b0 != 0));
+        if (oct >= 8) __builtin_amdgcn_s_setprio(3);
+        else if (oct >= 6) __builtin_amdgcn_s_setprio(2);
+        else if (oct >= 4) __builtin_amdgcn_s_setprio(1);
+        if (k < lane1) {
+            const CurveAxis a = load_axis(tpos, cpos, cweight, d);
+            solve_chain_lane(d, a, chain_t + d.out, mono + ci, stage);
+        }
+        __builtin_amdgcn_s_setprio(0);
+        item = __shfl(next, 0);
+        if (lane == 0 && item < items) next = n_waves + atomicAdd(work, 1);
+    }
+}
+
+// Crossings [i0, i1) of a chain, the first one from tstart, or from the value that solving crossings
+// [k0, i0) ends on (returned in guess).  Stores like solve_chain_lane_t; last is the last value.
+template <uint32_t T>
+__device__ inline void solve_segment_t(const ChainDesc& d, const CurveAxis& a, int k0, int i0, int i1,
+                                       float* __restrict__ out, float* __restrict__ stage, float& guess, float& last,
+                                       uint32_t& falls, uint32_t& rises) {
+    float tprev = d.t0, line = d.line0 + chain_step(d) * (float)k0;  // lines are small integers: exact
+    const uint32_t side = (uint32_t)chain_side(d);
+    ChainSolver<T> solver(a, chain_step(d), d.t1);
+    for (int k = k0; k < i1; ++k) {
+        const float ts = __all(solver.common(tprev)) ? solver.next_common(line, tprev, d.t1)
+                                                     : solver.next(line, tprev, d.t1);
+        const float v = bitsf((fbits(ts) & 0xFFFFFFFCu) | side);
+        if (k >= i0) {
+            const int j = (k - i0) & 15;
+            stage[j * kBlock] = v;
+            if (j == 15) {
+                float* dst = out + (k - 15);
+#pragma unroll
+                for (int u = 0; u < 16; ++u) dst[u] = stage[u * kBlock];
+            } else if (k == i1 - 1) {
+                float* dst = out + (k - j);
+                for (int u = 0; u <= j; ++u) dst[u] = stage[u * kBlock];
+            }
+            const float prev = k > 0 || side ? tprev : v;
+            falls |= !(v >= prev) ? 1u : 0u;
+            rises |= !(v <= prev) ? 1u : 0u;
+        } else {
+            guess = v;
+        }
+        tprev = v;
+        line += chain_step(d);
+    }
+    last = tprev;
+}
+
+// The same crossings again from a value that differs from the guess: up to the first that comes out
+// as it is stored, since everything after it is then equal too.  The order of the segment's
+// values is taken from the stored ones.
+template <uint32_t T>
+__device__ inline void resolve_segment_t(const ChainDesc& d, const CurveAxis& a, int i0, int i1, float tstart,
+                                         float* out, float& last, uint32_t& falls, uint32_t& rises) {
+    float tprev = tstart, line = d.line0 + chain_step(d) * (float)i0;
+    const uint32_t side = (uint32_t)chain_side(d);
+    ChainSolver<T, 6> solver(a, chain_step(d), d.t1);
+    int k = i0;
+    for (; k < i1; ++k) {
+        const float ts = solver.next(line, tprev, d.t1);
+        const float v = bitsf((fbits(ts) & 0xFFFFFFFCu) | side);
+        if (fbits(out[k]) == fbits(v)) break;
+        out[k] = v;
+        tprev = v;
+        line += chain_step(d);
+    }
+    if (k == i1) last = tprev;
+    falls = rises = 0;
+    tprev = tstart;
+    for (k = i0; k < i1; ++k) {
+        const float v = out[k];
+        falls |= !(v >= tprev) ? 1u : 0u;
+        rises |= !(v <= tprev) ? 1u : 0u;
+        tprev = v;
+    }
+}
+
+// About how many of a chain's crossings lie before parameter tau.
+__device__ inline int crossings_before(const ChainDesc& d, const CurveAxis& a, float tau) {
+    if (!(d.t0 < tau)) return 0;
+    const float v = eval_axis((uint32_t)d.type, tau, a.c[0], a.c[1], a.c[2], a.c[3]) - d.line0;
+    const float k = (chain_step(d) < 0.0f ? -v : v) * 0.5f + 2.0f;
+    return k >= (float)d.n ? d.n : (k > 0.0f ? (int)k : 0);
+}
+
+// Crossings solved to guess a segment's start, and the parameter that a chain's first segment reaches
+// past, in parts of its end (runs of the bisection from different starts fall together slowly near 0).
+constexpr int kWarm = 8;
+constexpr float kHeadTau = 0.03125f;
+// log2 of the lanes per chain: 2 in octave 8 (256 to 511 crossings), 4 in octave 9, 8 above.
+constexpr int kLanes8 = 1, kLanes9 = 2, kLanes10 = 3;
+
+// The chains of kHeavyCrossings and more, [0, *light_begin) in class order, cut into segments of 130 to 260
+// crossings (more in the few chains above 2,000), one lane each.  Longer segments waste less on
+// guesses, and no segment should outlast the light launch's chains beside it (255 crossings): at 4, 8 and
+// 16 lanes instead of 2, 4 and 8 a 4096^2 frame of 48.7 M crossings took 2.62 ms, with 1, 2 and 4 the
+// same 2.56 ms but one of 12.0 M 0.875 instead of 0.842 ms.  It replaces whole waves that speculated six
+// bisection levels at a time (13 times the arithmetic) for chains of 896 crossings and more, and single
+// lanes for those below: the heavy launch 1.10 -> 0.80 ms, the frame 2.72 -> 2.58 ms.
+__global__ __launch_bounds__(kBlock) void k_chain_segments(const float2* __restrict__ tpos,
+                                                           const uint32_t* __restrict__ cpos,
+                                                           const float* __restrict__ cweight,
+                                                           const ChainDesc* __restrict__ chains,
+                                                           const int32_t* __restrict__ order,
+                                                           const int32_t* __restrict__ class_off,
+                                                           const int32_t* __restrict__ light_begin,
+                                                           int32_t* __restrict__ work, float* __restrict__ chain_t,
+                                                           uint8_t* __restrict__ mono) {
+    __shared__ float s_stage[16 * kBlock];
+    float* stage = s_stage + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    // the chains of octaves 10 and up, 9 and 8 in class order: [0, b10), [b10, b9), [b9, lb)
+    const int32_t b10 = class_off[kHeavyClass + 7], b9 = class_off[kHeavyClass + 3], lb = *light_begin;
+    constexpr int P10 = 6 - kLanes10, P9 = 6 - kLanes9, P8 = 6 - kLanes8;  // log2 of a wave's chains
+    const int32_t n10 = (b10 + (1 << P10) - 1) >> P10, n9 = (b9 - b10 + (1 << P9) - 1) >> P9;
+    const int32_t items = n10 + n9 + ((lb - b9 + (1 << P8) - 1) >> P8);
+    const int32_t n_waves = (int32_t)gridDim.x * (kBlock / 64);
+    int32_t item = (int32_t)blockIdx.x * (kBlock / 64) + (int32_t)(threadIdx.x >> 6);
+    int32_t next = 0;
+    if (lane == 0 && item < items) next = n_waves + atomicAdd(work, 1);
+    while (item < items) {
+        const int p = item < n10 ? P10 : (item < n10 + n9 ? P9 : P8);  // log2 of the wave's chains
+        const int32_t c0 = item < n10 ? item << P10
+                                      : (item < n10 + n9 ? b10 + ((item - n10) << P9) : b9 + ((item - n10 - n9) << P8));
+        const int32_t end = item < n10 ? b10 : (item < n10 + n9 ? b9 : lb);
+        const int lanes = 64 >> p, j = lane & (lanes - 1);
+        const int32_t k = c0 + (lane >> (6 - p));
+        bool on = k < end;
+        const int32_t ci = on ? order[k] : 0;
+        ChainDesc d{};
+        CurveAxis a{};
+        if (on) {
+            d = chains[ci];
+            a = load_axis(tpos, cpos, cweight, d);
+        }
+        int i0 = 0, i1 = 0;
+        if (on) {
+            const int len = (d.n + kWarm * (lanes - 1) + lanes - 1) / lanes;  // steps per lane, guesses included
+            const int head = max(len, crossings_before(d, a, kHeadTau * d.t1));
+            const int rest = d.n - head >= lanes - 1 ? d.n - head : 0;
+            if (j == 0) {
+                i1 = d.n - rest;
+            } else {
+                on = rest > 0;
+                i0 = d.n - rest + (int)(((uint32_t)rest * (uint32_t)(j - 1)) / (uint32_t)(lanes - 1));
+                i1 = d.n - rest + (int)(((uint32_t)rest * (uint32_t)j) / (uint32_t)(lanes - 1));
+            }
+        }
+        float* out = chain_t + d.out;
+        float guess = d.t0, last = d.t0;
+        uint32_t falls = 0, rises = 0;
+        if (on) {
+            const uint32_t type = (uint32_t)d.type;
+            const int k0 = max(0, i0 - kWarm);
+            if (type == kCubic) solve_segment_t<kCubic>(d, a, k0, i0, i1, out, stage, guess, last, falls, rises);
+            else if (type == kQuad) solve_segment_t<kQuad>(d, a, k0, i0, i1, out, stage, guess, last, falls, rises);
+            else solve_segment_t<kArc>(d, a, k0, i0, i1, out, stage, guess, last, falls, rises);
+        }
+        // every guess against what the segment before ended on
+        for (;;) {
+            const float is = __shfl_up(last, 1);
+            const bool redo = on && j > 0 && fbits(is) != fbits(guess);
+            if (!__any(redo)) break;
+            if (redo) {
+                guess = is;
+                const uint32_t type = (uint32_t)d.type;
+                if (type == kCubic) resolve_segment_t<kCubic>(d, a, i0, i1, is, out, last, falls, rises);
+                else if (type == kQuad) resolve_segment_t<kQuad>(d, a, i0, i1, is, out, last, falls, rises);
+                else resolve_segment_t<kArc>(d, a, i0, i1, is, out, last, falls, rises);
+            }
+        }
+        // the order of the chain's values: any segment's
+        const unsigned long long own = (lanes == 64 ? ~0ull : ((1ull << lanes) - 1ull)) << (lane & ~(lanes - 1));
+        const bool f = (__ballot(falls != 0) & own) != 0ull, r = (__ballot(rises != 0) & own) != 0ull;
+        if (on && j == 0) mono[ci] = (uint8_t)((f ? 0 : 1) | (r ? 0 : 2));
         item = __shfl(next, 0);
         if (lane == 0 && item < items) next = n_waves + atomicAdd(work, 1);
     }
@@ -1033,25 +1025,26 @@ hipError_t launch_chain_prep(const float2* tpos, const uint32_t* cpos, const uin
 }
 
 hipError_t launch_chain_order(const uint8_t* chain_cls, uint32_t C, const int32_t* class_count,
-                              int32_t* class_off, int32_t* class_fill, int32_t* n_long, int32_t* light_begin,
-                              int32_t* n_long_light, int32_t* order, int n_cu, hipStream_t s) {
+                              int32_t* class_off, int32_t* class_fill, int32_t* light_begin, int32_t* order,
+                              int n_cu, hipStream_t s) {
     if (C == 0) return hipSuccess;
     unsigned g = grid_for((int64_t)C * 10);
     if (g > (unsigned)n_cu * 4) g = (unsigned)n_cu * 4;
-    k_chain_order<<<g, kBlock, 0, s>>>(chain_cls, (int64_t)C * 10, class_count, class_fill, class_off, n_long,
-                                       light_begin, n_long_light, order);
+    k_chain_order<<<g, kBlock, 0, s>>>(chain_cls, (int64_t)C * 10, class_count, class_fill, class_off,
+                                       light_begin, order);
     return hipGetLastError();
 }
 
 hipError_t launch_chain_solve(const float2* tpos, const uint32_t* cpos, const float* cweight,
-                              const ChainDesc* chains,
-                              const int32_t* order, const int32_t* class_off, const int32_t* n_long,
+                              const ChainDesc* chains, const int32_t* order, const int32_t* class_off,
                               const int32_t* light_begin, int heavy, int32_t* work, float* chain_t, uint8_t* mono,
                               int n_cu, hipStream_t s) {
-    // the heavy launch holds a few hundred long items: one wave per SIMD at most
-    const unsigned grid = heavy ? (unsigned)n_cu : (unsigned)(n_cu * 8);
-    k_chain_solve<<<grid, kBlock, 0, s>>>(tpos, cpos, cweight, chains, order, class_off, n_long, light_begin, heavy, work,
-                                          chain_t, mono);
+    if (heavy)
+        k_chain_segments<<<(unsigned)(n_cu * 4), kBlock, 0, s>>>(tpos, cpos, cweight, chains, order, class_off,
+                                                                 light_begin, work, chain_t, mono);
+    else
+        k_chain_solve<<<(unsigned)(n_cu * 8), kBlock, 0, s>>>(tpos, cpos, cweight, chains, order, class_off,
+                                                              light_begin, work, chain_t, mono);
     return hipGetLastError();
 }
 

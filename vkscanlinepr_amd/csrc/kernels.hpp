@@ -111,18 +111,16 @@ struct FragArgs {
 };
 // Chain length classes: cubic chains by quarter octave of their length (16 octaves x 4), then
 // line chains by octave.  The chain control block holds, as int32: class counts, class fill
-// counters, class offsets [kChainClasses + 1], the number of wave-solved chains, the work counter
-// of the persistent solve, the count of queued heavy pieces, the first light class's place, the
-// light solve's work counter, the count of queued wave pieces that wait on heavy chains and the
-// number of wave-solved chains at the head of the light launch.
+// counters, class offsets [kChainClasses + 1], the heavy solve's work counter, the count of queued
+// heavy pieces, the number of heavy chains (the first light chain's place), the light solve's work
+// counter and the count of queued wave pieces that wait on heavy chains.
 constexpr int kChainClasses = 80;
-constexpr int kCcFill = kChainClasses, kCcOff = 2 * kChainClasses, kCcNLong = 3 * kChainClasses + 1,
-              kCcWork = kCcNLong + 1, kCcHeavyPieces = kCcWork + 1, kCcLightBegin = kCcHeavyPieces + 1,
-              kCcWorkLight = kCcLightBegin + 1, kCcWavePieces = kCcWorkLight + 1, kCcNLongLight = kCcWavePieces + 1,
-              kCcWords = kCcNLongLight + 1;
-// Chains of at least kHeavyCrossings crossings are "heavy": they are solved by their own launch
-// (wave-solved and the longest lane-solved chains), and the pieces of at most kHeavyCrossings
-// entries, which never wait on them, are finished by a concurrent stream meanwhile.
+constexpr int kCcFill = kChainClasses, kCcOff = 2 * kChainClasses, kCcWork = 3 * kChainClasses + 1,
+              kCcHeavyPieces = kCcWork + 1, kCcLightBegin = kCcHeavyPieces + 1,
+              kCcWorkLight = kCcLightBegin + 1, kCcWavePieces = kCcWorkLight + 1, kCcWords = kCcWavePieces + 1;
+// Chains of at least kHeavyCrossings crossings are "heavy": they are cut into segments and solved by
+// their own launch, and the pieces of at most kHeavyCrossings entries, which never wait on them,
+// are finished by a concurrent stream meanwhile.
 constexpr int kHeavyCrossings = 256;
 // A frame whose buffers were sized before its counts were known (no host synchronisation): the
 // frame init compares the exact total offsets[C] with the budget; a frame over budget sets *over
@@ -140,16 +138,13 @@ hipError_t launch_chain_prep(const float2* tpos, const uint32_t* cpos, const uin
                              const uint32_t* ncuts, const int32_t* offsets, uint32_t C, int w, int h,
                              ChainDesc* chains, PieceDesc* pieces, uint8_t* chain_cls, int32_t* class_count,
                              int n_cu, hipStream_t s, const int32_t* over = nullptr, const int2* pcanvas = nullptr);
-// n_long / n_long_light: the wave-solved chains at the head of the heavy / light launch's range.
 hipError_t launch_chain_order(const uint8_t* chain_cls, uint32_t C, const int32_t* class_count,
-                              int32_t* class_off, int32_t* class_fill, int32_t* n_long, int32_t* light_begin,
-                              int32_t* n_long_light, int32_t* order, int n_cu, hipStream_t s);
-// heavy = 1: the chains of kHeavyCrossings and more; heavy = 0: the rest.  Each launch
-// wave-solves the first *n_long chains of its range and lane-solves the others.  The two
-// launches are independent.
+                              int32_t* class_off, int32_t* class_fill, int32_t* light_begin, int32_t* order,
+                              int n_cu, hipStream_t s);
+// heavy = 1: the chains of kHeavyCrossings and more; heavy = 0: the rest.  The two launches are
+// independent.
 hipError_t launch_chain_solve(const float2* tpos, const uint32_t* cpos, const float* cweight,
-                              const ChainDesc* chains,
-                              const int32_t* order, const int32_t* class_off, const int32_t* n_long,
+                              const ChainDesc* chains, const int32_t* order, const int32_t* class_off,
                               const int32_t* light_begin, int heavy, int32_t* work, float* chain_t, uint8_t* mono,
                               int n_cu, hipStream_t s);
 // Merges each piece's x and y chains into its (curve, t bits) entries, OR-merging equal t (the

@@ -114,7 +114,7 @@ void mvp_inverse(const float m[16], float out[9]) {
 // allocation counters.
 enum {
     kSumCells = 0, kSumSpans, kSumErr, kSumWaveChains, kSumHeavyPieces, kSumLongBands, kSumBigBands,
-    kSumTotal, kSumOver, kSumOverflow, kSumLive, kSumArena, kSumSorted, kSumCapR, kSumWaveChainsLight, kSumCount
+    kSumTotal, kSumOver, kSumOverflow, kSumLive, kSumArena, kSumSorted, kSumCapR, kSumCount
 };
 static_assert(kSumCount <= spr::kSummaryMax, "summary slots");
 
@@ -409,8 +409,7 @@ void chain_setup(spr_handle* H, int64_t n, int32_t* d_cc, const int2* pcanvas, c
                                    H->ncuts.p, H->counts.p, C, (int)H->w, (int)H->h, H->chains.p, H->pieces.p,
                                    H->chain_cls.p, d_cc, H->n_cu, s, over, pcanvas));
     SPR_HIP(spr::launch_chain_order(H->chain_cls.p, C, d_cc, d_cc + spr::kCcOff, d_cc + spr::kCcFill,
-                                    d_cc + spr::kCcNLong, d_cc + spr::kCcLightBegin, d_cc + spr::kCcNLongLight,
-                                    H->chain_order.p, H->n_cu, s));
+                                    d_cc + spr::kCcLightBegin, H->chain_order.p, H->n_cu, s));
 }
 
 // Chain solve and piece kernels of one frame, on two streams: the heavy solve runs on the main
@@ -423,16 +422,14 @@ void solve_and_pieces(spr_handle* H, uint32_t C, int32_t* d_cc, const spr::FragA
     // stages bracket exactly the device time of each stage's own kernels
     hipStream_t s = H->stream, s2 = serial(H) ? H->stream : H->stream2;
     const int32_t* d_coff = d_cc + spr::kCcOff;
-    const int32_t* d_nlong = d_cc + spr::kCcNLong;
     const int32_t* d_lb = d_cc + spr::kCcLightBegin;
     const spr::PieceLists L{H->lo_list.p, H->lo_cnt.p, H->wave_list.p, d_cc + spr::kCcWavePieces, H->heavy_list.p,
                             d_cc + spr::kCcHeavyPieces};
     SPR_HIP(hipEventRecord(H->ev_fork, s));
-    SPR_HIP(spr::launch_chain_solve(H->tpos.p, H->cpos.p, H->arcw(), H->chains.p, H->chain_order.p, d_coff, d_nlong, d_lb, 1,
+    SPR_HIP(spr::launch_chain_solve(H->tpos.p, H->cpos.p, H->arcw(), H->chains.p, H->chain_order.p, d_coff, d_lb, 1,
                                     d_cc + spr::kCcWork, H->chain_t.p, H->mono.p, n_cu_solve, s));
     SPR_HIP(hipStreamWaitEvent(s2, H->ev_fork, 0));
-    SPR_HIP(spr::launch_chain_solve(H->tpos.p, H->cpos.p, H->arcw(), H->chains.p, H->chain_order.p, d_coff,
-                                    d_cc + spr::kCcNLongLight, d_lb, 0,
+    SPR_HIP(spr::launch_chain_solve(H->tpos.p, H->cpos.p, H->arcw(), H->chains.p, H->chain_order.p, d_coff, d_lb, 0,
                                     d_cc + spr::kCcWorkLight, H->chain_t.p, H->mono.p, n_cu_solve, s2));
     if (s2 == s) stage_mark(H, 5);  // serial: both solves, then every piece kernel
     SPR_HIP(hipEventRecord(H->ev_light, s2));
@@ -655,8 +652,7 @@ void run_frame(spr_handle* H, bool record_begin = true) {
     S.p[kSumCells] = d_totals;
     S.p[kSumSpans] = d_totals + 1;
     S.p[kSumErr] = d_err;
-    S.p[kSumWaveChains] = gen ? d_cc + (by_chain ? spr::kCcNLong : kCcSplit) : nullptr;
-    S.p[kSumWaveChainsLight] = gen && by_chain ? d_cc + spr::kCcNLongLight : nullptr;
+    S.p[kSumWaveChains] = gen ? d_cc + (by_chain ? spr::kCcLightBegin : kCcSplit) : nullptr;
     S.p[kSumHeavyPieces] = gen ? d_cc + (by_chain ? spr::kCcHeavyPieces : kCcBigPieces) : nullptr;
     S.p[kSumLongBands] = reinterpret_cast<const int32_t*>(ctl_at(H, z.st_wind, z.ctr, 4).counter + 1);
     S.p[kSumBigBands] = d_bigcount;
@@ -1062,8 +1058,7 @@ void run_learned_frame(spr_handle* H) {
     S.p[kSumCells] = d_totals;
     S.p[kSumSpans] = d_totals + 1;
     S.p[kSumErr] = d_err;
-    S.p[kSumWaveChains] = C ? d_cc + (by_chain ? spr::kCcNLong : kCcSplit) : nullptr;
-    S.p[kSumWaveChainsLight] = C && by_chain ? d_cc + spr::kCcNLongLight : nullptr;
+    S.p[kSumWaveChains] = C ? d_cc + (by_chain ? spr::kCcLightBegin : kCcSplit) : nullptr;
     S.p[kSumHeavyPieces] = C ? d_cc + (by_chain ? spr::kCcHeavyPieces : kCcBigPieces) : nullptr;
     S.p[kSumLongBands] = reinterpret_cast<const int32_t*>(ticket + 1);
     S.p[kSumBigBands] = d_bigcount;
@@ -1230,7 +1225,7 @@ void sync_stats(spr_handle* H) {
     }
     H->stats.n_cells = H->sum(kSumCells);
     H->stats.n_spans = H->sum(kSumSpans);
-    H->stats.n_wave_chains = H->sum(kSumWaveChains) + H->sum(kSumWaveChainsLight);
+    H->stats.n_wave_chains = H->sum(kSumWaveChains);
     H->stats.n_heavy_pieces = H->sum(kSumHeavyPieces);
     H->stats.n_long_bands = H->sum(kSumLongBands);
     H->stats.n_big_bands = H->sum(kSumBigBands);
