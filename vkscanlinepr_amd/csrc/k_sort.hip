@@ -548,31 +548,161 @@ __global__ __launch_bounds__(kClassifyThreads) void k_band_classify2(const int32
     }
 }
 
+// The oversized bands of frames with emit, one workgroup each.  Such a band is one (path, cell
+// row) bucket, so its entries differ only in their cell column and need no sort: their winding
+// changes are summed per column in LDS (16 KiB for the widest canvas), and one scan over the
+// columns gives every cell's winding number, the cells and the spans.  The words are read once
+// and nothing but records is written; a merge sort of the band passed over it log2(n / 2048)
+// times through memory, on one compute unit.  The off-canvas bucket holds no cell: it has
+// no records, whatever its size.
+constexpr int kCols = 8192 / 2 + 3;  // columns -1 .. (w & ~1) / 2 + 1 of the widest canvas
+struct ColumnLds {
+    int32_t sum[kCols];
+    uint32_t has[(kCols + 31) / 32];
+    int32_t w[16], last[16];  // per wave
+};
+struct BigJob {
+    const int32_t* list;
+    const int32_t* excl;
+    const int32_t* count;
+};
+// Workgroup `group` of `groups`, of THREADS threads each.
+template <int THREADS>
+__device__ __forceinline__ void big_bands(const BigJob& G, const int32_t* __restrict__ band_start,
+                                          const uint32_t* __restrict__ src, const int2* __restrict__ band_pr,
+                                          const EmitArgs& E, int32_t group, int32_t groups, ColumnLds& L) {
+    static_assert(THREADS <= 16 * 64 && (kCols + THREADS - 1) / THREADS <= 32, "columns of a thread");
+    int32_t* s_sum = L.sum;
+    uint32_t* s_has = L.has;
+    int32_t* s_w = L.w;
+    int32_t* s_last = L.last;
+    const int32_t* __restrict__ big_list = G.list;
+    const int32_t* __restrict__ big_excl = G.excl;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int32_t nbig = *G.count;
+    for (int32_t q = group; q < nbig; q += groups) {
+        const int32_t band = big_list[q];
+        const int64_t s = band_start[band];
+        const int32_t n = (int32_t)(band_start[band + 1] - s);
+        const int2 pr = band_pr[band];
+        const BandPath b = band_path_of(E, band, pr, s);
+        const uint32_t* w = src + s;
+        const int loc = (int)(w[0] >> 17);
+        if (loc == pr.y) {
+            if (tid == 0) E.band_cnt[band] = make_int2(0, 0);
+            continue;
+        }
+        for (int i = tid; i < kCols; i += THREADS) s_sum[i] = 0;
+        for (int i = tid; i < (kCols + 31) / 32; i += THREADS) s_has[i] = 0u;
+        __syncthreads();
+        for (int32_t i = tid; i < n; i += THREADS) {
+            const uint32_t v = w[i];
+            const int col = min((int)((v >> 3) & 0x3FFFu), kCols - 1);
+            const int32_t wn = wn_of(v);
+            if (!((s_has[col >> 5] >> (col & 31)) & 1u)) atomicOr(&s_has[col >> 5], 1u << (col & 31));
+            if (wn) atomicAdd(&s_sum[col], wn);
+        }
+        __syncthreads();
+        // thread t owns columns t * per ..; what it needs of the columns before: their winding sum
+        // and the last one with an entry
+        constexpr int kPer = (kCols + THREADS - 1) / THREADS;
+        const int c0 = tid * kPer;
+        int32_t sum = 0, last = -1;
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            const int c = c0 + k;
+            if (c < kCols && ((s_has[c >> 5] >> (c & 31)) & 1u)) { sum = wadd(sum, s_sum[c]); last = c; }
+        }
+        int32_t tot;
+        int32_t run = wadd(big_excl[q], block_exclusive_add<int32_t, THREADS / 64>(sum, s_w, tot));
+        int32_t prev = last;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int32_t u = __shfl_up(prev, o);
+            if (lane >= o) prev = max(prev, u);
+        }
+        if (lane == 63) s_last[wave] = prev;
+        prev = __shfl_up(prev, 1);
+        if (lane == 0) prev = -1;
+        __syncthreads();
+        for (int k = 0; k < wave; ++k) prev = max(prev, s_last[k]);
+        const int y = loc < pr.y ? 2 * (pr.x + loc) : 0;
+        uint32_t cells = 0, spans = 0;
+        int32_t from = prev;
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            const int c = c0 + k;
+            if (c >= kCols || !((s_has[c >> 5] >> (c & 31)) & 1u)) continue;
+            const int x = 2 * c - 2;
+            const int32_t wn = (int32_t)((uint32_t)run - (uint32_t)b.wb);
+            const bool fills = (b.rule == 0u && wn != 0) || (b.rule == 1u && (wn & 1) != 0);
+            if (x >= 0 && x < b.cw && y < b.ch) cells |= 1u << k;
+            if (from >= 0 && from + 1 < c && fills) spans |= 1u << k;
+            run = wadd(run, s_sum[c]);
+            from = c;
+        }
+        __syncthreads();  // s_w is used again
+        int32_t total;
+        int32_t ex = block_exclusive_add<int32_t, THREADS / 64>(__popc(cells) | (__popc(spans) << 16), s_w, total);
+        int64_t pos = b.r0 + (ex & 0xFFFF) + (ex >> 16);
+        from = prev;
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            const int c = c0 + k;
+            if (c >= kCols || !((s_has[c >> 5] >> (c & 31)) & 1u)) continue;
+            const int x = 2 * c - 2;
+            if ((cells >> k) & 1u) E.crec[pos++] = (uint32_t)x | (2u << 16);
+            if ((spans >> k) & 1u) {
+                const int x0 = max(0, 2 * from);
+                E.crec[pos++] = (uint32_t)x0 | ((uint32_t)(x - x0) << 16);
+            }
+            from = c;
+        }
+        if (tid == 0) {
+            const int32_t nc = total & 0xFFFF, ns = total >> 16;
+            E.band_cnt[band] = make_int2(nc, ns);
+            if (y < b.ch && loc < pr.y + 2) E.brec[b.bb + loc] = make_int2((int32_t)b.r0, (int32_t)(b.r0 + nc + ns));
+        }
+        __syncthreads();  // the LDS is used again
+    }
+}
+
+constexpr int kColThreads = 1024;
+__global__ __launch_bounds__(kColThreads) void k_big_bands(const BigJob G, const int32_t* __restrict__ band_start,
+                                                           const uint32_t* __restrict__ src,
+                                                           const int2* __restrict__ band_pr, const EmitArgs E) {
+    __shared__ ColumnLds L;
+    big_bands<kColThreads>(G, band_start, src, band_pr, E, (int32_t)blockIdx.x, (int32_t)gridDim.x, L);
+}
+
 // CLS 0: every band of up to 512 words, one wave each (four per workgroup; the others are
 // skipped).  CLS 1: the listed bands of 513..1024 words (16 per lane).  CLS 2: the listed bands of
 // 1025..2048 words (32 per lane); k_band_classify2 queues the longer ones (single oversized
 // buckets) for k_big_bands.
+struct BandJob {
+    const int32_t* band_start;
+    const int32_t* n_bands;
+    const uint32_t* src;
+    const int32_t* bpre;
+    const int2* band_pr;
+    const int32_t* list;
+    int64_t cap;
+    const uint32_t* count;
+};
+constexpr int kClassWords(int cls) { return cls == 0 ? 8 : (cls == 1 ? 16 : 32); }  // per lane, at most
+
+// The band of wave w of a class's waves; lds: 128 * kClassWords words of the wave (the transposed load,
+// 64 R + 64 words, then the records, up to 128 R).
 template <int CLS>
-__global__ __launch_bounds__(256) void k_sort_bands_wave(const int32_t* __restrict__ band_start,
-                                                         const int32_t* __restrict__ n_bands,
-                                                         const uint32_t* __restrict__ src,
-                                                         const int32_t* __restrict__ bpre,
-                                                         const int2* __restrict__ band_pr,
-                                                         const int32_t* __restrict__ list, int64_t cap,
-                                                         const uint32_t* __restrict__ count, EmitArgs EA) {
-    constexpr int RMAX = CLS == 0 ? 8 : (CLS == 1 ? 16 : 32);
-    __shared__ uint32_t s_lds[4][128 * RMAX];  // the transposed load (64 R + 64), then the records (<= 128 R)
-    const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (w >= (CLS == 0 ? (int64_t)*n_bands : (int64_t)count[CLS - 1])) return;  // wave-uniform
-    const int64_t t = CLS == 0 ? w : (CLS == 1 ? list[w] : list[cap - 1 - w]);
-    const int64_t s = band_start[t], n = band_start[t + 1] - s;
+__device__ __forceinline__ void sort_band(const BandJob& J, const EmitArgs& EA, int64_t w, uint32_t* lds) {
+    if (w >= (CLS == 0 ? (int64_t)*J.n_bands : (int64_t)J.count[CLS - 1])) return;  // wave-uniform
+    const int64_t t = CLS == 0 ? w : (CLS == 1 ? J.list[w] : J.list[J.cap - 1 - w]);
+    const int64_t s = J.band_start[t], n = J.band_start[t + 1] - s;
     if (CLS == 0 && n > kSmallBandMax) return;
-    const uint32_t* p = src + s;
-    const int2 pr = band_pr[t];
-    const int32_t pre = bpre[t];
+    const uint32_t* p = J.src + s;
+    const int2 pr = J.band_pr[t];
+    const int32_t pre = J.bpre[t];
     const int m = (int)n;
-    uint32_t* lds = s_lds[threadIdx.x >> 6];
     if constexpr (CLS == 2) {
         wave_band<32>(p, m, t, s, pre, pr, EA, lds);
     } else if constexpr (CLS == 1) {
@@ -583,6 +713,36 @@ __global__ __launch_bounds__(256) void k_sort_bands_wave(const int32_t* __restri
         else if (m <= 256) wave_band<4>(p, m, t, s, pre, pr, EA, lds);
         else wave_band<8>(p, m, t, s, pre, pr, EA, lds);
     }
+}
+
+template <int CLS>
+__global__ __launch_bounds__(256) void k_sort_bands_wave(const BandJob J, const EmitArgs EA) {
+    __shared__ uint32_t s_lds[4][128 * kClassWords(CLS)];
+    const int wave = threadIdx.x >> 6;
+    sort_band<CLS>(J, EA, (int64_t)blockIdx.x * 4 + wave, s_lds[wave]);
+}
+
+// The three classes and the oversized bands in one launch, the longest first: frames of few bands,
+// where a launch costs 4.5 us and the launches would follow each other with the chip nearly empty.
+// Everything has the registers and the 64 KB of the longest class (two workgroups on a CU), so frames
+// of many bands keep a launch per class.  us a frame, four launches and one: 0.1 M entries in
+// 600 bands 270 and 258, 0.8 M in 1,600 132 and 127; 1.9 M in 20,000 short bands 412 and 432.
+__global__ __launch_bounds__(256) void k_sort_bands_all(const BandJob J, const BigJob G, const EmitArgs EA, int big,
+                                                        int large, int medium) {
+    __shared__ union {
+        uint32_t words[4][128 * kClassWords(2)];
+        ColumnLds columns;
+    } s_lds;
+    const int wave = threadIdx.x >> 6;
+    int b = (int)blockIdx.x;
+    if (b < big) {
+        big_bands<256>(G, J.band_start, J.src, J.band_pr, EA, b, big, s_lds.columns);
+        return;
+    }
+    b -= big;
+    if (b < large) sort_band<2>(J, EA, (int64_t)b * 4 + wave, s_lds.words[wave]);
+    else if (b < large + medium) sort_band<1>(J, EA, (int64_t)(b - large) * 4 + wave, s_lds.words[wave]);
+    else sort_band<0>(J, EA, (int64_t)(b - large - medium) * 4 + wave, s_lds.words[wave]);
 }
 
 // BIG = false: the bands of up to THREADS * kItems entries, the workgroups striding over all
@@ -714,113 +874,6 @@ __global__ __launch_bounds__(kBigThreads) void k_sort_big_bands(const int32_t* _
 
 namespace {
 
-// The oversized bands of frames with emit, one workgroup each.  Such a band is one (path, cell
-// row) bucket, so its entries differ only in their cell column and need no sort: their winding
-// changes are summed per column in LDS (16 KiB for the widest canvas), and one scan over the
-// columns gives every cell's winding number, the cells and the spans.  The words are read once
-// and nothing but records is written; a merge sort of the band passed over it log2(n / 2048)
-// times through memory, on one compute unit.  The off-canvas bucket holds no cell: it has
-// no records, whatever its size.
-constexpr int kColThreads = 1024;
-constexpr int kCols = 8192 / 2 + 3;  // columns -1 .. (w & ~1) / 2 + 1 of the widest canvas
-__global__ __launch_bounds__(kColThreads) void k_big_bands(const int32_t* __restrict__ band_start,
-                                                           const int32_t* __restrict__ big_list,
-                                                           const int32_t* __restrict__ big_excl,
-                                                           const int32_t* __restrict__ big_count,
-                                                           const uint32_t* __restrict__ src,
-                                                           const int2* __restrict__ band_pr, EmitArgs E) {
-    __shared__ int32_t s_sum[kCols];
-    __shared__ uint32_t s_has[(kCols + 31) / 32];
-    __shared__ int32_t s_w[kColThreads / 64], s_last[kColThreads / 64];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int32_t nbig = *big_count;
-    for (int32_t q = blockIdx.x; q < nbig; q += gridDim.x) {
-        const int32_t band = big_list[q];
-        const int64_t s = band_start[band];
-        const int32_t n = (int32_t)(band_start[band + 1] - s);
-        const int2 pr = band_pr[band];
-        const BandPath b = band_path_of(E, band, pr, s);
-        const uint32_t* w = src + s;
-        const int loc = (int)(w[0] >> 17);
-        if (loc == pr.y) {
-            if (tid == 0) E.band_cnt[band] = make_int2(0, 0);
-            continue;
-        }
-        for (int i = tid; i < kCols; i += kColThreads) s_sum[i] = 0;
-        for (int i = tid; i < (kCols + 31) / 32; i += kColThreads) s_has[i] = 0u;
-        __syncthreads();
-        for (int32_t i = tid; i < n; i += kColThreads) {
-            const uint32_t v = w[i];
-            const int col = min((int)((v >> 3) & 0x3FFFu), kCols - 1);
-            const int32_t wn = wn_of(v);
-            if (!((s_has[col >> 5] >> (col & 31)) & 1u)) atomicOr(&s_has[col >> 5], 1u << (col & 31));
-            if (wn) atomicAdd(&s_sum[col], wn);
-        }
-        __syncthreads();
-        // thread t owns columns t * per ..; what it needs of the columns before: their winding sum
-        // and the last one with an entry
-        constexpr int kPer = (kCols + kColThreads - 1) / kColThreads;
-        const int c0 = tid * kPer;
-        int32_t sum = 0, last = -1;
-#pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-            const int c = c0 + k;
-            if (c < kCols && ((s_has[c >> 5] >> (c & 31)) & 1u)) { sum = wadd(sum, s_sum[c]); last = c; }
-        }
-        int32_t tot;
-        int32_t run = wadd(big_excl[q], block_exclusive_add<int32_t, kColThreads / 64>(sum, s_w, tot));
-        int32_t prev = last;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int32_t u = __shfl_up(prev, o);
-            if (lane >= o) prev = max(prev, u);
-        }
-        if (lane == 63) s_last[wave] = prev;
-        prev = __shfl_up(prev, 1);
-        if (lane == 0) prev = -1;
-        __syncthreads();
-        for (int k = 0; k < wave; ++k) prev = max(prev, s_last[k]);
-        const int y = loc < pr.y ? 2 * (pr.x + loc) : 0;
-        uint32_t cells = 0, spans = 0;
-        int32_t from = prev;
-#pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-            const int c = c0 + k;
-            if (c >= kCols || !((s_has[c >> 5] >> (c & 31)) & 1u)) continue;
-            const int x = 2 * c - 2;
-            const int32_t wn = (int32_t)((uint32_t)run - (uint32_t)b.wb);
-            const bool fills = (b.rule == 0u && wn != 0) || (b.rule == 1u && (wn & 1) != 0);
-            if (x >= 0 && x < b.cw && y < b.ch) cells |= 1u << k;
-            if (from >= 0 && from + 1 < c && fills) spans |= 1u << k;
-            run = wadd(run, s_sum[c]);
-            from = c;
-        }
-        __syncthreads();  // s_w is used again
-        int32_t total;
-        int32_t ex = block_exclusive_add<int32_t, kColThreads / 64>(__popc(cells) | (__popc(spans) << 16), s_w, total);
-        int64_t pos = b.r0 + (ex & 0xFFFF) + (ex >> 16);
-        from = prev;
-#pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-            const int c = c0 + k;
-            if (c >= kCols || !((s_has[c >> 5] >> (c & 31)) & 1u)) continue;
-            const int x = 2 * c - 2;
-            if ((cells >> k) & 1u) E.crec[pos++] = (uint32_t)x | (2u << 16);
-            if ((spans >> k) & 1u) {
-                const int x0 = max(0, 2 * from);
-                E.crec[pos++] = (uint32_t)x0 | ((uint32_t)(x - x0) << 16);
-            }
-            from = c;
-        }
-        if (tid == 0) {
-            const int32_t nc = total & 0xFFFF, ns = total >> 16;
-            E.band_cnt[band] = make_int2(nc, ns);
-            if (y < b.ch && loc < pr.y + 2) E.brec[b.bb + loc] = make_int2((int32_t)b.r0, (int32_t)(b.r0 + nc + ns));
-        }
-        __syncthreads();  // the LDS is used again
-    }
-}
-
 // Workgroups per CU for a class: as many as the CU's 32 wave slots and 160 KiB of LDS allow.
 template <class T, int THREADS>
 unsigned class_grid(int64_t max_bands, int n_cu) {
@@ -863,24 +916,34 @@ hipError_t launch_sort_bands(const int32_t* band_start, const int32_t* n_bands, 
     return e;
 }
 
+constexpr int64_t kFewBands = 8192;  // k_sort_bands_all
+
 // The bands of frames with emit (after launch_band_classify): one wave per band, four bands per
 // workgroup; the bands above 512 words (at most N / 513 of them) in later launches.
 hipError_t launch_sort_bands_emit(const int32_t* band_start, const int32_t* n_bands, int64_t max_bands,
                                   const unsigned long long* src, const int32_t* big_list, const int32_t* bpre,
-                                  const uint32_t* ticket, const int2* band_pr, const EmitArgs& emit,
-                                  int64_t n_entries, hipStream_t s, hipStream_t s_small) {
+                                  const uint32_t* ticket, const int32_t* big_count, const int2* band_pr,
+                                  const EmitArgs& emit, int64_t n_entries, int n_cu, hipStream_t s,
+                                  hipStream_t s_small) {
     if (max_bands <= 0) return hipSuccess;
-    const uint32_t* w = reinterpret_cast<const uint32_t*>(src);
-    const int32_t* lists = big_list + 2 * max_bands;  // 2 * max_bands slots: both lists of long bands
-    const int64_t cap = 2 * max_bands;
-    k_sort_bands_wave<0><<<(unsigned)((max_bands + 3) / 4), 256, 0, s_small>>>(band_start, n_bands, w, bpre, band_pr,
-                                                                               lists, cap, ticket + 1, emit);
-    const int64_t max_med = std::min<int64_t>(max_bands, n_entries / (kSmallBandMax + 1) + 1);
-    k_sort_bands_wave<1><<<(unsigned)((max_med + 3) / 4), 256, 0, s>>>(band_start, n_bands, w, bpre, band_pr, lists,
-                                                                       cap, ticket + 1, emit);
-    const int64_t max_large = std::min<int64_t>(max_bands, n_entries / (kMediumBandMax + 1) + 1);
-    k_sort_bands_wave<2><<<(unsigned)((max_large + 3) / 4), 256, 0, s>>>(band_start, n_bands, w, bpre, band_pr, lists,
-                                                                         cap, ticket + 1, emit);
+    // 2 * max_bands slots: both lists of long bands
+    const BandJob J{band_start, n_bands, reinterpret_cast<const uint32_t*>(src), bpre, band_pr,
+                    big_list + 2 * max_bands, 2 * max_bands, ticket + 1};
+    auto groups = [](int64_t waves) { return (unsigned)((waves + 3) / 4); };
+    const unsigned large = groups(std::min<int64_t>(max_bands, n_entries / (kMediumBandMax + 1) + 1));
+    const unsigned medium = groups(std::min<int64_t>(max_bands, n_entries / (kSmallBandMax + 1) + 1));
+    const BigJob G{big_list, big_list + max_bands, big_count};
+    if (max_bands <= kFewBands && s == s_small) {
+        // a workgroup per band that N entries can make oversized, up to one per CU
+        const unsigned big = (unsigned)std::min<int64_t>(n_cu, n_entries / (kWaveBandMax + 1));
+        k_sort_bands_all<<<big + large + medium + groups(max_bands), 256, 0, s>>>(J, G, emit, (int)big, (int)large,
+                                                                                  (int)medium);
+        return hipGetLastError();
+    }
+    k_big_bands<<<(unsigned)n_cu, kColThreads, 0, s_small>>>(G, band_start, J.src, band_pr, emit);
+    k_sort_bands_wave<0><<<groups(max_bands), 256, 0, s_small>>>(J, emit);
+    k_sort_bands_wave<1><<<medium, 256, 0, s>>>(J, emit);
+    k_sort_bands_wave<2><<<large, 256, 0, s>>>(J, emit);
     return hipGetLastError();
 }
 
@@ -892,14 +955,6 @@ hipError_t launch_band_classify(const int32_t* band_start, const int32_t* n_band
     k_band_classify2<<<(unsigned)((max_bands + kClassifyThreads - 1) / kClassifyThreads), kClassifyThreads, 0, s>>>(
         band_start, n_bands, lists, 2 * max_bands, ticket + 1, bsum, ctl.status, ctl.counter, big_list, big_excl,
         big_count);
-    return hipGetLastError();
-}
-
-hipError_t launch_big_bands(const int32_t* band_start, const int32_t* big_list, const int32_t* big_excl,
-                            const int32_t* big_count, const unsigned long long* src, const int2* band_pr,
-                            const EmitArgs& emit, int n_cu, hipStream_t s) {
-    k_big_bands<<<(unsigned)n_cu, kColThreads, 0, s>>>(band_start, big_list, big_excl, big_count,
-                                                       reinterpret_cast<const uint32_t*>(src), band_pr, emit);
     return hipGetLastError();
 }
 

@@ -327,19 +327,17 @@ hipError_t launch_sort_big_bands(const int32_t* band_start, const int32_t* big_l
 // Bands of frames with emit (narrow words; EmitArgs).  launch_band_classify comes first: it scans the
 // bands' sums of winding changes in place, lists the bands of 513..1024 and 1025..2048 words
 // (ticket[1..2] count them) and queues the longer ones with their exclusive prefixes (big_count
-// zeroed).  launch_big_bands and the sort of the
-// bands of up to 512 words (s_small) may run on another stream, which the caller forks from s
-// after the classify pass and joins.  n_entries: an upper bound of the sorted entries.
+// zeroed).  launch_sort_bands_emit sorts and emits them all; in frames of many bands the oversized
+// ones and those of up to 512 words run on s_small, which may be another stream that the caller
+// forks from s after the classify pass and joins.  n_entries: an upper bound of the sorted entries.
 hipError_t launch_band_classify(const int32_t* band_start, const int32_t* n_bands, int64_t max_bands,
                                 int32_t* bsum, ScanCtl ctl, int32_t* big_list, int32_t* big_excl,
                                 int32_t* big_count, uint32_t* ticket, hipStream_t s);
 hipError_t launch_sort_bands_emit(const int32_t* band_start, const int32_t* n_bands, int64_t max_bands,
                                   const unsigned long long* src, const int32_t* big_list, const int32_t* bpre,
-                                  const uint32_t* ticket, const int2* band_pr, const EmitArgs& emit,
-                                  int64_t n_entries, hipStream_t s, hipStream_t s_small);
-hipError_t launch_big_bands(const int32_t* band_start, const int32_t* big_list, const int32_t* big_excl,
-                            const int32_t* big_count, const unsigned long long* src, const int2* band_pr,
-                            const EmitArgs& emit, int n_cu, hipStream_t s);
+                                  const uint32_t* ticket, const int32_t* big_count, const int2* band_pr,
+                                  const EmitArgs& emit, int64_t n_entries, int n_cu, hipStream_t s,
+                                  hipStream_t s_small);
 // ---- winding / mark / emit (a10 scan, a11); also writes each (path, row) bucket's record range
 hipError_t launch_mark_emit(const int32_t* skey, const int32_t* winding, const uint32_t* epath,
                             const uint32_t* rule, const uint32_t* fill, int64_t N, int w, int h,

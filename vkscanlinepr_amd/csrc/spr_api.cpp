@@ -612,10 +612,8 @@ void run_frame(spr_handle* H, bool record_begin = true) {
                 SPR_HIP(hipEventRecord(H->ev_sfork, s));
                 SPR_HIP(hipStreamWaitEvent(s2, H->ev_sfork, 0));
             }
-            SPR_HIP(spr::launch_big_bands(H->band_start.p, H->big_list.p, H->big_list.p + max_bands, d_bigcount,
-                                          H->sbig.p, H->band_pr.p, E, H->n_cu, s2));
             SPR_HIP(spr::launch_sort_bands_emit(H->band_start.p, H->bflag.p + NB, max_bands, H->sbig.p, H->big_list.p,
-                                                d_bsum, ticket, H->band_pr.p, E, N, s, s2));
+                                                d_bsum, ticket, d_bigcount, H->band_pr.p, E, N, H->n_cu, s, s2));
             if (s2 != s) {
                 SPR_HIP(hipEventRecord(H->ev_sjoin, s2));  // after the short bands' sort on s2
                 SPR_HIP(hipStreamWaitEvent(s, H->ev_sjoin, 0));
@@ -1022,10 +1020,8 @@ void run_learned_frame(spr_handle* H) {
             SPR_HIP(hipEventRecord(H->ev_sfork, s));
             SPR_HIP(hipStreamWaitEvent(sb, H->ev_sfork, 0));
         }
-        SPR_HIP(spr::launch_big_bands(H->band_start.p, H->big_list.p, H->big_list.p + max_bands, d_bigcount,
-                                      H->sbig.p, H->band_pr.p, E, H->n_cu, sb));
         SPR_HIP(spr::launch_sort_bands_emit(H->band_start.p, d_nbands, max_bands, H->sbig.p, H->big_list.p,
-                                            H->bsum_l.p, ticket, H->band_pr.p, E, nl, s, sb));
+                                            H->bsum_l.p, ticket, d_bigcount, H->band_pr.p, E, nl, H->n_cu, s, sb));
         if (sb != s) {
             SPR_HIP(hipEventRecord(H->ev_sjoin, sb));  // after the short bands' sort on sb
             SPR_HIP(hipStreamWaitEvent(s, H->ev_sjoin, 0));
