@@ -37,9 +37,9 @@
 //
 // Anti-aliased coverage (src-over): a boundary cell record whose 64-sample mask (k_aa.hip) is not
 // full appends, at each of its two columns, an entry (path of the batch, covered samples of row y,
-// of row y + 1) to that column's list in LDS (at most kAaSlots per column); the fold scales such
-// a path's premultiplied colour by count/16 in each row.  A batch whose lists would overflow is
-// redone with half as many paths (kAaSlots paths can never overflow).
+// of row y + 1) to that column's list in LDS (kAaSlots per column, and kAaMore more in a list for the
+// whole chunk); the fold scales such a path's premultiplied colour by count/16 in each row.  A batch
+// whose lists would overflow is redone with half as many paths (kAaSlots paths can never overflow).
 #include "device_common.hpp"
 #include "kernels.hpp"
 #include "scan_common.hpp"
@@ -51,6 +51,10 @@ namespace {
 constexpr int kStops = 512;                // gradient stops of one batch in LDS
 constexpr int kBatch = 64;                 // paths per coverage mask
 constexpr int kAaSlots = 4;                // partial-coverage entries per column and batch
+// entries of one batch beyond their column's: without them one column of 4,096 with a fifth entry had
+// half of all batches done over (4096^2: 1,284 us, with 16 more 1,150); a pixel with more than its slots
+// reads them all, so a long list (64, 128) costs denser scenes more than the batches it saves
+constexpr int kAaMore = 16;
 constexpr int kList = 512;                 // paths listed before their batches are folded
 constexpr int kListSub = 256;              // a listing step examines candidate paths in parts of this many
 constexpr int kUnroll = 4;                 // records loaded per thread before applying
@@ -255,7 +259,8 @@ __global__ __launch_bounds__(CHUNK / PIX) __attribute__((amdgpu_waves_per_eu(GRA
     // lcnt counts the column's entries
     __shared__ uint16_t lslot[AA ? kAaSlots * CHUNK : 1];
     __shared__ uint32_t lcnt[AA ? CHUNK / 4 : 1];
-    __shared__ int32_t lovf;
+    __shared__ uint32_t lmore[AA ? kAaMore : 1];  // the others: column << 16 | entry
+    __shared__ int32_t lmore_n;
     __shared__ u64 ev[CHUNK];
     __shared__ int2 list[kList];
     __shared__ uint32_t lcol[kList];
@@ -381,7 +386,7 @@ __global__ __launch_bounds__(CHUNK / PIX) __attribute__((amdgpu_waves_per_eu(GRA
             batch:
                 if constexpr (AA != 0) {
                     for (int k = tid; k < CHUNK / 4; k += BLOCK) lcnt[k] = 0u;
-                    if (tid == 0) lovf = 0;
+                    if (tid == 0) lmore_n = 0;
                 }
                 // clear the event words; the batch's colours; its records as one flat index space
 #pragma unroll
@@ -481,10 +486,13 @@ __global__ __launch_bounds__(CHUNK / PIX) __attribute__((amdgpu_waves_per_eu(GRA
                                     const uint32_t n1 = __popcll((cm >> (16 * (2 + px))) & 0xFFFFull);
                                     const uint32_t k = (atomicAdd(&lcnt[col >> 2], 1u << (8 * (col & 3))) >>
                                                         (8 * (col & 3))) & 0xFFu;
-                                    if (k < (uint32_t)kAaSlots)
-                                        lslot[k * CHUNK + col] = (uint16_t)((uint32_t)qi[u] | (n0 << 6) | (n1 << 11));
-                                    else
-                                        lovf = 1;
+                                    const uint32_t e = (uint32_t)qi[u] | (n0 << 6) | (n1 << 11);
+                                    if (k < (uint32_t)kAaSlots) {
+                                        lslot[k * CHUNK + col] = (uint16_t)e;
+                                    } else {
+                                        const int at = atomicAdd(&lmore_n, 1);
+                                        if (at < kAaMore) lmore[at] = ((uint32_t)col << 16) | e;
+                                    }
                                 }
                             }
                         }
@@ -492,7 +500,7 @@ __global__ __launch_bounds__(CHUNK / PIX) __attribute__((amdgpu_waves_per_eu(GRA
                 }
                 __syncthreads();
                 if constexpr (AA != 0) {
-                    if (lovf) {  // some column has more partial cells than slots: fewer paths
+                    if (lmore_n > kAaMore) {  // more partial cells than the lists hold: fewer paths
                         qn = qn / 2;
                         __syncthreads();
                         goto batch;
@@ -553,6 +561,9 @@ __global__ __launch_bounds__(CHUNK / PIX) __attribute__((amdgpu_waves_per_eu(GRA
                                     pm |= 1ull << (pe[k] & 63u);
                                 }
                             }
+                            if (np > (uint32_t)kAaSlots)
+                                for (int i = 0; i < lmore_n; ++i)
+                                    if ((int)(lmore[i] >> 16) == c) pm |= 1ull << (lmore[i] & 63u);
                         }
                     }
                     if constexpr (COMPOSE == 0) {
@@ -594,6 +605,9 @@ __global__ __launch_bounds__(CHUNK / PIX) __attribute__((amdgpu_waves_per_eu(GRA
 #pragma unroll
                                             for (int k = 0; k < kAaSlots; ++k)
                                                 if ((uint32_t)k < np && (pe[k] & 63u) == qq) e = pe[k];
+                                            if (np > (uint32_t)kAaSlots)
+                                                for (int i = 0; i < lmore_n; ++i)
+                                                    if (lmore[i] >> 16 == (uint32_t)c && (lmore[i] & 63u) == qq) e = lmore[i];
                                             s0 = scale(s0, (float)((e >> 6) & 31u) / 16.0f);
                                             s1 = scale(s1, (float)((e >> 11) & 31u) / 16.0f);
                                         }
