@@ -438,7 +438,7 @@ def main(argv=None):
     xc = cubic_crossings(r.export("counts"), r.export("cuts"), scene.arrays()["curve_type"])
     solve_ms = table["chain_solve"]["ms"]
     tflops = SOLVE_FLOP_PER_CUBIC_CROSSING * xc / (solve_ms * 1e-3) / 1e12
-    roof = {"bound": "valu", "kernel": "k_chain_solve (both launches)", "achieved": tflops,
+    roof = {"bound": "valu", "kernel": "k_chain_segments + k_chain_solve", "achieved": tflops,
             "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": tflops / FP32_PEAK_TFLOPS,
             "peak_no_fma_no_packed": VALU_NOFMA_PEAK_TOPS, "frac_no_fma_no_packed": tflops / VALU_NOFMA_PEAK_TOPS,
             "traffic": traffic.get("chain_solve"), "algorithmic_flop": SOLVE_FLOP_PER_CUBIC_CROSSING * xc,

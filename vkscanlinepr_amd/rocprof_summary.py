@@ -22,15 +22,14 @@ STAGE_KERNELS = {
     "transform": ["k_transform"],
     "count": ["k_count"],
     "chain_prep": ["k_chain_prep", "k_chain_order"],
-    "chain_solve": ["k_chain_solve"],
-    "piece_fragments": ["k_piece_small", "k_piece_fragments", "k_piece_waves", "k_piece_heavy"],
+    "chain_solve": ["k_chain_segments", "k_chain_solve"],
+    "piece_fragments": ["k_curves", "k_big_pieces", "k_piece_small", "k_piece_fragments", "k_piece_waves", "k_piece_heavy"],
     "gen_fragment": ["k_gen_fragment"],
-    "bucket_scatter": ["k_bucket_scatter", "k_band_flags", "k_band_emit"],
-    "band_sort": ["k_band_classify2", "k_sort_bands_wave", "k_sort_big_bands", "k_emit_big_bands",
-                  "k_band_totals"],
+    "bucket_scatter": ["k_bands", "k_bucket_scatter"],
+    "band_sort": ["k_band_classify2", "k_sort_bands_wave", "k_sort_bands_all", "k_big_bands"],
     # with mark + emit fused into the band sort (frames that export no stage), the whole sort
-    "sort": ["k_bucket_scatter", "k_band_flags", "k_band_emit", "k_band_classify2", "k_sort_bands_wave",
-             "k_sort_big_bands", "k_emit_big_bands", "k_band_totals", "k_mark_emit"],
+    "sort": ["k_bands", "k_bucket_scatter", "k_band_classify2", "k_sort_bands_wave", "k_sort_bands_all",
+             "k_big_bands", "k_mark_emit"],
     "mark_emit": ["k_mark_emit"],
     "cell_cover": ["k_cell_cover"],
     "composite": ["k_composite"],
