@@ -42,6 +42,8 @@
 #include "kernels.hpp"
 #include "scan_common.hpp"
 
+#include <type_traits>
+
 namespace spr {
 
 namespace {
@@ -59,6 +61,12 @@ constexpr int kStage = 4096;                    // big pieces up to this many en
 // segments that a batch is cut into (besides one per chain).
 constexpr int kWarm = 4, kWarm8 = 8, kWarm16 = 16, kSegMin = 4, kSegTarget = 112;
 constexpr int kSegs = 832;
+// Candidate starts of a batch's slow segments (a multiple of 8 each), and the chains that have any.
+constexpr int kCands = 384, kWalks = 16;
+constexpr int kCand16 = 16, kCand8 = 8;         // below t1 / 16, t1 / 8
+constexpr uint32_t kNoValue = 0xFFFFFFFFu;      // no entry, no value (solved values carry side bits 0 or 1)
+constexpr int64_t kFewWindows = 1024, kLongCurves = 8;  // k_curves
+static_assert(kCands / 8 < 64, "a segment's first candidate in 6 bits");
 // chains are 2 * 320; the segments after a chain's first hold X / kSegTarget or more of the
 // batch's X crossings in all but one of a chain, and only chains of 1.5 of them have any
 static_assert(2 * kSlots + kSegTarget + (2 * kSegTarget) / 3 <= kSegs, "segment list");
@@ -324,10 +332,19 @@ struct CurveBatch {
     unsigned long long starts[kCap / 64];  // bit per entry slot: a piece starts there
     uint16_t starts_before[kCap / 64];
     uint16_t head[2 * kSlots];           // length of each chain's first segment
-    uint32_t seg[kSegs];                 // chain | segment << 10 | crossings to guess its start from << 20
+    // chain | segment << 10 | crossings to guess its start from << 20, kHasCands | first candidate / 8 << 26
+    uint32_t seg[kSegs];
     int n_segs;
     int n_pieces, longest, n_slots, crossings;  // of the batch
 };
+
+struct Candidates {
+    uint32_t cand[kCands];   // chain | segment << 10 | candidate << 20; then the value it ends on
+    uint32_t start[kCands];  // the value it starts from; a segment's first: its predicted start
+    uint2 walk[kWalks];      // chain | segments of kCand16 << 10, of kCand8 << 20; first candidate
+    int n_cands, n_walks;
+};
+constexpr uint32_t kHasCands = 1u << 25;
 
 // The piece that entry slot e lies in or after, -1 before the first.
 __device__ inline int piece_of(const CurveBatch& B, int e) {
@@ -478,6 +495,48 @@ __device__ inline void seg_range(const CurveBatch& B, int ch, int j, int n, int 
     }
 }
 
+// Where t is small, a guess rarely comes true (see above), and correcting one segment after another
+// takes a round each.  The value before such a segment is one of few: the last midpoint of
+// a bisection lies within 2^-24 of its bracket from the root, and masked values are 4 ulp apart.  So the
+// idle threads solve these segments from each of the 16 (t < t1 / 16) or 8 (t < t1 / 8) masked
+// values around the root, one thread each, and one thread per chain then walks its segments from
+// candidate to candidate, which predicts every segment's start at once.  The predictions are
+// checked like all guesses.
+__device__ inline void try_candidates(const CurveBatch& B, Candidates& Q, int n_cands, int S, int len, float* none) {
+    // the waves without segments first; none: nothing is stored there
+    for (int c = ((int)threadIdx.x + kThreads - ((S + 63) & ~63)) & (kThreads - 1); c < n_cands; c += kThreads) {
+        const uint32_t e = Q.cand[c];
+        if (e == kNoValue) continue;
+        const int ch = (int)(e & 1023u), k = (int)(e >> 20);
+        const ChainRef r = chain_of(B, ch);
+        int i0, i1;
+        seg_range(B, ch, (int)((e >> 10) & 1023u), r.n, len, i0, i1);
+        const float root = solve_run_any(r.type, r.a, r.line0, r.neg, r.side, r.t1, i0 - 1, i0, i0, r.t0, false, none);
+        const uint32_t v = ((fbits(root) & 0xFFFFFFFCu) + (uint32_t)(4 * (k - kCand16))) | r.side;
+        Q.start[c] = v;
+        Q.cand[c] = fbits(solve_run_any(r.type, r.a, r.line0, r.neg, r.side, r.t1, i0, i1, i1, bitsf(v), false, none));
+    }
+}
+
+__device__ inline void walk_candidates(const CurveBatch& B, Candidates& Q, const uint2 w) {
+    const int ch = (int)(w.x & 1023u), n16 = (int)((w.x >> 10) & 1023u), n8 = (int)(w.x >> 20);
+    const ChainRef r = chain_of(B, ch);
+    uint32_t v = fbits(B.v[r.at + (int)B.head[ch] - 1]);
+    int c = (int)w.y;
+    for (int j = 0; j < n16 + n8; ++j) {
+        const int n = j < n16 ? kCand16 : kCand8;
+        uint32_t end = kNoValue;
+        if (v != kNoValue) {
+#pragma unroll 8
+            for (int k = 0; k < n; ++k)
+                if (Q.start[c + k] == v) end = Q.cand[c + k];
+        }
+        Q.start[c] = v;
+        v = end;
+        c += n;
+    }
+}
+
 // One workgroup per window of K.window entries.  first[b] is the curve that holds entry b * window.
 // Its span is latency (loads behind each other, chains of dependent solves, LDS searches), so the
 // waves that fit a CU decide its rate: one wave a window left 6 waves on a CU (23 KB of LDS each,
@@ -486,9 +545,17 @@ __device__ inline void seg_range(const CurveBatch& B, int ch, int j, int n, int 
 // the speculative solves per entry.  Frames in turn on three handles, us a frame, one wave and four:
 // 0.8 M entries on a few long curves 203 -> 134, 1.9 M on 20,000 glyphs 299 -> 261.  Two waves a
 // window: 138, 255; four to five per SIMD (96 to 128 VGPRs): 2 to 15% slower.
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6)))
+// CANDS: frames of at most kFewWindows windows, which last as long as their slowest window (a dozen rounds
+// of corrections: 109 us, the mean 42, for 16 paths at 512^2), try candidate starts.  us a frame without
+// and with: 16 paths at 512^2 250 and 229, 64 at 1024^2 126 and 119, a drawing of 0.15 M entries alone 311
+// and 291.  Frames of more windows fill the chip anyway, and the candidates' arithmetic costs more than the
+// rounds: 1.9 M entries 259 and 265, 6.2 M 894 and 939.  So do frames of very short curves, whose chains
+// are not cut: 0.4 M entries on 125,000 curves 203 and 210.
+template <bool CANDS>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CANDS ? 5 : 6)))
 void k_curves(const CurveArgs K, const FragArgs A) {
     __shared__ CurveBatch B;
+    __shared__ typename std::conditional<CANDS, Candidates, int>::type cands;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t total = K.n_dev ? min((int64_t)*K.n_dev, K.n) : K.n;
     const int64_t wb64 = (int64_t)blockIdx.x * K.window;
@@ -520,6 +587,10 @@ void k_curves(const CurveArgs K, const FragArgs A) {
             continue;
         }
         const int bb0 = max(wb, bo);  // the entry of slot 0
+        if constexpr (CANDS) {
+            for (int c = tid; c < kCands; c += kThreads) cands.cand[c] = kNoValue;
+            if (tid == 0) cands.n_cands = cands.n_walks = 0;
+        }
         const bool mine = o0 < wend && o1 > o0 && o1 > wb;
         if (wave == 0) {
             if (lane < kCap / 64) B.starts[lane] = 0ull;
@@ -622,8 +693,9 @@ void k_curves(const CurveArgs K, const FragArgs A) {
             int at = atomicAdd(&B.n_segs, 1 + m);
             B.seg[at++] = (uint32_t)ch;
             if (head >= r.n) continue;
+            const int first = at;
             ++n_split;
-            int k8 = 0, k16 = 0;
+            int k8 = 0, k16 = 0, n8 = 0, n16 = 0;
             if (r.type != kLine) {
                 k8 = crossings_before(r.type, r.a, r.line0, r.neg, r.t0, 0.125f * r.t1, r.n);
                 if (k8) k16 = crossings_before(r.type, r.a, r.line0, r.neg, r.t0, 0.0625f * r.t1, r.n);
@@ -632,10 +704,34 @@ void k_curves(const CurveArgs K, const FragArgs A) {
                 const int i0 = head + seg_begin(r.n - head, m, j);
                 const int warm = i0 >= k8 ? kWarm : (i0 >= k16 ? kWarm8 : kWarm16);
                 B.seg[at++] = (uint32_t)ch | ((uint32_t)(j + 1) << 10) | ((uint32_t)warm << 20);
+                n16 += i0 < k16 ? 1 : 0;
+                n8 += i0 >= k16 && i0 < k8 ? 1 : 0;
+            }
+            if constexpr (CANDS) {
+                // candidate starts for the segments below t1 / 8, as long as there is room
+                const int want = n16 * kCand16 + n8 * kCand8;
+                if (want == 0 || want > kCands) continue;
+                const int c0 = atomicAdd(&cands.n_cands, want);
+                if (c0 + want > kCands) continue;
+                const int w = atomicAdd(&cands.n_walks, 1);
+                if (w >= kWalks) continue;
+                cands.walk[w] = make_uint2((uint32_t)ch | ((uint32_t)n16 << 10) | ((uint32_t)n8 << 20), (uint32_t)c0);
+                for (int j = 0, c = c0; j < n16 + n8; ++j) {
+                    B.seg[first + j] |= kHasCands | ((uint32_t)(c >> 3) << 26);
+                    const int n = j < n16 ? kCand16 : kCand8;
+                    for (int k = 0; k < n; ++k, ++c)  // numbered around kCand16
+                        cands.cand[c] = (uint32_t)ch | ((uint32_t)(j + 1) << 10) | ((uint32_t)(kCand16 - n / 2 + k) << 20);
+                }
             }
         }
         __syncthreads();
         const int S = __builtin_amdgcn_readfirstlane(B.n_segs);
+        int n_cands = 0, n_walks = 0;
+        if constexpr (CANDS) {
+            // only beside a single round of segments
+            if (S <= kThreads) n_cands = min(__builtin_amdgcn_readfirstlane(cands.n_cands), kCands);
+            if (n_cands) n_walks = min(__builtin_amdgcn_readfirstlane(cands.n_walks), kWalks);
+        }
 
         // ---- the crossings, one segment per lane
         for (int s0 = 0; s0 < S; s0 += kThreads) {
@@ -649,15 +745,28 @@ void k_curves(const CurveArgs K, const FragArgs A) {
             // solve, then the guesses against what the segments before ended on: a segment whose
             // guess was off is solved again from there
             float g = r.t0, start = r.t0;
-            int k0 = max(0, i0 - (int)(e >> 20));
+            int k0 = max(0, i0 - (int)((e >> 20) & 31u));
             bool run = on, redo = false;
             for (;;) {
                 if (run) {
                     const float got = solve_run_any(r.type, r.a, r.line0, r.neg, r.side, r.t1, k0, i0, i1, start, redo, vs);
                     if (!redo) g = got;
                 }
+                if constexpr (CANDS) {
+                    if (n_walks && !redo) try_candidates(B, cands, n_cands, S, len, B.v);
+                }
                 __syncthreads();
-                const float is = on && i0 > 0 ? vs[i0 - 1] : g;
+                float is = on && i0 > 0 ? vs[i0 - 1] : g;
+                if constexpr (CANDS) {
+                    if (n_walks && !redo) {
+                        if (tid < n_walks) walk_candidates(B, cands, cands.walk[tid]);
+                        __syncthreads();
+                        if (on && (e & kHasCands)) {
+                            const uint32_t p = cands.start[(e >> 26) * 8];
+                            if (p != kNoValue) is = bitsf(p);
+                        }
+                    }
+                }
                 run = fbits(is) != fbits(g);
                 if (!__syncthreads_or(run ? 1 : 0)) break;
                 g = start = is;
@@ -886,7 +995,9 @@ hipError_t launch_curves(const CurveArgs& K, const FragArgs& A, hipStream_t s) {
     if (K.C == 0 || K.n == 0) return hipSuccess;
     if (K.window < kCurveWindowMin || K.window > kCurveWindowMax) return hipErrorInvalidValue;
     const int64_t g = (K.n + K.window - 1) / K.window;
-    k_curves<<<(unsigned)g, kThreads, 0, s>>>(K, A);
+    // entries per curve: with a few each, hardly a chain is long enough to be cut (see k_curves)
+    if (g <= kFewWindows && K.n >= kLongCurves * (int64_t)K.C) k_curves<true><<<(unsigned)g, kThreads, 0, s>>>(K, A);
+    else k_curves<false><<<(unsigned)g, kThreads, 0, s>>>(K, A);
     return hipGetLastError();
 }
 
