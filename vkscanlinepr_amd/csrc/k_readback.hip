@@ -34,11 +34,12 @@ __global__ __launch_bounds__(kReadThreads) void k_read_out(const uint8_t* __rest
         const uint32_t* s1 = reinterpret_cast<const uint32_t*>(src + o);
         uint32_t* d1 = reinterpret_cast<uint32_t*>(dst + o);
         for (int i = 4 * n16 + (int)threadIdx.x; i < n >> 2; i += kReadThreads) d1[i] = s1[i];
+        // every wave's stores have reached the host before the mark: a fence waits for the stores of
+        // its own wave only, and the barrier for none
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");  // system scope
         __syncthreads();
-        if (threadIdx.x == 0) {
-            __threadfence_system();
+        if (threadIdx.x == 0)
             __hip_atomic_store(&arrived[c], mark, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
     }
 }
 
