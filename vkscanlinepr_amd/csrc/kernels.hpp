@@ -55,7 +55,7 @@ struct CountArgs {
     float4* cuts;
     uint32_t* ncuts;
     int32_t* counts;            // [C + 1]
-    int32_t* seg;               // [Np + 1] entries of all curves of paths < p, or null
+    int32_t* seg;               // [Np + 1] entries of all curves of paths < p (not written without curves), or null
     int curve_tiles;
     unsigned long long* curve_status;
     uint32_t* curve_counter;

@@ -347,7 +347,8 @@ void stage_mark(spr_handle* H, int idx) {
     H->n_marks = idx + 1;
 }
 
-// Clears what the transform and the count pass start from, in one launch.
+// Clears what the transform and the count pass start from, in one launch.  The count pass writes the
+// path segments from its curves, so a scene without any has them cleared here.
 void clear_prefix(spr_handle* H, int64_t control_words) {
     spr::FrameInit init{};
     init.fill[0] = {(uint32_t*)H->zero.p, control_words, nullptr, 0, 0, 0u};
@@ -355,6 +356,7 @@ void clear_prefix(spr_handle* H, int64_t control_words) {
     init.fill[2] = {(uint32_t*)H->row_lo.p, H->Np, nullptr, 0, 0, 0x7FFFFFFFu};
     init.fill[3] = {(uint32_t*)H->row_hi.p, H->Np, nullptr, 0, 0, 0x80000000u};
     init.n_fills = 4;
+    if (!H->C) init.fill[init.n_fills++] = {(uint32_t*)H->seg.p, (int64_t)H->Np + 1, nullptr, 0, 0, 0u};
     SPR_HIP(spr::launch_frame_init(init, H->stream));
 }
 
