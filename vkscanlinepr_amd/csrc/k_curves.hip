@@ -887,7 +887,7 @@ __global__ __launch_bounds__(kBigThreads) void k_big_pieces(const CurveArgs K, c
     __shared__ uint32_t s_flags;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int32_t count = *K.big_count;
-    if (blockIdx.x == 0 && tid == 0 && count) atomicAdd(K.split_count, count);  // both of its chains are long
+    int n_split = 0;
     for (int32_t item = (int32_t)blockIdx.x; item < count; item += (int32_t)gridDim.x) {
         const int32_t slot = K.big[item];
         const uint32_t c = (uint32_t)slot / 5u;
@@ -916,6 +916,7 @@ __global__ __launch_bounds__(kBigThreads) void k_big_pieces(const CurveArgs K, c
         const int hx = min(g.nx, max(len, crossings_before(cv.type, ax, g.x0, g.xneg, g.t0, 0.03125f * g.t1, g.nx)));
         const int hy = min(g.ny, max(len, crossings_before(cv.type, ay, g.y0, g.yneg, g.t0, 0.03125f * g.t1, g.ny)));
         const int sx = g.nx ? 1 + seg_rest(g.nx, hx, len) : 0, sy = g.ny ? 1 + seg_rest(g.ny, hy, len) : 0;
+        n_split += (sx > 1 ? 1 : 0) + (sy > 1 ? 1 : 0);
         const bool on = tid < sx + sy, ys = tid >= sx;
         const int j = ys ? tid - sx : tid, nn = ys ? g.ny : g.nx, head = ys ? hy : hx, rest = max(1, (ys ? sy : sx) - 1);
         int i0 = 0, i1 = on ? head : 0;
@@ -987,6 +988,7 @@ __global__ __launch_bounds__(kBigThreads) void k_big_pieces(const CurveArgs K, c
         }
         __syncthreads();
     }
+    if (tid == 0 && n_split) atomicAdd(K.split_count, n_split);
 }
 
 }  // namespace
