@@ -40,3 +40,41 @@ def test_counts_the_chains_that_are_cut(spr, w, h, nx, ny, cut):
     assert abs(st.n_intersections - 2 * (1 + nx + ny)) <= 4  # both pieces have their long axes
     assert st.n_wave_chains == 2 * cut
     r.close()
+
+
+def _spans(k, n):
+    """A cubic's, quadratic's or line's points from 0 to 1, by k: slow at its start, even, or slow at its end."""
+    return {"slow": (0.0, 0.001, 0.02, 1.0), "even": (0.0, 1 / 3, 2 / 3, 1.0), "late": (0.0, 0.97, 0.999, 1.0),
+            "quad": (0.0, 0.01, 1.0), "line": (0.0, 1.0)}[k][:n]
+
+
+# pieces of 4,096 entries (the most that stay in LDS) and one more, and up to the longest of a canvas
+@pytest.mark.parametrize("w,h,nx,ny", [(64, 16384, 0, 4095), (64, 16384, 0, 4096), (8192, 512, 3850, 245),
+                                       (8192, 512, 3850, 246), (32, 16384, 9, 8180), (8192, 16, 4090, 5),
+                                       (8192, 8192, 4000, 4080)])
+@pytest.mark.parametrize("debug", [True, False])
+def test_pieces_beyond_lds_match_the_oracle(spr, orc, w, h, nx, ny, debug):
+    """Rising and falling curves of every type but arcs, slow and fast at their starts, each closed by a line."""
+    p0 = np.array([3.0, 3.0])
+    d = np.array([2.0 * nx + (0.5 if nx else 0.0), 2.0 * ny + (0.5 if ny else 0.0)])
+    curves = []
+    for k in ("slow", "even", "late", "quad", "line"):
+        pts = [p0 + d * t for t in _spans(k, 4)]
+        curves += [pts, pts[::-1], [np.array([w - q[0], q[1]]) for q in pts]]
+    a = _closed(curves)
+    print(f"[big-pieces] {w}x{h} {nx} {ny} debug={debug}", flush=True)
+    f = orc.Frame(a, w, h, threads=8)
+    o = f.get("inter").reshape(-1, 2)
+    assert np.bincount(o[:, 0]).min() >= 1 + nx + ny - 4  # every curve is one long piece
+    r = spr.Rasterizer(w, h, debug=debug)
+    _load(r, a)
+    r.render(readback=False)
+    st = r.stats()
+    assert st.n_heavy_pieces == len(a["curve_type"]) and st.n_intersections < 1 << 23
+    assert st.n_intersections == len(o)
+    if debug:
+        g = r.export("inter").reshape(-1, 2)
+        bad = np.flatnonzero((g != o).any(1))
+        assert bad.size == 0, (bad.size, bad[:4], g[bad[:4]], o[bad[:4]])
+    assert np.array_equal(r.export("image"), f.image().reshape(-1))
+    r.close()
