@@ -1585,6 +1585,7 @@ int spr_debug_export(spr_handle* H, int stage, void* dst, size_t cap, size_t* nb
     if (!H || !nbytes) { g_error = "null argument"; return SPR_ERR_INVALID; }
     return guarded(H, [&] {
         if (!H->frame_done) throw Fail{SPR_ERR_STATE, "no frame rendered"};
+        SPR_HIP(hipSetDevice(H->device));
         SPR_HIP(hipStreamSynchronize(H->stream));
         const bool debug = H->opts.debug != 0;
         const int64_t N = H->N;
@@ -1834,6 +1835,7 @@ int spr_batch_image(spr_handle* H, uint32_t doc, uint8_t* rgba_out, size_t cap) 
         const spr::DocDev& d = H->h_docs[doc];
         const size_t bytes = (size_t)4 * d.w * d.h;
         if (cap < bytes) throw Fail{SPR_ERR_CAPACITY, "destination too small"};
+        SPR_HIP(hipSetDevice(H->device));
         read_image(H, H->image.p + d.img_off, bytes, rgba_out);
     });
 }
@@ -1844,6 +1846,7 @@ int spr_autotune(spr_handle* H, uint32_t reps, spr_tune_report* out) {
         if (!H->loaded) throw Fail{SPR_ERR_STATE, "autotune before load"};
         if (H->inj) throw Fail{SPR_ERR_STATE, "autotune with injected intersections"};
         if (reps == 0) reps = 3;
+        SPR_HIP(hipSetDevice(H->device));
         const bool nosync = H->batch || (H->opts.mode == SPR_MODE_LEARNED && H->model.ready);
         const bool timing = H->stage_timing;
         H->stage_timing = false;
