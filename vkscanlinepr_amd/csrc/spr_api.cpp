@@ -677,6 +677,15 @@ void run_frame(spr_handle* H, bool record_begin = true) {
 constexpr int kReadSegChunks = 64;                                         // 2 MiB
 constexpr size_t kReadSeg = (size_t)kReadSegChunks * spr::kReadChunk;
 
+// The processor's hint for a polling loop, where it has one.
+inline void poll_hint() {
+#if defined(__x86_64__)
+    __builtin_ia32_pause();
+#elif defined(__aarch64__)
+    __asm__ volatile("yield");
+#endif
+}
+
 void read_image(spr_handle* H, const uint8_t* src, size_t bytes, uint8_t* dst) {
     hipStream_t s = H->stream;
     hipPointerAttribute_t attr{};
@@ -705,7 +714,7 @@ void read_image(spr_handle* H, const uint8_t* src, size_t bytes, uint8_t* dst) {
     // a chunk's mark; a stream that fails or ends without it is an error, not a wait for ever
     auto wait = [&](const uint32_t* a, uint32_t mark) {
         for (uint32_t spins = 1; __atomic_load_n(a, __ATOMIC_ACQUIRE) != mark; ++spins) {
-            __builtin_ia32_pause();
+            poll_hint();
             if (spins % 4096) continue;
             const hipError_t e = hipStreamQuery(s);
             if (e == hipErrorNotReady) { (void)hipGetLastError(); continue; }
