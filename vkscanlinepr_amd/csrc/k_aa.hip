@@ -35,11 +35,13 @@ constexpr int kBlock = 256;
 constexpr int kRecs = 4;                // records per thread and pass
 constexpr int kChunk = kRecs * kBlock;  // records per workgroup pass of the cover kernel
 // Cells of up to kRunMax chords (the run of sorted entries with the cell's key and path) keep what
-// their chords change in LDS; a cell of more is covered by a wave on its own.
-constexpr int kRunMax = 30;
+// their chords change in LDS; the cells of more come in a list, and a wave covers each.
+constexpr int kRunMax = kAaRunMax;
+constexpr int kDenseBlocks = 256;       // workgroups of the listed cells, in front of the others
 constexpr int kSlots = 5 * kBlock;      // chords in LDS at a time, besides the last cell's overhang
 constexpr uint32_t kNoEntry = 0xFFFFFFFFu;
 static_assert(kChunk <= 1024 && kRunMax < 32 && kChunk * kRunMax < 65536, "cell words");
+static_assert(kSlots >= 256 * (kBlock / 64), "words of the waves' listed cells");
 
 // Columns c of two pixels (32 of them, sample x = x0 + (c + 1/2) / 16) whose sample x lies above z:
 // those from the returned one on.  x32 = 32 x0, an integer below 2^20.  All values are exact: x > z
@@ -147,14 +149,21 @@ __device__ inline unsigned long long cell_mask(const uint32_t* head, const uint3
     return m;
 }
 
-// A cell of any number of chords by a whole wave, one sample a lane (lane = its bit in the mask), 64
-// chords loaded at a time.  All lanes take part.
-__device__ inline unsigned long long cover_open(int32_t f, const int32_t* __restrict__ skey,
+// Orders within one wave: LDS written by some lanes and then read by others.
+__device__ inline void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// A cell of any number of chords by a whole wave, 64 chords at a time: each chord's own values one lane per
+// chord, into the wave's words of `at` and `of` (LDS, four and three rows of 64), then what the chords change
+// one sample per lane (lane = its bit in the mask).  All lanes take part.
+__device__ inline unsigned long long cover_dense(int32_t f, const int32_t* __restrict__ skey,
                                                 const int32_t* __restrict__ sidx,
                                                 const int32_t* __restrict__ winding,
                                                 const uint32_t* __restrict__ epath,
                                                 const float4* __restrict__ chord, int64_t N,
-                                                const uint32_t* __restrict__ rule) {
+                                                const uint32_t* __restrict__ rule, uint32_t* at, uint32_t* of) {
     const int lane = threadIdx.x & 63;
     const int32_t key = skey[f];
     const uint32_t path = epath[f] & 0x3FFFFFFFu;
@@ -163,6 +172,7 @@ __device__ inline unsigned long long cover_open(int32_t f, const int32_t* __rest
     const float yc = (float)(ry + 1);
     const float xs = (float)(rx + px) + ((float)((7 * j) & 15) + 0.5f) / 16.0f;
     const float ys = (float)(ry + py) + ((float)j + 0.5f) / 16.0f;
+    const bool upper = py != 0;
     int32_t W = winding[f];
     int n = 64;
     for (int64_t g0 = f; n == 64; g0 += 64) {
@@ -170,18 +180,42 @@ __device__ inline unsigned long long cover_open(int32_t f, const int32_t* __rest
         const bool own = g < N && skey[g] == key && (epath[g] & 0x3FFFFFFFu) == path;
         const unsigned long long other = __ballot(!own);
         n = other ? __ffsll((long long)other) - 1 : 64;
-        float4 ch = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (own) ch = chord[sidx[g]];
-        for (int k = 0; k < n; ++k) {
-            const float ax = __shfl(ch.x, k), ay = __shfl(ch.y, k), bx = __shfl(ch.z, k), by = __shfl(ch.w, k);
+        if (own) {
+            const float4 ch = chord[sidx[g]];
+            const float ax = ch.x, ay = ch.y, bx = ch.z, by = ch.w;
             const int sr = (ay < yc && yc <= by) ? -1 : ((by < yc && yc <= ay) ? 1 : 0);
-            const float xc = ax + (yc - ay) * ((bx - ax) / (by - ay));
             const bool rightward = ax < bx;
-            const float lo = rightward ? ax : bx, hi = rightward ? bx : ax;
-            const float v = ay + (xs - ax) * ((by - ay) / (bx - ax));
-            const bool hit = lo < xs && xs <= hi && (py ? yc <= v && v < ys : ys < v && v <= yc);
-            W = wadd(W, (xs > xc ? sr : 0) + (hit ? (rightward == (py != 0) ? 1 : -1) : 0));
+            at[lane] = fbits(ax + (yc - ay) * ((bx - ax) / (by - ay)));
+            at[64 + lane] = fbits(rightward ? ax : bx);
+            at[128 + lane] = fbits(rightward ? bx : ax);
+            at[192 + lane] = (uint32_t)(sr + 1) | (rightward ? 4u : 0u);
+            of[lane] = fbits(ax);
+            of[64 + lane] = fbits(ay);
+            of[128 + lane] = fbits((by - ay) / (bx - ax));
         }
+        wave_sync();
+        // four chords a step, their words loaded together; those past the last one change nothing
+        for (int k = 0; k < n; k += 4) {
+            float xc[4], lo[4], hi[4], ax[4], ay[4], sl[4];
+            uint32_t e[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                xc[u] = bitsf(at[k + u]); lo[u] = bitsf(at[64 + k + u]); hi[u] = bitsf(at[128 + k + u]);
+                e[u] = at[192 + k + u];
+                ax[u] = bitsf(of[k + u]); ay[u] = bitsf(of[64 + k + u]); sl[u] = bitsf(of[128 + k + u]);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const float v = ay[u] + (xs - ax[u]) * sl[u];
+                // no short circuit: no branches
+                const bool in = (lo[u] < xs) & (xs <= hi[u]);
+                const bool hit = in & (((ys < v) & (v <= yc) & !upper) | ((yc <= v) & (v < ys) & upper));
+                const int32_t row = ((int)(e[u] & 3u) - 1) & -(int)(xs > xc[u]);
+                const int32_t column = (1 - 2 * (int)((e[u] >> 2) ^ (uint32_t)py)) & -(int)hit;
+                W = wadd(W, (row + column) & -(int)(k + u < n));
+            }
+        }
+        wave_sync();  // the words are used again
     }
     return __ballot(rule[path] == 1u ? (W & 1) != 0 : W != 0);
 }
@@ -235,20 +269,35 @@ __device__ inline int run_length(int32_t f, const Four& q, const int32_t* __rest
 // lane walking the cell's chords: 2.5 ms; one lane per cell with the bits below: 1.9 ms, of which 0.4 ms
 // were arithmetic, since the longest cell of a wave held the other lanes back and each of its chords
 // waited on two dependent loads.  Five waves per SIMD: four or six were 6% slower.
+// Cells of more than kRunMax chords are few, but lie side by side (a path's dense spots): taken by the waves
+// whose records they were, one after another, 54 of them made this kernel 534 us instead of 130 in a
+// drawing at four times its size.  k_mark_emit lists them, and waves of their own spread over the chip.
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5)))
 void k_cell_cover(const int32_t* __restrict__ cell_first, const int32_t* __restrict__ totals, int64_t rec_cap,
                   const int32_t* __restrict__ skey, const int32_t* __restrict__ sidx,
                   const int32_t* __restrict__ winding, const uint32_t* __restrict__ epath,
                   const float4* __restrict__ chord, int64_t N, const uint32_t* __restrict__ rule,
-                  unsigned long long* __restrict__ cmask) {
+                  unsigned long long* __restrict__ cmask, const int2* __restrict__ dense,
+                  const int32_t* __restrict__ n_dense) {
     // per chord: its entry and its cell's key, then its ChordBits
     __shared__ uint32_t s_head[kSlots + kRunMax], s_low[kSlots + kRunMax], s_high[kSlots + kRunMax];
     // per cell: place of its chords | chords << 16 | even-odd << 21 | record << 22, winding number
     __shared__ uint2 s_cell[kChunk];
     __shared__ int32_t s_wave[kBlock / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (blockIdx.x < kDenseBlocks) {
+        const int32_t nd = *n_dense;
+        for (int32_t i = (int32_t)blockIdx.x + kDenseBlocks * wave; i < nd; i += kDenseBlocks * (kBlock / 64)) {
+            const int2 d = dense[i];
+            const unsigned long long m = cover_dense(__builtin_amdgcn_readfirstlane(d.y), skey, sidx, winding, epath,
+                                                     chord, N, rule, s_head + 256 * wave, s_low + 256 * wave);
+            if (lane == 0) cmask[d.x] = m;
+        }
+        return;
+    }
     const int64_t R = min((int64_t)totals[0] + (int64_t)totals[1], rec_cap);
-    for (int64_t c0 = (int64_t)blockIdx.x * kChunk; c0 < R; c0 += (int64_t)gridDim.x * kChunk) {
+    const int64_t stride = (int64_t)(gridDim.x - kDenseBlocks) * kChunk;
+    for (int64_t c0 = (int64_t)(blockIdx.x - kDenseBlocks) * kChunk; c0 < R; c0 += stride) {
         // what a cell needs of its entries, all records of a thread at once (a span loads entry 0)
         int32_t fr[kRecs], key[kRecs];
         int n[kRecs], at[kRecs];
@@ -277,13 +326,7 @@ void k_cell_cover(const int32_t* __restrict__ cell_first, const int32_t* __restr
         int mine = 0;  // chords | cells << 16
 #pragma unroll
         for (int u = 0; u < kRecs; ++u) {
-            for (unsigned long long open = __ballot(n[u] > kRunMax); open; open &= open - 1) {
-                const int l = __ffsll((long long)open) - 1;
-                const unsigned long long m =
-                    cover_open(__builtin_amdgcn_readlane(fr[u], l), skey, sidx, winding, epath, chord, N, rule);
-                if (lane == l) cmask[c0 + u * kBlock + tid] = m;
-            }
-            if (n[u] > kRunMax) n[u] = 0;
+            if (n[u] > kRunMax) n[u] = 0;  // listed
             mine += n[u] + (n[u] > 0 ? 1 << 16 : 0);
         }
         // the cells' places among the chunk's chords
@@ -364,12 +407,12 @@ void k_cell_cover(const int32_t* __restrict__ cell_first, const int32_t* __restr
 hipError_t launch_cell_cover(const int32_t* cell_first, const int32_t* totals, int64_t rec_cap,
                              const int32_t* skey, const int32_t* sidx, const int32_t* winding,
                              const uint32_t* epath, const float4* chord, int64_t N, const uint32_t* rule,
-                             unsigned long long* cmask, hipStream_t s) {
+                             unsigned long long* cmask, const int2* dense, const int32_t* n_dense, hipStream_t s) {
     if (rec_cap <= 0 || N <= 0) return hipSuccess;
     int64_t g = (rec_cap + kChunk - 1) / kChunk;
     g = g < 65536 ? g : 65536;  // few passes each: passes differ in cost (3% faster than 4,096 workgroups)
-    k_cell_cover<<<(unsigned)g, kBlock, 0, s>>>(cell_first, totals, rec_cap, skey, sidx, winding, epath, chord, N,
-                                                rule, cmask);
+    k_cell_cover<<<(unsigned)g + kDenseBlocks, kBlock, 0, s>>>(cell_first, totals, rec_cap, skey, sidx, winding, epath, chord, N,
+                                                rule, cmask, dense, n_dense);
     return hipGetLastError();
 }
 

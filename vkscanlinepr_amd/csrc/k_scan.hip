@@ -167,7 +167,8 @@ __global__ __launch_bounds__(kMarkThreads) void k_mark_emit(
     int32_t* __restrict__ totals,
     const int32_t* __restrict__ bucket_base, const int2* __restrict__ prow, int2* __restrict__ brec,
     int32_t* __restrict__ err, const int2* __restrict__ pcanvas, const int32_t* __restrict__ wbase,
-    int32_t* __restrict__ cell_first) {
+    int32_t* __restrict__ cell_first, int2* __restrict__ dense, int32_t* __restrict__ n_dense) {
+    static_assert(kAaRunMax >= kScanItems, "a longer run of entries leaves its thread");
     __shared__ int32_t s_tile;
     __shared__ unsigned long long s_w[kMarkThreads / 64];
     __shared__ unsigned long long s_prefix;
@@ -228,6 +229,7 @@ __global__ __launch_bounds__(kMarkThreads) void k_mark_emit(
     const int2 pr_a = prow[pa], pr_z = prow[pz];
     const int32_t bb_a = bucket_base[pa], bb_z = bucket_base[pz];
     uint32_t cellbits = 0, spanbits = 0;
+    int tail = -1;  // where the thread's last run of equal entries starts, when it is a cell that starts here
 #pragma unroll
     for (int j = 0; j < kScanItems; ++j) {
         const int64_t f = i0 + j;
@@ -250,9 +252,17 @@ __global__ __launch_bounds__(kMarkThreads) void k_mark_emit(
             const bool wf = (r == 0u && wn != 0) || (r == 1u && (wn & 1) != 0);
             span = (y0 == y1) && (x0 + 2 < x1) && (pprev == p1) && wf;
         }
+        if (cell) tail = j;
+        else if (pprev != p1 || kprev != k1) tail = -1;
         cellbits |= (uint32_t)cell << j;
         spanbits |= (uint32_t)span << j;
         kprev = k1; pprev = p1;
+    }
+    // a cell of more than kAaRunMax entries is the last one of its thread, or none
+    if (!dense || inext >= N || knext_out != keys[kScanItems - 1] || pnext_out != pz) tail = -1;
+    if (tail >= 0) {
+        const int64_t e = i0 + tail + kAaRunMax;
+        if (e >= N || skey[e] != knext_out || cur.at(e) != pz) tail = -1;
     }
     const unsigned long long mine = (unsigned long long)__popc(cellbits) | ((unsigned long long)__popc(spanbits) << 32);
     unsigned long long total;
@@ -267,6 +277,16 @@ __global__ __launch_bounds__(kMarkThreads) void k_mark_emit(
     int32_t spans_before = (int32_t)(off >> 32);
     const int64_t tile_rec0 = (int64_t)(s_prefix & 0xFFFFFFFFull) + (int64_t)(s_prefix >> 32);
     const int64_t tile_recs = (int64_t)(total & 0xFFFFFFFFull) + (int64_t)(total >> 32);
+    const unsigned long long dense_lanes = __ballot(tail >= 0);
+    if (dense_lanes) {
+        const int lane = threadIdx.x & 63, leader = __ffsll((long long)dense_lanes) - 1;
+        int32_t at = 0;
+        if (lane == leader) at = atomicAdd(n_dense, (int32_t)__popcll(dense_lanes));
+        at = __shfl(at, leader) + (int32_t)__popcll(dense_lanes & ((1ull << lane) - 1ull));
+        const uint32_t before = tail >= 0 ? (1u << tail) - 1u : 0u;
+        const int32_t o = cells_before + spans_before + __popc(cellbits & before) + __popc(spanbits & before);
+        if (tail >= 0) dense[at] = make_int2(o < rec_cap ? o : 0, (int32_t)(i0 + tail));
+    }
     if (i0 < N) {
         int32_t kp = (i0 > 0) ? k_before : 0;
         uint32_t pp = (i0 > 0) ? p_before : 0xFFFFFFFFu;
@@ -419,13 +439,14 @@ hipError_t launch_mark_emit(const int32_t* skey, const int32_t* winding, const u
                             ScanCtl ctl, int4* records, uint32_t* crec, int32_t* flags, int32_t* totals,
                             const int32_t* bucket_base, const int2* prow, int2* brec, hipStream_t s,
                             const int32_t* n_dev, const int32_t* sstart, uint32_t Np, int64_t rec_cap,
-                            int32_t* err, const int2* pcanvas, const int32_t* wbase, int32_t* cell_first) {
+                            int32_t* err, const int2* pcanvas, const int32_t* wbase, int32_t* cell_first,
+                            int2* dense, int32_t* n_dense) {
     if (N == 0) return hipSuccess;
     k_mark_emit<<<(unsigned)((N + kMarkTile - 1) / kMarkTile), kMarkThreads, 0, s>>>(skey, winding, epath, rule, fill, N, n_dev,
                                                                  sstart, Np, rec_cap, w, h, ctl.status,
                                                                  ctl.counter, records, crec, flags, totals,
                                                                  bucket_base, prow, brec, err, pcanvas, wbase,
-                                                                 cell_first);
+                                                                 cell_first, dense, n_dense);
     return hipGetLastError();
 }
 

@@ -339,13 +339,17 @@ hipError_t launch_sort_bands_emit(const int32_t* band_start, const int32_t* n_ba
                                   const EmitArgs& emit, int64_t n_entries, int n_cu, hipStream_t s,
                                   hipStream_t s_small);
 // ---- winding / mark / emit (a10 scan, a11); also writes each (path, row) bucket's record range
+// cell_first (anti-aliased frames): each record's first sorted entry, -1 for a span; dense: the cells of more
+// than kAaRunMax entries in any order (record, first entry), at most N / (kAaRunMax + 1), counted in *n_dense
+// (zeroed).
+constexpr int kAaRunMax = 30;
 hipError_t launch_mark_emit(const int32_t* skey, const int32_t* winding, const uint32_t* epath,
                             const uint32_t* rule, const uint32_t* fill, int64_t N, int w, int h,
                             ScanCtl ctl, int4* records, uint32_t* crec, int32_t* flags, int32_t* totals,
                             const int32_t* bucket_base, const int2* prow, int2* brec, hipStream_t s,
                             const int32_t* n_dev, const int32_t* sstart, uint32_t Np, int64_t rec_cap,
                             int32_t* err, const int2* pcanvas = nullptr, const int32_t* wbase = nullptr,
-                            int32_t* cell_first = nullptr);
+                            int32_t* cell_first = nullptr, int2* dense = nullptr, int32_t* n_dense = nullptr);
 
 // ---- anti-aliased coverage (k_aa.hip): the 64-sample mask of every boundary cell record (2x2
 // pixels x 16 samples, bit (2 py + px) * 16 + j), ~0 for spans.  cell_first[o] = the record's
@@ -355,7 +359,7 @@ constexpr int kAaSamples = 16;
 hipError_t launch_cell_cover(const int32_t* cell_first, const int32_t* totals, int64_t rec_cap,
                              const int32_t* skey, const int32_t* sidx, const int32_t* winding,
                              const uint32_t* epath, const float4* chord, int64_t N, const uint32_t* rule,
-                             unsigned long long* cmask, hipStream_t s);
+                             unsigned long long* cmask, const int2* dense, const int32_t* n_dense, hipStream_t s);
 
 // ---- learned single-pass allocation (k_learned.hip)
 constexpr int kMlpIn = 16, kMlpHidden = 64, kMlpOut = 2;

@@ -172,6 +172,7 @@ struct spr_handle {
     DBuf<int32_t> skey, sidx, winding, flags;
     DBuf<int4> records;     // full records, kept only with the debug option
     DBuf<int32_t> cell_first;            // anti-aliased frames: each record's first sorted entry
+    DBuf<int2> dense;                    // and the cells of many entries: record, first entry
     DBuf<unsigned long long> cmask;      // anti-aliased frames: each record's sample coverage
     DBuf<float4> chord;                  // anti-aliased frames: each entry's chord
     DBuf<uint32_t> crec;    // compact records (x | width << 16) read by the composite
@@ -276,7 +277,7 @@ enum { kCcBigPieces = spr::kCcWords, kCcSplit, kCcWords };
 struct ZeroLayout {
     size_t a_words = 0, total = 0;
     size_t ctr_a = 0, st_count = 0, st_pbase = 0;
-    size_t ctr = 0, totals = 0, misc = 0, chainctl = 0, st_hist = 0, st_band = 0, st_wind = 0, st_mark = 0;
+    size_t ctr = 0, totals = 0, misc = 0, dense = 0, chainctl = 0, st_hist = 0, st_band = 0, st_wind = 0, st_mark = 0;
     size_t hist = 0, fill = 0, bsum = 0, brec = 0;
 };
 
@@ -290,6 +291,7 @@ ZeroLayout zero_layout(uint32_t C, uint32_t Np, int64_t N, int64_t NB) {
     z.ctr = o; o += 4;                 // eight u32 counters of the phase-B scans
     z.totals = o; o += 2;              // int32 cells, spans, R, ended tally workgroups
     z.misc = o; o += 1;                // int32 error flag, big-band count
+    z.dense = o; o += 1;               // int32 dense cells (anti-aliased frames), spare
     z.chainctl = o; o += (kCcWords + 1) / 2;  // counters of the curve pass (int32)
     z.st_hist = o; o += (size_t)spr::bucket_band_tiles(NB);
     z.st_band = o; o += (size_t)spr::bucket_band_tiles(NB);
@@ -534,7 +536,10 @@ void run_frame(spr_handle* H, bool record_begin = true) {
     H->big_list.ensure(4 * (size_t)max_bands);  // oversized band ids, their winding prefixes, two lists of long bands
     if (debug) { H->flags.ensure(2 * n1); H->records.ensure(2 * n1); }
     if (keep) H->sidx.ensure(n1);
-    if (aa) { H->cell_first.ensure(2 * n1); H->cmask.ensure(2 * n1); H->chord.ensure(n1); }
+    if (aa) {
+        H->cell_first.ensure(2 * n1); H->cmask.ensure(2 * n1); H->chord.ensure(n1);
+        H->dense.ensure(n1 / (spr::kAaRunMax + 1) + 1);
+    }
     H->crec.ensure(2 * n1);
     H->image.ensure((size_t)4 * H->w * H->h);
     const bool gen = !H->inj && N > 0, by_chain = N >= spr::kChainFrame;
@@ -554,6 +559,7 @@ void run_frame(spr_handle* H, bool record_begin = true) {
     int32_t* d_totals = reinterpret_cast<int32_t*>(H->zero.p + z.totals);
     int32_t* d_err = reinterpret_cast<int32_t*>(H->zero.p + z.misc);
     int32_t* d_bigcount = d_err + 1;
+    int32_t* d_dense = reinterpret_cast<int32_t*>(H->zero.p + z.dense);
     int32_t* d_hist = reinterpret_cast<int32_t*>(H->zero.p + z.hist);
     int32_t* d_fill = reinterpret_cast<int32_t*>(H->zero.p + z.fill);
     int32_t* d_bsum = reinterpret_cast<int32_t*>(H->zero.p + z.bsum);
@@ -637,10 +643,11 @@ void run_frame(spr_handle* H, bool record_begin = true) {
                                       ctl_at(H, z.st_mark, z.ctr, 3), debug ? H->records.p : nullptr, H->crec.p,
                                       debug ? H->flags.p : nullptr, d_totals, H->bucket_base.p, H->prow.p, d_brec,
                                       s, nullptr, nullptr, Np, (int64_t)(2 * n1), d_err, nullptr, nullptr,
-                                      aa ? H->cell_first.p : nullptr));
+                                      aa ? H->cell_first.p : nullptr, aa ? H->dense.p : nullptr, d_dense));
     if (aa)
         SPR_HIP(spr::launch_cell_cover(H->cell_first.p, d_totals, (int64_t)(2 * n1), H->skey.p, H->sidx.p,
-                                       H->winding.p, H->epath.p, H->chord.p, N, H->rule.p, H->cmask.p, s));
+                                       H->winding.p, H->epath.p, H->chord.p, N, H->rule.p, H->cmask.p, H->dense.p,
+                                       d_dense, s));
     H->last_brec = d_brec;
     H->last_learned = false;
     H->last_fused = narrow;
@@ -1413,7 +1420,7 @@ int spr_destroy(spr_handle* H) {
     H->chain_cls.release(); H->mono.release(); H->win_first.release(); H->key.release(); H->wn.release(); H->epath.release(); H->sorted.release();
     H->sbig.release(); H->stmp.release(); H->skey.release(); H->sidx.release();
     H->winding.release(); H->flags.release(); H->records.release(); H->crec.release();
-    H->cell_first.release(); H->cmask.release(); H->chord.release();
+    H->cell_first.release(); H->cmask.release(); H->chord.release(); H->dense.release();
     H->row_lo.release(); H->row_hi.release(); H->bucket_base.release(); H->bflag.release();
     H->band_start.release(); H->band_pr.release(); H->big_list.release(); H->prow.release(); H->image.release(); H->zero.release();
     drop_graph(H);
