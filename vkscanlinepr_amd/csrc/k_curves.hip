@@ -32,6 +32,12 @@
 // t1 / 32.  Segments that start there solve more crossings before their own (8 and 16 instead of
 // 4), and a chain's first segment reaches past t = t1 / 32.
 //
+// A view of the first part of large curves has hundreds of crossings there, and hardly a guess comes true:
+// segments corrected one after another cost more than the chain solved in order.  A chain with a long start
+// (more than 64 crossings before t1 / 32) therefore has all those before t1 / 8 in its first segment, and a whole
+// wave solves that (wave_solve.hpp).  us a frame: 64 scribbles at 32 and 8 times their size on 1024^2 813 -> 432
+// and 767 -> 490, an illustration at 8 times its size on 4096^2 3,343 -> 1,758.
+//
 // This is the pass of small frames (launch_curves' caller chooses), whose span would otherwise be
 // their longest chain: whole chains take about 1 us a crossing one after another, and the passes
 // over the chains (k_chain.hip) cost a launch each.  The speculation costs about twice the
@@ -41,6 +47,7 @@
 #include "device_common.hpp"
 #include "kernels.hpp"
 #include "scan_common.hpp"
+#include "wave_solve.hpp"
 
 #include <type_traits>
 
@@ -61,6 +68,11 @@ constexpr int kStage = 4096;                    // big pieces up to this many en
 // segments that a batch is cut into (besides one per chain).
 constexpr int kWarm = 4, kWarm8 = 8, kWarm16 = 16, kSegMin = 4, kSegTarget = 112;
 constexpr int kSegs = 832;
+// A chain with a long start has all crossings before t1 / 8 in its first segment, which a whole wave solves; a
+// batch has at most so many.
+constexpr int kLongHeads = 8;
+constexpr int kBigLongHead = 16;                // for kLongHead in k_big_pieces, whose waves would wait anyway
+constexpr uint32_t kByWave = 1u << 20;          // on a chain's first segment in the list
 // Candidate starts of a batch's slow segments (a multiple of 8 each), and the chains that have any.
 constexpr int kCands = 384, kWalks = 16;
 constexpr int kCand16 = 16, kCand8 = 8;         // below t1 / 16, t1 / 8
@@ -336,6 +348,8 @@ struct CurveBatch {
     uint32_t seg[kSegs];
     int n_segs;
     int n_pieces, longest, n_slots, crossings;  // of the batch
+    int n_long;                          // chains with a long start
+    uint16_t longs[kLongHeads];          // those that waves solve
 };
 
 struct Candidates {
@@ -451,14 +465,6 @@ __device__ inline void store_gap(const FragArgs& A, int64_t i, int curve, uint32
 // Segments of a chain of n crossings whose first one has `head` of them: 1 + rest, the others of
 // (nearly) equal lengths near `len`.
 __device__ inline int seg_rest(int n, int head, int len) { return (n - head + len - 1) / len; }
-
-// Crossings of a chain that lie before parameter tau, about.
-__device__ inline int crossings_before(uint32_t type, const CurveAxis& a, float line0, bool neg, float t0, float tau, int n) {
-    if (!(t0 < tau)) return 0;
-    const float d = eval_axis(type, tau, a.c[0], a.c[1], a.c[2], a.c[3]) - line0;
-    const float k = (neg ? -d : d) * 0.5f + 2.0f;
-    return k >= (float)n ? n : (k > 0.0f ? (int)k : 0);
-}
 
 // A chain of the batch: its piece's values for one axis.
 struct ChainRef {
@@ -666,7 +672,7 @@ void k_curves(const CurveArgs K, const FragArgs A) {
             if (lane < kCap / 64) B.starts_before[lane] = (uint16_t)(upto - here);
             if (lane == 63) {
                 B.n_pieces = before; B.crossings = x_upto; B.longest = longest; B.n_slots = n_slots;
-                B.n_segs = 0;
+                B.n_segs = B.n_long = 0;
             }
         }
         __syncthreads();
@@ -681,25 +687,32 @@ void k_curves(const CurveArgs K, const FragArgs A) {
             if ((B.pa[ch >> 1].x & 0xFFFFu) == kNoPiece) continue;
             const ChainRef r = chain_of(B, ch);
             if (r.n == 0) continue;
-            int head = r.n;
+            int head = r.n, k8 = 0;
+            uint32_t by_wave = 0;
             if (r.n > len + len / 2) {
                 head = len;
-                if (r.type != kLine)
-                    head = max(len, crossings_before(r.type, r.a, r.line0, r.neg, r.t0, 0.03125f * r.t1, r.n));
+                if (r.type != kLine) {
+                    k8 = crossings_before(r.type, r.a, r.line0, r.neg, r.t0, 0.125f * r.t1, r.n);
+                    if (k8) head = max(len, crossings_before(r.type, r.a, r.line0, r.neg, r.t0, kHeadTau * r.t1, r.n));
+                    int w = kLongHeads;
+                    if (head > kLongHead) w = atomicAdd(&B.n_long, 1);
+                    if (w < kLongHeads) {
+                        B.longs[w] = (uint16_t)ch;
+                        by_wave = kByWave;
+                        head = max(head, k8);
+                    }
+                }
                 if (r.n - head < len / 2) head = r.n;
             }
             B.head[ch] = (uint16_t)head;
             const int m = seg_rest(r.n, head, len);
             int at = atomicAdd(&B.n_segs, 1 + m);
-            B.seg[at++] = (uint32_t)ch;
+            B.seg[at++] = (uint32_t)ch | by_wave;
             if (head >= r.n) continue;
             const int first = at;
             ++n_split;
-            int k8 = 0, k16 = 0, n8 = 0, n16 = 0;
-            if (r.type != kLine) {
-                k8 = crossings_before(r.type, r.a, r.line0, r.neg, r.t0, 0.125f * r.t1, r.n);
-                if (k8) k16 = crossings_before(r.type, r.a, r.line0, r.neg, r.t0, 0.0625f * r.t1, r.n);
-            }
+            int k16 = 0, n8 = 0, n16 = 0;
+            if (k8) k16 = crossings_before(r.type, r.a, r.line0, r.neg, r.t0, 0.0625f * r.t1, r.n);
             for (int j = 0; j < m; ++j) {
                 const int i0 = head + seg_begin(r.n - head, m, j);
                 const int warm = i0 >= k8 ? kWarm : (i0 >= k16 ? kWarm8 : kWarm16);
@@ -733,6 +746,20 @@ void k_curves(const CurveArgs K, const FragArgs A) {
             if (n_cands) n_walks = min(__builtin_amdgcn_readfirstlane(cands.n_walks), kWalks);
         }
 
+        // ---- the long starts, a wave each
+        const int n_long = min(__builtin_amdgcn_readfirstlane(B.n_long), kLongHeads);
+        if (n_long) {
+            const TreeNode N = tree_node(lane);
+#pragma unroll 1
+            for (int i = wave; i < n_long; i += kWaves) {
+                const int ch = __builtin_amdgcn_readfirstlane((int)B.longs[i]);
+                const ChainRef r = chain_of(B, ch);
+                float* vs = B.v + r.at;
+                solve_wave_any(N, r.type, r.a, r.line0, r.neg ? -2.0f : 2.0f, r.side, r.t1, (int)B.head[ch], r.t0,
+                               [&](int k, float v) { if (lane == 0) vs[k] = v; });
+            }
+        }
+
         // ---- the crossings, one segment per lane
         for (int s0 = 0; s0 < S; s0 += kThreads) {
             const bool on = s0 + tid < S;
@@ -746,7 +773,7 @@ void k_curves(const CurveArgs K, const FragArgs A) {
             // guess was off is solved again from there
             float g = r.t0, start = r.t0;
             int k0 = max(0, i0 - (int)((e >> 20) & 31u));
-            bool run = on, redo = false;
+            bool run = on && !(i0 == 0 && (e & kByWave)), redo = false;
             for (;;) {
                 if (run) {
                     const float got = solve_run_any(r.type, r.a, r.line0, r.neg, r.side, r.t1, k0, i0, i1, start, redo, vs);
@@ -913,8 +940,13 @@ __global__ __launch_bounds__(kBigThreads) void k_big_pieces(const CurveArgs K, c
         // segments: one per thread (as in k_curves)
         const int len = max(kSegMin, (nv + kBigThreads - 5) / (kBigThreads - 4));
         const CurveAxis ax = {{cv.x[0], cv.x[1], cv.x[2], cv.x[3]}}, ay = {{cv.y[0], cv.y[1], cv.y[2], cv.y[3]}};
-        const int hx = min(g.nx, max(len, crossings_before(cv.type, ax, g.x0, g.xneg, g.t0, 0.03125f * g.t1, g.nx)));
-        const int hy = min(g.ny, max(len, crossings_before(cv.type, ay, g.y0, g.yneg, g.t0, 0.03125f * g.t1, g.ny)));
+        const int kx = crossings_before(cv.type, ax, g.x0, g.xneg, g.t0, 0.125f * g.t1, g.nx);
+        const int ky = crossings_before(cv.type, ay, g.y0, g.yneg, g.t0, 0.125f * g.t1, g.ny);
+        int hx = min(g.nx, max(len, crossings_before(cv.type, ax, g.x0, g.xneg, g.t0, kHeadTau * g.t1, g.nx)));
+        int hy = min(g.ny, max(len, crossings_before(cv.type, ay, g.y0, g.yneg, g.t0, kHeadTau * g.t1, g.ny)));
+        const bool wx = cv.type != kLine && hx > kBigLongHead, wy = cv.type != kLine && hy > kBigLongHead;  // by a wave
+        if (wx) hx = max(hx, kx);
+        if (wy) hy = max(hy, ky);
         const int sx = g.nx ? 1 + seg_rest(g.nx, hx, len) : 0, sy = g.ny ? 1 + seg_rest(g.ny, hy, len) : 0;
         n_split += (sx > 1 ? 1 : 0) + (sy > 1 ? 1 : 0);
         const bool on = tid < sx + sy, ys = tid >= sx;
@@ -941,7 +973,19 @@ __global__ __launch_bounds__(kBigThreads) void k_big_pieces(const CurveArgs K, c
         };
         const int warm = beyond(0.125f * g.t1) ? kWarm : (beyond(0.0625f * g.t1) ? kWarm8 : kWarm16);
         int k0 = max(0, i0 - warm);
-        bool run = on, redo = false;
+        // the long first segments by a wave each (as in k_curves)
+        if (wave == 0 ? wx : (wave == 1 && wy)) {
+            const TreeNode N = tree_node(lane);
+            const CurveAxis aw = wave ? ay : ax;
+            const int at = wave ? g.nx : 0;
+            const float line_w = wave ? g.y0 : g.x0, step_w = (wave ? g.yneg : g.xneg) ? -2.0f : 2.0f;
+            const int head_w = wave ? hy : hx;
+            if (local) solve_wave_any(N, cv.type, aw, line_w, step_w, (uint32_t)wave, g.t1, head_w, g.t0,
+                                      [&](int k, float v) { if (lane == 0) st_in[at + k] = v; });
+            else solve_wave_any(N, cv.type, aw, line_w, step_w, (uint32_t)wave, g.t1, head_w, g.t0,
+                                [&](int k, float v) { if (lane == 0) gt[at + k] = v; });
+        }
+        bool run = on && !(j == 0 && (ys ? wy : wx)), redo = false;
         for (;;) {
             if (run) {
                 // the two branches keep every pointer in one address space (no flat accesses)
