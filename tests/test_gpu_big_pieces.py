@@ -78,3 +78,33 @@ def test_pieces_beyond_lds_match_the_oracle(spr, orc, w, h, nx, ny, debug):
         assert bad.size == 0, (bad.size, bad[:4], g[bad[:4]], o[bad[:4]])
     assert np.array_equal(r.export("image"), f.image().reshape(-1))
     r.close()
+
+
+@pytest.mark.parametrize("far", [1e5, 5e8, 9.99e8, 1.01e9, 2.1e9, 4.4e9, 1e12, 1e30])
+def test_far_ends_match_the_oracle(spr, orc, far):
+    """Curves through the canvas whose ends lie far outside, where the count and the write pass round differently: the
+    pieces that the count pass lists are those that the windows leave out.  Beyond 2^32 the count reserves
+    entries that are not written, which the reference leaves undefined: there the two kinds of frame agree."""
+    w = h = 3000
+    mid = np.array([w / 2 + 0.3, h / 2 - 0.7])
+    curves = []
+    for dx, dy in ((1.0, 1.0), (1.0, 0.4), (-0.7, 1.0), (1e-9, 1.0), (1.0, -1e-9)):
+        d = np.array([dx, dy]) * far
+        curves += [[mid - d, mid - d / 3, mid + d / 3, mid + d], [mid + d, mid, mid - d],
+                   [mid, mid + d * 1e-3, mid + d / 2, mid + d], [mid - d, mid + 1.0]]
+    a = _closed(curves)
+    print(f"[big-pieces] far {far}", flush=True)
+    images = []
+    for debug in (True, False):
+        r = spr.Rasterizer(w, h, debug=debug)
+        _load(r, a)
+        r.render(readback=False)
+        images.append(r.export("image"))
+        if debug:
+            g = r.export("inter")
+        r.close()
+    assert np.array_equal(images[0], images[1])
+    if far < 2.0**32:
+        f = orc.Frame(a, w, h, threads=8)
+        assert np.array_equal(g, f.get("inter"))
+        assert np.array_equal(images[0], f.image().reshape(-1))

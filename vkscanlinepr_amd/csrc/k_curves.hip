@@ -43,7 +43,7 @@
 // over the chains (k_chain.hip) cost a launch each.  The speculation costs about twice the
 // arithmetic, so frames that fill the chip with chains take k_chain.hip.
 //
-// Pieces of more than kBigPiece entries are queued for k_big_pieces, one workgroup each.
+// Pieces of more than kBigPiece entries, which the count pass lists, take k_big_pieces, one workgroup each.
 #include "device_common.hpp"
 #include "kernels.hpp"
 #include "scan_common.hpp"
@@ -633,7 +633,6 @@ void k_curves(const CurveArgs K, const FragArgs A) {
                         else { needs = true; needs_at = prev; after = g; }
                     }
                     prev = in ? at : -1;
-                    if (starts && !in) K.big[atomicAdd(K.big_count, 1)] = (int32_t)(5 * c + k);
                     if (in) {
                         const int rel = g.base - bb0;
                         // a grid line is only meaningful (and then in [0, 16386]) on an axis with crossings
@@ -913,7 +912,7 @@ __global__ __launch_bounds__(kBigThreads) void k_big_pieces(const CurveArgs K, c
     __shared__ uint32_t st_out[kStage];
     __shared__ uint32_t s_flags;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int32_t count = *K.big_count;
+    const int32_t count = K.n_dev && *K.n_dev == 0 ? 0 : *K.big_count;  // a frame over its budget has no entries
     int n_split = 0;
     for (int32_t item = (int32_t)blockIdx.x; item < count; item += (int32_t)gridDim.x) {
         const int32_t slot = K.big[item];
@@ -927,13 +926,14 @@ __global__ __launch_bounds__(kBigThreads) void k_big_pieces(const CurveArgs K, c
         const uint32_t bb = (uint32_t)A.bucket_base[path];
         const int2 pr = A.prow[path];
         PieceGeom g, after;
-        g.base = g.nx = g.ny = 0; g.x0 = g.y0 = g.t0 = g.t1 = 0.0f; g.xneg = g.yneg = false;
+        g.base = g.nx = g.ny = 0; g.x0 = g.y0 = g.t0 = g.t1 = 0.0f; g.xneg = g.yneg = g.ok = false;
         after = g;
         bool has_after = false;
         walk_pieces(cv, qq, K.ncuts[c], K.offsets[c], K.offsets[c + 1], w, h, [&](int k, const PieceGeom& x) {
             if (k == kk) g = x;
             if (k == kk + 1 && x.ok) { after = x; has_after = true; }
         });
+        if (!g.ok) continue;  // counted but not written: left to k_curves as gaps
         const float t_end = has_after ? first_entry_t(cv, after) : 1.0f;
         const int nv = g.nx + g.ny, n = g.n();
         const bool local = n <= kStage;

@@ -191,7 +191,18 @@ __global__ __launch_bounds__(kBlock) void k_count(const CountArgs K) {
                 if (k > n) break;
                 const float t = k < n ? q[k < 4 ? k : 3] : 1.0f;
                 const float p1x = cv.ex(t), p1y = cv.ey(t);
-                cnt += piece_count(p0x, p0y, p1x, p1y, w, h);
+                const int pc = piece_count(p0x, p0y, p1x, p1y, w, h);
+                cnt += pc;
+                // as the curve pass counts it: the two round differently only far outside any canvas
+                const float far = 1e9f;
+                if (pc > kCurvePieceMax ||
+                    !(fabsf(p0x) < far && fabsf(p0y) < far && fabsf(p1x) < far && fabsf(p1y) < far)) {
+                    const PieceGrid G = piece_grid(p0x, p0y, p1x, p1y, w, h);
+                    if (1 + G.nx + G.ny > kCurvePieceMax) {
+                        K.big[atomicAdd(K.n_big, 1)] = (int32_t)(5 * c + k);
+                        if (K.host) __hip_atomic_store(&K.host[2], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    }
+                }
                 p0x = p1x; p0y = p1y;
             }
         }

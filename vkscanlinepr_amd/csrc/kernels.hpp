@@ -42,6 +42,7 @@ hipError_t launch_transform(const float2* pos, const uint32_t* pos_path, uint32_
 // Count pass with the exclusive scans of the per-curve counts and of the paths' bucket counts.
 // Statuses and counters zeroed; tiles of kCountTile curves or paths, at least one of each.
 constexpr int kCountTile = 256;
+constexpr int kCurvePieceMax = 1024;  // entries of a piece that a window of the curve pass takes
 inline int count_tiles(int64_t n) { return (int)(n > 0 ? (n + kCountTile - 1) / kCountTile : 1); }
 struct CountArgs {
     const float2* tpos;
@@ -69,7 +70,9 @@ struct CountArgs {
     unsigned long long* path_status;
     uint32_t* path_counter;
     const int2* pcanvas;        // per-path canvas of a batch, or null
-    int32_t* host;              // the two totals in host memory, or null
+    int32_t* host;              // the two totals and a word set with the first big piece, in host memory, or null
+    int32_t* big;               // [5 C] the pieces of more than kCurvePieceMax entries: 5 curve + piece, in any order
+    int32_t* n_big;             // zeroed
 };
 hipError_t launch_count(const CountArgs& K, hipStream_t s);
 hipError_t launch_segment_stats(const int32_t* seg, uint32_t Np, int32_t* max_len, hipStream_t s);
@@ -204,13 +207,14 @@ hipError_t launch_read_out(const uint8_t* src, uint8_t* dst, int64_t bytes, uint
 // The intersection write and the fragment keys: one workgroup per window of `window`
 // entries takes the pieces that start there from the curve data to their keys (or sort words),
 // winding changes and bucket counts, without storing the entries unless A.inter is set.  Pieces
-// of more than kCurvePieceMax entries are queued in `big` for launch_big_pieces.
+// of more than kCurvePieceMax entries are left to launch_big_pieces, which needs nothing of launch_curves
+// and may run beside it.
 // Frames of this many entries take the chain passes: they fill the chip with whole chains sorted by
 // length, which costs half the arithmetic of the curve pass, but has their longest chain and seven
 // launches as its span.  ms a frame alone, by chains and by curves: 6.2 M entries 1.00 and 0.85,
 // 12.0 M 1.22 and 1.54, 24.7 M 1.85 and 2.65, 48.7 M 2.99 and 5.26.
 constexpr int64_t kChainFrame = (int64_t)1 << 23;
-constexpr int kCurveWindowMin = 64, kCurveWindowMax = 1024, kCurvePieceMax = 1024;
+constexpr int kCurveWindowMin = 64, kCurveWindowMax = 1024;
 struct CurveArgs {
     const int32_t* offsets;
     const float4* cuts;
@@ -220,8 +224,8 @@ struct CurveArgs {
     const int32_t* n_dev;
     int32_t window;
     const int32_t* first;
-    int32_t* big;              // [5 C] queue of piece slots 5 curve + piece
-    int32_t* big_count;        // zeroed
+    const int32_t* big;        // the count pass's big pieces
+    const int32_t* big_count;
     int32_t* split_count;      // zeroed: += chains solved by several lanes side by side
     uint32_t* scratch;         // n words
     float* chain_t;            // n values: parameters of pieces beyond LDS

@@ -268,9 +268,8 @@ const spr::PaintArgs* paint_args(const spr_handle* H, spr::PaintArgs& pa) {
 
 namespace {
 
-// Counters of the curve pass (int32), after the chain passes' control words: queued big pieces,
-// chains solved by several lanes.
-enum { kCcBigPieces = spr::kCcWords, kCcSplit, kCcWords };
+// Counter of the curve pass (int32), after the chain passes' control words: chains solved by several lanes.
+enum { kCcSplit = spr::kCcWords, kCcWords };
 
 // Per-frame zeroed control region, in 64-bit words.  Phase A is cleared at frame start (before
 // the host sync), phase B once N and the bucket count NB are known.
@@ -349,15 +348,22 @@ void stage_mark(spr_handle* H, int idx) {
     H->n_marks = idx + 1;
 }
 
+// The number of big pieces that the count pass lists, behind the list (the control words can move
+// to another buffer between the count and the curve pass).
+int32_t* big_pieces(const spr_handle* H) { return H->heavy_list.p + 5 * (size_t)H->C; }
+
 // Clears what the transform and the count pass start from, in one launch.  The count pass writes the
 // path segments from its curves, so a scene without any has them cleared here.
 void clear_prefix(spr_handle* H, int64_t control_words) {
+    H->heavy_list.ensure(5 * (size_t)H->C + 1);
+    H->h_pinned[2] = 0;
     spr::FrameInit init{};
     init.fill[0] = {(uint32_t*)H->zero.p, control_words, nullptr, 0, 0, 0u};
     init.fill[1] = {(uint32_t*)H->visible.p, H->Np, nullptr, 0, 0, 0u};
     init.fill[2] = {(uint32_t*)H->row_lo.p, H->Np, nullptr, 0, 0, 0x7FFFFFFFu};
     init.fill[3] = {(uint32_t*)H->row_hi.p, H->Np, nullptr, 0, 0, 0x80000000u};
-    init.n_fills = 4;
+    init.fill[4] = {(uint32_t*)big_pieces(H), 1, nullptr, 0, 0, 0u};
+    init.n_fills = 5;
     if (!H->C) init.fill[init.n_fills++] = {(uint32_t*)H->seg.p, (int64_t)H->Np + 1, nullptr, 0, 0, 0u};
     SPR_HIP(spr::launch_frame_init(init, H->stream));
 }
@@ -368,7 +374,7 @@ spr::CountArgs count_args(spr_handle* H, int rmax, spr::ScanCtl curves, spr::Sca
     return spr::CountArgs{H->tpos.p, H->cpos.p, H->ctype.p, H->arcw(), H->cpath.p, H->visible.p, H->C, (int)H->w,
                           (int)H->h, H->cuts.p, H->ncuts.p, H->counts.p, seg, spr::count_tiles(H->C), curves.status,
                           curves.counter, H->row_lo.p, H->row_hi.p, H->Np, rmax, H->bucket_base.p, H->prow.p,
-                          spr::count_tiles(H->Np), paths.status, paths.counter, pcanvas, host};
+                          spr::count_tiles(H->Np), paths.status, paths.counter, pcanvas, host, H->heavy_list.p, big_pieces(H)};
 }
 
 // Entries per window of the curve pass.  A workgroup takes one window, and 1,536 workgroups are
@@ -384,16 +390,30 @@ int32_t curve_window(const spr_handle* H, int64_t n) {
 }
 
 // Intersections and fragment keys of a frame below spr::kChainFrame entries (stage marks 4 and 6
-// are the caller's).
-void curve_pass(spr_handle* H, int32_t* d_cc, const spr::FragArgs& A, int64_t n, const int32_t* n_dev, int32_t window) {
+// are the caller's).  known: the frame has pieces beyond a window (without a host wait, n_dev, it may).
+// Known ones run on the second stream, beside the windows.  2.3 M entries of a drawing at eight times its size
+// on 4096^2, 640 us of windows and 840 of big pieces: 1,724 us a frame one after the other, 1,140 beside each other.
+void curve_pass(spr_handle* H, int32_t* d_cc, const spr::FragArgs& A, int64_t n, const int32_t* n_dev, int32_t window,
+                bool known) {
+    hipStream_t s = H->stream, s2 = known && !serial(H) ? H->stream2 : H->stream;
     const spr::CurveArgs K{H->counts.p, H->cuts.p, H->ncuts.p, H->C, n, n_dev, window, H->win_first.p, H->heavy_list.p,
-                           d_cc + kCcBigPieces, d_cc + kCcSplit, (uint32_t*)H->sbig.p, (float*)H->stmp.p};
-    SPR_HIP(spr::launch_curves(K, A, H->stream));
+                           big_pieces(H), d_cc + kCcSplit, (uint32_t*)H->sbig.p, (float*)H->stmp.p};
+    if (s2 != s) {
+        SPR_HIP(hipEventRecord(H->ev_fork, s));
+        SPR_HIP(hipStreamWaitEvent(s2, H->ev_fork, 0));
+        SPR_HIP(spr::launch_big_pieces(K, A, H->n_cu * H->merge_k / 8, s2));
+        SPR_HIP(hipEventRecord(H->ev_join, s2));
+    }
+    SPR_HIP(spr::launch_curves(K, A, s));
     stage_mark(H, 5);
-    // a piece holds its start and at most the grid lines of each axis inside the canvas and one beyond
-    const int w = H->batch ? H->max_w : (int)H->w, h = H->batch ? H->max_h : (int)H->h;
-    if (1 + (w / 2 + 2) + (h / 2 + 2) > spr::kCurvePieceMax)
-        SPR_HIP(spr::launch_big_pieces(K, A, H->n_cu * H->merge_k / 8, H->stream));
+    if (s2 != s) {
+        SPR_HIP(hipStreamWaitEvent(s, H->ev_join, 0));
+    } else if (known || n_dev) {
+        // a piece holds its start and at most the grid lines of each axis inside the canvas and one beyond
+        const int w = H->batch ? H->max_w : (int)H->w, h = H->batch ? H->max_h : (int)H->h;
+        if (1 + (w / 2 + 2) + (h / 2 + 2) > spr::kCurvePieceMax)
+            SPR_HIP(spr::launch_big_pieces(K, A, H->n_cu * H->merge_k / 8, s));
+    }
 }
 
 // Buffers and descriptors of the chain passes.
@@ -548,7 +568,6 @@ void run_frame(spr_handle* H, bool record_begin = true) {
     init.fill[0] = {(uint32_t*)(H->zero.p + z.a_words), 2 * (int64_t)(z.total - z.a_words), nullptr, 0, 0, 0u};
     init.n_fills = 1;
     if (gen) {
-        H->heavy_list.ensure((size_t)C * 5);
         if (!by_chain) {
             H->win_first.ensure((size_t)ceil_div(N, window));
             init.offsets = H->counts.p; init.C = C; init.window = window;
@@ -576,7 +595,7 @@ void run_frame(spr_handle* H, bool record_begin = true) {
                               keep ? H->inter.p : nullptr, aa ? H->chord.p : nullptr,
                               narrow ? H->epath.p : nullptr};
         if (by_chain) solve_and_pieces(H, C, d_cc, A, (int64_t)n1, H->n_cu * H->chain_k / 8, H->n_cu * H->merge_k / 8);
-        else curve_pass(H, d_cc, A, N, nullptr, window);
+        else curve_pass(H, d_cc, A, N, nullptr, window, H->h_pinned[2] != 0);
     } else {
         stage_mark(H, 5);
     }
@@ -660,7 +679,7 @@ void run_frame(spr_handle* H, bool record_begin = true) {
     S.p[kSumSpans] = d_totals + 1;
     S.p[kSumErr] = d_err;
     S.p[kSumWaveChains] = gen ? d_cc + (by_chain ? spr::kCcLightBegin : kCcSplit) : nullptr;
-    S.p[kSumHeavyPieces] = gen ? d_cc + (by_chain ? spr::kCcHeavyPieces : kCcBigPieces) : nullptr;
+    S.p[kSumHeavyPieces] = !gen ? nullptr : (by_chain ? d_cc + spr::kCcHeavyPieces : big_pieces(H));
     S.p[kSumLongBands] = reinterpret_cast<const int32_t*>(ctl_at(H, z.st_wind, z.ctr, 4).counter + 1);
     S.p[kSumBigBands] = d_bigcount;
     S.p[kSumTotal] = H->inj ? nullptr : H->counts.p + C;
@@ -981,7 +1000,6 @@ void run_learned_frame(spr_handle* H) {
     init.fill[3] = {(uint32_t*)H->brec_l.p, 2 * nb_budget, d_nb, 2, 0, 0u};
     init.n_fills = 4;
     if (C) {
-        H->heavy_list.ensure((size_t)C * 5);
         H->win_first.ensure((size_t)ceil_div(nl, window));
         init.offsets = H->counts.p; init.C = C; init.window = window;
         init.first = H->win_first.p; init.n_first = ceil_div(nl, window);
@@ -998,7 +1016,7 @@ void run_learned_frame(spr_handle* H) {
                               H->key.p, H->wn.p, H->epath.p, H->bucket_base.p, H->prow.p, H->hist_l.p, d_err,
                               debug ? H->inter.p : nullptr, nullptr, narrow ? H->epath.p : nullptr};
         if (by_chain) solve_and_pieces(H, C, d_cc, A, nl, H->n_cu * H->chain_k / 8, H->n_cu * H->merge_k / 8);
-        else curve_pass(H, d_cc, A, nl, d_live, window);
+        else curve_pass(H, d_cc, A, nl, d_live, window, false);
     } else {
         stage_mark(H, 5);
     }
@@ -1073,7 +1091,7 @@ void run_learned_frame(spr_handle* H) {
     S.p[kSumSpans] = d_totals + 1;
     S.p[kSumErr] = d_err;
     S.p[kSumWaveChains] = C ? d_cc + (by_chain ? spr::kCcLightBegin : kCcSplit) : nullptr;
-    S.p[kSumHeavyPieces] = C ? d_cc + (by_chain ? spr::kCcHeavyPieces : kCcBigPieces) : nullptr;
+    S.p[kSumHeavyPieces] = !C ? nullptr : (by_chain ? d_cc + spr::kCcHeavyPieces : big_pieces(H));
     S.p[kSumLongBands] = reinterpret_cast<const int32_t*>(ticket + 1);
     S.p[kSumBigBands] = d_bigcount;
     S.p[kSumTotal] = H->counts.p + C;
