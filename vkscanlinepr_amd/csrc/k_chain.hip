@@ -33,6 +33,7 @@
 //     1024 entries (and short ones whose next piece waits on a heavy chain) go to k_piece_heavy,
 //     which does the same with a whole workgroup per piece and more LDS.
 #include "device_common.hpp"
+#include "fragments.hpp"
 #include "kernels.hpp"
 
 namespace spr {
@@ -70,14 +71,15 @@ __device__ inline int class_cost_octave(int cls) { return cls < 64 ? cls >> 2 : 
 // piece k-1 (flagged end parameter and end point) to its own end, and its entries start after
 // the 1 + nx + ny entries of each earlier piece.  Each of the curve's 5 piece slots gets a
 // descriptor (base = -1: no piece), each non-empty chain a descriptor and every chain slot its
-// class byte (0xFF: no chain).
+// class byte (0xFF: no chain).  Entries that the count pass reserved and no piece writes get their
+// fragments here.
 __global__ __launch_bounds__(kBlock) void k_chain_prep(
     const float2* __restrict__ tpos, const uint32_t* __restrict__ cpos,
     const uint32_t* __restrict__ ctype, const float* __restrict__ cweight, const uint32_t* __restrict__ cpath,
     const int32_t* __restrict__ visible, const float4* __restrict__ cuts,
     const uint32_t* __restrict__ ncuts, const int32_t* __restrict__ offsets, uint32_t C, int w,
     int h, ChainDesc* __restrict__ chains, PieceDesc* __restrict__ pieces, uint8_t* __restrict__ chain_cls,
-    int32_t* __restrict__ class_count, const int32_t* __restrict__ over, const int2* __restrict__ pcanvas) {
+    int32_t* __restrict__ class_count, const int32_t* __restrict__ over, const FragArgs A) {
     __shared__ int32_t hist[kClasses];
     if (threadIdx.x < kClasses) hist[threadIdx.x] = 0;
     __syncthreads();
@@ -89,7 +91,7 @@ __global__ __launch_bounds__(kBlock) void k_chain_prep(
         const uint32_t path = cpath[c];
         const uint32_t nc = !skip && visible_mask(visible[path]) ? ncuts[c] : 0xFFFFFFFFu;  // all slots empty
         int cw = w, ch = h;
-        if (pcanvas && nc != 0xFFFFFFFFu) { const int2 cvs = pcanvas[path]; cw = cvs.x; ch = cvs.y; }
+        if (A.pcanvas && nc != 0xFFFFFFFFu) { const int2 cvs = A.pcanvas[path]; cw = cvs.x; ch = cvs.y; }
         const uint32_t type = ctype[c];
         CurvePts cv;
         float q[4] = {1.0f, 1.0f, 1.0f, 1.0f};
@@ -103,7 +105,7 @@ __global__ __launch_bounds__(kBlock) void k_chain_prep(
         }
         float t0 = 0.0f, p0x = 0.0f, p0y = 0.0f;
         if (nc != 0xFFFFFFFFu) { p0x = cv.x[0]; p0y = cv.y[0]; }
-        int off = 0;
+        int off = 0, written = base0;
 #pragma unroll
         for (int k = 0; k < 5; ++k) {
             PieceDesc pd;
@@ -116,6 +118,7 @@ __global__ __launch_bounds__(kBlock) void k_chain_prep(
                 const PieceGrid G = piece_grid(p0x, p0y, p1x, p1y, cw, ch);
                 const int base = base0 + off;
                 if (base + G.nx + G.ny + 1 <= limit) {  // count and write passes agree
+                    written = base + G.nx + G.ny + 1;
                     pd.base = base; pd.nx = G.nx; pd.ny = G.ny; pd.curve = (int32_t)c; pd.t0 = t0;
                     // the last piece's last segment runs to t = 1; the others run to the next
                     // piece's first entry
@@ -145,6 +148,11 @@ __global__ __launch_bounds__(kBlock) void k_chain_prep(
             }
             pieces[5 * (int64_t)c + k] = pd;
             reinterpret_cast<uint16_t*>(chain_cls)[5 * (int64_t)c + k] = (uint16_t)(k0 | (k1 << 8));
+        }
+        if (written < limit) {
+            const uint32_t bb = (uint32_t)A.bucket_base[path];
+            const int2 pr = A.prow[path];
+            for (int i = written; i < limit; ++i) store_gap(A, i, (int)c, path, bb, pr);
         }
     }
     __syncthreads();
@@ -657,26 +665,6 @@ __device__ inline PieceMeta meta_of_lane(const PieceMeta& m, int k) {
     return r;
 }
 
-// An entry's fragment outputs; returns its global bucket.  Frames with narrow sort words store the
-// bucket (in key) and the narrow word (bucket inside the path, x + 2 or 0 in the off-canvas
-// bucket, winding change + 1), which is all their scatter needs; the others store the key, the
-// winding change and the path.
-__device__ inline uint32_t store_fragment(const FragArgs& A, int64_t i, uint32_t yx, int swn, uint32_t path,
-                                          uint32_t bb, int2 pr) {
-    const uint32_t loc = bucket_local((int32_t)yx, pr, A.err);
-    const uint32_t bucket = bb + loc;
-    if (A.nword) {
-        const uint32_t xl = loc == (uint32_t)pr.y ? 0u : (yx & 0xFFFFu) - kNarrowX0;
-        A.key[i] = (int32_t)bucket;
-        A.nword[i] = (loc << 17) | (xl << 2) | (uint32_t)(swn + 1);
-    } else {
-        A.key[i] = (int32_t)yx;
-        A.wn[i] = (int8_t)swn;
-        A.epath[i] = path;
-    }
-    return bucket;
-}
-
 // gen_fragment for the entries of one piece, fin[0..n) = their final t bits: entry o's segment
 // runs to entry o+1, the last one's to m.t_end.  Keys, winding changes and paths are written
 // coalesced; bucket counts are aggregated over runs of the wave.  Every lane of the n_waves
@@ -1015,12 +1003,12 @@ hipError_t launch_chain_prep(const float2* tpos, const uint32_t* cpos, const uin
                              const float* cweight, const uint32_t* cpath, const int32_t* visible, const float4* cuts,
                              const uint32_t* ncuts, const int32_t* offsets, uint32_t C, int w, int h,
                              ChainDesc* chains, PieceDesc* pieces, uint8_t* chain_cls, int32_t* class_count,
-                             int n_cu, hipStream_t s, const int32_t* over, const int2* pcanvas) {
+                             const FragArgs& A, int n_cu, hipStream_t s, const int32_t* over) {
     if (C == 0) return hipSuccess;
     unsigned g = grid_for((int64_t)C);
     if (g > (unsigned)n_cu * 8) g = (unsigned)n_cu * 8;
     k_chain_prep<<<g, kBlock, 0, s>>>(tpos, cpos, ctype, cweight, cpath, visible, cuts, ncuts, offsets, C, w, h, chains,
-                                      pieces, chain_cls, class_count, over, pcanvas);
+                                      pieces, chain_cls, class_count, over, A);
     return hipGetLastError();
 }
 

@@ -45,6 +45,7 @@
 //
 // Pieces of more than kBigPiece entries, which the count pass lists, take k_big_pieces, one workgroup each.
 #include "device_common.hpp"
+#include "fragments.hpp"
 #include "kernels.hpp"
 #include "scan_common.hpp"
 #include "wave_solve.hpp"
@@ -190,26 +191,6 @@ __device__ inline uint32_t or_merged(const uint32_t* v, int n, int o) {
     for (int s = o; s > 0 && (v[s - 1] & 0xFFFFFFFCu) == m; --s) acc |= v[s - 1];
     if (o + 1 < n && (v[o + 1] & 0xFFFFFFFCu) == m) acc |= v[o + 1];
     return acc;
-}
-
-// An entry's fragment outputs; returns its global bucket.  Frames with narrow sort words store the
-// bucket (in key) and the narrow word (bucket inside the path, x + 2 or 0 in the off-canvas
-// bucket, winding change + 1), which is all their scatter needs; the others store the key, the
-// winding change and the path.
-__device__ inline uint32_t store_fragment(const FragArgs& A, int64_t i, uint32_t yx, int swn, uint32_t path,
-                                          uint32_t bb, int2 pr) {
-    const uint32_t loc = bucket_local((int32_t)yx, pr, A.err);
-    const uint32_t bucket = bb + loc;
-    if (A.nword) {
-        const uint32_t xl = loc == (uint32_t)pr.y ? 0u : (yx & 0xFFFFu) - kNarrowX0;
-        A.key[i] = (int32_t)bucket;
-        A.nword[i] = (loc << 17) | (xl << 2) | (uint32_t)(swn + 1);
-    } else {
-        A.key[i] = (int32_t)yx;
-        A.wn[i] = (int8_t)swn;
-        A.epath[i] = path;
-    }
-    return bucket;
 }
 
 // gen_fragment for the entries of one piece, v[0..n) = their merged t bits: entry o's segment
@@ -452,14 +433,6 @@ __device__ inline void merge_slots(CurveBatch& B, int s0, int s1, int longest, b
     for (int j = 0; j < kPerLane; ++j)
         if (dest[j] >= 0) B.v[dest[j] + rank[j]] = v[j];
     __syncthreads();
-}
-
-// An entry without a segment: the off-canvas cell, no winding change.
-__device__ inline void store_gap(const FragArgs& A, int64_t i, int curve, uint32_t path, uint32_t bb, int2 pr) {
-    const uint32_t bucket = store_fragment(A, i, kSentinelKey, 0, path, bb, pr);
-    atomicAdd(&A.hist[bucket], 1);
-    if (A.inter) A.inter[i] = make_int2(curve, 0);
-    if (A.chord) A.chord[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 }
 
 // Segments of a chain of n crossings whose first one has `head` of them: 1 + rest, the others of

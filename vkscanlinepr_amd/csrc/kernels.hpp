@@ -140,7 +140,7 @@ hipError_t launch_chain_prep(const float2* tpos, const uint32_t* cpos, const uin
                              const float* cweight, const uint32_t* cpath, const int32_t* visible, const float4* cuts,
                              const uint32_t* ncuts, const int32_t* offsets, uint32_t C, int w, int h,
                              ChainDesc* chains, PieceDesc* pieces, uint8_t* chain_cls, int32_t* class_count,
-                             int n_cu, hipStream_t s, const int32_t* over = nullptr, const int2* pcanvas = nullptr);
+                             const FragArgs& A, int n_cu, hipStream_t s, const int32_t* over = nullptr);
 hipError_t launch_chain_order(const uint8_t* chain_cls, uint32_t C, const int32_t* class_count,
                               int32_t* class_off, int32_t* class_fill, int32_t* light_begin, int32_t* order,
                               int n_cu, hipStream_t s);

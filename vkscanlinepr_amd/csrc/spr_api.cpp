@@ -417,7 +417,7 @@ void curve_pass(spr_handle* H, int32_t* d_cc, const spr::FragArgs& A, int64_t n,
 }
 
 // Buffers and descriptors of the chain passes.
-void chain_setup(spr_handle* H, int64_t n, int32_t* d_cc, const int2* pcanvas, const int32_t* over) {
+void chain_setup(spr_handle* H, int64_t n, int32_t* d_cc, const spr::FragArgs& A, const int32_t* over) {
     const uint32_t C = H->C;
     hipStream_t s = H->stream;
     H->chain_t.ensure((size_t)std::max<int64_t>(n, 1));
@@ -431,7 +431,7 @@ void chain_setup(spr_handle* H, int64_t n, int32_t* d_cc, const int2* pcanvas, c
     H->mono.ensure((size_t)C * 10);
     SPR_HIP(spr::launch_chain_prep(H->tpos.p, H->cpos.p, H->ctype.p, H->arcw(), H->cpath.p, H->visible.p, H->cuts.p,
                                    H->ncuts.p, H->counts.p, C, (int)H->w, (int)H->h, H->chains.p, H->pieces.p,
-                                   H->chain_cls.p, d_cc, H->n_cu, s, over, pcanvas));
+                                   H->chain_cls.p, d_cc, A, H->n_cu, s, over));
     SPR_HIP(spr::launch_chain_order(H->chain_cls.p, C, d_cc, d_cc + spr::kCcOff, d_cc + spr::kCcFill,
                                     d_cc + spr::kCcLightBegin, H->chain_order.p, H->n_cu, s));
 }
@@ -586,14 +586,13 @@ void run_frame(spr_handle* H, bool record_begin = true) {
 
     int32_t* d_cc = reinterpret_cast<int32_t*>(H->zero.p + z.chainctl);
     if (H->inj) SPR_HIP(hipMemcpyAsync(H->inter.p, H->inj_inter.data(), (size_t)N * 8, hipMemcpyHostToDevice, s));
-    if (gen && by_chain) chain_setup(H, N, d_cc, nullptr, nullptr);
+    // narrow frames: the curve pass stores each entry's bucket (key) and sort word (epath)
+    const spr::FragArgs A{H->cpos.p, H->ctype.p, H->arcw(), H->cpath.p, H->tpos.p, w, h, nullptr,
+                          H->key.p, H->wn.p, H->epath.p, H->bucket_base.p, H->prow.p, d_hist, d_err,
+                          keep ? H->inter.p : nullptr, aa ? H->chord.p : nullptr, narrow ? H->epath.p : nullptr};
+    if (gen && by_chain) chain_setup(H, N, d_cc, A, nullptr);
     stage_mark(H, 4);
     if (gen) {
-        // narrow frames: the curve pass stores each entry's bucket (key) and sort word (epath)
-        const spr::FragArgs A{H->cpos.p, H->ctype.p, H->arcw(), H->cpath.p, H->tpos.p, w, h, nullptr,
-                              H->key.p, H->wn.p, H->epath.p, H->bucket_base.p, H->prow.p, d_hist, d_err,
-                              keep ? H->inter.p : nullptr, aa ? H->chord.p : nullptr,
-                              narrow ? H->epath.p : nullptr};
         if (by_chain) solve_and_pieces(H, C, d_cc, A, (int64_t)n1, H->n_cu * H->chain_k / 8, H->n_cu * H->merge_k / 8);
         else curve_pass(H, d_cc, A, N, nullptr, window, H->h_pinned[2] != 0);
     } else {
@@ -1009,12 +1008,12 @@ void run_learned_frame(spr_handle* H) {
 
     // phase 2: the plain stages on device counts, within the budget
     int32_t* d_cc = reinterpret_cast<int32_t*>(H->zero.p + z.chainctl);
-    if (C && by_chain) chain_setup(H, nl, d_cc, pcv, d_over);
+    const spr::FragArgs A{H->cpos.p, H->ctype.p, H->arcw(), H->cpath.p, H->tpos.p, w, h, pcv,
+                          H->key.p, H->wn.p, H->epath.p, H->bucket_base.p, H->prow.p, H->hist_l.p, d_err,
+                          debug ? H->inter.p : nullptr, nullptr, narrow ? H->epath.p : nullptr};
+    if (C && by_chain) chain_setup(H, nl, d_cc, A, d_over);
     stage_mark(H, 4);
     if (C) {
-        const spr::FragArgs A{H->cpos.p, H->ctype.p, H->arcw(), H->cpath.p, H->tpos.p, w, h, pcv,
-                              H->key.p, H->wn.p, H->epath.p, H->bucket_base.p, H->prow.p, H->hist_l.p, d_err,
-                              debug ? H->inter.p : nullptr, nullptr, narrow ? H->epath.p : nullptr};
         if (by_chain) solve_and_pieces(H, C, d_cc, A, nl, H->n_cu * H->chain_k / 8, H->n_cu * H->merge_k / 8);
         else curve_pass(H, d_cc, A, nl, d_live, window, false);
     } else {
