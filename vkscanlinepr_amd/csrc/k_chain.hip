@@ -1,5 +1,5 @@
 // k_chain.hip -- intersection write (make_intersection_1.comp:217-447) for gfx950, in passes over
-// whole chains: the form of large frames (k_curves.hip is that of the others).
+// whole chains: the form of large frames and of those with many long starts (k_curves.hip is that of the others).
 //
 // Inside one monotone piece the reference interleaves x-grid and y-grid crossings, but every
 // bisection for the next crossing on one axis starts from the previous crossing of the SAME axis
@@ -16,7 +16,8 @@
 //     one chain per lane, in descending length.  k_chain_segments takes the longer ones, several
 //     lanes per chain: each lane solves a segment from a guess of the value before it, and the
 //     segments whose guess was off are solved again from the true one, so that the results are the
-//     sequential chain's (the reasons stand in k_curves.hip).  The first item of every wave is its
+//     sequential chain's (the reasons stand in k_curves.hip).  Of the longer ones, those with a long
+//     start (wave_solve.hpp), where guesses do not pay, take a whole wave each.  The first item of every wave is its
 //     global wave index (the first waves of a launch sit on distinct SIMDs, so the costliest items
 //     do not share one), later items come from an atomic counter; issue priority follows the item's
 //     cost.
@@ -35,6 +36,7 @@
 #include "device_common.hpp"
 #include "fragments.hpp"
 #include "kernels.hpp"
+#include "wave_solve.hpp"
 
 namespace spr {
 
@@ -45,6 +47,13 @@ constexpr int kStage = 4096;       // piece values staged in LDS by the merging 
 constexpr int kClasses = kChainClasses;  // 0..63: cubic chains (4 per octave), 64..79: line chains
 // first heavy cubic class: a quarter-octave class 4*l + sub holds lengths >= 2^l (l = 8: 256)
 constexpr int kHeavyClass = 4 * 8;
+// Heavy chains with a long start (wave_solve.hpp) that holds two thirds of them: segments still pay for the rest of a
+// longer chain.  300 cubics whose first part crosses 2000^2: 2,683 us a frame without this class, 786 with it.  Every
+// long start in it cost an illustration of 48.7 M entries on 4096^2 140 us of 2,720, and at twice its size 650 of
+// 2,300; this rule costs them nothing.  (Of 1/2, 3/5, 2/3, 3/4 and all, 1/2 and 3/5 cost drawings up to 40%
+// and 9%, 3/4 and all leave shorter starts to the segments: 300 arcs 1,189 and 1,544 instead of 914.)  The costliest
+// class of all; no length reaches it.
+constexpr int kLongClass = 63;
 static_assert(kHeavyCrossings == 1 << 8, "heavy class boundary");
 static_assert(kFrag == 2, "chain descriptors keep only the sign of the grid step");
 
@@ -138,7 +147,14 @@ __global__ __launch_bounds__(kBlock) void k_chain_prep(
                         d.t1 = t1;
                         d.type = (int16_t)type;
                         chains[2 * (5 * (int64_t)c + k) + side] = d;
-                        const uint32_t kc = (uint32_t)chain_class(n, type != kLine);
+                        uint32_t kc = (uint32_t)chain_class(n, type != kLine);
+                        if (kc >= (uint32_t)kHeavyClass && kc < 64u) {
+                            const float* p = side ? cv.y : cv.x;
+                            const CurveAxis a = {{p[0], p[1], p[2], p[3]}};
+                            const bool neg = (d.flags & 2) != 0;
+                            const int early = crossings_before(type, a, d.line0, neg, t0, kEighth * t1, n);
+                            if (3 * early > 2 * n && long_start(type, a, d.line0, neg, t0, t1, n)) kc = (uint32_t)kLongClass;
+                        }
                         atomicAdd(&hist[kc], 1);
                         if (side) k1 = kc; else k0 = kc;
                     }
@@ -394,20 +410,37 @@ __device__ inline void resolve_segment_t(const ChainDesc& d, const CurveAxis& a,
     }
 }
 
-// About how many of a chain's crossings lie before parameter tau.
-__device__ inline int crossings_before(const ChainDesc& d, const CurveAxis& a, float tau) {
-    if (!(d.t0 < tau)) return 0;
-    const float v = eval_axis((uint32_t)d.type, tau, a.c[0], a.c[1], a.c[2], a.c[3]) - d.line0;
-    const float k = (chain_step(d) < 0.0f ? -v : v) * 0.5f + 2.0f;
-    return k >= (float)d.n ? d.n : (k > 0.0f ? (int)k : 0);
-}
-
-// Crossings solved to guess a segment's start, and the parameter that a chain's first segment reaches
-// past, in parts of its end (runs of the bisection from different starts fall together slowly near 0).
+// Crossings solved to guess a segment's start.
 constexpr int kWarm = 8;
-constexpr float kHeadTau = 0.03125f;
 // log2 of the lanes per chain: 2 in octave 8 (256 to 511 crossings), 4 in octave 9, 8 above.
 constexpr int kLanes8 = 1, kLanes9 = 2, kLanes10 = 3;
+
+// A chain by a whole wave, all of its crossings in order; stores like solve_chain_lane_t, 64 values at a time.
+__device__ inline void solve_chain_wave(const ChainDesc& d, const CurveAxis& a, float* __restrict__ chain_t,
+                                        uint8_t* __restrict__ mono) {
+    const int lane = threadIdx.x & 63;
+    const TreeNode N = tree_node(lane);
+    float* out = chain_t + d.out;
+    float prev = d.t0, kept = 0.0f;
+    uint32_t rises = 0, falls = 0;
+    const uint32_t side = (uint32_t)chain_side(d);
+    solve_wave_any(N, (uint32_t)d.type, a, d.line0, chain_step(d), side, d.t1, d.n, d.t0, [&](int k, float v) {
+        const float before = k > 0 || side ? prev : v;
+        falls |= !(v >= before) ? 1u : 0u;
+        rises |= !(v <= before) ? 1u : 0u;
+        prev = v;
+        kept = (k & 63) == lane ? v : kept;
+        if ((k & 63) == 63 || k == d.n - 1)
+            if (lane <= (k & 63)) out[(k & ~63) + lane] = kept;
+    });
+    if (lane == 0) *mono = (uint8_t)((falls ? 0 : 1) | (rises ? 0 : 2));
+}
+
+// Chains with long starts up to this many are solved by a wave each, more by a lane each: a wave takes a crossing in
+// half a lane's time and 64 times its share of the chip.  us a frame, by waves and by lanes: 3,000 chains of 800
+// crossings 1,431 and 1,737 or 1,143 and 1,166 (arcs, cubics), 2,400 of 320 552 and 550, 10,000 of 400 1,585 and 917,
+// 10,000 of 800 2,999 and 1,499.
+constexpr int32_t kLongByWave = 2048;
 
 // The chains of kHeavyCrossings and more, [0, *light_begin) in class order, cut into segments of 130 to 260
 // crossings (more in the few chains above 2,000), one lane each.  Longer segments waste less on
@@ -428,20 +461,38 @@ __global__ __launch_bounds__(kBlock) void k_chain_segments(const float2* __restr
     __shared__ float s_stage[16 * kBlock];
     float* stage = s_stage + threadIdx.x;
     const int lane = threadIdx.x & 63;
-    // the chains of octaves 10 and up, 9 and 8 in class order: [0, b10), [b10, b9), [b9, lb)
+    // the chains with long starts, then those of octaves 10 and up, 9 and 8 in class order: [0, nl),
+    // [nl, b10), [b10, b9), [b9, lb)
+    const int32_t nl = class_off[kLongClass - 1];
+    const bool by_wave = nl <= kLongByWave;
+    const int32_t n_long = by_wave ? nl : (nl + 63) >> 6;
     const int32_t b10 = class_off[kHeavyClass + 7], b9 = class_off[kHeavyClass + 3], lb = *light_begin;
     constexpr int P10 = 6 - kLanes10, P9 = 6 - kLanes9, P8 = 6 - kLanes8;  // log2 of a wave's chains
-    const int32_t n10 = (b10 + (1 << P10) - 1) >> P10, n9 = (b9 - b10 + (1 << P9) - 1) >> P9;
-    const int32_t items = n10 + n9 + ((lb - b9 + (1 << P8) - 1) >> P8);
+    const int32_t n10 = (b10 - nl + (1 << P10) - 1) >> P10, n9 = (b9 - b10 + (1 << P9) - 1) >> P9;
+    const int32_t items = n_long + n10 + n9 + ((lb - b9 + (1 << P8) - 1) >> P8);
     const int32_t n_waves = (int32_t)gridDim.x * (kBlock / 64);
     int32_t item = (int32_t)blockIdx.x * (kBlock / 64) + (int32_t)(threadIdx.x >> 6);
     int32_t next = 0;
     if (lane == 0 && item < items) next = n_waves + atomicAdd(work, 1);
     while (item < items) {
-        const int p = item < n10 ? P10 : (item < n10 + n9 ? P9 : P8);  // log2 of the wave's chains
-        const int32_t c0 = item < n10 ? item << P10
-                                      : (item < n10 + n9 ? b10 + ((item - n10) << P9) : b9 + ((item - n10 - n9) << P8));
-        const int32_t end = item < n10 ? b10 : (item < n10 + n9 ? b9 : lb);
+        if (item < n_long) {
+            if (by_wave) {
+                const int32_t ci = __builtin_amdgcn_readfirstlane(order[item]);
+                solve_chain_wave(chains[ci], load_axis(tpos, cpos, cweight, chains[ci]), chain_t, mono + ci);
+            } else if (item * 64 + lane < nl) {
+                const int32_t ci = order[item * 64 + lane];
+                const ChainDesc d = chains[ci];
+                solve_chain_lane(d, load_axis(tpos, cpos, cweight, d), chain_t + d.out, mono + ci, stage);
+            }
+            item = __shfl(next, 0);
+            if (lane == 0 && item < items) next = n_waves + atomicAdd(work, 1);
+            continue;
+        }
+        const int32_t it = item - n_long;
+        const int p = it < n10 ? P10 : (it < n10 + n9 ? P9 : P8);  // log2 of the wave's chains
+        const int32_t c0 = it < n10 ? nl + (it << P10)
+                                    : (it < n10 + n9 ? b10 + ((it - n10) << P9) : b9 + ((it - n10 - n9) << P8));
+        const int32_t end = it < n10 ? b10 : (it < n10 + n9 ? b9 : lb);
         const int lanes = 64 >> p, j = lane & (lanes - 1);
         const int32_t k = c0 + (lane >> (6 - p));
         bool on = k < end;
@@ -455,7 +506,8 @@ __global__ __launch_bounds__(kBlock) void k_chain_segments(const float2* __restr
         int i0 = 0, i1 = 0;
         if (on) {
             const int len = (d.n + kWarm * (lanes - 1) + lanes - 1) / lanes;  // steps per lane, guesses included
-            const int head = max(len, crossings_before(d, a, kHeadTau * d.t1));
+            const int head = max(len, crossings_before((uint32_t)d.type, a, d.line0, chain_step(d) < 0.0f, d.t0,
+                                                       kHeadTau * d.t1, d.n));
             const int rest = d.n - head >= lanes - 1 ? d.n - head : 0;
             if (j == 0) {
                 i1 = d.n - rest;

@@ -664,10 +664,10 @@ void k_curves(const CurveArgs K, const FragArgs A) {
             if (r.n > len + len / 2) {
                 head = len;
                 if (r.type != kLine) {
-                    k8 = crossings_before(r.type, r.a, r.line0, r.neg, r.t0, 0.125f * r.t1, r.n);
+                    k8 = crossings_before(r.type, r.a, r.line0, r.neg, r.t0, kEighth * r.t1, r.n);
                     if (k8) head = max(len, crossings_before(r.type, r.a, r.line0, r.neg, r.t0, kHeadTau * r.t1, r.n));
                     int w = kLongHeads;
-                    if (head > kLongHead) w = atomicAdd(&B.n_long, 1);
+                    if (head > kLongHead || k8 > kLongEighth) w = atomicAdd(&B.n_long, 1);
                     if (w < kLongHeads) {
                         B.longs[w] = (uint16_t)ch;
                         by_wave = kByWave;
@@ -913,8 +913,8 @@ __global__ __launch_bounds__(kBigThreads) void k_big_pieces(const CurveArgs K, c
         // segments: one per thread (as in k_curves)
         const int len = max(kSegMin, (nv + kBigThreads - 5) / (kBigThreads - 4));
         const CurveAxis ax = {{cv.x[0], cv.x[1], cv.x[2], cv.x[3]}}, ay = {{cv.y[0], cv.y[1], cv.y[2], cv.y[3]}};
-        const int kx = crossings_before(cv.type, ax, g.x0, g.xneg, g.t0, 0.125f * g.t1, g.nx);
-        const int ky = crossings_before(cv.type, ay, g.y0, g.yneg, g.t0, 0.125f * g.t1, g.ny);
+        const int kx = crossings_before(cv.type, ax, g.x0, g.xneg, g.t0, kEighth * g.t1, g.nx);
+        const int ky = crossings_before(cv.type, ay, g.y0, g.yneg, g.t0, kEighth * g.t1, g.ny);
         int hx = min(g.nx, max(len, crossings_before(cv.type, ax, g.x0, g.xneg, g.t0, kHeadTau * g.t1, g.nx)));
         int hy = min(g.ny, max(len, crossings_before(cv.type, ay, g.y0, g.yneg, g.t0, kHeadTau * g.t1, g.ny)));
         const bool wx = cv.type != kLine && hx > kBigLongHead, wy = cv.type != kLine && hy > kBigLongHead;  // by a wave

@@ -3,6 +3,7 @@
 #include "device_common.hpp"
 #include "kernels.hpp"
 #include "scan_common.hpp"
+#include "wave_solve.hpp"
 
 namespace spr {
 
@@ -185,7 +186,11 @@ __global__ __launch_bounds__(kBlock) void k_count(const CountArgs K) {
         K.cuts[c] = make_float4(q[0], q[1], q[2], q[3]);
         K.ncuts[c] = n;
         if (vis) {
-            float p0x = cv.x[0], p0y = cv.y[0];
+            float p0x = cv.x[0], p0y = cv.y[0], t_first = -1.0f, end_x = 0.0f, end_y = 0.0f;
+            // a piece beyond the curve pass's windows, perhaps: its grid rounds differently from the count far
+            // outside any canvas
+            const float far = 1e9f;
+            bool big = !(fabsf(p0x) < far) | !(fabsf(p0y) < far);
 #pragma unroll
             for (uint32_t k = 0; k < 5; ++k) {
                 if (k > n) break;
@@ -193,10 +198,17 @@ __global__ __launch_bounds__(kBlock) void k_count(const CountArgs K) {
                 const float p1x = cv.ex(t), p1y = cv.ey(t);
                 const int pc = piece_count(p0x, p0y, p1x, p1y, w, h);
                 cnt += pc;
-                // as the curve pass counts it: the two round differently only far outside any canvas
-                const float far = 1e9f;
-                if (pc > kCurvePieceMax ||
-                    !(fabsf(p0x) < far && fabsf(p0y) < far && fabsf(p1x) < far && fabsf(p1y) < far)) {
+                big = big | (pc > kCurvePieceMax) | !(fabsf(p1x) < far) | !(fabsf(p1y) < far);
+                if (k == 0 && pc > kLongHead && cv.type != kLine) { t_first = t; end_x = p1x; end_y = p1y; }
+                p0x = p1x; p0y = p1y;
+            }
+            if (big) {
+                p0x = cv.x[0]; p0y = cv.y[0];
+#pragma unroll 1
+                for (uint32_t k = 0; k <= n && k < 5; ++k) {
+                    const float qk = k < 2 ? (k == 0 ? q[0] : q[1]) : (k == 2 ? q[2] : q[3]);
+                    const float t = k < n ? qk : 1.0f;
+                    const float p1x = cv.ex(t), p1y = cv.ey(t);
                     const PieceGrid G = piece_grid(p0x, p0y, p1x, p1y, w, h);
                     if (1 + G.nx + G.ny > kCurvePieceMax) {
                         const int32_t at = atomicAdd(K.n_big, 1);
@@ -204,8 +216,25 @@ __global__ __launch_bounds__(kBlock) void k_count(const CountArgs K) {
                         if (at == 0 && K.host)  // one store: an illustration of 34 M entries lost 110 us to one for each
                             __hip_atomic_store(&K.host[2], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                     }
+                    p0x = p1x; p0y = p1y;
                 }
-                p0x = p1x; p0y = p1y;
+            }
+            // the first piece's chains with many crossings before t1 / 32 (only the choice of a pass hangs on them)
+            int n_long = 0;
+            float reach = cv.type == kArc ? INFINITY : 0.0f;  // 128 pixels before t / 32 need 1,400 in all
+#pragma unroll
+            for (int i = 1; i < 4; ++i)
+                reach = fmaxf(reach, fmaxf(fabsf(cv.x[i] - cv.x[0]), fabsf(cv.y[i] - cv.y[0])));
+            if (t_first >= 0.0f && reach > 1024.0f) {
+                const PieceGrid G = piece_grid(cv.x[0], cv.y[0], end_x, end_y, w, h);
+                const float t32 = kHeadTau * t_first, x32 = cv.ex(t32), y32 = cv.ey(t32);
+                n_long = (G.nx > kLongHead && 0.25f * G.dx * (x32 - G.x0) > (float)kLongHead ? 1 : 0) +
+                         (G.ny > kLongHead && 0.25f * G.dy * (y32 - G.y0) > (float)kLongHead ? 1 : 0);
+            }
+            if (n_long) {
+                const int before = atomicAdd(K.n_long, n_long);
+                if (K.host && before <= kManyLong && before + n_long > kManyLong)
+                    __hip_atomic_store(&K.host[3], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             }
         }
     }

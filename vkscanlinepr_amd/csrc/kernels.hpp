@@ -43,6 +43,11 @@ hipError_t launch_transform(const float2* pos, const uint32_t* pos_path, uint32_
 // Statuses and counters zeroed; tiles of kCountTile curves or paths, at least one of each.
 constexpr int kCountTile = 256;
 constexpr int kCurvePieceMax = 1024;  // entries of a piece that a window of the curve pass takes
+// Frames with more chains with long starts than this take the chain passes, where a light chain has a lane and a
+// heavy one a wave up to some number of them: the curve pass has a wave for each, which fills the chip.  us a frame,
+// curve pass and chain passes: 4,200 such cubics at 400^2 894 and 578, 5,000 at 800^2 1,934 and 902, 300 at 2000^2
+// 870 and 789; 64 instead made drawings with a few closer views of long curves slower.
+constexpr int kManyLong = 256;
 inline int count_tiles(int64_t n) { return (int)(n > 0 ? (n + kCountTile - 1) / kCountTile : 1); }
 struct CountArgs {
     const float2* tpos;
@@ -70,9 +75,11 @@ struct CountArgs {
     unsigned long long* path_status;
     uint32_t* path_counter;
     const int2* pcanvas;        // per-path canvas of a batch, or null
-    int32_t* host;              // the two totals and a word set with the first big piece, in host memory, or null
+    int32_t* host;              // in host memory, or null: the two totals, a word set with the first big piece and
+                                // one set when n_long exceeds kManyLong
     int32_t* big;               // [5 C] the pieces of more than kCurvePieceMax entries: 5 curve + piece, in any order
     int32_t* n_big;             // zeroed
+    int32_t* n_long;            // zeroed: += first pieces' chains with long starts (wave_solve.hpp)
 };
 hipError_t launch_count(const CountArgs& K, hipStream_t s);
 hipError_t launch_segment_stats(const int32_t* seg, uint32_t Np, int32_t* max_len, hipStream_t s);

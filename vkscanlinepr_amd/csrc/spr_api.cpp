@@ -114,7 +114,7 @@ void mvp_inverse(const float m[16], float out[9]) {
 // allocation counters.
 enum {
     kSumCells = 0, kSumSpans, kSumErr, kSumWaveChains, kSumHeavyPieces, kSumLongBands, kSumBigBands,
-    kSumTotal, kSumOver, kSumOverflow, kSumLive, kSumArena, kSumSorted, kSumCapR, kSumCount
+    kSumTotal, kSumOver, kSumOverflow, kSumLive, kSumArena, kSumSorted, kSumCapR, kSumLong, kSumCount
 };
 static_assert(kSumCount <= spr::kSummaryMax, "summary slots");
 
@@ -216,6 +216,7 @@ struct spr_handle {
     DBuf<int2> brec_l;
     int64_t lb_n = 0, lb_r = 0;                     // learned frame budgets (entries, records)
     int64_t total_seen = 0, route_n = 0;            // most entries a learned frame of the scene had; what chose the route
+    bool long_seen = false, route_long = false;     // its last frame had many chains with long starts; as above
     bool need_prediction = true;                    // scene or model changed: read the prediction back
     bool lb_dirty = true;                           // scene, MVP, model or margin changed: the graph is stale
     int64_t n_live = 0;                             // entries of the last learned frame
@@ -348,21 +349,22 @@ void stage_mark(spr_handle* H, int idx) {
     H->n_marks = idx + 1;
 }
 
-// The number of big pieces that the count pass lists, behind the list (the control words can move
-// to another buffer between the count and the curve pass).
+// The number of big pieces that the count pass lists and of chains with long starts, behind the list (the
+// control words can move to another buffer between the count and the curve pass).
 int32_t* big_pieces(const spr_handle* H) { return H->heavy_list.p + 5 * (size_t)H->C; }
+int32_t* long_chains(const spr_handle* H) { return big_pieces(H) + 1; }
 
 // Clears what the transform and the count pass start from, in one launch.  The count pass writes the
 // path segments from its curves, so a scene without any has them cleared here.
 void clear_prefix(spr_handle* H, int64_t control_words) {
-    H->heavy_list.ensure(5 * (size_t)H->C + 1);
-    H->h_pinned[2] = 0;
+    H->heavy_list.ensure(5 * (size_t)H->C + 2);
+    H->h_pinned[2] = H->h_pinned[3] = 0;
     spr::FrameInit init{};
     init.fill[0] = {(uint32_t*)H->zero.p, control_words, nullptr, 0, 0, 0u};
     init.fill[1] = {(uint32_t*)H->visible.p, H->Np, nullptr, 0, 0, 0u};
     init.fill[2] = {(uint32_t*)H->row_lo.p, H->Np, nullptr, 0, 0, 0x7FFFFFFFu};
     init.fill[3] = {(uint32_t*)H->row_hi.p, H->Np, nullptr, 0, 0, 0x80000000u};
-    init.fill[4] = {(uint32_t*)big_pieces(H), 1, nullptr, 0, 0, 0u};
+    init.fill[4] = {(uint32_t*)big_pieces(H), 2, nullptr, 0, 0, 0u};
     init.n_fills = 5;
     if (!H->C) init.fill[init.n_fills++] = {(uint32_t*)H->seg.p, (int64_t)H->Np + 1, nullptr, 0, 0, 0u};
     SPR_HIP(spr::launch_frame_init(init, H->stream));
@@ -374,7 +376,8 @@ spr::CountArgs count_args(spr_handle* H, int rmax, spr::ScanCtl curves, spr::Sca
     return spr::CountArgs{H->tpos.p, H->cpos.p, H->ctype.p, H->arcw(), H->cpath.p, H->visible.p, H->C, (int)H->w,
                           (int)H->h, H->cuts.p, H->ncuts.p, H->counts.p, seg, spr::count_tiles(H->C), curves.status,
                           curves.counter, H->row_lo.p, H->row_hi.p, H->Np, rmax, H->bucket_base.p, H->prow.p,
-                          spr::count_tiles(H->Np), paths.status, paths.counter, pcanvas, host, H->heavy_list.p, big_pieces(H)};
+                          spr::count_tiles(H->Np), paths.status, paths.counter, pcanvas, host, H->heavy_list.p, big_pieces(H),
+                          long_chains(H)};
 }
 
 // Entries per window of the curve pass.  A workgroup takes one window, and 1,536 workgroups are
@@ -562,7 +565,7 @@ void run_frame(spr_handle* H, bool record_begin = true) {
     }
     H->crec.ensure(2 * n1);
     H->image.ensure((size_t)4 * H->w * H->h);
-    const bool gen = !H->inj && N > 0, by_chain = N >= spr::kChainFrame;
+    const bool gen = !H->inj && N > 0, by_chain = N >= spr::kChainFrame || H->h_pinned[3] != 0;
     const int32_t window = curve_window(H, N);
     spr::FrameInit init{};
     init.fill[0] = {(uint32_t*)(H->zero.p + z.a_words), 2 * (int64_t)(z.total - z.a_words), nullptr, 0, 0, 0u};
@@ -989,9 +992,12 @@ void run_learned_frame(spr_handle* H) {
     // the prediction (or a batch's proven bound) can put far above it: a 6.2 M entry pan at 1920x1080
     // on a budget above 2^24 took 1007 us by chains, 925 by curves.  A captured frame takes the route
     // of the eager one before it, whose buffers are there.
-    if (!H->capturing) H->route_n = H->total_seen > 0 ? std::min(H->total_seen, nl) : nl;
+    if (!H->capturing) {
+        H->route_n = H->total_seen > 0 ? std::min(H->total_seen, nl) : nl;
+        H->route_long = H->long_seen;
+    }
     const int32_t window = curve_window(H, H->route_n);
-    const bool by_chain = H->route_n >= spr::kChainFrame;
+    const bool by_chain = H->route_n >= spr::kChainFrame || H->route_long;
     spr::FrameInit init{};
     init.fill[0] = {(uint32_t*)H->hist_l.p, nb_budget + 1, d_nb, 1, 1, 0u};
     init.fill[1] = {(uint32_t*)H->fill_l.p, nb_budget, d_nb, 1, 0, 0u};
@@ -1100,6 +1106,7 @@ void run_learned_frame(spr_handle* H) {
     S.p[kSumArena] = H->arena.p + Np;
     S.p[kSumSorted] = d_nsorted;
     S.p[kSumCapR] = d_capr;
+    S.p[kSumLong] = long_chains(H);
     const spr::TallyArgs T = tally_args(H, narrow ? H->band_cnt.p : nullptr, d_nbands, max_bands, d_totals, S);
     spr::PaintArgs pa;
     SPR_HIP(spr::launch_composite(H->crec.p, H->brec_l.p, H->bucket_base.p, H->prow.p, H->fill.p, Np,
@@ -1120,6 +1127,7 @@ void learned_finish(spr_handle* H) {
     const int64_t total = H->sum(kSumTotal);
     const int64_t overflow_paths = H->sum(kSumOverflow);
     H->total_seen = std::max(H->total_seen, total);
+    H->long_seen = H->sum(kSumLong) > spr::kManyLong;
     H->frame_done = true;
     H->last_learned = true;
     H->last_fallback = false;
@@ -1363,6 +1371,7 @@ void load_arrays(spr_handle* H, const float* pos, const uint32_t* pos_path, uint
     H->inj = false;
     H->inj_inter.clear();
     H->total_seen = 0;
+    H->long_seen = false;
     H->lb_dirty = true;
     H->need_prediction = true;
     H->batch = false;
@@ -1854,6 +1863,7 @@ int spr_load_batch(spr_handle* H, const spr_scene* const* docs, const uint32_t* 
         H->max_h = max_h;
         H->img_bytes = img;
         H->total_seen = 0;
+        H->long_seen = false;
         H->lb_dirty = true;
         H->need_prediction = true;
     });

@@ -123,9 +123,15 @@ __device__ inline int crossings_before(uint32_t type, const CurveAxis& a, float 
     return k >= (float)n ? n : (k > 0.0f ? (int)k : 0);
 }
 
-// A chain has a long start when more crossings than this lie before kHeadTau of its end parameter: there two
-// runs of the bisection from different starts hardly ever fall together (k_curves.hip).
-constexpr int kLongHead = 64;
-constexpr float kHeadTau = 0.03125f;
+// A chain has a long start when many crossings lie near t = 0, where two runs of the bisection from different starts
+// hardly ever fall together (k_curves.hip): more than kLongHead before 1/32 of its end parameter, or more than
+// kLongEighth before 1/8.
+constexpr int kLongHead = 64, kLongEighth = 224;
+constexpr float kHeadTau = 0.03125f, kEighth = 0.125f;
+__device__ inline bool long_start(uint32_t type, const CurveAxis& a, float line0, bool neg, float t0, float t1, int n) {
+    return n > kLongHead && t0 < kEighth * t1 &&
+           (crossings_before(type, a, line0, neg, t0, kEighth * t1, n) > kLongEighth ||
+            crossings_before(type, a, line0, neg, t0, kHeadTau * t1, n) > kLongHead);
+}
 
 }  // namespace spr
