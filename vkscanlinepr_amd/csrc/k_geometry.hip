@@ -203,6 +203,7 @@ __global__ __launch_bounds__(kBlock) void k_count(const CountArgs K) {
                 p0x = p1x; p0y = p1y;
             }
             if (big) {
+                uint32_t pieces = 0;
                 p0x = cv.x[0]; p0y = cv.y[0];
 #pragma unroll 1
                 for (uint32_t k = 0; k <= n && k < 5; ++k) {
@@ -210,13 +211,14 @@ __global__ __launch_bounds__(kBlock) void k_count(const CountArgs K) {
                     const float t = k < n ? qk : 1.0f;
                     const float p1x = cv.ex(t), p1y = cv.ey(t);
                     const PieceGrid G = piece_grid(p0x, p0y, p1x, p1y, w, h);
-                    if (1 + G.nx + G.ny > kCurvePieceMax) {
-                        const int32_t at = atomicAdd(K.n_big, 1);
-                        K.big[at] = (int32_t)(5 * c + k);
-                        if (at == 0 && K.host)  // one store: an illustration of 34 M entries lost 110 us to one for each
-                            __hip_atomic_store(&K.host[2], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                    }
+                    pieces |= 1 + G.nx + G.ny > kCurvePieceMax ? 1u << k : 0u;
                     p0x = p1x; p0y = p1y;
+                }
+                if (pieces) {
+                    int32_t at = atomicAdd(K.n_big, (int32_t)__popc(pieces));
+                    if (at == 0 && K.host)  // one store: an illustration of 34 M entries lost 110 us to one for each
+                        __hip_atomic_store(&K.host[2], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    for (; pieces; pieces &= pieces - 1u) K.big[at++] = (int32_t)(5 * c + (uint32_t)__ffs(pieces) - 1u);
                 }
             }
             // the first piece's chains with many crossings before t1 / 32 (only the choice of a pass hangs on them)
