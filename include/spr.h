@@ -79,15 +79,16 @@ typedef struct spr_stats {
                                   rendered with the plain method (the allocation then grows) */
     /* Which kernel routes the last frame took (each route has its own kernel or mode): */
     int64_t n_wave_chains;     /* crossing chains that several lanes share, cut into segments that are
-                                  solved side by side (frames of 2^23 intersections and more: the
+                                  solved side by side (frames of 2^23 intersections and more, or of
+                                  more than 256 curves with many crossings near their start: the
                                   chains of 256 or more crossings) */
     int64_t n_heavy_pieces;    /* monotone pieces merged by a 256-thread workgroup each (more than
-                                  1024 entries, or, in frames of 2^23 intersections and more, whose
-                                  last segment waits on a chain of 256 or more crossings of the
-                                  next piece) */
+                                  1024 entries, or, in the same frames, whose last segment waits on
+                                  a chain of 256 or more crossings of the next piece) */
     int64_t n_long_bands;      /* sort bands of more than 512 words (one wave at 16 or 32 words per
-                                  lane; 256-thread LDS sorts in frames that export a stage) */
-    int64_t n_big_bands;       /* sort bands of more than 2048 words (global merge-path sort) */
+                                  lane; 256-thread LDS sorts in debug and anti-aliased frames) */
+    int64_t n_big_bands;       /* sort bands of more than 2048 words (sums per column, a workgroup
+                                  each; a global merge-path sort in debug and anti-aliased frames) */
     int64_t graph_captures;    /* LEARNED and batches: frames captured as a HIP graph so far (a new
                                   scene, model, margin, tuning or budget needs a new capture; a
                                   still frame and a frame after a new MVP have a graph each, and

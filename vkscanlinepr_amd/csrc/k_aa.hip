@@ -265,10 +265,10 @@ __device__ inline int run_length(int32_t f, const Four& q, const int32_t* __rest
 // time and each cell's side by side, and every lane computes the changes of one chord (all lanes the
 // same straight line of about 550 instructions, the next chord on its way); then every lane adds up
 // the changes of one cell (about 40 instructions a chord).  Bound by that arithmetic.  On 48.7 M chords in
-// 36.6 M cells of a 4096^2 frame 1.43 ms.  Four lanes per cell with 16 integer winding numbers each, every
-// lane walking the cell's chords: 2.5 ms; one lane per cell with the bits below: 1.9 ms, of which 0.4 ms
-// were arithmetic, since the longest cell of a wave held the other lanes back and each of its chords
-// waited on two dependent loads.  Five waves per SIMD: four or six were 6% slower.
+// 36.6 M cells of a 4096^2 frame 1.43 ms (1.21 with the dense cells in a list, below).  Four lanes per cell
+// with 16 integer winding numbers each, every lane walking the cell's chords: 2.5 ms; one lane per cell with the
+// bits below: 1.9 ms, of which 0.4 ms were arithmetic, since the longest cell of a wave held the other lanes back
+// and each of its chords waited on two dependent loads.  Five waves per SIMD: four or six were 6% slower.
 // Cells of more than kRunMax chords are few, but lie side by side (a path's dense spots): taken by the waves
 // whose records they were, one after another, 54 of them made this kernel 534 us instead of 130 in a
 // drawing at four times its size.  k_mark_emit lists them, and waves of their own spread over the chip.

@@ -22,7 +22,7 @@
 //
 // The prefix takes consecutive columns in one thread, the fold in consecutive lanes, through LDS: 64
 // neighbouring pixels are mostly covered by the same paths, so a wave's lanes take the same number of
-// steps, read the same colours and evaluate the same paints.  With PIX consecutive pixels per thread a
+// steps, read the same colours and evaluate the same paints.  Folding PIX consecutive pixels per thread, a
 // wave's lanes lay PIX pixels apart, each step lasted as long as the most covered of them, and
 // 4096^2 pixels under 55 paths each took 611 us instead of 457; 64 opaque paths on 1024^2 30 instead of
 // 16; a drawing with gradients at 1800x1200 289 instead of 94; anti-aliased 4096^2 1,597 instead of 1,281.
@@ -245,7 +245,7 @@ __global__ __launch_bounds__(CHUNK / PIX) __attribute__((amdgpu_waves_per_eu(GRA
                                                       const unsigned long long* __restrict__ cmask,
                                                       const TallyArgs T) {
     constexpr int TWO = (GRAD || AA) ? 1 : 0;            // the two rows of a cell row differ
-    constexpr int BLOCK = CHUNK / PIX;                   // threads; each keeps PIX consecutive pixels
+    constexpr int BLOCK = CHUNK / PIX;                   // threads; each keeps PIX pixels, BLOCK columns apart
     static_assert(PIX <= 32 && PIX % (AA ? 4 : 2) == 0 && BLOCK % kListSub == 0, "composite shape");
     // Parts of a listing step.  Four at a time, their rows loaded a step ahead, took the composite of
     // 20,000 paths on 2048^2 from 70 to 58 us (one at a time: 79 steps that wait on two loads each);
@@ -659,9 +659,11 @@ __global__ __launch_bounds__(CHUNK / PIX) __attribute__((amdgpu_waves_per_eu(GRA
 
 // Chunk and pixels per thread by the widest row: the narrowest of 512, 1024 and 2048 columns in
 // workgroups of 256 threads that holds it, else 4096 columns at 8 pixels per thread (512 threads; with
-// coverage two rows of accumulators, 128 VGPRs, 4 waves per SIMD).  Above kFewPaths paths, where
+// coverage two rows of accumulators, 128 VGPRs, 4 waves per SIMD, and 27 VGPRs spilled, 112 bytes a
+// lane).  Above kFewPaths paths, where
 // listing them is most of the work, src-over takes 16 pixels in 256 threads.  4096^2, three frames in
-// turn: 5,000 paths 2.33 ms against 2.48 with 16, 20,000 glyphs 370 us against 330.  Overwrite takes
+// turn: 5,000 paths 2.33 ms against 2.48 with 16 (6 VGPRs spilled), 20,000 glyphs 370 us against 330; the
+// line lies somewhere between these two, and what it stands for is the paths on a row.  Overwrite takes
 // 16 (its pixels need one register each).  With paints always 1024 columns at 4 per thread.
 constexpr uint32_t kFewPaths = 8192;
 hipError_t launch_composite(const uint32_t* records, const int2* brec, const int32_t* bucket_base,

@@ -519,7 +519,8 @@ __device__ inline void walk_candidates(const CurveBatch& B, Candidates& Q, const
 // One workgroup per window of K.window entries.  first[b] is the curve that holds entry b * window.
 // Its span is latency (loads behind each other, chains of dependent solves, LDS searches), so the
 // waves that fit a CU decide its rate: one wave a window left 6 waves on a CU (23 KB of LDS each,
-// 160 VGPRs); four waves to the same LDS put 24 there (6 per SIMD, at most 80 VGPRs).  Four waves
+// 160 VGPRs); four waves to the same LDS put 24 there (6 per SIMD: at most 80 VGPRs, for which 22 are
+// spilled, 84 bytes a lane; with CANDS 5 per SIMD, 96 VGPRs and 17 spilled, 72 bytes).  Four waves
 // also take a window of 1024 entries in about the time that one took 128, with a quarter of
 // the speculative solves per entry.  Frames in turn on three handles, us a frame, one wave and four:
 // 0.8 M entries on a few long curves 203 -> 134, 1.9 M on 20,000 glyphs 299 -> 261.  Two waves a
@@ -529,7 +530,8 @@ __device__ inline void walk_candidates(const CurveBatch& B, Candidates& Q, const
 // and with: 16 paths at 512^2 250 and 229, 64 at 1024^2 126 and 119, a drawing of 0.15 M entries alone 311
 // and 291.  Frames of more windows fill the chip anyway, and the candidates' arithmetic costs more than the
 // rounds: 1.9 M entries 259 and 265, 6.2 M 894 and 939.  So do frames of very short curves, whose chains
-// are not cut: 0.4 M entries on 125,000 curves 203 and 210.
+// are not cut: 0.4 M entries on 125,000 curves 203 and 210.  Both lines lie somewhere between two measured
+// scenes: kFewWindows between 670 windows and 1,860, kLongCurves between 3 entries a curve and 13.
 template <bool CANDS>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CANDS ? 5 : 6)))
 void k_curves(const CurveArgs K, const FragArgs A) {

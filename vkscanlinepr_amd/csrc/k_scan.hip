@@ -407,7 +407,6 @@ hipError_t launch_scan_i32_noalloc(const int32_t* in, int32_t* out, int64_t n, h
     ScanCtl c;
     c.status = ws;
     c.counter = reinterpret_cast<uint32_t*>(ws + tiles);
-    c.epoch = 0;
     return launch_scan_i32(in, out, n, c, s);
 }
 

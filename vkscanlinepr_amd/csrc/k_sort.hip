@@ -726,7 +726,7 @@ __global__ __launch_bounds__(256) void k_sort_bands_wave(const BandJob J, const 
 // where a launch costs 4.5 us and the launches would follow each other with the chip nearly empty.
 // Everything has the registers and the 64 KB of the longest class (two workgroups on a CU), so frames
 // of many bands keep a launch per class.  us a frame, four launches and one: 0.1 M entries in
-// 600 bands 270 and 258, 0.8 M in 1,600 132 and 127; 1.9 M in 20,000 short bands 412 and 432.
+// 600 bands 270 and 258, 0.8 M in 1,600 132 and 127; 1.9 M in 20,000 short bands 412 and 432 (kFewBands lies somewhere between).
 __global__ __launch_bounds__(256) void k_sort_bands_all(const BandJob J, const BigJob G, const EmitArgs EA, int big,
                                                         int large, int medium) {
     __shared__ union {

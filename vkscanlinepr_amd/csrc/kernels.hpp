@@ -11,12 +11,11 @@ namespace spr {
 
 struct Mvp { float m[16]; };
 
-// Scan control: a tile-status array tagged with an epoch so it never needs clearing, and an
-// atomic counter that hands out tile ids in dispatch order.
+// Scan control: a tile-status array and an atomic counter that hands out tile ids in dispatch
+// order, both zero before a scan.
 struct ScanCtl {
     unsigned long long* status;  // >= tiles entries
-    uint32_t* counter;           // one u32, zero before the first use of the frame
-    uint32_t epoch;              // distinct per scan invocation inside a frame sequence
+    uint32_t* counter;           // one u32
     int shape = 0;               // tile of the scans of 2^20 elements and more (kScanShapes; tuned)
 };
 // Tile shapes (int4 per thread, threads) of the large scans: 8 x 1024 (the default), 8 x 512,
@@ -128,8 +127,8 @@ constexpr int kChainClasses = 80;
 constexpr int kCcFill = kChainClasses, kCcOff = 2 * kChainClasses, kCcWork = 3 * kChainClasses + 1,
               kCcHeavyPieces = kCcWork + 1, kCcLightBegin = kCcHeavyPieces + 1,
               kCcWorkLight = kCcLightBegin + 1, kCcWavePieces = kCcWorkLight + 1, kCcWords = kCcWavePieces + 1;
-// Chains of at least kHeavyCrossings crossings are "heavy": they are cut into segments and solved by
-// their own launch, and the pieces of at most kHeavyCrossings entries, which never wait on them,
+// Chains of at least kHeavyCrossings crossings are "heavy": they are cut into segments (or, with a
+// long start, solved by a wave each) by their own launch, and the pieces of at most kHeavyCrossings entries, which never wait on them,
 // are finished by a concurrent stream meanwhile.
 constexpr int kHeavyCrossings = 256;
 // A frame whose buffers were sized before its counts were known (no host synchronisation): the
@@ -141,7 +140,8 @@ struct Budget {
     int32_t* live;
     int32_t* over;
 };
-// The chain passes (k_chain.hip): frames of kChainFrame entries and more.  over (optional): frames
+// The chain passes (k_chain.hip): frames of kChainFrame entries and more, or of more than kManyLong chains with
+// long starts.  over (optional): frames
 // with *over != 0 write no chain and no piece.
 hipError_t launch_chain_prep(const float2* tpos, const uint32_t* cpos, const uint32_t* ctype,
                              const float* cweight, const uint32_t* cpath, const int32_t* visible, const float4* cuts,
@@ -210,7 +210,7 @@ constexpr int kReadChunk = 32768;
 hipError_t launch_read_out(const uint8_t* src, uint8_t* dst, int64_t bytes, uint32_t* arrived, uint32_t mark,
                            hipStream_t s);
 
-// The curve pass (k_curves.hip): frames below kChainFrame entries.
+// The curve pass (k_curves.hip): the other frames.
 // The intersection write and the fragment keys: one workgroup per window of `window`
 // entries takes the pieces that start there from the curve data to their keys (or sort words),
 // winding changes and bucket counts, without storing the entries unless A.inter is set.  Pieces

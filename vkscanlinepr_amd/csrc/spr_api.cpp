@@ -328,7 +328,6 @@ spr::ScanCtl ctl_at(spr_handle* H, size_t st, size_t ctr_word, int counter) {
     spr::ScanCtl c;
     c.status = H->zero.p + st;
     c.counter = reinterpret_cast<uint32_t*>(H->zero.p + ctr_word) + counter;
-    c.epoch = 0;
     c.shape = H->scan_shape;
     return c;
 }
@@ -1602,7 +1601,6 @@ int spr_scan_i32(spr_handle* H, const int32_t* d_in, int32_t* d_out, uint64_t n,
         spr::ScanCtl c;
         c.status = H->scan_ws.p;
         c.counter = reinterpret_cast<uint32_t*>(H->scan_ws.p + tiles);
-        c.epoch = 0;
         c.shape = H->scan_shape;
         SPR_HIP(spr::launch_scan_i32(d_in, d_out, (int64_t)n, c, s));
     });
